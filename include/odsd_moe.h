@@ -115,6 +115,13 @@ int odsd_w4_pack(const uint8_t *q, const uint16_t *scale, const uint16_t *zero,
                  int64_t N, int64_t Kd, int32_t block_stride, int32_t block_offset,
                  uint32_t *qp, uint16_t *sz, void *stream);
 
+/* Quantise-on-load: one expert's gate [I, H], up [I, H] and down [H, I] weights (fp32 or bf16, each
+ * with its dtype code, 16-byte aligned) straight into the streaming layout, one launch; the bits are
+ * those of odsd_w4_quantize followed by odsd_w4_pack.  H and I multiples of 128. */
+int odsd_w4_load_expert(const void *gate, int32_t gate_dtype, const void *up, int32_t up_dtype,
+                        const void *down, int32_t down_dtype, int64_t H, int64_t I, uint32_t *gu_q,
+                        uint16_t *gu_sz, uint32_t *dn_q, uint16_t *dn_sz, void *stream);
+
 /* ---- RMSNorm ------------------------------------------------------------------------ */
 /* out = cast(x * rsqrt(mean(x^2) + eps)) * weight, cast BEFORE the weight multiply. */
 int odsd_rmsnorm(const void *x, const void *weight, int32_t dtype, int32_t T, int32_t H,

@@ -37,6 +37,8 @@ SIGNATURES = {
     "odsd_w4_packed_q_bytes": (C.c_size_t, [C.c_int64, C.c_int64]),
     "odsd_w4_packed_sz_bytes": (C.c_size_t, [C.c_int64, C.c_int64]),
     "odsd_w4_pack": (C.c_int, [_P, _P, _P, C.c_int64, C.c_int64, C.c_int32, C.c_int32, _P, _P, _P]),
+    "odsd_w4_load_expert": (C.c_int, [_P, C.c_int32, _P, C.c_int32, _P, C.c_int32, C.c_int64, C.c_int64,
+                                      _P, _P, _P, _P, _P]),
     "odsd_rmsnorm": (C.c_int, [_P, _P, C.c_int32, C.c_int32, C.c_int32, C.c_float, _P, _P]),
     "odsd_add_rmsnorm": (C.c_int, [_P, _P, _P, C.c_int32, C.c_int32, C.c_int32, C.c_float, _P, _P, _P]),
     "odsd_router_workspace_bytes": (C.c_size_t, [_SP]),

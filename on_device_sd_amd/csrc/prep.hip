@@ -3,13 +3,33 @@
 #include "common.h"
 
 // -----------------------------------------------------------------------------------------
-// Quantiser: one wavefront per (row, group of 128 columns); lane l owns columns 2l, 2l+1.
-// Arithmetic follows quantize_tensor (pre_exp/expert_skip_prediction/quant.py:99-106) per
+// Arithmetic of the quantiser, per (row, group of 128 columns).  It follows quantize_tensor (pre_exp/expert_skip_prediction/quant.py:99-106) per
 // group with 4 bits: scale=(max-min)/15, zero=0-min/scale (a float, never rounded to an
 // integer), q=clamp(round(w/scale+zero),0,15).  scale and zero are rounded to fp16 before
 // the codes are computed.  Every fp32 step is a single correctly rounded operation
 // (__f*_rn) so that a CPU restatement gets the same bits.
 // -----------------------------------------------------------------------------------------
+struct QuantParams {
+    half_t s16, z16;     // as stored
+    float sf, zf;        // the same values, what the codes are computed with
+};
+__device__ __forceinline__ QuantParams quant_params(const float mn, const float mx) {
+    const float s32 = __fdiv_rn(__fsub_rn(mx, mn), 15.0f);
+    half_t s16 = (half_t)s32;
+    if (!(s16 > (half_t)0.0f)) s16 = (half_t)1.0f;
+    if (__builtin_isinf((float)s16)) s16 = (half_t)ODSD_FP16_MAX;
+    const float sf = (float)s16;
+    float z32 = __fsub_rn(0.0f, __fdiv_rn(mn, sf));
+    z32 = fminf(fmaxf(z32, -ODSD_FP16_MAX), ODSD_FP16_MAX);
+    const half_t z16 = (half_t)z32;
+    return QuantParams{s16, z16, sf, (float)z16};
+}
+__device__ __forceinline__ uint32_t quant_code(const float w, const QuantParams &p) {
+    const float t = rintf(__fadd_rn(__fdiv_rn(w, p.sf), p.zf));
+    return (uint32_t)fminf(fmaxf(t, 0.0f), 15.0f);
+}
+
+// Canonical form: one wavefront per (row, group); lane l owns columns 2l, 2l+1.
 template <typename WT>
 __global__ __launch_bounds__(256) void w4_quantize_kernel(const WT *__restrict__ w, int64_t n_units,
                                                           int64_t G, uint8_t *__restrict__ q,
@@ -23,23 +43,12 @@ __global__ __launch_bounds__(256) void w4_quantize_kernel(const WT *__restrict__
     const float w1 = ActIO<WT>::load(w, base + 1);
     const float mn = wave_min(fminf(w0, w1));
     const float mx = wave_max(fmaxf(w0, w1));
-    const float s32 = __fdiv_rn(__fsub_rn(mx, mn), 15.0f);
-    half_t s16 = (half_t)s32;
-    if (!(s16 > (half_t)0.0f)) s16 = (half_t)1.0f;
-    if (__builtin_isinf((float)s16)) s16 = (half_t)ODSD_FP16_MAX;
-    const float sf = (float)s16;
-    float z32 = __fsub_rn(0.0f, __fdiv_rn(mn, sf));
-    z32 = fminf(fmaxf(z32, -ODSD_FP16_MAX), ODSD_FP16_MAX);
-    const half_t z16 = (half_t)z32;
-    const float zf = (float)z16;
-    const float t0 = rintf(__fadd_rn(__fdiv_rn(w0, sf), zf));
-    const float t1 = rintf(__fadd_rn(__fdiv_rn(w1, sf), zf));
-    const uint32_t c0 = (uint32_t)fminf(fmaxf(t0, 0.0f), 15.0f);
-    const uint32_t c1 = (uint32_t)fminf(fmaxf(t1, 0.0f), 15.0f);
+    const QuantParams qp = quant_params(mn, mx);
+    const uint32_t c0 = quant_code(w0, qp), c1 = quant_code(w1, qp);
     q[(size_t)unit * (ODSD_GROUP / 2) + lane] = (uint8_t)(c0 | (c1 << 4));
     if (lane == 0) {
-        scale[unit] = __builtin_bit_cast(uint16_t, s16);
-        zero[unit] = __builtin_bit_cast(uint16_t, z16);
+        scale[unit] = __builtin_bit_cast(uint16_t, qp.s16);
+        zero[unit] = __builtin_bit_cast(uint16_t, qp.z16);
     }
 }
 
@@ -93,6 +102,109 @@ __global__ __launch_bounds__(256) void w4_pack_kernel(const uint8_t *__restrict_
         const uint32_t s = scale[row * G + g], z = zero[row * G + g];
         sz[(bd * G + g) * 16 + r] = s | (z << 16);
     }
+}
+
+// -----------------------------------------------------------------------------------------
+// Quantise-on-load of one expert: gate, up and down weights -> streaming layout in ONE launch, with no
+// canonical copy in between.  A wavefront takes one [16 rows x 128 columns] tile; its lane (r = l%16,
+// kq = l/16) reads columns 32j + 8kq .. + 7 of row r (j = 0..3), which are exactly the codes of its
+// four packed words, so the group's minimum and maximum need two exchanges between lanes and the tile
+// leaves as one contiguous 1 KiB store.  Consecutive wavefronts take consecutive groups of a row
+// block.  16 experts of [768, 2048] in bf16: 115 us, bound by the host's 7 us per call (kernel 6.0 us,
+// 12 MB: launch, one round trip and the divisions; 7.4 us with the compiler's division).  As three
+// quantise and three pack launches with a canonical copy in between, 96 calls in all, 766 us.
+// -----------------------------------------------------------------------------------------
+struct LoadMatrix {
+    const void *w;
+    uint4_t *qp;
+    uint32_t *sz;
+    int f32;                     // 1: fp32 weights, 0: bf16
+    int G;                       // groups per row
+    int first;                   // first tile of this matrix in the launch
+    int bstride, boffset;        // destination block = b * bstride + boffset
+};
+struct LoadParams {
+    LoadMatrix m[3];
+    int n_tiles;
+};
+__global__ __launch_bounds__(256) void w4_load_expert_kernel(const LoadParams p) {
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tile >= p.n_tiles) return;
+    const int which = __builtin_amdgcn_readfirstlane((tile >= p.m[1].first) + (tile >= p.m[2].first));
+    const LoadMatrix m = p.m[which];
+    const int t = tile - m.first;
+    const int b = t / m.G, g = t - b * m.G;
+    const int lane = lane_id(), r = lane & 15, kq = lane >> 4;
+    const size_t at = ((size_t)(b * 16 + r) * m.G + g) * ODSD_GROUP + kq * 8;
+    float w[4][8];
+    if (m.f32) {
+        const float *src = (const float *)m.w + at;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float4_t lo = *(const float4_t *)(src + 32 * j), hi = *(const float4_t *)(src + 32 * j + 4);
+            w[j][0] = lo.x; w[j][1] = lo.y; w[j][2] = lo.z; w[j][3] = lo.w;
+            w[j][4] = hi.x; w[j][5] = hi.y; w[j][6] = hi.z; w[j][7] = hi.w;
+        }
+    } else {
+        const uint16_t *src = (const uint16_t *)m.w + at;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint4_t v = *(const uint4_t *)(src + 32 * j);
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                w[j][2 * i] = __uint_as_float(u[i] << 16);
+                w[j][2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
+            }
+        }
+    }
+    float mn = w[0][0], mx = w[0][0];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            mn = fminf(mn, w[j][i]);
+            mx = fmaxf(mx, w[j][i]);
+        }
+#pragma unroll
+    for (int d = 16; d <= 32; d <<= 1) {
+        mn = fminf(mn, __shfl_xor(mn, d, ODSD_WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, d, ODSD_WAVE));
+    }
+    const QuantParams qp = quant_params(mn, mx);
+    // w / scale, correctly rounded, in three instructions: q0 = w y with y = 1 / scale correctly rounded is
+    // within 1.5 units of the quotient, its residual w - q0 scale is exact, and one correction leaves an
+    // error below 2^-23 units before the last rounding.  scale has 11 significant bits (it is an fp16
+    // value), so a quotient that is not itself halfway between two floats is at least 2^-12 units away
+    // from that point, and no 24-bit w has a quotient exactly there: the last rounding is the right one.
+    // (Quotients too small for that argument vanish when the zero point is added.)  Groups with
+    // infinities take the division.
+    const bool finite = mx - mn < INFINITY;
+    const float y = __fdiv_rn(1.0f, qp.sf);
+    uint32_t out[4];
+    constexpr int pos[8] = {0, 16, 4, 20, 8, 24, 12, 28};      // permute_nibbles: code i -> bit position
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] = 0;
+    if (__all(finite)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float q0 = __fmul_rn(w[j][i], y);
+                const float q = fmaf(fmaf(-q0, qp.sf, w[j][i]), y, q0);
+                const float t = rintf(__fadd_rn(q, qp.zf));
+                out[j] |= (uint32_t)__builtin_amdgcn_fmed3f(t, 0.0f, 15.0f) << pos[i];
+            }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[j] |= quant_code(w[j][i], qp) << pos[i];
+    }
+    const size_t dst = (size_t)(b * m.bstride + m.boffset) * m.G + g;
+    m.qp[dst * 64 + lane] = uint4_t{out[0], out[1], out[2], out[3]};
+    if (kq == 0)
+        m.sz[dst * 16 + r] = (uint32_t)__builtin_bit_cast(uint16_t, qp.s16) | ((uint32_t)__builtin_bit_cast(uint16_t, qp.z16) << 16);
 }
 
 // -----------------------------------------------------------------------------------------
@@ -209,6 +321,28 @@ extern "C" int odsd_w4_pack(const uint8_t *q, const uint16_t *scale, const uint1
     if ((total + 255) / 256 > 0x7fffffffLL) return ODSD_ERR_SHAPE;
     w4_pack_kernel<<<dim3((unsigned)((total + 255) / 256)), 256, 0, (hipStream_t)stream>>>(
         q, scale, zero, nb, G, block_stride, block_offset, (uint4_t *)qp, (uint32_t *)sz);
+    ODSD_CHECK_LAUNCH();
+    return ODSD_OK;
+}
+
+extern "C" int odsd_w4_load_expert(const void *gate, int32_t gate_dtype, const void *up, int32_t up_dtype,
+                                   const void *down, int32_t down_dtype, int64_t H, int64_t I, uint32_t *gu_q,
+                                   uint16_t *gu_sz, uint32_t *dn_q, uint16_t *dn_sz, void *stream) {
+    if (!gate || !up || !down || !gu_q || !gu_sz || !dn_q || !dn_sz) return ODSD_ERR_NULL;
+    if (H <= 0 || I <= 0 || H % ODSD_GROUP || I % ODSD_GROUP || H * I > (1LL << 40)) return ODSD_ERR_SHAPE;
+    for (const int32_t d : {gate_dtype, up_dtype, down_dtype})
+        if (d != ODSD_DT_F32 && d != ODSD_DT_BF16) return ODSD_ERR_DTYPE;
+    for (const void *q : {gate, up, down, (const void *)gu_q, (const void *)dn_q})
+        if (!odsd_aligned16(q)) return ODSD_ERR_ALIGN;
+    if ((((uintptr_t)gu_sz) | ((uintptr_t)dn_sz)) & 3u) return ODSD_ERR_ALIGN;
+    const int64_t tiles = I / 16 * (H / ODSD_GROUP), tiles_dn = H / 16 * (I / ODSD_GROUP);   // the same number
+    if (2 * tiles + tiles_dn > 0x7fffffffLL / 4) return ODSD_ERR_SHAPE;
+    const int Gu = (int)(H / ODSD_GROUP), Gd = (int)(I / ODSD_GROUP);
+    const LoadParams p{{{gate, (uint4_t *)gu_q, (uint32_t *)gu_sz, gate_dtype == ODSD_DT_F32, Gu, 0, 2, 0},
+                        {up, (uint4_t *)gu_q, (uint32_t *)gu_sz, up_dtype == ODSD_DT_F32, Gu, (int)tiles, 2, 1},
+                        {down, (uint4_t *)dn_q, (uint32_t *)dn_sz, down_dtype == ODSD_DT_F32, Gd, (int)(2 * tiles), 1, 0}},
+                       (int)(2 * tiles + tiles_dn)};
+    w4_load_expert_kernel<<<dim3((unsigned)((p.n_tiles + 3) / 4)), 256, 0, (hipStream_t)stream>>>(p);
     ODSD_CHECK_LAUNCH();
     return ODSD_OK;
 }

@@ -107,6 +107,23 @@ def w4_pack_into(q: torch.Tensor, scale: torch.Tensor, zero: torch.Tensor, qp: t
                                 qp.data_ptr(), sz.data_ptr(), _stream()), "odsd_w4_pack")
 
 
+def w4_load_expert(gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor,
+                   dst: Tuple[int, int, int, int]) -> None:
+    """gate [I,H], up [I,H], down [H,I] (float32 / bfloat16) -> the streaming layout at the four device
+    addresses ``dst`` (gate_up codes, gate_up (scale, zero), down codes, down (scale, zero)), in one launch."""
+    _require_cuda(gate, up, down)
+    I, H = gate.shape
+    if up.shape != gate.shape or down.shape != (H, I):
+        raise ValueError(f"expert weights do not belong together: {tuple(gate.shape)}, {tuple(up.shape)}, {tuple(down.shape)}")
+    gate, up, down = gate.contiguous(), up.contiguous(), down.contiguous()
+    a, b, c = gate.data_ptr(), up.data_ptr(), down.data_ptr()
+    if (a | b | c) % 16:                                          # the kernel reads 16 bytes at a time
+        gate, up, down = gate.clone(), up.clone(), down.clone()
+        a, b, c = gate.data_ptr(), up.data_ptr(), down.data_ptr()
+    _lib.check(_lib.load().odsd_w4_load_expert(a, _dtype_code(gate.dtype), b, _dtype_code(up.dtype), c,
+                                               _dtype_code(down.dtype), H, I, *dst, _stream()), "odsd_w4_load_expert")
+
+
 # ------------------------------------------------------------------------------------------
 # RMSNorm / conversion
 # ------------------------------------------------------------------------------------------

@@ -115,10 +115,18 @@ class W4ExpertBank:
 
     def load_expert(self, e: int, gate_w: torch.Tensor, up_w: torch.Tensor, down_w: torch.Tensor,
                     keep_canonical: bool = False):
-        """Quantise one expert's [I,H], [I,H], [H,I] weights on the device and pack them."""
-        canon = tuple(ops.w4_quantize(w.to(self.device)) for w in (gate_w, up_w, down_w))
-        self.load_canonical(e, *canon)
-        return canon if keep_canonical else None
+        """Quantise one expert's [I,H], [I,H], [H,I] weights on the device and pack them: in one launch, or
+        through the canonical arrays when the caller wants those as well."""
+        ws = [w if w.is_cuda else w.to(self.device) for w in (gate_w, up_w, down_w)]
+        if keep_canonical:
+            canon = tuple(ops.w4_quantize(w) for w in ws)
+            self.load_canonical(e, *canon)
+            return canon
+        if ws[0].shape != (self.inter, self.hidden):
+            raise ValueError(f"expert weights of shape {tuple(ws[0].shape)}: this bank holds [{self.inter}, {self.hidden}]")
+        ops.w4_load_expert(*ws, self._ptrs[e])
+        self.mark_loaded(e)
+        return None
 
     EXPERT_WEIGHT_NAME = "model.layers.{layer}.mlp.experts.{expert}.{proj}_proj.weight"
 
