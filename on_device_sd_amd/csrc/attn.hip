@@ -32,56 +32,7 @@
 // of the cached K/V by slot, repeat_interleave for GQA, causal mask with offset k_len - q_len,
 // scaled_dot_product_attention), the flash_attn_with_kvcache call it stands in for (:252-272) and
 // the flash_attn_varlen_func call of the prefill branch (:229-240).
-#include "common.h"
-#include <type_traits>
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
-
-struct AttnParams {
-    const void *q;             // [n_tokens, H, HD]
-    const void *k_cache;       // [num_slots, KVH * HD]
-    const void *v_cache;
-    void *out;                 // [n_tokens, H, HD]
-    const int32_t *q_lens;     // [n_seqs] or null (1 each)
-    const int32_t *context_lens;
-    const int32_t *block_tables;   // [n_seqs, max_blocks]
-    int n_seqs, H, KVH, max_blocks, block_size;
-    int64_t num_slots;
-    float scale_log2e;         // softmax scale * log2(e)
-    // variable-length mode (prefill): q / k / v rows of sequence s are q[cu_q[s] ..], k[cu_k[s] ..]
-    // (contiguous, no block table); both null in paged mode
-    const int32_t *cu_q, *cu_k;
-    int splits;                // workgroups sharing one sequence's keys (blockIdx.z)
-    float *part;               // splits > 1: partial results [seq, kvh, row group][split][64][HD + 4]
-};
-
-template <typename T> struct AttnT;
-template <> struct AttnT<half_t> {
-    typedef half8_t V8;
-    __device__ static __forceinline__ float4_t mfma(V8 a, V8 b, float4_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-    }
-    __device__ static __forceinline__ uint16_t from_f32(float v) { return __builtin_bit_cast(uint16_t, (half_t)v); }
-    // two values, round to nearest even, as one 32-bit word (a in the low half)
-    __device__ static __forceinline__ uint32_t pack2(float a, float b) {
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        typedef float f2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
-    }
-};
-template <> struct AttnT<__bf16> {
-    typedef bf16x8_t V8;
-    __device__ static __forceinline__ float4_t mfma(V8 a, V8 b, float4_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-    }
-    __device__ static __forceinline__ uint16_t from_f32(float v) { return f32_to_bf16(v); }
-    __device__ static __forceinline__ uint32_t pack2(float a, float b) {   // v_cvt_pk_bf16_f32
-        typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-        typedef float f2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
-    }
-};
+#include "attn.h"
 
 // first query token of sequence seq: the sum of the query lengths before it, one wavefront-wide pass
 __device__ __forceinline__ int attn_first_token(const int32_t *q_lens, int seq) {
@@ -622,6 +573,11 @@ extern "C" int odsd_varlen_attention(const void *q, const void *k, const void *v
     const int64_t rows = (int64_t)max_seqlen_q * (num_heads / num_kv_heads);
     if ((rows + 63) / 64 > 65535) return ODSD_ERR_UNSUPPORTED;     // grid.y
     const int rg = (int)((rows + 63) / 64);
+    if (odsd_attn_prefill_supported(p, head_dim, max_seqlen_q, max_seqlen_k)) {
+        odsd_launch_attn_prefill(p, dtype, head_dim, max_seqlen_q, (hipStream_t)stream);
+        ODSD_CHECK_LAUNCH();
+        return ODSD_OK;
+    }
     p.splits = attn_splits(n_seqs, num_kv_heads, rg, p.max_blocks, 32);
     if (p.splits > 1) {
         const size_t need = odsd_varlen_attention_workspace_bytes(n_seqs, max_seqlen_q, max_seqlen_k, num_heads,
