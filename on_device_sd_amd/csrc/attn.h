@@ -15,14 +15,16 @@ struct AttnParams {
     const int32_t *q_lens;     // [n_seqs] or null (1 each)
     const int32_t *context_lens;
     const int32_t *block_tables;   // [n_seqs, max_blocks]
-    int n_seqs, H, KVH, max_blocks, block_size;
+    int n_seqs, H, KVH, Gq, max_blocks, block_size;   // Gq: query heads per KV head
     int64_t num_slots;
     float scale_log2e;         // softmax scale * log2(e)
     // variable-length mode (prefill): q / k / v rows of sequence s are q[cu_q[s] ..], k[cu_k[s] ..]
     // (contiguous, no block table); both null in paged mode
     const int32_t *cu_q, *cu_k;
-    int splits;                // workgroups sharing one sequence's keys (blockIdx.z)
-    float *part;               // splits > 1: partial results [seq, kvh, row group][split][64][HD + 4]
+    int n_wg;                  // streaming kernels: workgroups that share the work
+    int whole;                 // no unit is split
+    int v_once;                // V is read nontemporally
+    float *part;               // its partial results, two slots per workgroup: [rows][HD + 4]
 };
 
 template <typename T> struct AttnT;

@@ -1,29 +1,30 @@
-// Causal attention over cached or packed keys (gfx950): the decode / verify step over the paged KV
-// cache, and the prefill step over the step's own variable-length sequences.
+// Causal attention over cached or packed keys with few query rows per sequence: the decode / verify
+// step over the paged KV cache, and packed calls that the prefill kernel does not take.
 //
-// One workgroup per (sequence, KV head, group of 64 query rows, slice of the keys); a query row is
-// one (token, query head) pair of the KV head's group, so with grouped-query attention a verify
-// step of 8 tokens and 8 query heads per KV head fills the 64 rows.  Each of the 4 wavefronts owns
-// 16 rows; the workgroup walks its keys 32 at a time:
-//   * the tile's K and V rows are fetched once per workgroup (two tiles ahead, into registers) and
-//     put into LDS one tile ahead, both as stored ([key][head_dim], 16- and 32-byte segments of a
-//     row XORed with the key against bank conflicts); all wavefronts read their operands from
-//     there (double buffered, one barrier per tile);
-//   * S^T = K Q^T on the matrix cores (v_mfma_f32_16x16x32, keys as the A operand, the
-//     wavefront's Q rows as the B operand held in registers), which leaves the scores of one
-//     query row in the 4 lanes that share lane % 16 -- the layout the P operand of the second
-//     product needs, so the probabilities never move between lanes;
-//   * softmax in fp32 in the exp2 domain with the scale folded in; a row's reference point (the
-//     value subtracted before exp2) follows its running maximum lazily, and the sum of the
-//     probabilities stays a per-lane partial sum until the end, so most tiles exchange nothing
-//     between lanes;
-//   * O += P V with V^T as the B operand: a lane needs one head dimension of 8 keys, which
-//     ds_read_b64_tr_b16 delivers from the row-major tile (the 16 lanes of a group read 4 keys x
-//     16 dimensions and each gets one dimension's column of 4), so V is never transposed in memory.
-// A verify step has few (sequence, KV head) pairs and long key lists, so the keys of one sequence
-// are cut into `splits` slices handled by different workgroups; each leaves its reference point,
-// sum and unnormalised output, and a small second kernel merges the slices of a row (the usual
-// rescaling by exp2(m_slice - m_all)), in slice order.
+// A query row is one (token, query head) pair of a KV head's group; up to 16, 32 or 64 rows of one
+// (sequence, KV head) -- a unit -- are worked on together, so one pass over the keys serves a whole group
+// of query heads and all draft tokens.  What the kernels have to do is stream K and V from HBM.  The keys
+// of all units are laid end to end and dealt out in equal contiguous shares to as many workgroups as the
+// chip holds at once.  A share may begin and end in the middle of a unit: such pieces leave partial results
+// that a second kernel merges, whole units are finished in place.  Sequences of mixed lengths then cost
+// what their bytes cost; with a fixed number of slices per sequence, as before, the longest sequence set
+// the time.  Two forms:
+//   * up to 16 rows (decode; 32 with a lot of keys), attn_stream_kernel: each of the 4 wavefronts takes
+//     its own 32 keys of every 128, for all rows of the unit, with no barrier in the loop.  K goes from
+//     memory straight into the registers that S^T = K Q^T wants as its A operand (v_mfma_f32_16x16x32); V
+//     goes through a piece of LDS that belongs to the wavefront, because O^T = V^T P^T needs its transpose
+//     (ds_read_b64_tr_b16).  A tile's registers are refilled as soon as it has been multiplied (K) or put
+//     into LDS (V); three wavefronts per SIMD hide what is left of the latency;
+//   * more rows, attn_tile_kernel: a wavefront cannot hold the rows next to its keys, so the workgroup
+//     shares the keys through LDS.
+// In both the scores of one query row stay in the 4 lanes that share lane % 16, in the order in which P^T
+// is wanted as the B operand, and O^T keeps the row there too: maximum, sum and rescaling factor are lane
+// values.  Softmax in fp32 in the exp2 domain; a row's reference point follows its running maximum lazily.
+// Measured (32 query / 4 KV heads of 128, bf16, kernel + merge, before -> now): 64 sequences of 750 to 3000
+// keys, one query each, 263 MB: 64.1 -> 47.5 us (the kernel alone 6.1 TB/s: bound by HBM); 64 of 2048
+// keys 53.3 -> 45.9; one of 4000 13.9 -> 13.0; 16 of 300 13.3 -> 7.7 (no merge).  32 sequences of 512 to 2048
+// keys x 8 queries, 85 MB: 31.8 -> 30.8: start-up, pieces and merge are as long as the stream there.
+//
 // Paged form: the cache is addressed through the sequence's block table exactly as the reference
 // gathers it: position p lives in slot block_table[p / block_size] * block_size + p % block_size.
 // Packed form: the keys of sequence s are rows cu_seqlens_k[s] .. of k / v.
@@ -33,442 +34,748 @@
 // scaled_dot_product_attention), the flash_attn_with_kvcache call it stands in for (:252-272) and
 // the flash_attn_varlen_func call of the prefill branch (:229-240).
 #include "attn.h"
+#include "w4_gemm.h"
+#include <type_traits>
 
-// first query token of sequence seq: the sum of the query lengths before it, one wavefront-wide pass
-__device__ __forceinline__ int attn_first_token(const int32_t *q_lens, int seq) {
-    int part = 0;
-    for (int i = threadIdx.x & 63; i < seq; i += 64) part += q_lens[i];
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) part += __shfl_xor(part, d, ODSD_WAVE);
-    return part;
+#define ATTN_WG 512          // workgroups that share the work: two per CU
+// Granularities of the list in keys: it is cut at multiples of FINE when that gives every workgroup at least
+// COARSE keys, otherwise at multiples of COARSE; with no sequence longer than WHOLE nothing is split and
+// there is nothing to merge.  (A merge costs 4 to 6 us, what a workgroup needs for WHOLE keys: 16 sequences
+// of 300 keys, decode, 7.7 us whole against 10.2 split.)
+#define ATTN_STREAM_FINE 128
+#define ATTN_STREAM_COARSE 128
+#define ATTN_STREAM_WHOLE 512
+#define ATTN_TILE_FINE 32
+#define ATTN_TILE_COARSE 256
+#define ATTN_TILE_WHOLE 256
+
+// ---- how the work is dealt out -----------------------------------------------------------------------
+// A sequence is KVH * rg units, each of `steps` list steps of g keys (a sequence without keys still owns
+// output rows, which are written as zeros: one step).
+struct SeqCost {
+    int L, ql, rg, steps, cost;
+};
+__device__ __forceinline__ void seq_steps(const AttnParams &p, SeqCost &c, const int g) {
+    c.steps = max(1, (c.L + g - 1) / g);
+    c.cost = c.rg * p.KVH * c.steps;
+}
+__device__ __forceinline__ SeqCost seq_cost(const AttnParams &p, const int s, const int rows_per_unit, const int g) {
+    SeqCost c{0, 0, 0, 0, 0};
+    if (s < p.n_seqs) {
+        if (p.cu_k) {
+            c.L = p.cu_k[s + 1] - p.cu_k[s];
+            c.ql = p.cu_q[s + 1] - p.cu_q[s];
+        } else {
+            c.L = p.context_lens[s];
+            c.ql = p.q_lens ? p.q_lens[s] : 1;
+        }
+        c.ql = max(c.ql, 0);
+        c.rg = (c.ql * p.Gq + rows_per_unit - 1) / rows_per_unit;
+        seq_steps(p, c, g);
+    }
+    return c;
+}
+// inclusive prefix sum over the wavefront
+__device__ __forceinline__ int wave_scan(int v) {
+#define ATTN_SCAN(CTRL, ROWMASK) v += __builtin_amdgcn_update_dpp(0, v, CTRL, ROWMASK, 0xF, false)
+    ATTN_SCAN(0x111, 0xF);   // row_shr:1, 2, 4, 8
+    ATTN_SCAN(0x112, 0xF);
+    ATTN_SCAN(0x114, 0xF);
+    ATTN_SCAN(0x118, 0xF);
+    ATTN_SCAN(0x142, 0xA);   // row_bcast:15 into rows 1 and 3
+    ATTN_SCAN(0x143, 0xC);   // row_bcast:31 into rows 2 and 3
+#undef ATTN_SCAN
+    return v;
+}
+__device__ __forceinline__ int lane_value(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+
+// Where a sequence stands in the list: found either by a position in the list or by its number.
+struct SeqAt {
+    int seq, L, ql, rg, steps;
+    int first;       // list position of its first step
+    int q0;          // its first query token
+};
+struct ListPlan {
+    int g;                   // keys per list step
+    int total, share;        // steps in all, steps per workgroup
+    SeqAt at;
+    bool found;
+};
+// fine, coarse: the two granularities.  The list is cut at multiples of `fine` keys when every workgroup gets at
+// least `coarse` keys that way; otherwise at multiples of `coarse`, so that short units stay whole.
+template <bool BY_SEQ>
+__device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int rows_per_unit, const int fine,
+                                              const int coarse, const int who) {
+    const int lane = lane_id();
+    ListPlan pl;
+    pl.g = p.whole ? 1 << 30 : fine;          // (longer than any sequence: one step per unit, whatever its length)
+    SeqCost c0 = seq_cost(p, lane, rows_per_unit, pl.g);
+    int s0, total;
+    for (;;) {
+        s0 = wave_scan(c0.cost);
+        total = lane_value(s0, 63);
+        for (int b = 64; b < p.n_seqs; b += 64)
+            total += lane_value(wave_scan(seq_cost(p, b + lane, rows_per_unit, pl.g).cost), 63);
+        if (p.whole || pl.g == coarse || total >= (coarse / fine) * p.n_wg) break;
+        pl.g = coarse;
+        seq_steps(p, c0, coarse);
+    }
+    pl.total = total;
+    pl.share = max(1, (total + p.n_wg - 1) / p.n_wg);
+    pl.found = false;
+    const int target = BY_SEQ ? 0 : who * pl.share;
+    if (!BY_SEQ && target >= total) return pl;
+    int before = 0, tok = 0;
+    SeqCost c = c0;
+    int sc = s0;
+    for (int b = 0; b < p.n_seqs; b += 64) {
+        if (b > 0) {
+            c = seq_cost(p, b + lane, rows_per_unit, pl.g);
+            sc = wave_scan(c.cost);
+        }
+        const int tc = wave_scan(c.ql);
+        const int sum = lane_value(sc, 63);
+        if (BY_SEQ ? who < b + 64 : target < before + sum) {
+            const int l = BY_SEQ ? who - b : __builtin_ctzll(__ballot(before + sc > target));
+            pl.at = SeqAt{b + l, lane_value(c.L, l), lane_value(c.ql, l), lane_value(c.rg, l), lane_value(c.steps, l),
+                          before + lane_value(sc, l) - lane_value(c.cost, l),
+                          tok + lane_value(tc, l) - lane_value(c.ql, l)};
+            pl.found = true;
+            return pl;
+        }
+        before += sum;
+        tok += lane_value(tc, 63);
+    }
+    return pl;
 }
 
-template <typename T, int HD, bool ALIGNED>
-__global__ __launch_bounds__(256, 2) void paged_attn_kernel(const AttnParams p) {
+// the unit after this one: of the same sequence, or of the next one that has any
+__device__ __forceinline__ void next_unit(const AttnParams &p, SeqAt &sq, int &unit, int &step, const int rows_per_unit,
+                                          const int g) {
+    step = 0;
+    if (++unit < p.KVH * sq.rg) return;
+    unit = 0;
+    sq.first += p.KVH * sq.rg * sq.steps;
+    do {                                                   // (a sequence without queries has no units)
+        sq.q0 += sq.ql;
+        ++sq.seq;
+        const SeqCost nx = seq_cost(p, sq.seq, rows_per_unit, g);
+        sq.L = __builtin_amdgcn_readfirstlane(nx.L);
+        sq.ql = __builtin_amdgcn_readfirstlane(nx.ql);
+        sq.rg = __builtin_amdgcn_readfirstlane(nx.rg);
+        sq.steps = __builtin_amdgcn_readfirstlane(nx.steps);
+    } while (sq.rg == 0);
+}
+
+// ---- one 32-key tile of 16 query rows -----------------------------------------------------------------
+// Lane (c, kq) holds the scores of keys 16 t + 4 kq + i of query row c (a[4 t + i], before the softmax
+// scale, masked ones -inf); returns the probabilities as the B operand of O^T = V^T P^T and keeps the row's
+// reference point, this lane's part of its sum, and O^T.  The reference point moves only when some score of
+// the wavefront exceeds it by more than 2^8 (probabilities up to 256 are as exact in fp16 / bf16 as those
+// below 1, and the sums are fp32): most tiles then need no exchange between lanes at all.
+template <typename T, int NDB>
+__device__ __forceinline__ typename AttnT<T>::V8 softmax_tile(const float (&a)[8], const float sc, float &m_run,
+                                                              float &l_run, float4_t (&o)[NDB]) {
+    float mx = fmaxf(fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])), fmaxf(fmaxf(a[4], a[5]), fmaxf(a[6], a[7])));
+    if (__any(mx * sc > m_run + 8.0f)) {
+        mx = fmaxf(mx, __shfl_xor(mx, 16, ODSD_WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, ODSD_WAVE));
+        const float m_new = fmaxf(m_run, mx * sc);
+        // a row with nothing to attend yet keeps m = -inf: use 0 as the reference point then
+        const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));   // m_run = -inf -> 0
+        l_run *= alpha;
+        m_run = m_new;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) { o[db].x *= alpha; o[db].y *= alpha; o[db].z *= alpha; o[db].w *= alpha; }
+    }
+    const float neg_ref = m_run == -INFINITY ? 0.0f : -m_run;
+    float pe[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) pe[e] = __builtin_amdgcn_exp2f(fmaf(a[e], sc, neg_ref));   // masked -> 0
+    l_run += ((pe[0] + pe[1]) + (pe[2] + pe[3])) + ((pe[4] + pe[5]) + (pe[6] + pe[7]));
+    return __builtin_bit_cast(typename AttnT<T>::V8,
+                              uint4_t{AttnT<T>::pack2(pe[0], pe[1]), AttnT<T>::pack2(pe[2], pe[3]),
+                                      AttnT<T>::pack2(pe[4], pe[5]), AttnT<T>::pack2(pe[6], pe[7])});
+}
+// A operand of O^T = V^T P^T: this lane's dimension of keys 4 kq .. + 3 (at `at`) and 16 + 4 kq .. + 3
+// (`further` bytes on), the keys of the lane's 8 probabilities
+template <typename V8>
+__device__ __forceinline__ V8 read_vt(const char *at, const int further) {
+    typedef short s4_t __attribute__((ext_vector_type(4)));
+    typedef short s8_t __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) s4_t lds_s4;
+    const s4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)at);
+    const s4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(at + further));
+    return __builtin_bit_cast(V8, s8_t{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w});
+}
+
+template <typename T, int HD, int RB, bool ALIGNED>
+__global__ __launch_bounds__(256, RB == 1 ? 3 : 2) void attn_stream_kernel(const AttnParams p) {
     typedef typename AttnT<T>::V8 V8;
     constexpr int NJ = HD / 32;          // 32-dim steps of the score product
-    constexpr int NDB = HD / 16;         // 16-dim column blocks of the output
-    constexpr int PIECES = 32 * (HD / 8) / 256;   // 16-byte pieces of a V tile per thread
-    // V tile as stored ([key][HD]); the 32-byte segment (16 dims) of a row is XORed with vswz(key):
-    // a transposing read touches 8 consecutive keys' segments of one column block per half wavefront
-    __shared__ __attribute__((aligned(16))) uint16_t vs[2][32 * HD];
-    auto vswz = [](int key) { return HD == 128 ? (key & 7) : ((key >> 1) & 3); };
-    // K tile as stored ([key][HD]), 16-byte pieces of a row XORed with the key so that the 16 lanes
-    // reading the same piece of 16 different keys hit different banks
-    __shared__ __attribute__((aligned(16))) uint16_t kt[2][32 * HD];
-
-    const int seq = blockIdx.x / p.KVH, kvh = blockIdx.x % p.KVH;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NDB = HD / 16;         // 16-dim blocks of the output
+    constexpr int NP = HD / 8;           // 16-byte pieces of a row
+    constexpr int NV = 32 * NP / 64;     // 16-byte pieces of a 32-key V tile per lane
+    constexpr int RPI = 64 / NP;         // rows per V load
+    constexpr int ROWS = 16 * RB;        // rows of a unit
+    constexpr int STEP = 128;            // keys of a turn, 32 per wavefront
+    constexpr int VT = 32 * HD * 2;      // bytes of a V tile
+    constexpr int XROW = HD + 4;         // floats per row of the exchange area (and of partial results)
+    constexpr int LDS_BYTES = 4 * ROWS * XROW * 4 > 4 * VT ? 4 * ROWS * XROW * 4 : 4 * VT;
+    __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];   // V tiles, one per wavefront; then the exchange
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, kq = lane >> 4;
-    const int Gq = p.H / p.KVH;
-    const bool varlen = p.cu_k != nullptr;
-    const int k_start = varlen ? p.cu_k[seq] : 0;
-    const int L = varlen ? p.cu_k[seq + 1] - k_start : p.context_lens[seq];
-    const int ql = varlen ? p.cu_q[seq + 1] - p.cu_q[seq] : (p.q_lens ? p.q_lens[seq] : 1);
-    const int rows_total = ql * Gq;
-    // (a sequence without cached keys still owns output rows: they are written as zeros below)
-    if (ql <= 0 || (int)blockIdx.y * 64 >= rows_total) return;
-    const int row0 = ((int)blockIdx.y * 4 + wave) * 16;
-    const bool wave_active = row0 < rows_total;
-    const int D = p.KVH * HD;
-    const uint16_t *kc = (const uint16_t *)p.k_cache, *vc = (const uint16_t *)p.v_cache;
-    const int32_t *bt = p.block_tables + (size_t)seq * p.max_blocks;
+    char *vt = lds + wave * VT;
+    float *xch = (float *)lds;
+    auto vswz = [](int key) { return HD == 128 ? (key & 7) : ((key >> 1) & 3); };
 
-    // this lane's query row (B operand of S^T = K Q^T: lane (c, kq) holds Q[row c][32 j + 8 kq ..]);
-    // fetched after the first K / V tiles are on their way (the first token of the sequence is a
-    // prefix sum over the query lengths: a dependent chain that nothing else waits for)
-    const int row = row0 + c;
-    const bool row_ok = wave_active && row < rows_total;
-    const int tok = row_ok ? row / Gq : 0, hq = row_ok ? row % Gq : 0;
-    V8 qf[NJ];
-    int q0 = seq;
-    auto first_token = [&]() {
-        if (varlen) q0 = p.cu_q[seq];
-        else if (p.q_lens) q0 = attn_first_token(p.q_lens, seq);
+    const ListPlan pl = list_plan<false>(p, ROWS, ATTN_STREAM_FINE, ATTN_STREAM_COARSE, blockIdx.x);
+    if (!pl.found) return;
+    int pos = blockIdx.x * pl.share;                       // list position of the next step
+    const int end = min(pl.total, pos + pl.share);
+    SeqAt sq = pl.at;
+    int unit = (pos - sq.first) / sq.steps;                // unit of the sequence, step inside the unit
+    int step = (pos - sq.first) - unit * sq.steps;
+
+    const int D = p.KVH * HD;
+    const float sc = p.scale_log2e;
+    const uint32_t rowb = (uint32_t)(D * 2);
+    const char *kc = (const char *)p.k_cache, *vc = (const char *)p.v_cache;
+    // V tile in LDS as stored, 32-byte segments of a row XORed with vswz(key): where this lane's pieces go ...
+    const int vrow0 = lane / NP, vpc = lane % NP;
+    // (vswz(RPI u + vrow0): with 4 rows per load the odd ones differ by 4, with 8 all are alike)
+    const uint32_t vw_at[2] = {(uint32_t)(vrow0 * HD * 2 + ((vpc >> 1) ^ vswz(vrow0)) * 32 + (vpc & 1) * 16),
+                               (uint32_t)(vrow0 * HD * 2 + ((vpc >> 1) ^ vswz(vrow0 + RPI)) * 32 + (vpc & 1) * 16)};
+    // ... and where it reads: dims 16 db + c of keys 4 kq .. + 3 (lane c of a group of 16 addresses key c / 4, 4 dims)
+    const int rkey = 4 * kq + (c >> 2);
+    uint32_t vr_at[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) vr_at[db] = (uint32_t)(rkey * HD * 2 + (db ^ vswz(rkey)) * 32 + (c & 3) * 8);
+
+    while (pos < end) {
+        // ---- one piece: steps step .. step + n - 1 of one unit ----------------------------------------
+        const int n = min(end - pos, sq.steps - step);
+        const int kvh = unit / sq.rg, rg = unit - kvh * sq.rg;
+        const int L = sq.L, ql = sq.ql, k_last = L - 1;
+        const int rows_total = ql * p.Gq, row0 = rg * ROWS;
+        const int rows_here = min(ROWS, rows_total - row0);
+        const int k_start = p.cu_k ? __builtin_amdgcn_readfirstlane(p.cu_k[sq.seq]) : 0;
+        const int32_t *bt = p.block_tables + (size_t)sq.seq * p.max_blocks;
+
+        V8 qf[RB][NJ];
+        int kmax[RB];                                      // last position that row attends
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int row = row0 + 16 * rb + c;
+            const bool ok = row < rows_total;
+            const int tok = ok ? row / p.Gq : 0, hq = ok ? row - tok * p.Gq : 0;
+            kmax[rb] = ok ? L - ql + tok : -1;
+            const uint16_t *qp = (const uint16_t *)p.q + ((size_t)(sq.q0 + tok) * p.H + kvh * p.Gq + hq) * HD + 8 * kq;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                uint4_t raw = {0u, 0u, 0u, 0u};
+                if (ok) raw = *(const uint4_t *)(qp + 32 * j);
+                qf[rb][j] = __builtin_bit_cast(V8, raw);
+            }
+        }
+        const int kmin = L - ql + row0 / p.Gq;            // the unit's first row: tiles that end at or before it need no mask
+
+        float m_run[RB], l_run[RB];
+        float4_t o[RB][NDB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            m_run[rb] = -INFINITY;
+            l_run[rb] = 0.0f;
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) o[rb][db] = float4_t{0.f, 0.f, 0.f, 0.f};
+        }
+
+        // this wavefront's tiles: 32 keys from 32 * wave on, every STEP; 64 of them at a time (their
+        // table entries sit one per lane)
+        const char *kh = kc + kvh * (HD * 2), *vh = vc + kvh * (HD * 2);
+        const int key_end = min(L, pl.g * (step + n));
+        for (int key0 = pl.g * step + 32 * wave; key0 < key_end; key0 += 64 * STEP) {
+            const int nt = min(64, (key_end - key0 + STEP - 1) / STEP);
+            // ALIGNED: the slot of each tile's first key and the last row of the tile that may be read, one
+            // tile per lane (an entry that is negative or beyond the cache reads slot 0)
+            int slot_l = 0, lim_l = 0;
+            if constexpr (ALIGNED) {
+                const int kp = min(key0 + STEP * lane, k_last & ~31);
+                if (p.cu_k) {
+                    slot_l = k_start + kp;
+                    lim_l = k_last - kp;
+                } else {
+                    const int blk = kp / p.block_size;
+                    const int32_t b = bt[min(blk, p.max_blocks - 1)];
+                    const bool ok = b >= 0 && blk < p.max_blocks && ((int64_t)b + 1) * p.block_size <= p.num_slots;
+                    slot_l = ok ? b * p.block_size + (kp - blk * p.block_size) : 0;
+                    lim_l = ok ? k_last - kp : 0;
+                }
+            }
+            // !ALIGNED: lane l (and l + 32) looks up the slot of key l of a tile, one tile ahead of its fetch
+            auto entry = [&](const int i) -> int {
+                const int pc = min(key0 + STEP * i + (lane & 31), k_last);
+                return bt[min(pc / p.block_size, p.max_blocks - 1)];
+            };
+            auto slot_of = [&](const int i, const int b) -> int {
+                const int pc = min(key0 + STEP * i + (lane & 31), k_last);
+                const int blk = pc / p.block_size;
+                const int64_t sl = (int64_t)b * p.block_size + (pc - blk * p.block_size);
+                return (b >= 0 && blk < p.max_blocks && sl < p.num_slots) ? (int)sl : 0;
+            };
+            uint4_t kreg[2][NJ], vreg[NV];
+            int pend = 0, slot_v = 0;
+            auto fetch_k = [&](const int i) {
+                if constexpr (ALIGNED) {
+                    const uint32_t lim = (uint32_t)lane_value(lim_l, i);
+                    const char *kb = kh + (uint64_t)(uint32_t)lane_value(slot_l, i) * rowb;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const uint32_t off = min((uint32_t)(16 * t + c), lim) * rowb + kq * 16u;
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) kreg[t][j] = *(const uint4_t *)(kb + off + 64 * j);
+                    }
+                } else {
+                    slot_v = slot_of(i, pend);
+                    pend = entry(i + 1);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const uint32_t s = (uint32_t)__shfl(slot_v, 16 * t + c, ODSD_WAVE);
+                        const char *kb = kh + (uint64_t)s * rowb + kq * 16;
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) kreg[t][j] = *(const uint4_t *)(kb + 64 * j);
+                    }
+                }
+            };
+            auto fetch_v = [&](const int i) {      // (after fetch_k of the same tile)
+                if constexpr (ALIGNED) {
+                    const uint32_t lim = (uint32_t)lane_value(lim_l, i);
+                    const char *vb = vh + (uint64_t)(uint32_t)lane_value(slot_l, i) * rowb;
+#pragma unroll
+                    for (int u = 0; u < NV; ++u)
+                        vreg[u] = __builtin_nontemporal_load((const uint4_t *)(vb + (min((uint32_t)(RPI * u + vrow0), lim) * rowb + vpc * 16u)));
+                } else {
+#pragma unroll
+                    for (int u = 0; u < NV; ++u) {
+                        const uint32_t s = (uint32_t)__shfl(slot_v, RPI * u + vrow0, ODSD_WAVE);
+                        vreg[u] = __builtin_nontemporal_load((const uint4_t *)(vh + (uint64_t)s * rowb + vpc * 16));
+                    }
+                }
+            };
+            // one tile.  FETCH: there is a next one; it is requested into the registers this one has just left
+            auto tile = [&](auto fetch_c, const int i) {
+                const int k0 = key0 + STEP * i;
+                float4_t st[RB][2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) {
+                        st[rb][t] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+                            st[rb][t] = AttnT<T>::mfma(__builtin_bit_cast(V8, kreg[t][j]), qf[rb][j], st[rb][t]);
+                    }
+                if constexpr (decltype(fetch_c)::value) fetch_k(i + 1);
+#pragma unroll
+                for (int u = 0; u < NV; ++u) *(uint4_t *)(vt + vw_at[u & 1] + RPI * u * HD * 2) = vreg[u];
+                if constexpr (decltype(fetch_c)::value) fetch_v(i + 1);
+                V8 pf[RB];
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) {
+                    // lane (c, kq) holds keys k0 + 16 t + 4 kq + i of query row c (raw scores)
+                    float a[8] = {st[rb][0].x, st[rb][0].y, st[rb][0].z, st[rb][0].w, st[rb][1].x, st[rb][1].y, st[rb][1].z, st[rb][1].w};
+                    if (k0 + 31 > kmin) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            a[e] = k0 + 16 * (e >> 2) + 4 * kq + (e & 3) <= kmax[rb] ? a[e] : -INFINITY;
+                    }
+                    pf[rb] = softmax_tile<T, NDB>(a, sc, m_run[rb], l_run[rb], o[rb]);
+                }
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) {
+                    const V8 vf = read_vt<V8>(vt + vr_at[db], 16 * HD * 2);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) o[rb][db] = AttnT<T>::mfma(vf, pf[rb], o[rb][db]);
+                }
+            };
+            if constexpr (!ALIGNED) pend = entry(0);
+            fetch_k(0);
+            fetch_v(0);
+            int i = 0;
+            for (; i + 1 < nt; ++i) tile(std::true_type{}, i);
+            tile(std::false_type{}, i);
+        }
+
+        // ---- the four wavefronts' sums, through LDS -----------------------------------------------------
+        const bool whole = n == sq.steps;
+        __syncthreads();                                   // every wavefront is done with its V tile
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            float *xr = xch + (wave * ROWS + 16 * rb + c) * XROW;
+            float l = l_run[rb];
+            l += __shfl_xor(l, 16, ODSD_WAVE);
+            l += __shfl_xor(l, 32, ODSD_WAVE);
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) *(float4_t *)(xr + 16 * db + 4 * kq) = o[rb][db];
+            if (kq == 0) {
+                xr[HD] = m_run[rb];
+                xr[HD + 1] = l;
+            }
+        }
+        __syncthreads();
+        // (a piece that begins where its workgroup's share begins goes to the workgroup's first slot)
+        float *part = p.part + (size_t)(2 * blockIdx.x + (pos > (int)blockIdx.x * pl.share ? 1 : 0)) * (ROWS * XROW);
+        for (int it = tid; it < rows_here * (HD / 4); it += 256) {
+            const int row = it / (HD / 4), d = 4 * (it % (HD / 4));
+            const float *xr = xch + row * XROW;
+            float m = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) m = fmaxf(m, xr[w * ROWS * XROW + HD]);
+            const float ref = m == -INFINITY ? 0.0f : m;
+            float l = 0.0f;
+            float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const float f = __builtin_amdgcn_exp2f(xr[w * ROWS * XROW + HD] - ref);      // -inf -> 0
+                const float4_t v = *(const float4_t *)(xr + w * ROWS * XROW + d);
+                l += f * xr[w * ROWS * XROW + HD + 1];
+                acc.x += f * v.x; acc.y += f * v.y; acc.z += f * v.z; acc.w += f * v.w;
+            }
+            if (whole) {
+                const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+                const int r = row0 + row, tok = r / p.Gq, hq = r - tok * p.Gq;
+                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+                *(u32x2 *)((uint16_t *)p.out + ((size_t)(sq.q0 + tok) * p.H + kvh * p.Gq + hq) * HD + d) =
+                    u32x2{AttnT<T>::pack2(acc.x * inv, acc.y * inv), AttnT<T>::pack2(acc.z * inv, acc.w * inv)};
+            } else {
+                *(float4_t *)(part + row * XROW + d) = acc;
+                if (d == 0) {
+                    part[row * XROW + HD] = m;
+                    part[row * XROW + HD + 1] = l;
+                }
+            }
+        }
+        pos += n;
+        if (pos < end) {
+            __syncthreads();                               // the exchange area becomes V tiles again
+            next_unit(p, sq, unit, step, ROWS, pl.g);
+        }
+    }
+}
+
+// The form for more than 32 rows per sequence (a verify step of a model with many query heads per KV head): a
+// wavefront cannot hold 64 rows next to its keys, so here the four wavefronts own 16 rows each and share
+// the keys through LDS, 32 at a time.  K and V rows are copied there asynchronously, three tiles ahead (a
+// ring of four, one barrier per tile, waits that leave the younger copies in flight) and on across the end
+// of a piece; the rows of the keys are looked up for many tiles at a time and kept in LDS.
+template <typename T, int HD>
+__global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
+    typedef typename AttnT<T>::V8 V8;
+    constexpr int NJ = HD / 32, NDB = HD / 16;
+    constexpr int NP = HD / 8;           // 16-byte pieces of a row
+    constexpr int RPC = 64 / NP;         // rows of one copy
+    constexpr int COPIES = 32 / RPC / 4; // copies per wavefront, tile and matrix
+    constexpr int ROWS = 64, XROW = HD + 4;
+    constexpr int TILEB = 32 * HD * 2;
+    constexpr int NBUF = 4;
+    constexpr int MOST = 64;             // tiles whose rows are looked up at a time
+    __shared__ __attribute__((aligned(16))) char lds[NBUF * 2 * TILEB];
+    __shared__ uint32_t slots[MOST * 32];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, kq = lane >> 4;
+    auto vswz = [](int key) { return HD == 128 ? (key & 7) : ((key >> 1) & 3); };
+
+    const ListPlan pl = list_plan<false>(p, ROWS, ATTN_TILE_FINE, ATTN_TILE_COARSE, blockIdx.x);
+    if (!pl.found) return;
+    const int first_pos = blockIdx.x * pl.share, end = min(pl.total, first_pos + pl.share);
+    const float sc = p.scale_log2e;
+
+    // copies: row RPC * (wave + 4 i) + lane / NP of a tile, stored piece lane % NP (16-byte pieces of a K row and
+    // 32-byte segments of a V row XORed with the key against bank conflicts)
+    const int crow = lane / NP, cslot = lane % NP;
+    uint32_t kp_at[COPIES], vp_at[COPIES];
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) {
+        const int key = RPC * (wave + 4 * i) + crow;
+        kp_at[i] = (uint32_t)(cslot ^ (key & (NP - 1))) * 16u;
+        vp_at[i] = (uint32_t)(2 * ((cslot >> 1) ^ vswz(key)) + (cslot & 1)) * 16u;
+    }
+    // fragments: K (A operand: key 16 t + c, dims 32 j + 8 kq ..), V^T (dims 16 db + c of keys 4 kq .. and 16 + 4 kq ..)
+    uint32_t k_at[NJ], v_at[NDB];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) k_at[j] = (uint32_t)(c * HD * 2 + ((4 * j + kq) ^ (c & (NP - 1))) * 16);
+    const int rkey = 4 * kq + (c >> 2);
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) v_at[db] = (uint32_t)(rkey * HD * 2 + (db ^ vswz(rkey)) * 32 + (c & 3) * 8);
+
+    // The workgroup's share as pieces (consecutive steps of one unit).  Two cursors walk them: `ahead` looks up
+    // the rows of the next tiles' keys, `now` is what is being computed.
+    struct Cursor {
+        SeqAt sq;
+        int pos, unit, step, n;      // list position, unit, first step and steps of the piece
+        int key, key_end;            // next key and end of the piece's keys
     };
-    auto load_q = [&]() {
-        first_token();
-        const uint16_t *qp = (const uint16_t *)p.q + ((size_t)(q0 + tok) * p.H + kvh * Gq + hq) * HD + 8 * kq;
+    auto set_piece = [&](Cursor &q) {
+        q.n = min(end - q.pos, q.sq.steps - q.step);
+        q.key = pl.g * q.step;
+        q.key_end = min(q.sq.L, pl.g * (q.step + q.n));
+    };
+    auto next_piece = [&](Cursor &q) {
+        q.pos += q.n;
+        if (q.pos < end) {
+            next_unit(p, q.sq, q.unit, q.step, ROWS, pl.g);
+            set_piece(q);
+        }
+    };
+    Cursor now;
+    now.sq = pl.at;
+    now.pos = first_pos;
+    now.unit = (first_pos - pl.at.first) / pl.at.steps;
+    now.step = (first_pos - pl.at.first) - now.unit * pl.at.steps;
+    set_piece(now);
+    Cursor ahead = now;
+
+    // of the piece being computed
+    bool fresh = true;                                     // its rows have not been set up yet
+    bool active = false, ok = false;
+    int tok = 0, hq = 0, kmax = -1, kmin = 0, kvh = 0;
+    V8 qf[NJ];
+    float m_run = 0.0f, l_run = 0.0f;
+    float4_t o[NDB];
+    auto begin_piece = [&]() {
+        kvh = now.unit / now.sq.rg;
+        const int rg = now.unit - kvh * now.sq.rg;
+        const int rows_total = now.sq.ql * p.Gq, row0 = rg * ROWS + 16 * wave;
+        const int row = row0 + c;
+        active = row0 < rows_total;
+        ok = row < rows_total;
+        tok = ok ? row / p.Gq : 0;
+        hq = ok ? row - tok * p.Gq : 0;
+        kmax = ok ? now.sq.L - now.sq.ql + tok : -1;       // last position this row attends
+        kmin = now.sq.L - now.sq.ql + row0 / p.Gq;
+        const uint16_t *qp = (const uint16_t *)p.q + ((size_t)(now.sq.q0 + tok) * p.H + kvh * p.Gq + hq) * HD + 8 * kq;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             uint4_t raw = {0u, 0u, 0u, 0u};
-            if (row_ok) raw = *(const uint4_t *)(qp + 32 * j);
+            if (ok) raw = *(const uint4_t *)(qp + 32 * j);
             qf[j] = __builtin_bit_cast(V8, raw);
         }
+        m_run = -INFINITY;
+        l_run = 0.0f;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) o[db] = float4_t{0.f, 0.f, 0.f, 0.f};
+        fresh = false;
     };
-    const int kmax = row_ok ? L - ql + tok : -1;      // last position this row attends
-    int kmin_wave = row_ok ? kmax : 0x7fffffff;        // tiles ending at or before it need no mask
+    auto end_piece = [&]() {
+        float l = l_run;
+        l += __shfl_xor(l, 16, ODSD_WAVE);
+        l += __shfl_xor(l, 32, ODSD_WAVE);
+        if (ok) {
+            if (now.n == now.sq.steps) {
+                const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+                uint16_t *op = (uint16_t *)p.out + ((size_t)(now.sq.q0 + tok) * p.H + kvh * p.Gq + hq) * HD + 4 * kq;
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) kmin_wave = min(kmin_wave, __shfl_xor(kmin_wave, d, ODSD_WAVE));
-    const float sc = p.scale_log2e;
-
-    // per query row c: the reference point of its exponentials (the same in its 4 kq lanes) and
-    // this lane's share of the sum of its probabilities
-    float m_run = -INFINITY, l_run = 0.0f;
-    float4_t o[NDB];
+                for (int db = 0; db < NDB; ++db)
+                    *(u32x2 *)(op + 16 * db) = u32x2{AttnT<T>::pack2(o[db].x * inv, o[db].y * inv),
+                                                     AttnT<T>::pack2(o[db].z * inv, o[db].w * inv)};
+            } else {
+                // (a piece that begins where its workgroup's share begins goes to the workgroup's first slot)
+                float *part = p.part + (size_t)(2 * blockIdx.x + (now.pos > first_pos ? 1 : 0)) * (ROWS * XROW) + (16 * wave + c) * XROW;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) o[db] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-    // Software pipeline over the 32-key tiles, two tiles deep.  A tile's K and V rows are fetched
-    // once per workgroup, 16 bytes per thread and piece (piece = tid + 256 u -> key = piece /
-    // (HD / 8), dims 8 * (piece % (HD / 8)) ..), two tiles ahead into one of two register sets;
-    // one tile ahead they go to LDS, as stored, and every wavefront reads its
-    // MFMA operands from there (K fetched per wavefront instead costs four times the L2 traffic
-    // and was what bounded the kernel).  During tile `it`: the set that held tile `it` is refilled
-    // with tile it + 2, the other set (tile it + 1) goes to the other LDS buffers, and the
-    // block-table entries of tile it + 3 are requested BEFORE the fetches (the load counter retires
-    // in order: a younger table read awaited by the next tile would otherwise drain the big
-    // fetches issued before it).  The steady-state tiles fetch unconditionally and the last two
-    // tiles are compiled without the fetch, so that no wait is placed after a join of "fetched"
-    // and "did not fetch".
-    // ALIGNED (block_size a multiple of 32): a tile lies in one cache block, so its table entry is
-    // one wavefront-uniform read; otherwise every lane reads the entries of its own keys.
-    constexpr int NE = ALIGNED ? 1 : PIECES;            // table entries a tile needs per lane
-    const int k_last = L - 1;
-    const int bs = p.block_size;
-    auto entry_at = [&](int pos) -> int32_t { return varlen ? 0 : bt[min(min(pos, k_last) / bs, p.max_blocks - 1)]; };
-    auto request = [&](int k0, int32_t (&e)[NE]) {
-        if constexpr (ALIGNED) {
-            e[0] = entry_at(k0);
-        } else {
-#pragma unroll
-            for (int u = 0; u < PIECES; ++u) e[u] = entry_at(k0 + (tid + 256 * u) / (HD / 8));
-        }
-    };
-    // slot of position pos (clamped into the sequence) in the block whose table entry is b; an
-    // entry that is negative, beyond the table or beyond the cache reads slot 0
-    auto slot_in = [&](int32_t b, int pos) -> int64_t {
-        const int pc = min(pos, k_last);
-        const int blk = pc / bs;
-        const int64_t sl = (int64_t)b * bs + (pc - blk * bs);
-        return (b >= 0 && blk < p.max_blocks && sl < p.num_slots) ? sl : 0;
-    };
-    uint4_t kreg[2][PIECES], vreg[2][PIECES];
-    // fetch of the tile at k0, whose table entries are e
-    auto fetch = [&](auto set, int k0, const int32_t (&e)[NE]) {
-        constexpr int S = decltype(set)::value;
-        if constexpr (ALIGNED) {
-            // everything about the block is wavefront-uniform: one 64-bit base per tile, and a lane
-            // adds the 32-bit offset of its row (clamped to the sequence's last key in the tile)
-            const int k0c = min(k0, k_last & ~31);
-            const int blk = k0c / bs;
-            const int32_t b = e[0];
-            const bool ok = varlen || (b >= 0 && blk < p.max_blocks && ((int64_t)b + 1) * bs <= p.num_slots);
-            const int64_t slot0 = varlen ? (int64_t)k_start + k0c : (ok ? (int64_t)b * bs + (k0c - blk * bs) : 0);
-            const int lim = ok ? k_last - k0c : 0;
-            const size_t base = (size_t)slot0 * D + kvh * HD;
-            const uint16_t *kb = kc + base, *vb = vc + base;
-#pragma unroll
-            for (int u = 0; u < PIECES; ++u) {
-                const int piece = tid + 256 * u;
-                const uint32_t off = (uint32_t)min(piece / (HD / 8), lim) * (uint32_t)D + 8 * (piece % (HD / 8));
-                kreg[S][u] = *(const uint4_t *)(kb + off);
-                vreg[S][u] = *(const uint4_t *)(vb + off);
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < PIECES; ++u) {
-                const int piece = tid + 256 * u;
-                const int64_t sl = slot_in(e[u], k0 + piece / (HD / 8));
-                const size_t off = (size_t)sl * D + kvh * HD + 8 * (piece % (HD / 8));
-                kreg[S][u] = *(const uint4_t *)(kc + off);
-                vreg[S][u] = *(const uint4_t *)(vc + off);
-            }
-        }
-    };
-    // a tile's K and V rows into the LDS buffers `buf`, 16 bytes per thread and piece, as stored
-    auto store_kv = [&](auto set, int buf) {
-        constexpr int S = decltype(set)::value;
-#pragma unroll
-        for (int u = 0; u < PIECES; ++u) {
-            const int piece = tid + 256 * u;
-            const int key = piece / (HD / 8), ch = piece % (HD / 8);
-            *(uint4_t *)&vs[buf][key * HD + 16 * ((ch >> 1) ^ vswz(key)) + 8 * (ch & 1)] = vreg[S][u];
-            *(uint4_t *)&kt[buf][key * HD + 8 * (ch ^ (key & (HD / 8 - 1)))] = kreg[S][u];
-        }
-    };
-
-    // this workgroup's slice of the 32-key tiles
-    // (keys past the last one that any row of this workgroup attends are never visited: in a
-    // prefill the early row groups stop long before the end of the sequence)
-    const int last_tok = min(ql - 1, ((int)blockIdx.y * 64 + 63) / Gq);
-    const int k_end = max(0, min(L, L - ql + last_tok + 1));   // no visible key at all: no tiles, zeros out
-    const int all_tiles = (k_end + 31) / 32;
-    const int per_split = (all_tiles + p.splits - 1) / p.splits;
-    const int t_begin = min(all_tiles, (int)blockIdx.z * per_split);
-    const int n_tiles = min(all_tiles, t_begin + per_split) - t_begin;
-    const int kbase = t_begin * 32;
-    int32_t pend[NE];                                   // entries of the tile after the newest fetched one
-
-    // one tile; S: the register set that held it (free now). FETCH: tile it + 2 exists and is fetched (and
-    // the entries of tile it + 3 requested); STORE: tile it + 1 exists and its V goes to LDS
-    auto tile = [&](auto set, auto fetch_c, auto store_c, int it) {
-        constexpr int S = decltype(set)::value;
-        constexpr bool FETCH = decltype(fetch_c)::value, STORE = decltype(store_c)::value;
-        const int k0 = kbase + it * 32, buf = it & 1;
-        float4_t st[2];
-        if (wave_active) {
-            // scores S^T[key][row] for the two 16-key halves
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                float4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                    const int key = 16 * t + c;
-                    const uint4_t kraw = *(const uint4_t *)&kt[buf][key * HD + 8 * ((4 * j + kq) ^ (key & (HD / 8 - 1)))];
-                    acc = AttnT<T>::mfma(__builtin_bit_cast(V8, kraw), qf[j], acc);
+                for (int db = 0; db < NDB; ++db) *(float4_t *)(part + 16 * db + 4 * kq) = o[db];
+                if (kq == 0) {
+                    part[HD] = m_run;
+                    part[HD + 1] = l;
                 }
-                st[t] = acc;
             }
         }
-        if constexpr (FETCH) {
-            int32_t now[NE];
-#pragma unroll
-            for (int i = 0; i < NE; ++i) now[i] = pend[i];
-            request(k0 + 96, pend);
-            fetch(set, k0 + 64, now);
-        }
-        if (wave_active) {
-            // lane (c, kq) holds keys k0 + 16 t + 4 kq + i of query row c (raw scores, before the
-            // softmax scale).  Only tiles that reach past the first row's last key need the mask.
-            float a[8] = {st[0].x, st[0].y, st[0].z, st[0].w, st[1].x, st[1].y, st[1].z, st[1].w};
-            if (k0 + 31 > kmin_wave) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    a[i] = k0 + 16 * (i >> 2) + 4 * kq + (i & 3) <= kmax ? a[i] : -INFINITY;
+        next_piece(now);
+        fresh = true;
+    };
+
+    while (now.pos < end) {
+        if (fresh) begin_piece();
+        // rows of K / V (slot * KVH + kvh) of the next tiles' keys, at most MOST tiles: positions past a
+        // piece's last key repeat that key's row; an entry that is negative or beyond the cache reads slot 0
+        int nt = 0;
+        while (nt < MOST && ahead.pos < end) {
+            const int L = ahead.sq.L, here = min(MOST - nt, max(0, (ahead.key_end - ahead.key + 31) / 32));
+            const int ks = p.cu_k ? p.cu_k[ahead.sq.seq] : 0;
+            const int h = ahead.unit / ahead.sq.rg;
+            const int32_t *bt = p.block_tables + (size_t)ahead.sq.seq * p.max_blocks;
+            for (int i = tid; i < 32 * here; i += 256) {
+                const int pc = min(ahead.key + i, L - 1);
+                uint32_t sl;
+                if (p.cu_k) {
+                    sl = (uint32_t)(ks + pc);
+                } else {
+                    const int blk = pc / p.block_size;
+                    const int32_t b = bt[min(blk, p.max_blocks - 1)];
+                    const int64_t s = (int64_t)b * p.block_size + (pc - blk * p.block_size);
+                    sl = (b >= 0 && blk < p.max_blocks && s < p.num_slots) ? (uint32_t)s : 0u;
+                }
+                slots[32 * nt + i] = sl * (uint32_t)p.KVH + (uint32_t)h;
             }
-            float mx = fmaxf(fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])), fmaxf(fmaxf(a[4], a[5]), fmaxf(a[6], a[7])));
-            // The reference point m_run of a row moves only when some score of the wavefront
-            // exceeds it by more than 2^8 (probabilities up to 256 are as exact in fp16 / bf16 as
-            // those below 1, and the sums are fp32): most tiles then need no exchange between
-            // lanes at all -- no maximum, no rescaling of the output, no sum (l_run stays a
-            // per-lane partial sum until the end).
-            if (__any(mx * sc > m_run + 8.0f)) {
-                mx = fmaxf(mx, __shfl_xor(mx, 16, ODSD_WAVE));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, ODSD_WAVE));
-                const float m_new = fmaxf(m_run, mx * sc);
-                // a row with nothing to attend yet keeps m = -inf: use 0 as the reference point then
-                const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));   // m_run = -inf -> 0
-                l_run *= alpha;
-                m_run = m_new;
-                // the output tile holds rows 4 kq + i in lane (dim, kq): fetch those rows' alpha
-                float al[4];
+            nt += here;
+            ahead.key += 32 * here;
+            if (ahead.key >= ahead.key_end) next_piece(ahead);
+        }
+        nt = __builtin_amdgcn_readfirstlane(nt);
+        __syncthreads();
+        // (Q has come in before the table entries; without this the compiler would wait for it, and with it for
+        // every copy, at its first use)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) al[i] = __shfl(alpha, 4 * kq + i, ODSD_WAVE);
+        for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(qf[j]));
+        auto copy_tile = [&](const int i) {
+            char *dst = lds + (i & (NBUF - 1)) * (2 * TILEB);
+            uint32_t sl[COPIES];
+#pragma unroll
+            for (int u = 0; u < COPIES; ++u) sl[u] = slots[32 * i + RPC * (wave + 4 * u) + crow];
+#pragma unroll
+            for (int u = 0; u < COPIES; ++u) {
+                const uint64_t off = (uint64_t)sl[u] * (HD * 2);
+                dma16_from_to_lds((const char *)p.k_cache + off + kp_at[u], (lds_void *)(dst + RPC * (wave + 4 * u) * HD * 2));
+                const char *vfrom = (const char *)p.v_cache + off + vp_at[u];
+                lds_void *vto = (lds_void *)(dst + TILEB + RPC * (wave + 4 * u) * HD * 2);
+                if (p.v_once) dma16_from_to_lds_nt(vfrom, vto);
+                else dma16_from_to_lds(vfrom, vto);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < NBUF - 1; ++i)
+            if (i < nt) copy_tile(i);
+        for (int i = 0; i < nt; ++i) {
+            while (now.key >= now.key_end) {               // (a piece without keys ends as it begins)
+                if (fresh) begin_piece();
+                end_piece();
+            }
+            if (fresh) begin_piece();
+            // tile i has landed once only the copies of the younger tiles are outstanding
+            if (i + 2 < nt) ODSD_WAIT_VMCNT_LGKM0(2 * 2 * COPIES);
+            else if (i + 1 < nt) ODSD_WAIT_VMCNT_LGKM0(2 * COPIES);
+            else ODSD_WAIT_VMCNT_LGKM0(0);
+            __builtin_amdgcn_s_barrier();                  // ... for every wavefront, and all are done with tile i - 1
+            if (i + NBUF - 1 < nt) copy_tile(i + NBUF - 1);
+            if (active) {
+                const char *kt = lds + (i & (NBUF - 1)) * (2 * TILEB), *vt = kt + TILEB;
+                const int k0 = now.key;
+                float4_t st[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    st[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        st[t] = AttnT<T>::mfma(*(const V8 *)(kt + k_at[j] + t * 16 * HD * 2), qf[j], st[t]);
+                }
+                float a[8] = {st[0].x, st[0].y, st[0].z, st[0].w, st[1].x, st[1].y, st[1].z, st[1].w};
+                if (k0 + 31 > kmin) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        a[e] = k0 + 16 * (e >> 2) + 4 * kq + (e & 3) <= kmax ? a[e] : -INFINITY;
+                }
+                const V8 pf = softmax_tile<T, NDB>(a, sc, m_run, l_run, o);
 #pragma unroll
                 for (int db = 0; db < NDB; ++db) {
-                    o[db].x *= al[0]; o[db].y *= al[1]; o[db].z *= al[2]; o[db].w *= al[3];
+                    const V8 vf = read_vt<V8>(vt + v_at[db], 16 * HD * 2);
+                    o[db] = AttnT<T>::mfma(vf, pf, o[db]);
                 }
             }
-            const float neg_ref = m_run == -INFINITY ? 0.0f : -m_run;
-            float pe[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) pe[i] = __builtin_amdgcn_exp2f(fmaf(a[i], sc, neg_ref));   // masked -> 0
-            l_run += ((pe[0] + pe[1]) + (pe[2] + pe[3])) + ((pe[4] + pe[5]) + (pe[6] + pe[7]));
-            const V8 pf = __builtin_bit_cast(V8, uint4_t{AttnT<T>::pack2(pe[0], pe[1]), AttnT<T>::pack2(pe[2], pe[3]),
-                                                          AttnT<T>::pack2(pe[4], pe[5]), AttnT<T>::pack2(pe[6], pe[7])});
-            // B operand of column block db: dimension 16 db + c of keys 4 kq .. + 3 and 16 + 4 kq .. + 3
-            // (the keys of pf's 8 probabilities).  Lane c of a group addresses key 4 kq + c / 4,
-            // dimensions 16 db + 4 (c % 4) .. + 3; the read hands it column c of the group's 4 x 16 block.
-            const int key_a = 4 * kq + (c >> 2), key_b = key_a + 16;
-            const uint16_t *va = &vs[buf][key_a * HD + 4 * (c & 3)], *vb = &vs[buf][key_b * HD + 4 * (c & 3)];
-            const int swa = vswz(key_a), swb = vswz(key_b);
-#pragma unroll
-            for (int db = 0; db < NDB; ++db) {
-                typedef short s4_t __attribute__((ext_vector_type(4)));
-                typedef __attribute__((address_space(3))) s4_t lds_s4;
-                const s4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(va + 16 * (db ^ swa)));
-                const s4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(vb + 16 * (db ^ swb)));
-                typedef short s8_t __attribute__((ext_vector_type(8)));
-                const V8 vf = __builtin_bit_cast(V8, s8_t{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w});
-                o[db] = AttnT<T>::mfma(pf, vf, o[db]);
-            }
+            now.key += 32;
         }
-        // K and V of tile it + 1 (other set, fetched during tile it - 1) into the other LDS buffers
-        if constexpr (STORE) store_kv(std::integral_constant<int, S ^ 1>{}, buf ^ 1);
-        __syncthreads();
-    };
-
-    if (n_tiles > 0) {
-        const std::integral_constant<int, 0> s0;
-        const std::integral_constant<int, 1> s1;
-        const std::true_type yes;
-        const std::false_type no;
-        // prologue: tiles 0 and 1 fetched, tile 0 in LDS, the entries of tile 2 requested
-        request(kbase, pend);
-        fetch(s0, kbase, pend);
-        if (n_tiles > 1) {
-            request(kbase + 32, pend);
-            fetch(s1, kbase + 32, pend);
+        // (pieces that end with the list, or had no keys at all)
+        while (now.pos < end && now.key >= now.key_end) {
+            if (fresh) begin_piece();
+            end_piece();
         }
-        request(kbase + 64, pend);
-        load_q();
-        store_kv(s0, 0);
-        __syncthreads();
-        int it = 0;
-        for (; it + 3 < n_tiles; it += 2) {
-            tile(s0, yes, yes, it);
-            tile(s1, yes, yes, it + 1);
-        }
-        // one to three tiles are left, `it` is even
-        const int left = n_tiles - it;
-        if (left == 3) {
-            tile(s0, yes, yes, it);
-            tile(s1, no, yes, it + 1);
-            tile(s0, no, no, it + 2);
-        } else if (left == 2) {
-            tile(s0, no, yes, it);
-            tile(s1, no, no, it + 1);
-        } else {
-            tile(s0, no, no, it);
-        }
-    } else {
-        first_token();     // the rows are still written (zeros): they need the sequence's first row
-    }
-
-    l_run += __shfl_xor(l_run, 16, ODSD_WAVE);
-    l_run += __shfl_xor(l_run, 32, ODSD_WAVE);
-    if (wave_active && p.splits > 1) {
-        // partial result of this slice: rows of the workgroup's 64, [HD] unnormalised output, m, l
-        float *base = p.part + ((((size_t)blockIdx.x * gridDim.y + blockIdx.y) * p.splits + blockIdx.z) * 64) * (HD + 4);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float *rowp = base + (size_t)(wave * 16 + 4 * kq + i) * (HD + 4);
-#pragma unroll
-            for (int db = 0; db < NDB; ++db)
-                rowp[16 * db + c] = i == 0 ? o[db].x : i == 1 ? o[db].y : i == 2 ? o[db].z : o[db].w;
-        }
-        if (kq == 0) {
-            float *rowp = base + (size_t)(wave * 16 + c) * (HD + 4);
-            rowp[HD] = m_run;
-            rowp[HD + 1] = l_run;
-        }
-        return;
-    }
-    if (wave_active) {
-        float inv[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float l = __shfl(l_run, 4 * kq + i, ODSD_WAVE);
-            inv[i] = l > 0.0f ? 1.0f / l : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = row0 + 4 * kq + i;
-            if (r < rows_total) {
-                const int t2 = r / Gq, h2 = r % Gq;
-                uint16_t *op = (uint16_t *)p.out + ((size_t)(q0 + t2) * p.H + kvh * Gq + h2) * HD + c;
-#pragma unroll
-                for (int db = 0; db < NDB; ++db) {
-                    const float v = (i == 0 ? o[db].x : i == 1 ? o[db].y : i == 2 ? o[db].z : o[db].w) * inv[i];
-                    op[16 * db] = AttnT<T>::from_f32(v);
-                }
-            }
-        }
+        ODSD_WAIT_VMCNT_LGKM0(0);
+        __builtin_amdgcn_s_barrier();                      // buffers and slots are free again
     }
 }
 
-// Merge of the key slices: out[row] = sum_s exp2(m_s - m) O_s / sum_s exp2(m_s - m) l_s, slices in
-// order. One workgroup per (sequence, KV head, row group, 256 VEC / HD rows): a thread owns VEC
-// neighbouring output elements of a row and walks the slices.  VEC = 4 (one 16-byte load per slice;
-// rows of the partial results are HD + 4 floats apart so that they stay 16-byte aligned) when there
-// are at most 4 slices: a quarter of the workgroups and of the exponentials; with more slices there
-// are few rows, and one element per thread keeps more of the chip busy.  (More rows per workgroup,
-// taken in turn, measured slower: each turn is one more exposed load latency.)
-template <typename T, int HD, int SB, int VEC>
-__global__ __launch_bounds__(256) void paged_attn_merge_kernel(const AttnParams p) {
-    static_assert(VEC == 1 || VEC == 4, "one element or one 16-byte vector per thread");
-    constexpr int TPR = HD / VEC;                       // threads per row
-    constexpr int RPW = 256 / TPR;                      // rows per workgroup
-    const int seq = blockIdx.x / p.KVH, kvh = blockIdx.x % p.KVH;
-    const int Gq = p.H / p.KVH;
-    const bool varlen = p.cu_k != nullptr;
-    const int ql = varlen ? p.cu_q[seq + 1] - p.cu_q[seq] : (p.q_lens ? p.q_lens[seq] : 1);
-    const int rows_total = ql * Gq;
-    // the sequence's first token: a chain of its own (a wavefront-wide sum over the query lengths),
-    // started before the partial results are requested and by every lane of the wavefront
-    int q0 = seq;
-    if (varlen) q0 = p.cu_q[seq];
-    else if (p.q_lens) q0 = attn_first_token(p.q_lens, seq);
-    const int d = VEC * ((int)threadIdx.x % TPR);
-    const int r = (int)blockIdx.z * RPW + (int)threadIdx.x / TPR;
-    const int row = (int)blockIdx.y * 64 + r;
-    if (row >= rows_total) return;
-    const float *base = p.part + ((((size_t)blockIdx.x * gridDim.y + blockIdx.y) * p.splits) * 64 + r) * (HD + 4);
-    const size_t stride = (size_t)64 * (HD + 4);
-    // one pass, SB slices at a time (all their loads in flight together; SB = 4 when there are no
-    // more than 4 slices, so that none is fetched twice), rescaling the running
-    // sums whenever a batch raises the reference point
+// Merge of the pieces of a unit: out[row] = sum_s exp2(m_s - m) O_s / sum_s exp2(m_s - m) l_s, pieces in
+// order.  One workgroup per (sequence, KV head, unit, 1024 / HD rows): a thread owns 4 neighbouring output
+// elements of a row and walks the pieces, 4 at a time.  Units that were finished in place are left alone.
+template <typename T, int HD, int ROWS, int FINE, int COARSE>
+__global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
+    constexpr int XROW = HD + 4;
+    constexpr int TPR = HD / 4, RPW = 256 / TPR;
+    const int seq = blockIdx.x / p.KVH, kvh = blockIdx.x - seq * p.KVH;
+    const int rg = blockIdx.y;
+    const ListPlan pl = list_plan<true>(p, ROWS, FINE, COARSE, seq);
+    const SeqAt &sq = pl.at;
+    if (rg >= sq.rg) return;
+    const int a = sq.first + (kvh * sq.rg + rg) * sq.steps;        // list positions of the unit's steps
+    const int wa = a / pl.share, wb = (a + sq.steps - 1) / pl.share;
+    if (wa == wb) return;
+    const int row = (int)blockIdx.z * RPW + (int)threadIdx.x / TPR, d = 4 * ((int)threadIdx.x % TPR);
+    const int r = rg * ROWS + row;
+    if (row >= ROWS || r >= sq.ql * p.Gq) return;
+    const float *base = p.part + row * XROW;
+    const size_t slot = (size_t)ROWS * XROW;
+    auto piece = [&](const int w) { return base + (size_t)(2 * w + (w == wa && a > wa * pl.share ? 1 : 0)) * slot; };
     float m = -INFINITY, l = 0.0f;
-    float acc[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
-    for (int s0 = 0; s0 < p.splits; s0 += SB) {
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int SB = 4;
+    for (int w0 = wa; w0 <= wb; w0 += SB) {
         float ms[SB], ls[SB];
-        float os[SB][VEC];
+        float4_t os[SB];
 #pragma unroll
         for (int u = 0; u < SB; ++u) {
-            // (every load unconditional, on a clamped slice: loads under a branch serialise)
-            const float *rp = base + (size_t)min(s0 + u, p.splits - 1) * stride;
+            // (every load unconditional, on a clamped piece: loads under a branch serialise)
+            const float *rp = piece(min(w0 + u, wb));
             const float2_t ml = *(const float2_t *)(rp + HD);
             ms[u] = ml.x;
             ls[u] = ml.y;
-            if constexpr (VEC == 4) {
-                const float4_t v = *(const float4_t *)(rp + d);
-                os[u][0] = v.x; os[u][1] = v.y; os[u][2] = v.z; os[u][3] = v.w;
-            } else {
-                os[u][0] = rp[d];
-            }
+            os[u] = *(const float4_t *)(rp + d);
         }
 #pragma unroll
         for (int u = 0; u < SB; ++u) {
-            if (s0 + u >= p.splits) {
+            if (w0 + u > wb) {
                 ms[u] = -INFINITY;
                 ls[u] = 0.0f;
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) os[u][i] = 0.0f;
+                os[u] = float4_t{0.f, 0.f, 0.f, 0.f};
             }
         }
         float mb = m;
 #pragma unroll
         for (int u = 0; u < SB; ++u) mb = fmaxf(mb, ms[u]);
         const float ref = mb == -INFINITY ? 0.0f : mb;
-        const float keep = exp2f(m - ref);            // m = -inf -> 0
+        const float keep = __builtin_amdgcn_exp2f(m - ref);            // m = -inf -> 0
         l *= keep;
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) acc[i] *= keep;
+        acc.x *= keep; acc.y *= keep; acc.z *= keep; acc.w *= keep;
 #pragma unroll
         for (int u = 0; u < SB; ++u) {
-            const float f = exp2f(ms[u] - ref);
+            const float f = __builtin_amdgcn_exp2f(ms[u] - ref);
             l += f * ls[u];
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[i] += f * os[u][i];
+            acc.x += f * os[u].x; acc.y += f * os[u].y; acc.z += f * os[u].z; acc.w += f * os[u].w;
         }
         m = mb;
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const int tok = row / Gq, hq = row % Gq;
-    uint16_t *op = (uint16_t *)p.out + ((size_t)(q0 + tok) * p.H + kvh * Gq + hq) * HD + d;
-    if constexpr (VEC == 4) {
-        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-        *(u16x4 *)op = u16x4{AttnT<T>::from_f32(acc[0] * inv), AttnT<T>::from_f32(acc[1] * inv),
-                             AttnT<T>::from_f32(acc[2] * inv), AttnT<T>::from_f32(acc[3] * inv)};
-    } else {
-        op[0] = AttnT<T>::from_f32(acc[0] * inv);
-    }
+    const int tok = r / p.Gq, hq = r - tok * p.Gq;
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    *(u32x2 *)((uint16_t *)p.out + ((size_t)(sq.q0 + tok) * p.H + kvh * p.Gq + hq) * HD + d) =
+        u32x2{AttnT<T>::pack2(acc.x * inv, acc.y * inv), AttnT<T>::pack2(acc.z * inv, acc.w * inv)};
 }
 
-#ifndef ATTN_TARGET_WGS
-#define ATTN_TARGET_WGS 512
-#endif
-// key slices per sequence: enough workgroups to fill the chip, at least 8 tiles of keys each
-static int attn_splits(int n_seqs, int kvh, int row_groups, int max_blocks, int block_size) {
-    const long base = (long)n_seqs * kvh * row_groups;
-    const long max_tiles = ((long)max_blocks * block_size + 31) / 32;
-    long s = (ATTN_TARGET_WGS + base - 1) / base;
-    if (s > max_tiles / 8) s = max_tiles / 8;
-    if (s > 64) s = 64;
-    return s < 1 ? 1 : (int)s;
+// ---- host side -----------------------------------------------------------------------------------------
+// Form of the kernel by the query rows of a sequence and the bytes that the keys can have
+struct AttnForm {
+    int rows;            // per unit
+    int fine, whole;
+};
+static int64_t attn_kv_bytes(int64_t n_seqs, int64_t max_keys, int kvh, int head_dim) {
+    return n_seqs * max_keys * kvh * head_dim * 4;
+}
+static AttnForm attn_form(int64_t rows, int64_t kv_bytes) {
+    // 17 to 32 rows: two row blocks per wavefront pay with a lot of keys (64 sequences of up to 2000, 338 MB,
+    // 5 queries of 4 heads: 62.6 against 68.3 us), the shared tiles with fewer (16 of up to 1000: 17.3 against 19.9)
+    const bool wide = rows > 16 && rows <= 32 && kv_bytes > (256LL << 20);
+    if (rows <= 16 || wide) return AttnForm{wide ? 32 : 16, ATTN_STREAM_FINE, ATTN_STREAM_WHOLE};
+    return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_WHOLE};
 }
 
 extern "C" size_t odsd_paged_attention_workspace_bytes(int32_t n_seqs, int32_t max_q_len, int32_t num_heads,
@@ -479,10 +786,64 @@ extern "C" size_t odsd_paged_attention_workspace_bytes(int32_t n_seqs, int32_t m
         return 0;
     const int64_t rows = (int64_t)max_q_len * (num_heads / num_kv_heads);
     if ((rows + 63) / 64 > 65535) return 0;
-    const int rg = (int)((rows + 63) / 64);
-    const int splits = attn_splits(n_seqs, num_kv_heads, rg, max_blocks, block_size);
-    if (splits == 1) return 256;
-    return odsd_round_up((size_t)n_seqs * num_kv_heads * rg * splits * 64 * (head_dim + 4) * sizeof(float), 256);
+    const int64_t max_keys = (int64_t)max_blocks * block_size;
+    const AttnForm f = attn_form(rows, attn_kv_bytes(n_seqs, max_keys, num_kv_heads, head_dim));
+    if (max_keys <= f.whole) return 256;                              // every unit stays whole: nothing to merge
+    return odsd_round_up((size_t)2 * ATTN_WG * f.rows * (head_dim + 4) * sizeof(float), 256);
+}
+
+// p: everything but Gq, n_wg, part; max_keys: no sequence has more
+static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_t rows, int64_t max_keys, bool aligned,
+                              void *workspace, size_t workspace_bytes, size_t need, hipStream_t st) {
+    const int64_t kv_bytes = attn_kv_bytes(p.n_seqs, max_keys, p.KVH, head_dim);
+    const AttnForm f = attn_form(rows, kv_bytes);
+    p.Gq = p.H / p.KVH;
+    const int64_t rg = (rows + f.rows - 1) / f.rows;
+    if (rg > 65535) return ODSD_ERR_UNSUPPORTED;                      // grid.y of the merge
+    const int64_t steps = (max_keys + f.fine - 1) / f.fine;
+    const bool merge = max_keys > f.whole;
+    const int64_t units = (int64_t)p.n_seqs * p.KVH * rg;
+    if (merge) {
+        if (!workspace) return ODSD_ERR_NULL;
+        if (!odsd_aligned16(workspace)) return ODSD_ERR_ALIGN;
+        if (workspace_bytes < need) return ODSD_ERR_WORKSPACE;
+        p.part = (float *)workspace;
+        p.n_wg = ATTN_WG;
+        p.whole = 0;
+    } else {
+        p.n_wg = (int)min(units, (int64_t)0x7fffffff);                // each a workgroup of its own, finished in place
+        p.whole = 1;
+    }
+    const unsigned grid = (unsigned)min((int64_t)p.n_wg, units * steps);
+    // (keys that fit the 256 MB memory-side cache may still be there from the call before)
+    p.v_once = kv_bytes > (100 << 20);
+    const dim3 mgrid((unsigned)(p.n_seqs * p.KVH), (unsigned)rg, (unsigned)((f.rows * head_dim + 1023) / 1024));
+#define ATTN_GO(T, HDV, RBV)                                                                     \
+    do {                                                                                         \
+        if (aligned) attn_stream_kernel<T, HDV, RBV, true><<<grid, 256, 0, st>>>(p);             \
+        else attn_stream_kernel<T, HDV, RBV, false><<<grid, 256, 0, st>>>(p);                    \
+        if (merge) attn_merge_kernel<T, HDV, 16 * RBV, ATTN_STREAM_FINE, ATTN_STREAM_COARSE><<<mgrid, 256, 0, st>>>(p);           \
+    } while (0)
+#define ATTN_GO_RB(T, HDV)                                                                       \
+    do {                                                                                         \
+        if (f.rows == 16) ATTN_GO(T, HDV, 1);                                                    \
+        else if (f.rows == 32) ATTN_GO(T, HDV, 2);                                               \
+        else {                                                                                   \
+            attn_tile_kernel<T, HDV><<<grid, 256, 0, st>>>(p);                                   \
+            if (merge) attn_merge_kernel<T, HDV, 64, ATTN_TILE_FINE, ATTN_TILE_COARSE><<<mgrid, 256, 0, st>>>(p);              \
+        }                                                                                        \
+    } while (0)
+    if (dtype == ODSD_DT_F16) {
+        if (head_dim == 128) ATTN_GO_RB(half_t, 128);
+        else ATTN_GO_RB(half_t, 64);
+    } else {
+        if (head_dim == 128) ATTN_GO_RB(__bf16, 128);
+        else ATTN_GO_RB(__bf16, 64);
+    }
+#undef ATTN_GO_RB
+#undef ATTN_GO
+    ODSD_CHECK_LAUNCH();
+    return ODSD_OK;
 }
 
 extern "C" int odsd_paged_attention(const void *q, const void *k_cache, const void *v_cache,
@@ -507,39 +868,11 @@ extern "C" int odsd_paged_attention(const void *q, const void *k_cache, const vo
     p.n_seqs = n_seqs; p.H = num_heads; p.KVH = num_kv_heads; p.max_blocks = max_blocks;
     p.block_size = block_size; p.num_slots = num_slots;
     p.scale_log2e = softmax_scale * 1.4426950408889634f;
-    const int64_t rows = (int64_t)max_q_len * (num_heads / num_kv_heads);
-    if ((rows + 63) / 64 > 65535) return ODSD_ERR_UNSUPPORTED;     // grid.y
-    const int rg = (int)((rows + 63) / 64);
-    p.splits = attn_splits(n_seqs, num_kv_heads, rg, max_blocks, block_size);
-    if (p.splits > 1) {
-        const size_t need = odsd_paged_attention_workspace_bytes(n_seqs, max_q_len, num_heads, num_kv_heads,
-                                                                 head_dim, block_size, max_blocks);
-        if (!workspace) return ODSD_ERR_NULL;
-        if (!odsd_aligned16(workspace)) return ODSD_ERR_ALIGN;
-        if (workspace_bytes < need) return ODSD_ERR_WORKSPACE;
-        p.part = (float *)workspace;
-    }
-    const dim3 grid((unsigned)(n_seqs * num_kv_heads), (unsigned)rg, (unsigned)p.splits);
-    const int mvec = p.splits > 4 ? 1 : 4;
-    const dim3 mgrid((unsigned)(n_seqs * num_kv_heads), (unsigned)rg, (unsigned)(64 / (256 * mvec / head_dim)));
-    hipStream_t st = (hipStream_t)stream;
-#define ATTN_GO(T, HDV)                                                              \
-    do {                                                                             \
-        if (block_size % 32 == 0) paged_attn_kernel<T, HDV, true><<<grid, 256, 0, st>>>(p);  \
-        else paged_attn_kernel<T, HDV, false><<<grid, 256, 0, st>>>(p);              \
-        if (p.splits > 4) paged_attn_merge_kernel<T, HDV, 8, 1><<<mgrid, 256, 0, st>>>(p);      \
-        else if (p.splits > 1) paged_attn_merge_kernel<T, HDV, 4, 4><<<mgrid, 256, 0, st>>>(p); \
-    } while (0)
-    if (dtype == ODSD_DT_F16) {
-        if (head_dim == 128) ATTN_GO(half_t, 128);
-        else ATTN_GO(half_t, 64);
-    } else {
-        if (head_dim == 128) ATTN_GO(__bf16, 128);
-        else ATTN_GO(__bf16, 64);
-    }
-#undef ATTN_GO
-    ODSD_CHECK_LAUNCH();
-    return ODSD_OK;
+    const size_t need = odsd_paged_attention_workspace_bytes(n_seqs, max_q_len, num_heads, num_kv_heads, head_dim,
+                                                             block_size, max_blocks);
+    return attn_stream_launch(p, dtype, head_dim, (int64_t)max_q_len * (num_heads / num_kv_heads),
+                              (int64_t)max_blocks * block_size, block_size % 32 == 0, workspace, workspace_bytes, need,
+                              (hipStream_t)stream);
 }
 
 // ---- variable-length (prefill) form ----------------------------------------------------------------
@@ -572,39 +905,13 @@ extern "C" int odsd_varlen_attention(const void *q, const void *k, const void *v
     p.scale_log2e = softmax_scale * 1.4426950408889634f;
     const int64_t rows = (int64_t)max_seqlen_q * (num_heads / num_kv_heads);
     if ((rows + 63) / 64 > 65535) return ODSD_ERR_UNSUPPORTED;     // grid.y
-    const int rg = (int)((rows + 63) / 64);
     if (odsd_attn_prefill_supported(p, head_dim, max_seqlen_q, max_seqlen_k)) {
         odsd_launch_attn_prefill(p, dtype, head_dim, max_seqlen_q, (hipStream_t)stream);
         ODSD_CHECK_LAUNCH();
         return ODSD_OK;
     }
-    p.splits = attn_splits(n_seqs, num_kv_heads, rg, p.max_blocks, 32);
-    if (p.splits > 1) {
-        const size_t need = odsd_varlen_attention_workspace_bytes(n_seqs, max_seqlen_q, max_seqlen_k, num_heads,
-                                                                  num_kv_heads, head_dim);
-        if (!workspace) return ODSD_ERR_NULL;
-        if (!odsd_aligned16(workspace)) return ODSD_ERR_ALIGN;
-        if (workspace_bytes < need) return ODSD_ERR_WORKSPACE;
-        p.part = (float *)workspace;
-    }
-    const dim3 grid((unsigned)(n_seqs * num_kv_heads), (unsigned)rg, (unsigned)p.splits);
-    const int mvec = p.splits > 4 ? 1 : 4;
-    const dim3 mgrid((unsigned)(n_seqs * num_kv_heads), (unsigned)rg, (unsigned)(64 / (256 * mvec / head_dim)));
-    hipStream_t st = (hipStream_t)stream;
-#define ATTN_GO(T, HDV)                                                              \
-    do {                                                                             \
-        paged_attn_kernel<T, HDV, true><<<grid, 256, 0, st>>>(p);                    \
-        if (p.splits > 4) paged_attn_merge_kernel<T, HDV, 8, 1><<<mgrid, 256, 0, st>>>(p);      \
-        else if (p.splits > 1) paged_attn_merge_kernel<T, HDV, 4, 4><<<mgrid, 256, 0, st>>>(p); \
-    } while (0)
-    if (dtype == ODSD_DT_F16) {
-        if (head_dim == 128) ATTN_GO(half_t, 128);
-        else ATTN_GO(half_t, 64);
-    } else {
-        if (head_dim == 128) ATTN_GO(__bf16, 128);
-        else ATTN_GO(__bf16, 64);
-    }
-#undef ATTN_GO
-    ODSD_CHECK_LAUNCH();
-    return ODSD_OK;
+    const size_t need = odsd_varlen_attention_workspace_bytes(n_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads,
+                                                              head_dim);
+    return attn_stream_launch(p, dtype, head_dim, rows, max_seqlen_k, true, workspace, workspace_bytes, need,
+                              (hipStream_t)stream);
 }

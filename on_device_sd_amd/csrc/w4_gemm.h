@@ -126,6 +126,8 @@ __device__ __forceinline__ float silu_f32(float g) { return g / (1.0f + __expf(-
 // s_waitcnt vmcnt(N) only (gfx9 encoding: vmcnt = bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
 #define ODSD_WAIT_VMCNT_LGKM0(N) \
     __builtin_amdgcn_s_waitcnt(((N) & 0xF) | (((N) >> 4) << 14) | (7 << 4) | (0x0 << 8))
+#define ODSD_WAIT_LGKM0() \
+    __builtin_amdgcn_s_waitcnt(0xF | (3 << 14) | (7 << 4) | (0x0 << 8))
 #define ODSD_WAIT_VMCNT(N) \
     __builtin_amdgcn_s_waitcnt(((N) & 0xF) | (((N) >> 4) << 14) | (7 << 4) | (0xF << 8))
 
@@ -163,3 +165,19 @@ __device__ __forceinline__ void dma16_to_lds(const global_char *base, uint32_t b
                  : "memory");   // m0 is a reserved register: the compiler sets it itself before every use
 }
 
+// The same with a 64-bit address per lane.
+__device__ __forceinline__ void dma16_from_to_lds(const char *from, lds_void *dst) {
+    const uint32_t m0v = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(m0v), "v"(from)
+                 : "memory");
+}
+// Nontemporal: data that is read once.
+__device__ __forceinline__ void dma16_from_to_lds_nt(const char *from, lds_void *dst) {
+    const uint32_t m0v = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt"
+                 :
+                 : "s"(m0v), "v"(from)
+                 : "memory");
+}

@@ -1,0 +1,91 @@
+"""The decode / verify attention kernels against the oracle where their division of the work can go wrong:
+16 / 17, 32 / 33 and 64 / 65 query rows per KV head, contexts around the 32-key tiles, the 128-key turns and
+the bounds below which nothing is split, pieces that begin and end inside a sequence, more than 64 sequences
+(the list is laid out 64 at a time), sequences without queries or without keys, and table widths that choose
+the two-row-block form."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(dev, dtype, H, KVH, HD, bs, seqs, pad_blocks=0, seed=0):
+    """seqs: (context_len, q_len) per sequence; returns what the call needs and the oracle's answer."""
+    g = torch.Generator().manual_seed(seed)
+    nbs = [max(1, -(-L // bs)) for L, _ in seqs]
+    perm = torch.randperm(sum(nbs) + 2, generator=g).tolist()
+    tables, at = [], 0
+    for nb in nbs:
+        tables.append(perm[at:at + nb]); at += nb
+    mb = max(nbs) + pad_blocks
+    bt = torch.tensor([t + [-1] * (mb - len(t)) for t in tables], dtype=torch.int32)
+    D = KVH * HD
+    kc = torch.randn((sum(nbs) + 2) * bs, D, generator=g).to(dtype)
+    vc = torch.randn((sum(nbs) + 2) * bs, D, generator=g).to(dtype)
+    qls = [q for _, q in seqs]
+    q = torch.randn(sum(qls), H, HD, generator=g)
+    q[::5] *= 5.0                                    # peaked rows: the reference point of the exponentials moves
+    q = q.to(dtype)
+    ref = orc.paged_attention(q, kc, vc, bt.tolist(), [L for L, _ in seqs], qls, KVH, bs, HD ** -0.5)
+    ctx = {"block_tables": bt.to(dev), "context_lens": torch.tensor([L for L, _ in seqs], dtype=torch.int32, device=dev),
+           "verify_query_lens": torch.tensor(qls, dtype=torch.int32, device=dev)}
+    return q.to(dev), kc.to(dev), vc.to(dev), ctx, max(qls), ref
+
+
+def _edges(lens, q):
+    return [(max(L, q), q) for L in lens]
+
+
+CASES = {
+    # rows per KV head either side of the forms' bounds
+    "rows16": (torch.bfloat16, 16, 1, 128, 32, _edges([600, 33, 1300], 1), 0),
+    "rows17": (torch.bfloat16, 17, 1, 128, 32, _edges([600, 33, 1300], 1), 0),
+    "rows33": (torch.float16, 11, 1, 64, 32, _edges([700, 5, 901], 3), 0),
+    "rows64": (torch.bfloat16, 16, 2, 128, 64, _edges([257, 1024, 255, 700], 8), 0),
+    "rows65": (torch.float16, 13, 1, 128, 16, _edges([900, 300], 5), 0),
+    # contexts at the tiles' and turns' edges, everything whole / something split
+    "whole512": (torch.bfloat16, 8, 2, 128, 32, _edges([1, 31, 32, 33, 127, 128, 129, 511, 512], 1), 0),
+    "split513": (torch.bfloat16, 8, 2, 128, 32, _edges([1, 31, 32, 33, 127, 128, 129, 512, 513], 1), 0),
+    "tile256": (torch.bfloat16, 16, 2, 128, 32, _edges([9, 31, 64, 65, 255, 256], 6), 0),
+    "tile257": (torch.bfloat16, 16, 2, 128, 32, _edges([9, 31, 64, 65, 255, 257], 6), 0),
+    # table entries of single keys (block sizes that are no multiple of 32)
+    "block16": (torch.float16, 8, 2, 128, 16, _edges([1000, 17, 129, 640], 1), 0),
+    "block3_hd64": (torch.bfloat16, 8, 4, 64, 3, _edges([800, 95, 1, 333], 2), 0),
+    # many sequences: the list is scanned 64 at a time; shares that span several of them
+    "seqs150": (torch.bfloat16, 4, 2, 64, 32, [(1 + (i * 37) % 900, 1) for i in range(150)], 0),
+    "seqs70_tile": (torch.float16, 16, 1, 64, 32, [(8 + (i * 53) % 700, 1 + i % 5) for i in range(70)], 0),
+    # no keys, no queries, fewer keys than queries
+    "holes": (torch.bfloat16, 8, 2, 128, 32, [(0, 2), (700, 1), (3, 4), (40, 0), (1200, 2), (0, 1)], 0),
+    "holes_tile": (torch.bfloat16, 24, 1, 128, 32, [(0, 2), (700, 3), (40, 0), (2, 3), (1200, 2), (0, 1)], 0),
+    # a table wide enough for 256 MB of keys: 17 to 32 rows in two row blocks
+    "wide": (torch.bfloat16, 32, 8, 128, 64, _edges([1500, 300, 129, 77], 5), 256),
+    "wide_block48": (torch.float16, 24, 8, 64, 48, _edges([1500, 300, 129, 77], 8), 800),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_paged_attention_shares(dev, name):
+    import on_device_sd_amd as odsd
+    dtype, H, KVH, HD, bs, seqs, pad = CASES[name]
+    print("attention shares", name, flush=True)
+    q, kc, vc, ctx, mq, ref = _case(dev, dtype, H, KVH, HD, bs, seqs, pad, seed=len(name))
+    out = odsd.paged_attention(q, kc, vc, ctx, KVH, bs, max_q_len=mq)
+    err = (out.float().cpu() - ref).abs()
+    # probabilities and output are rounded to the storage type: 2^-9 (bf16) or 2^-12 of values up to ~4
+    tol = 2e-2 if dtype == torch.bfloat16 else 3e-3
+    print(f"  max-abs error {err.max().item():.3e}", flush=True)
+    assert err.max().item() <= tol
+    assert torch.equal(out, odsd.paged_attention(q, kc, vc, ctx, KVH, bs, max_q_len=mq))
+
+
+def test_context_longer_than_its_table(dev):
+    """A context_len beyond the table's width (the positions past it read slot 0, as documented for entries
+    beyond the cache) stays inside the buffers: the bound that keeps units whole comes from the table."""
+    import on_device_sd_amd as odsd
+    q, kc, vc, ctx, mq, _ = _case(dev, torch.bfloat16, 8, 2, 128, 32, [(100, 1), (64, 1)])
+    ctx["context_lens"] = torch.tensor([100, 1500], dtype=torch.int32, device=dev)
+    out = odsd.paged_attention(q, kc, vc, ctx, 2, 32, max_q_len=mq)
+    assert torch.isfinite(out.float()).all()
