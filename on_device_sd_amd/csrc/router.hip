@@ -261,7 +261,7 @@ __device__ __forceinline__ int topk_token(const double *__restrict__ partial, co
                 }
             }
         }
-        const int we = wave_argmax(bk, be);   // the same in every lane
+        const int we = wave_best(bk, be);   // the same in every lane
         // the winner's logit sits in lane (we & 63), slot (we >> 6)
         double cand = lg[0];
 #pragma unroll
