@@ -63,12 +63,10 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
     __shared__ int32_t wsum[2][DISP ? WAVES : 1];        // DISP: per-wavefront totals (pairs of e, pairs below e)
 
     // workgroup -> (expert, row chunk, k split).  Hardware deals workgroups round-robin over
-    // the 8 XCDs.  With many token rows per expert (MB >= 6) consecutive logical ids are kept
-    // on one XCD so that an expert's rows stay in one L2; with few rows that locality is worth
-    // nothing and would leave an XCD idle for every expert without tokens, so the chunks of
-    // one expert are spread over all XCDs instead.
-    const int b = blockIdx.x;
-    const int L = MB >= 6 ? (b & 7) * p.wg_per_xcd + (b >> 3) : b;
+    // the 8 XCDs: the chunks of one expert are spread over all of them.  (Keeping an expert's rows
+    // in one L2 is worth nothing with few rows, and would leave an XCD idle for every expert
+    // without tokens.)
+    const int L = blockIdx.x;
     if (L >= p.n_wg) return;
     const int ks = L % p.KS;
     const int chunk = (L / p.KS) % p.nchunks;
@@ -656,7 +654,7 @@ struct ExpertsPlan {
     int WK_gu, WK_dn;  // wavefronts splitting K inside a workgroup (MB == 1 path)
     int KS;          // split of the down projection's reduction dimension across workgroups
     int PS_gu, PS_dn;  // prefill tile kernel: workgroups sharing the row passes of one tile
-    int tile;        // MB == 8: the 256 x 256 tile kernel instead of the streaming kernel
+    int tile;        // the tile kernel (experts_prefill.hip) instead of the streaming kernel
     int y_f16;       // down-projection outputs kept as fp16 (unsplit reduction) instead of fp32 partials
     int fused;       // whole-block calls run gate_up and down as one launch (experts_fused.hip)
     int S;           // fused: workgroups per expert = fp16 partial-sum slices of the down projection
@@ -674,16 +672,17 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     const long P = (long)s->T * s->K;
     const long mean_rows = (P + s->E - 1) / s->E;
     // token blocks per pass follow the mean number of rows per expert; an expert with more
-    // rows than one pass holds takes further passes over its weights.  Measured crossovers
-    // (uniform routing, Mixtral and Qwen3-235B expert shapes): 64-row passes win up to ~60 rows
-    // per expert, 128-row streaming passes up to ~130, the 256-row tile kernel beyond.
+    // rows than one pass holds takes further passes over its weights.  Crossover between the
+    // streaming kernel's 64-row passes and the tile kernel, whole layer on uniform routing, us,
+    // streaming / tile: Mixtral 25 rows per expert 180 / 202, 40 rows 200 / 215; Qwen3-30B 32 rows
+    // 113 / 129, 62 rows 164 (128-row passes) / 157.
     p.tile = 0;
     if (s->T <= 16) p.MB = 1;
     else if (s->T <= 32) p.MB = 2;
     else if (s->T <= 64) p.MB = 4;      // no expert can have more rows than a 64-row pass holds
     else if (mean_rows <= 16) p.MB = 2;
     else if (mean_rows <= 52) p.MB = 4;
-    else { p.MB = 8; p.tile = mean_rows > 136; }
+    else { p.MB = 8; p.tile = 1; }
     const long active = s->E < P ? s->E : P;       // upper bound of experts with rows
     const long slots = 512;                        // 256 CUs x 2 workgroups
     const int G_gu = s->H / ODSD_GROUP, G_dn = s->I / ODSD_GROUP;
@@ -701,10 +700,10 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
         const int gper = (G_dn + KS - 1) / KS;
         p.WK_dn = gper >= 8 ? 4 : (gper >= 4 ? 2 : 1);
     } else if (p.tile) {
-        // 256 x 256 tiles: with few experts the tiles alone do not fill 256 CUs.  First hand the
-        // row passes of one tile (it re-reads its weights per pass anyway) to several workgroups,
-        // then split the down projection's reduction.
-        const long mean_passes = (mean_rows + 255) / 256;
+        // 256 weight rows x up to 128 token rows, two workgroups per CU: with few experts the tiles
+        // alone do not fill 256 CUs.  First hand the row passes of one tile (it re-reads its weights
+        // per pass anyway) to several workgroups, then split the down projection's reduction.
+        const long mean_passes = (mean_rows + 127) / 128;
         const long tiles_gu = active * ((2 * s->I / 16 + 15) / 16), tiles_dn = active * ((s->H / 16 + 15) / 16);
         while (tiles_gu * p.PS_gu < slots && p.PS_gu * 2 <= mean_passes) p.PS_gu *= 2;
         while (tiles_dn * p.PS_dn < slots && p.PS_dn * 2 <= mean_passes) p.PS_dn *= 2;
@@ -712,17 +711,11 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
         while (tiles_dn * p.PS_dn * KS < slots && KS * 2 <= G_dn / 4 && KS < 16) KS *= 2;
         p.KS = KS;
     } else {
-        if (p.MB <= 4) {
-            const long wg_gu = active * ((2 * s->I / 16 + 15) / 16);
-            if (wg_gu < 4 * slots) p.NB = 2;
-        } else {
-            p.NB = 2;
-        }
+        const long wg_gu = active * ((2 * s->I / 16 + 15) / 16);
+        if (wg_gu < 4 * slots) p.NB = 2;
         const int nchunks_dn = (s->H / 16 + 4 * p.NB - 1) / (4 * p.NB);
-        // up to 4 workgroups per CU with at most 4 token blocks, 2 with 8
-        const long want = p.MB <= 4 ? 2 * slots : slots;
         int KS = 1;
-        while (KS * 2 <= G_dn / 2 && active * nchunks_dn * KS < want && KS < 16) KS *= 2;
+        while (KS * 2 <= G_dn / 2 && active * nchunks_dn * KS < 2 * slots && KS < 16) KS *= 2;   // up to 4 workgroups per CU
         p.KS = KS;
     }
     // every split must own at least one group
@@ -818,10 +811,8 @@ static void launch_gemm_plan(const ExpertsPlan &pl, GemmParams &gp, hipStream_t 
     } else if (pl.MB == 4) {
         if (pl.NB == 2) launch_gemm<2, 4, MODE, 2, 2, 1, false, 4>(gp, st);
         else launch_gemm<4, 4, MODE, 2, 2, 1, false, 2>(gp, st);
-    } else if (pl.tile) {
-        odsd_launch_gemm_prefill<MODE>(gp, st);
     } else {
-        launch_gemm<2, 8, MODE, 2, 2, 1, false, 2>(gp, st);
+        odsd_launch_gemm_prefill<MODE>(gp, st);
     }
 }
 

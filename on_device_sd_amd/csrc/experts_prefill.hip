@@ -1,41 +1,45 @@
-// Grouped W4A16 expert product for prefill-shaped calls (hundreds of token rows per expert).
+// Grouped W4A16 expert product for calls with more than 52 token rows per expert on average.
 //
-// With many rows per expert the product is bound by the matrix cores, and what matters is that
-// every packed weight is expanded to fp16 exactly once per expert and then shared.  One
-// workgroup of 8 wavefronts (two per SIMD, so that one's expansion and LDS traffic hide under
-// the other's MFMAs) owns a tile of 256 weight rows x BM token rows and walks the reduction
-// dimension in stages of 64 columns:
-//   * each wavefront expands 2 of the 16 weight tiles of the stage (int4 -> fp16 in registers,
-//     the same bit trick as the streaming kernel) and writes them to LDS in MFMA A-fragment
-//     order, [tile][32-column step][lane] x 16 bytes, which every wavefront reads back without
-//     bank conflicts;
-//   * the token rows of the stage arrive by asynchronous global -> LDS DMA (128 bytes per row,
-//     16-byte segments XOR-swizzled by (row >> 1) & 7, conflict-free for the B-fragment reads);
-//   * wavefront (wn, wm) multiplies weight tiles 4*wn..4*wn+3 (64 rows) with token blocks
-//     MBW*wm..MBW*wm+MBW-1 (16 rows each) on v_mfma_f32_16x16x32_f16: per 32-column step
-//     4 A fragments and MBW B fragments feed 4*MBW MFMAs (0.375 KiB of LDS reads per MFMA);
-//   * both LDS areas are double buffered; stage s+1 is produced while stage s is multiplied,
-//     one raw s_barrier per stage.
-// Epilogues are those of the streaming kernel (SiLU(gate)*up -> fp16 h, or fp32 y).
+// One workgroup of 4 wavefronts owns 256 weight rows x up to 128 token rows, two workgroups per CU;
+// a wavefront owns 64 of the weight rows and ALL of the token rows (2 x NM blocks of 32 x 32 on
+// v_mfma_f32_32x32x16_f16, NM = 1 .. 4 compiled separately, chosen per pass by the rows there are).
+//   * The weights never pass through LDS: a wavefront expands its own rows (int4 -> fp16 in
+//     registers, once per pass), straight from the packed tiles.  Two 16-row tiles make a 32-row A
+//     operand: lane l takes row l % 16 of tile (l >> 4) & 1, columns 32 j + 16 (l >> 5) + 8 i + 0..7
+//     for step (i, j), which is one word of the packed layout.  In gate_up the two tiles are a gate
+//     and an up block, so accumulator registers q and q + 8 of a lane are gate and up of one feature.
+//   * The token rows of a 128-column group arrive by asynchronous global -> LDS copies, 256 bytes a
+//     row, 16-byte segments XORed with the row (mod 16): no bank conflicts in the loop.  Double
+//     buffered, one barrier per group.
+//   * A group is 8 steps of 16 columns.  Each step's MFMAs run with the fragment reads and the
+//     expansion of the next step between them; the last step crosses the barrier and takes the first
+//     fragments of the next group.
+//   * fp16 results leave through LDS in whole rows of the tile.
+// Passes: an expert with more rows than a pass holds shares its 32-row blocks evenly between passes.
+//
+// What bounds it: before, weights went expanded through LDS (192 KB read + 64 KB written per 64-column
+// stage of 2048 matrix cycles, the 128 bytes per cycle that LDS has).  Now LDS reads are half of that,
+// and the matrix unit is busy 58 % of the time at the 1.6 GHz that the load takes the clock down to
+// (Qwen3-235B experts, T = 4096: gate_up 987 -> 830 us, 990 TFLOP/s, down 578 -> 425 us, 970 TFLOP/s;
+// the library's fp16 product of 8192^3 reaches 1160 on the same card).  At 62 rows per expert vector
+// and matrix instructions share the time (57 % and 49 % of the cycles with workgroups).
+// Variants: one wavefront per SIMD with 256 token rows per pass, i.e. half the expansion: 1.50 against
+// 1.45 ms for that layer (nothing runs under its barriers, prologue and epilogue).
 //
 // Replaces the same reference code as the streaming kernel: the three F.linear calls of
 // expert_forward_with_weights (demo/src/layers/mlp.py:227-230) inside the per-expert loop of
 // demo/src/model/qwen3_runner.py:303-380.
 #include "w4_gemm.h"
 
-template <int MODE, int MBW>
-__global__ __launch_bounds__(512, 2) void w4_gemm_prefill_kernel(const GemmParams p) {
-    constexpr int BM = 2 * 16 * MBW;           // token rows per pass
-    constexpr int XPT = BM * 8 / 512;          // 16-byte pieces of one token-row stage per thread
-    static_assert((BM * 8) % 512 == 0, "token-row pieces must divide among the threads");
-    constexpr int XS_STAGE = BM * 128;         // bytes: BM rows x 64 fp16
-    constexpr int WS_STAGE = 16 * 2 * 1024;    // bytes: 16 tiles x 2 steps x 64 lanes x 16 B
-    // one object per buffer: the compiler must see that the DMA into one buffer cannot alias
-    // the reads of the other, or it drains every outstanding load before each LDS read
-    __shared__ __attribute__((aligned(16))) char xs0[XS_STAGE];
-    __shared__ __attribute__((aligned(16))) char xs1[XS_STAGE];
-    __shared__ __attribute__((aligned(16))) char ws0[WS_STAGE];
-    __shared__ __attribute__((aligned(16))) char ws1[WS_STAGE];
+#include <type_traits>
+
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void w4_gemm_prefill_kernel(const GemmParams p) {
+    constexpr int MAXNM = 4;                   // 32-row token blocks per pass
+    constexpr int XS_BUF = MAXNM * 32 * 256;   // one group of the token rows
+    __shared__ __attribute__((aligned(16))) char xs[2 * XS_BUF];
 
     // consecutive logical ids stay on one XCD: the row tiles of one expert share its token rows
     const int b = blockIdx.x;
@@ -54,270 +58,203 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_prefill_kernel(const GemmParam
     const uint64_t t_present = trow[0];
     const uint64_t t_q = MODE == 0 ? trow[0] : trow[2], t_sz = MODE == 0 ? trow[1] : trow[3];
     if (M_e == 0 || t_present == 0) return;
-    const global_char *qp_c = (const global_char *)t_q;
-    const global_char *szp_c = (const global_char *)t_sz;
     const global_char *src_c = (const global_char *)p.src;
-    // gate_up reads its weights through buffer loads: resource in scalar registers, constant
-    // per-lane offset, the group as the scalar offset -- no vector instruction per address
-    const __amdgpu_buffer_rsrc_t rsrc_q = __builtin_amdgcn_make_buffer_rsrc((void *)(uintptr_t)qp_c, 0, p.NBLK * p.G * 1024, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrc_sz = __builtin_amdgcn_make_buffer_rsrc((void *)(uintptr_t)szp_c, 0, p.NBLK * p.G * 64, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_q = __builtin_amdgcn_make_buffer_rsrc((void *)(uintptr_t)t_q, 0, p.NBLK * p.G * 1024, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_sz = __builtin_amdgcn_make_buffer_rsrc((void *)(uintptr_t)t_sz, 0, p.NBLK * p.G * 64, 0x00020000);
 
     const DequantConsts dc = dequant_consts();
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int r = lane & 15, kq = lane >> 4;
-    const int wn = wave & 3, wm = wave >> 2;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, kh = lane >> 5;
     const int G = p.G;
-    const int NST = 2 * G;                     // stages of 64 columns
     const int g_begin = ks * p.gper, g_end = min(G, g_begin + p.gper);   // this K slice (never empty)
 
-    // expansion duty: tiles 2*wave and 2*wave+1 of this row chunk (clamped, never out of range)
+    // this wavefront's tiles 4 wave .. 4 wave + 3 of the chunk: all inside the matrix or none
+    // (its row blocks are a multiple of 8); a wavefront without tiles works on tile 0 and stores nothing
+    const int cblk0 = chunk * 16 + 4 * wave;
+    const bool blk_ok = cblk0 < p.NBLK;
     uint32_t wq_off[2], sz_off[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        uint32_t blk = chunk * 16 + 2 * wave + i;
-        if (blk >= (uint32_t)p.NBLK) blk = 0;
-        wq_off[i] = (blk * G * 64 + lane) * 16u;
-        sz_off[i] = (blk * G * 16 + r) * 4u;
+    for (int rb = 0; rb < 2; ++rb) {
+        const uint32_t blk = (blk_ok ? cblk0 : 0) + 2 * rb + ((lane >> 4) & 1);
+        wq_off[rb] = (blk * G * 64 + (lane & 15) + 32 * kh) * 16u;
+        sz_off[rb] = (blk * G * 16 + (lane & 15)) * 4u;
     }
-    // product duty: tiles 4*wn .. 4*wn+3
-    const int cblk0 = chunk * 16 + 4 * wn;
-    bool blk_ok[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) blk_ok[i] = cblk0 + i < p.NBLK;
+    // this lane's B fragment of step s = (i, j) = (s & 1, s >> 1): token row n, segment 4 j + 2 kh + i
+    const uint32_t frag0 = (uint32_t)(n * 256 + (((2 * kh) ^ (n & 15)) << 4));
+    auto frag = [&](const int s) { return frag0 ^ (uint32_t)((4 * (s >> 1) + (s & 1)) << 4); };
 
-    for (int m0 = ps * BM; m0 < M_e; m0 += p.PS * BM) {
-        const int mcnt = min(M_e - m0, BM);
-        const int mrows_w = max(0, min(mcnt - wm * 16 * MBW, 16 * MBW));   // rows of this M half
-        const int nmb = (mrows_w + 15) >> 4;
+    const int nblk = (M_e + 31) >> 5;                   // 32-row token blocks of this expert
+    const int npass = (nblk + MAXNM - 1) / MAXNM;
 
-        // token-row pieces of this thread: piece = i*512 + tid -> row = piece/8, segment = piece%8,
-        // fetched from source segment  segment ^ ((row >> 1) & 7)
-        uint32_t st_off[XPT];
+    auto run_pass = [&](auto nm_c, const int m0, const int mcnt) {
+        constexpr int NM = decltype(nm_c)::value;
+        // copies of this wavefront: token rows 16 i + 4 wave + lane / 16, source segment (lane % 16) ^ (row % 16);
+        // rows past the expert's last one copy its first: what they feed is never stored
+        uint32_t st_off[2 * NM];
 #pragma unroll
-        for (int i = 0; i < XPT; ++i) {
-            const int piece = i * 512 + tid;
-            const int row = piece >> 3, seg = piece & 7;
+        for (int i = 0; i < 2 * NM; ++i) {
+            const int row = 16 * i + 4 * wave + (lane >> 4);
             const int slot = base + m0 + (row < mcnt ? row : 0);
             const int srow = p.rowmap ? p.rowmap[slot] : slot;
-            st_off[i] = ((uint32_t)srow * (uint32_t)p.src_ld + (seg ^ ((row >> 1) & 7)) * 8) * 2u;
+            st_off[i] = ((uint32_t)srow * (uint32_t)p.src_ld + ((lane & 15) ^ (row & 15)) * 8) * 2u;
         }
-
-        float4_t acc[4][MBW];
+        float16_t acc[2][NM];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-            for (int m = 0; m < MBW; ++m) acc[i][m] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-        uint4_t wq[2][2];      // [ring slot = group parity][duty tile]
-        uint32_t wsz[2][2];
-
-        auto load_w = [&](int slot, int g) {
-            const uint32_t gc = (uint32_t)min(g, G - 1);
+            for (int m = 0; m < NM; ++m)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                if (MODE == 0) {
-                    wq[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_q, (int)wq_off[i], (int)(gc * 1024u), 2 /* nt */);
-                    wsz[slot][i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_sz, (int)sz_off[i], (int)(gc * 64u), 0);
-                } else {
-                    // (the down projection measured 14 % slower with buffer loads)
-                    wq[slot][i] = __builtin_nontemporal_load((const global_u4 *)(qp_c + (wq_off[i] + gc * 1024u)));
-                    wsz[slot][i] = *(const global_u32 *)(szp_c + (sz_off[i] + gc * 64u));
-                }
+                for (int i = 0; i < 16; ++i) acc[rb][m][i] = 0.0f;
+
+        // Packed weights in registers: those of the group at hand (wq) and F groups on their way, fetched
+        // behind the copies of the token rows that have to land before them, so that the wait for those
+        // copies leaves the youngest in flight.  (F == 2 with four blocks of rows spills.)
+        constexpr int F = NM <= 3 ? 2 : 1;
+        uint4_t wq[2][2], wq_f[F][2][2];       // [slot = group % F][row block][i], words j = 0..3
+        uint32_t wsz_f[F][2];
+        auto load_w = [&](auto slot_c, const int g) {
+            constexpr int slot = decltype(slot_c)::value % F;
+            const int gc = min(g, g_end - 1);
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) {
+                wq_f[slot][rb][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_q, (int)wq_off[rb], gc * 1024, 2 /* nt */);
+                wq_f[slot][rb][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_q, (int)wq_off[rb] + 256, gc * 1024, 2 /* nt */);
+                wsz_f[slot][rb] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_sz, (int)sz_off[rb], gc * 64, 0);
             }
         };
-        auto dma_x = [&](char *xs, int st) {
-            const uint32_t sc = (uint32_t)min(st, NST - 1);
+        auto dma_piece = [&](const uint32_t buf, const int g, const int i) {
+            lds_void *dst = (lds_void *)(xs + buf + (16 * i + 4 * wave) * 256);
+            dma16_to_lds(src_c + (size_t)g * (ODSD_GROUP * 2u), st_off[i], dst);
+        };
+        half8_t a[2][2], bx[2][NM];  // [step parity]
+        DequantPrep pr[2];
+        auto expand = [&](const int par, const int s) {
 #pragma unroll
-            for (int i = 0; i < XPT; ++i) {
-                // piece i covers rows 64 i .. 64 i + 63 of the pass: nothing to fetch past its last row
-                if (i * 64 < mcnt) {
-                    lds_void *dst = (lds_void *)(xs + (i * 512 + wave * 64) * 16);
-                    dma16_to_lds(src_c, st_off[i] + sc * 128u, dst);
-                }
+            for (int rb = 0; rb < 2; ++rb) a[par][rb] = dequant_word(dc, pr[rb], wq[rb][s & 1][s >> 1]);
+        };
+        // group g's weights have landed and become those at hand; past the slice's end their scale is zero
+        auto take_w = [&](auto slot_c, const int g) {
+            constexpr int slot = decltype(slot_c)::value % F;
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) {
+                wq[rb][0] = wq_f[slot][rb][0];
+                wq[rb][1] = wq_f[slot][rb][1];
+                pr[rb] = dequant_prep(F == 1 || g < g_end ? wsz_f[slot][rb] : 0u);
             }
         };
-        // expand the two 32-column steps `half` (0: words x,y  1: words z,w) of ring slot `slot`
-        // into weight buffer `buf`
-        auto expand = [&](int slot, int half, char *ws) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const DequantPrep pr = dequant_prep(wsz[slot][i]);
-                const uint32_t w0 = half ? wq[slot][i].z : wq[slot][i].x;
-                const uint32_t w1 = half ? wq[slot][i].w : wq[slot][i].y;
-                char *dst = ws + (((2 * wave + i) * 2) * 64 + lane) * 16;
-                *(half8_t *)dst = dequant_word(dc, pr, w0);
-                *(half8_t *)(dst + 1024) = dequant_word(dc, pr, w1);
-            }
-        };
-        // one quarter of expand(): duty tile i, word w of the half
-        auto expand_piece = [&](int slot, int half, char *ws, int i, int w) {
-            const DequantPrep pr = dequant_prep(wsz[slot][i]);
-            const uint32_t word = half ? (w ? wq[slot][i].w : wq[slot][i].z) : (w ? wq[slot][i].y : wq[slot][i].x);
-            char *dst = ws + (((2 * wave + i) * 2) * 64 + lane) * 16 + w * 1024;
-            *(half8_t *)dst = dequant_word(dc, pr, word);
-        };
-        // multiply stage (xs, ws) and, in the same scheduling region, expand the next stage's
-        // weights (ring slot eslot, half ehalf) into ews, so that the vector work and the LDS
-        // writes of the expansion sit between the MFMAs instead of in front of them
-        auto mma_stage = [&](const char *xs, const char *ws, int eslot, int ehalf, char *ews) {
-            if (nmb == MBW) {
-                // Every token block of this wavefront is in use: branch-free and software
-                // pipelined.  The stage is cut into units of 2 token blocks x one 32-column
-                // step.  The LDS reads of unit u+1 are issued, then (behind a scheduling fence
-                // that keeps them there) the 8 MFMAs of unit u, so the read latency hides under
-                // the matrix work of the same wavefront.  The expansion of the next stage's
-                // weights is cut into 4 pieces that ride along with the first 4 units.
-                static_assert(MBW % 2 == 0, "token blocks are processed in pairs");
-                constexpr int UPJ = MBW / 2;           // units per 32-column step
-                auto read_a = [&](int jj, half8_t (&a)[4]) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        a[i] = *(const half8_t *)(ws + ((((4 * wn + i) * 2) + jj) * 64 + lane) * 16);
-                };
-                auto read_b = [&](int jj, int m, half8_t &bx) {
-                    const int row = wm * 16 * MBW + m * 16 + r;
-                    const int seg = (4 * jj + kq) ^ ((row >> 1) & 7);
-                    bx = *(const half8_t *)(xs + row * 128 + seg * 16);
-                };
-                half8_t a_cur[4], a_nxt[4], b_cur[2], b_nxt[2];
-                read_a(0, a_cur);
-                read_b(0, 0, b_cur[0]);
-                read_b(0, 1, b_cur[1]);
-#define PF_UNIT(U)                                                                                      \
-    {                                                                                                   \
-        constexpr int mp = (U) % UPJ;                                                                   \
-        if ((U) + 1 < 2 * UPJ) {                                                                        \
-            constexpr int jn = ((U) + 1) / UPJ, mn = ((U) + 1) % UPJ;                                   \
-            if (mn == 0) read_a(jn, a_nxt);                                                             \
-            read_b(jn, 2 * mn, b_nxt[0]);                                                               \
-            read_b(jn, 2 * mn + 1, b_nxt[1]);                                                           \
-        }                                                                                               \
-        __builtin_amdgcn_sched_barrier(0);                                                              \
-        if ((U) < 4) expand_piece(eslot, ehalf, ews, (U) >> 1, (U) & 1);                                \
-        _Pragma("unroll") for (int q = 0; q < 2; ++q)                                                   \
-        _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                   \
-            acc[i][2 * mp + q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_cur[i], b_cur[q], acc[i][2 * mp + q], 0, 0, 0);                       \
-        __builtin_amdgcn_sched_barrier(0);                                                              \
-        if ((U) + 1 < 2 * UPJ) {                                                                        \
-            if (((U) + 1) % UPJ == 0) {                                                                 \
-                _Pragma("unroll") for (int i = 0; i < 4; ++i) a_cur[i] = a_nxt[i];                      \
-            }                                                                                           \
-            b_cur[0] = b_nxt[0];                                                                        \
-            b_cur[1] = b_nxt[1];                                                                        \
-        }                                                                                               \
-    }
-                static_assert(MBW == 8, "the unit list below is written out for 8 token blocks");
-                PF_UNIT(0) PF_UNIT(1) PF_UNIT(2) PF_UNIT(3)
-                PF_UNIT(4) PF_UNIT(5) PF_UNIT(6) PF_UNIT(7)
-#undef PF_UNIT
-            } else {
-                expand(eslot, ehalf, ews);
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj) {
-                    half8_t a[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        a[i] = *(const half8_t *)(ws + ((((4 * wn + i) * 2) + jj) * 64 + lane) * 16);
-#pragma unroll
-                    for (int m = 0; m < MBW; ++m) {
-                        if (m < nmb) {
-                            const int row = wm * 16 * MBW + m * 16 + r;
-                            const int seg = (4 * jj + kq) ^ ((row >> 1) & 7);
-                            const half8_t bx = *(const half8_t *)(xs + row * 128 + seg * 16);
-#pragma unroll
-                            for (int i = 0; i < 4; ++i)
-                                acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], bx, acc[i][m], 0, 0, 0);
-                        }
-                    }
-                }
-            }
-        };
+        using Slot0 = std::integral_constant<int, 0>;
+        using Slot1 = std::integral_constant<int, 1>;
 
-        // prologue: stage 0 in place
-        __builtin_amdgcn_s_barrier();          // the previous pass is done with both LDS areas
-        dma_x(xs0, 2 * g_begin);
-        load_w(0, g_begin);
-        load_w(1, g_begin + 1);
+        __builtin_amdgcn_s_barrier();          // the previous pass is done with the token rows
+#pragma unroll
+        for (int i = 0; i < 2 * NM; ++i) dma_piece(0, g_begin, i);
+        load_w(Slot0{}, g_begin);
+        if (F == 2) load_w(Slot1{}, g_begin + 1);
         __builtin_amdgcn_sched_barrier(0);
-        expand(0, 0, ws0);
-        __builtin_amdgcn_sched_barrier(0);
-        ODSD_WAIT_VMCNT_LGKM0(4);              // all but the second group's 4 loads have landed
+        ODSD_WAIT_VMCNT_LGKM0((F - 1) * 6);
         __builtin_amdgcn_s_barrier();
+        uint32_t cur = 0;                      // byte offset of the buffer of the group at hand
+#pragma unroll
+        for (int m = 0; m < NM; ++m) bx[0][m] = *(const half8_t *)(xs + frag(0) + m * 8192);
+        take_w(Slot0{}, g_begin);
+        expand(0, 0);
 
-        // two groups (four stages) per trip: ring slots and buffers are compile-time constants
-        for (int g = g_begin; g < g_end; g += 2) {
-            // stage 4k   : group g, first half.   produce (g, second half) -> x buf 1, w buf 1
-            dma_x(xs1, 2 * g + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            mma_stage(xs0, ws0, 0, 1, ws1);
-            __builtin_amdgcn_sched_barrier(0);
-            load_w(0, g + 2);                  // slot 0 is fully expanded
-            __builtin_amdgcn_sched_barrier(0);
-            ODSD_WAIT_VMCNT_LGKM0(4);          // the DMA is older than the 4 refill loads
-            __builtin_amdgcn_s_barrier();
-            // stage 4k+1 : group g, second half.  produce (g+1, first half) -> x buf 0, w buf 0
-            dma_x(xs0, 2 * g + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            mma_stage(xs1, ws1, 1, 0, ws0);
-            __builtin_amdgcn_sched_barrier(0);
-            ODSD_WAIT_VMCNT_LGKM0(0);
-            __builtin_amdgcn_s_barrier();
-            if (g + 1 >= g_end) break;
-            // stage 4k+2 : group g+1, first half.  produce (g+1, second half) -> buffers 1
-            dma_x(xs1, 2 * g + 3);
-            __builtin_amdgcn_sched_barrier(0);
-            mma_stage(xs0, ws0, 1, 1, ws1);
-            __builtin_amdgcn_sched_barrier(0);
-            load_w(1, g + 3);
-            __builtin_amdgcn_sched_barrier(0);
-            ODSD_WAIT_VMCNT_LGKM0(4);
-            __builtin_amdgcn_s_barrier();
-            // stage 4k+3 : group g+1, second half.  produce (g+2, first half) -> buffers 0
-            dma_x(xs0, 2 * g + 4);
-            __builtin_amdgcn_sched_barrier(0);
-            mma_stage(xs1, ws1, 0, 0, ws0);
-            __builtin_amdgcn_sched_barrier(0);
-            ODSD_WAIT_VMCNT_LGKM0(0);
-            __builtin_amdgcn_s_barrier();
-        }
-
-        // epilogue: lane holds rows 4*kq..4*kq+3 of each 16-row tile, token column r
+        // One group.  Every load is issued whatever follows (past the slice's end: its last group again).
+        auto group = [&](auto slot_c, const int g) {
+            constexpr int slot = decltype(slot_c)::value;
+            const char *xb = xs + cur;
+            const int gx = min(g + 1, g_end - 1);
 #pragma unroll
-        for (int m = 0; m < MBW; ++m) {
-            const int row = wm * 16 * MBW + m * 16 + r;
-            if (m < nmb && row < mcnt) {
-                const size_t slot = (size_t)(base + m0 + row);
-                if (MODE == 0) {
-#pragma unroll
-                    for (int i = 0; i < 4; i += 2) {
-                        if (blk_ok[i]) {
-                            const float4_t gt = acc[i][m], up = acc[i + 1][m];
-                            half4_t h;
-                            h.x = f32_to_f16_sat(silu_f32(gt.x) * up.x);
-                            h.y = f32_to_f16_sat(silu_f32(gt.y) * up.y);
-                            h.z = f32_to_f16_sat(silu_f32(gt.z) * up.z);
-                            h.w = f32_to_f16_sat(silu_f32(gt.w) * up.w);
-                            const int feat = ((cblk0 + i) >> 1) * 16 + kq * 4;
-                            *(half4_t *)(p.h16 + slot * p.ldo + feat) = h;
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if (blk_ok[i]) {
-                            const int n = (cblk0 + i) * 16 + kq * 4;
-                            if (p.y_f16) {
-                                const float4_t v = acc[i][m];
-                                *(half4_t *)((half_t *)p.y + ((size_t)ks * p.P + slot) * p.ldo + n) =
-                                    half4_t{f32_to_f16_sat(v.x), f32_to_f16_sat(v.y), f32_to_f16_sat(v.z), f32_to_f16_sat(v.w)};
-                            } else {
-                                *(float4_t *)(p.y + ((size_t)ks * p.P + slot) * p.ldo + n) = acc[i][m];
-                            }
-                        }
-                    }
+            for (int s = 0; s < 8; ++s) {
+                const int par = s & 1;
+                __builtin_amdgcn_sched_barrier(0);
+                if (s == 7) {
+                    // into the next group: this wavefront's copies and its next weights have landed, its
+                    // reads of this group's rows are complete; then the same of every wavefront
+                    ODSD_WAIT_VMCNT_LGKM0((F - 1) * 6);
+                    __builtin_amdgcn_s_barrier();
+                    xb = xs + (cur ^ XS_BUF);
                 }
+#pragma unroll
+                for (int m = 0; m < NM; ++m) bx[par ^ 1][m] = *(const half8_t *)(xb + frag((s + 1) & 7) + m * 8192);
+                if (s == 7) take_w(std::integral_constant<int, slot ^ 1>{}, g + 1);
+                expand(par ^ 1, (s + 1) & 7);
+#pragma unroll
+                for (int m = 0; m < NM; ++m)
+#pragma unroll
+                    for (int rb = 0; rb < 2; ++rb)
+                        acc[rb][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[par][rb], bx[par][m], acc[rb][m], 0, 0, 0);
+                constexpr int NV = (27 + 2 * NM - 1) / (2 * NM);
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // LDS read
+                    __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);    // vector
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);
+                }
+                // the next group's copies, two a step (into the buffer of the group before this one); the
+                // weights of the next group in front of them (F == 1), or those of the group after it behind them
+                if (s <= NM) __builtin_amdgcn_sched_barrier(0);
+                if (F == 1 && s == 0) load_w(Slot0{}, g + 1);
+                if (s < NM) {
+                    dma_piece(cur ^ XS_BUF, gx, 2 * s);
+                    dma_piece(cur ^ XS_BUF, gx, 2 * s + 1);
+                }
+                if (F == 2 && s == NM) load_w(slot_c, g + 2);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            cur ^= XS_BUF;
+        };
+        for (int g = g_begin; g < g_end; g += F) {
+            group(Slot0{}, g);
+            if (F == 2) group(Slot1{}, g + 1);
+        }
+        ODSD_WAIT_VMCNT_LGKM0(0);              // the copies that nobody waited for must not land in the results
+
+        // epilogue: register 4 q + u of a lane is row 8 q + 4 kh + u of the 32-row block, token n
+        // The results (fp16 in both modes: this plan keeps fp16 sums) go through LDS (16-byte pieces of a token's row XORed with the token), so that
+        // they leave in whole rows of the tile
+        constexpr int OUTB = MODE == 0 ? 256 : 512;    // bytes of one token's results in this tile
+        constexpr int PIECES = OUTB / 16;
+        __builtin_amdgcn_s_barrier();                  // every wavefront has read its last fragments
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const int row = m * 32 + n;
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+                for (int q = 0; q < (MODE == 0 ? 2 : 4); ++q) {
+                    half4_t h;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        h[u] = f32_to_f16_sat(MODE == 0 ? silu_f32(acc[rb][m][4 * q + u]) * acc[rb][m][(8 + 4 * q + u) & 15] : acc[rb][m][4 * q + u]);
+                    const int piece = MODE == 0 ? 4 * wave + 2 * rb + q : 8 * wave + 4 * rb + q;
+                    *(half4_t *)(xs + row * OUTB + ((piece ^ (n & (PIECES - 1))) << 4) + 8 * kh) = h;
+                }
+        }
+        __syncthreads();
+        char *out = MODE == 0 ? (char *)p.h16 : (char *)p.y + (size_t)ks * p.P * p.ldo * 2;
+        const int width = min(OUTB, (int)(p.ldo * 2 - chunk * OUTB));     // the matrix may end inside the tile
+        const int piece = lane & (PIECES - 1), sub = lane / PIECES;
+        for (int row = wave * (64 / PIECES) + sub; row < mcnt; row += 256 / PIECES) {
+            const uint4_t v = *(const uint4_t *)(xs + row * OUTB + ((piece ^ (row & (PIECES - 1))) << 4));
+            if (piece * 16 < width)
+                *(uint4_t *)(out + (size_t)(base + m0 + row) * p.ldo * 2 + (size_t)chunk * OUTB + piece * 16) = v;
+        }
+        __syncthreads();                               // the next pass copies into the same memory
+    };
+
+    for (int q = ps; q < npass; q += p.PS) {
+        const int per = nblk / npass, rest = nblk % npass;       // the first `rest` passes take one block more
+        const int b0 = q * per + min(q, rest), nm = per + (q < rest);
+        const int m0 = b0 * 32, mcnt = min(M_e - m0, nm * 32);
+        switch (nm) {
+#define PASS(N) case N: run_pass(std::integral_constant<int, N>{}, m0, mcnt); break;
+            PASS(1) PASS(2) PASS(3) PASS(4)
+#undef PASS
         }
     }
 }
@@ -328,8 +265,7 @@ void odsd_launch_gemm_prefill(GemmParams &gp, hipStream_t st) {
     if (gp.PS < 1) gp.PS = 1;
     gp.n_wg = gp.E * gp.nchunks * gp.KS * gp.PS;
     gp.wg_per_xcd = (gp.n_wg + 7) / 8;
-    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_gemm_prefill_kernel<MODE, 8>),
-                gp.wg_per_xcd * 8, 512, st, gp);
+    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_gemm_prefill_kernel<MODE>), gp.wg_per_xcd * 8, 256, st, gp);
 }
 
 template void odsd_launch_gemm_prefill<0>(GemmParams &, hipStream_t);
