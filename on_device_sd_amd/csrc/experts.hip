@@ -14,7 +14,7 @@
 //                    (summed in a fixed order by the combine, so split-K stays deterministic)
 //
 // Token rows of one expert are shared by the 4 wavefronts of a workgroup through LDS
-// (double buffered, one 128-column group per stage, loads for the next stage in flight
+// (two or three buffers, one 128-column group per stage, loads for the next stages in flight
 // while the current one is multiplied).
 //
 // Replaces: expert_forward_with_weights (demo/src/layers/mlp.py:227-230) inside the
@@ -31,7 +31,7 @@
 // DIRECT == true  (MB == 1): token rows are never staged; each wavefront reads its B
 //       fragments straight from L1/L2 as part of the ring slot -- no barrier in the loop.
 // DIRECT == false (WK == 1): token rows go global -> LDS by asynchronous DMA loads
-//       (global_load_lds, no registers), double buffered, 16-byte segments XOR-swizzled
+//       (global_load_lds, no registers), two or three buffers, 16-byte segments XOR-swizzled
 //       by the row so that the B-fragment reads are bank-conflict free; one raw s_barrier
 //       per group, preceded by a vmcnt wait that leaves the newest loads in flight.
 // DISP  (gate_up only) the workgroup dispatches for itself: it scans the [P] expert ids (P <= 4
@@ -53,7 +53,13 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
     constexpr int RING_TRIPS = DEPTH == 2 ? 4 : 1;
     constexpr int XPT = DIRECT ? 1 : 4 * MB / WAVES;   // 16-byte pieces of a token-row chunk per thread
     constexpr int ROWS_PER_PIECE = 4 * WAVES;     // rows covered by one piece index (16 threads per row)
-    constexpr int XS_BYTES = 2 * 16 * MB * 256;
+    // Token-row buffers: copies of the rows run NXB - 1 groups ahead.  Waiting for a group's rows also waits
+    // for every load issued before them, so with two buffers a ring of any depth has only its youngest slot
+    // in flight across a barrier; a third buffer makes that two (down projection, I = 1536, 8 tokens:
+    // 35.2 -> 31.7 us).  For one token block only: with more copies per group the waits for the ring, which do
+    // not know of the copies, take the second slot away again (MB = 2 equal, MB = 4 5 to 8 % slower).
+    constexpr int NXB = !DIRECT && MB == 1 && DEPTH == 3 ? 3 : 2;
+    constexpr int XS_BYTES = NXB * 16 * MB * 256;
     constexpr int RED_FLOATS = WK > 1 ? (WK - 1) * RSUB * 64 * NB * 4 : 1;
     // one LDS object: token-row buffers (LDS path) or the K-part reduction area (direct path)
     constexpr int LDS_BYTES = DIRECT ? (WK > 1 ? RED_FLOATS * 4 : 16) : XS_BYTES;
@@ -199,7 +205,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
     for (int m0 = 0; m0 < M_e; m0 += 16 * MB) {
         const int mcnt = min(M_e - m0, 16 * MB);
         const int nmb = (mcnt + 15) >> 4;
-        const int mcnt_s = DIRECT ? mcnt : scalar_int(mcnt);
+        const int mcnt_s = MB == 1 ? mcnt : scalar_int(mcnt);
         if (DISP && m0 > 0) scan_rows(m0, false);   // the tokens of this pass's rows
 
         // byte offsets of the token rows this thread fetches
@@ -260,7 +266,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
             for (int i = 0; i < XPT; ++i) {
                 // piece i covers ROWS_PER_PIECE rows from row ROWS_PER_PIECE * i on: nothing to
                 // fetch for a token block without rows
-                if (i * ROWS_PER_PIECE < mcnt_s) {
+                if (MB == 1 || i * ROWS_PER_PIECE < mcnt_s) {
                     lds_void *dst = (lds_void *)(xs_raw + buf * (16 * MB * 256) + (i * 64 * WAVES + wave * 64) * 16);
                     dma16_to_lds(xg, st_off[i], dst);
                 }
@@ -270,6 +276,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
         if (!DIRECT) {
             __builtin_amdgcn_s_barrier();   // the previous pass is done with xs
             dma_x(0, g_begin);
+            if (NXB == 3) dma_x(1, g_begin + 1);
         }
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
@@ -277,7 +284,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
             if (DIRECT) load_xd(d, g_begin + d);
         }
         if (!DIRECT) {
-            // x(g_begin) has landed once at most the loads issued after it are outstanding
+            // the token rows have landed once at most the loads issued after them are outstanding
             ODSD_WAIT_VMCNT(DEPTH * 2 * NB);
             __builtin_amdgcn_s_barrier();
         }
@@ -303,7 +310,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
             const char *xfrag[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) xfrag[j] = xs_raw + (uint32_t)(xb * (16 * MB * 256)) + lds_frag[j];
-            const int nmb_s = DIRECT ? nmb : scalar_int(nmb);
+            const int nmb_s = MB == 1 ? 1 : scalar_int(nmb);
 #pragma unroll
             for (int h = 0; h < NB; h += NA) {
                 half8_t a[NA][4];
@@ -311,7 +318,8 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
                 for (int i = 0; i < NA; ++i) dequant_tile(dc, wq[d][h + i], wsz[d][h + i], a[i]);
                 if (h + NA >= NB) {
                     __builtin_amdgcn_sched_barrier(0);
-                    if (!DIRECT && (REFILL || g + 1 < g_end)) dma_x(xb ^ 1, g + 1);
+                    // (into the buffer that the previous step read)
+                    if (!DIRECT && (REFILL || g + NXB - 1 < g_end)) dma_x(xb == 0 ? NXB - 1 : xb - 1, g + NXB - 1);
                     if (REFILL) load_w(d, g + DEPTH);      // ring slot d is free again
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -337,15 +345,16 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
                 __builtin_amdgcn_sched_barrier(0);
                 // x(g+1) was issued in this step, before this step's refill: once only the
                 // refill is outstanding it has landed (and so has the previous step's refill,
-                // which the next step starts with anyway)
-                if (REFILL) ODSD_WAIT_VMCNT(2 * NB);
+                // which the next step starts with anyway).  Three buffers: x(g+1) was issued in the step
+                // before, and after it that step's refill, x(g+2) (one copy at least) and this refill
+                if (REFILL) ODSD_WAIT_VMCNT(NXB == 3 ? 4 * NB + 1 : 2 * NB);
                 else ODSD_WAIT_VMCNT(0);
                 __builtin_amdgcn_s_barrier();
             }
         };
-        // with an even number of steps per trip the token buffer of a step is known at compile
-        // time (every trip starts on an even step) and becomes an immediate offset
-        constexpr bool XB_STATIC = DEPTH % 2 == 0;
+        // where the buffers divide the steps of a trip the token buffer of a step is known at compile
+        // time (every trip starts on buffer 0) and becomes an immediate offset
+        constexpr bool XB_STATIC = DEPTH % NXB == 0;
         int it = 0, g = g_begin;
         // Main part: whole trips round the ring while more than DEPTH groups remain (a trip whose
         // later refills run past the last group clamps them: at most DEPTH - 1 tiles per block).
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
             for (int t = 0; t < RING_TRIPS; ++t) {
 #pragma unroll
                 for (int d = 0; d < DEPTH; ++d) {
-                    step(std::true_type{}, d, XB_STATIC ? (d & 1) : (it & 1), g);
+                    step(std::true_type{}, d, XB_STATIC ? d % NXB : it % NXB, g);
                     ++g;
                     ++it;
                 }
@@ -368,7 +377,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             if (g < g_end) {
-                step(std::false_type{}, d, XB_STATIC ? (d & 1) : (it & 1), g);
+                step(std::false_type{}, d, XB_STATIC ? d % NXB : it % NXB, g);
                 ++g;
                 ++it;
             }
@@ -647,11 +656,14 @@ __global__ __launch_bounds__(1024) void combine_norm_kernel(const float *__restr
     }
 }
 
+#define STREAM_DISPATCH_CHUNKS 32   // most gate_up workgroups per expert that each scan the ids (stream_dispatch_supported)
+
 // ---- host side ---------------------------------------------------------------------------------
 struct ExpertsPlan {
     int MB;          // 16-row token blocks held per pass
     int NB;          // 16-row weight blocks per wavefront
-    int WK_gu, WK_dn;  // wavefronts splitting K inside a workgroup (MB == 1 path)
+    int NB_dn;       // MB == 1, LDS path: the same of the down projection
+    int WK_gu, WK_dn;  // MB == 1: wavefronts of a workgroup that split K on the direct path, 0: the LDS path
     int KS;          // split of the down projection's reduction dimension across workgroups
     int PS_gu, PS_dn;  // prefill tile kernel: workgroups sharing the row passes of one tile
     int tile;        // the tile kernel (experts_prefill.hip) instead of the streaming kernel
@@ -688,17 +700,31 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     const int G_gu = s->H / ODSD_GROUP, G_dn = s->I / ODSD_GROUP;
     p.NB = 4;
     p.WK_gu = p.WK_dn = 1;
+    p.NB_dn = 2;
     p.KS = 1;
     p.PS_gu = p.PS_dn = 1;
     if (p.MB == 1) {
         // many small work items: 4 wavefronts split K when each still gets >= 2 groups
         p.WK_gu = G_gu >= 8 ? 4 : (G_gu >= 4 ? 2 : 1);
-        const long chunks_dn = (s->H / 16 + 4 - 1) / 4;   // with WK = 4: 64 rows per workgroup
+        const long chunks_dn = (s->H / 16 + 4 - 1) / 4;   // 64 rows per workgroup
         int KS = 1;
         while (KS * 2 <= G_dn / 8 && active * chunks_dn * KS < 4 * slots && KS < 16) KS *= 2;
         p.KS = KS;
         const int gper = (G_dn + KS - 1) / KS;
-        p.WK_dn = gper >= 8 ? 4 : (gper >= 4 ? 2 : 1);
+        // gate_up through LDS where it then dispatches for itself and the experts with rows fill the chip
+        // without a split of K: layer at H = 2048, I = 768, E = 128, K = 8, us, direct / LDS: T = 4 41.8 / 42.9,
+        // T = 6 46.8 / 46.8, T = 8 54.0 / 49.4, T = 16 68.7 / 62.5; H = 4096, I = 1536: T = 4 82.5 / 82.3,
+        // T = 8 119 / 119, T = 16 168 / 161.  (E = 8, I = 14336 has too many workgroups per expert to dispatch
+        // inside; there the direct form is faster at any T, T = 5 68 / 72 us, T = 16 89 / 92.)
+        if (P >= 48 && (2 * s->I / 16 + 7) / 8 <= STREAM_DISPATCH_CHUNKS) p.WK_gu = 0;
+        // down through LDS (direct / LDS, us): H = 4096, I = 1536, E = 128: T = 1 13.7 / 12.4, T = 8 43.9 / 31.7,
+        // T = 16 63.5 / 46.1; I = 14336, E = 8: T = 3 28.7 / 22.9, T = 5 35.9 / 35.7, T = 16 47.4 / 42.4.
+        // Reductions of under 4 groups end before a pipeline is worth its start (2 groups: 4.7 / 5.2).
+        // Two weight blocks per wavefront for long reductions on a full chip (I = 1536, one / two blocks:
+        // T = 2 16.4 / 17.3, T = 4 23.7 / 20.8, T = 8 32.6 / 31.7), one for short ones (I = 768: T = 8
+        // 11.7 / 12.1, T = 16 15.7 / 16.5).
+        p.WK_dn = gper >= 4 ? 0 : 1;
+        p.NB_dn = gper >= 8 && active * ((s->H / 16 + 7) / 8) * KS >= 2 * slots ? 2 : 1;
     } else if (p.tile) {
         // 256 weight rows x up to 128 token rows, two workgroups per CU: with few experts the tiles
         // alone do not fill 256 CUs.  First hand the row passes of one tile (it re-reads its weights
@@ -801,10 +827,15 @@ template <int MODE>
 static void launch_gemm_plan(const ExpertsPlan &pl, GemmParams &gp, hipStream_t st) {
     const int wk = MODE == 0 ? pl.WK_gu : pl.WK_dn;
     gp.y_f16 = pl.y_f16;
-    if (pl.MB == 1) {
-        if (wk == 4) launch_gemm<4, 1, MODE, 2, 2, 4, true, 2>(gp, st);
-        else if (wk == 2) launch_gemm<4, 1, MODE, 3, 2, 2, true, 2>(gp, st);
-        else launch_gemm<4, 1, MODE, 3, 2, 1, true, 2>(gp, st);
+    if (pl.MB == 1 && wk == 0) {
+        if (MODE == 0 || pl.NB_dn == 2) launch_gemm<2, 1, MODE, 3, 2, 1, false, 4>(gp, st);
+        else if constexpr (MODE == 1) launch_gemm<1, 1, MODE, 3, 1, 1, false, 4>(gp, st);
+    } else if (pl.MB == 1) {
+        if constexpr (MODE == 0) {
+            if (wk == 4) { launch_gemm<4, 1, MODE, 2, 2, 4, true, 2>(gp, st); return; }
+            if (wk == 2) { launch_gemm<4, 1, MODE, 3, 2, 2, true, 2>(gp, st); return; }
+        }
+        launch_gemm<4, 1, MODE, 3, 2, 1, true, 2>(gp, st);
     } else if (pl.MB == 2) {
         if (pl.NB == 2) launch_gemm<2, 2, MODE, 2, 2, 1, false, 4>(gp, st);
         else launch_gemm<4, 2, MODE, 3, 4, 1, false, 2>(gp, st);
@@ -828,8 +859,9 @@ static int experts_args_ok(const odsd_moe_shape *s) {
 // expert it costs gate_up more than the launch it saves: +7 us at the Mixtral T = 160 shape, +6 us
 // at T = 5, so those plans keep the dispatch kernel)
 static bool stream_dispatch_supported(const ExpertsPlan &pl, const odsd_moe_shape *s) {
-    const int chunks = (2 * s->I / 16 + 4 * pl.NB - 1) / (4 * pl.NB);     // gate_up workgroups per expert
-    return !pl.tile && (pl.MB == 2 || pl.MB == 4) && chunks <= 32 && s->T * s->K <= 4 * 256;
+    const int nb = pl.MB == 1 ? 2 : pl.NB;
+    const int chunks = (2 * s->I / 16 + 4 * nb - 1) / (4 * nb);     // gate_up workgroups per expert
+    return !pl.tile && (pl.MB > 1 || pl.WK_gu == 0) && chunks <= STREAM_DISPATCH_CHUNKS && s->T * s->K <= 4 * 256;
 }
 
 // idx + dispatch_out: the dispatch arrays have not been filled; the kernel dispatches for itself
