@@ -17,6 +17,8 @@
 #include "common.h"
 #include "router_topk.h"
 
+#include <type_traits>
+
 #define ROUTER_MAX_NE 4    // expert tiles (of 16) per wavefront
 #define ROUTER_MAX_V 8     // most logits per lane in the top-k kernel -> E <= 512
 
@@ -47,7 +49,14 @@ template <> struct Row8<float> {
 };
 
 // unit = (token tile, expert group, k split); 4 units (wavefronts) per workgroup.
-template <typename XT, int NE, bool REDUCE4>
+// At thousands of tokens the fp64 matrix cores bound it (4.3 GFLOP at T = 4096, H = 4096, E = 128: 55 us at
+// 78 TFLOP/s).  So the loop holds nothing but loads, conversions and products: no branch (NORMED is compiled, the
+// fp16 copy has a loop of its own), no masking (rows past T or E are read from row 0 and their results not
+// stored), and neighbouring products belong to two accumulators in turn (all four in turn need every row's
+// load at the start of a chunk: 118 us where this takes 103).  With branches and masks in the loop, before / now,
+// us: E = 128, H = 2048: T = 256 6.4 / 5.9, T = 512 10.7 / 9.4, T = 1000 17.6 / 16.3, T = 2200 41.8 / 37.7;
+// H = 4096: T = 4096 113 / 103 (42 TFLOP/s, at the clock that the expert kernels in between leave).
+template <typename XT, int NE, bool REDUCE4, bool NORMED>
 __global__ __launch_bounds__(256) void router_partial_kernel(const XT *__restrict__ x,
                                                              const XT *__restrict__ wg,
                                                              double *__restrict__ partial,
@@ -55,7 +64,7 @@ __global__ __launch_bounds__(256) void router_partial_kernel(const XT *__restric
                                                              int E, int S, int EG, int n_units,
                                                              const double *__restrict__ norm_ss,
                                                              const XT *__restrict__ norm_w, double eps) {
-    const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (unit >= n_units) return;
     const int lane = lane_id();
     const int r = lane & 15, kg = lane >> 4;
@@ -86,9 +95,8 @@ __global__ __launch_bounds__(256) void router_partial_kernel(const XT *__restric
 
     // fused RMSNorm (demo/src/layers/layernorm.py:21-27): the row statistic comes from the kernel
     // that produced x; the arithmetic per element is that of the stand-alone RMSNorm kernel
-    const bool normed = norm_ss != nullptr;
     double rstd = 1.0;
-    if (normed) {
+    if (NORMED) {
         const int nchunk = (H + 1023) / 1024;   // the statistic arrives as per-chunk sums
         double tot = 0.0;
         for (int c = 0; c < nchunk; ++c) tot += norm_ss[(size_t)(t_ok ? t : 0) * nchunk + c];
@@ -96,12 +104,10 @@ __global__ __launch_bounds__(256) void router_partial_kernel(const XT *__restric
     }
     const XT *xrow = x + (size_t)(t_ok ? t : 0) * H;
     const XT *wrow[NE];
-    bool e_ok[NE];
 #pragma unroll
     for (int i = 0; i < NE; ++i) {
         const int e = (eg * NE + i) * 16 + r;
-        e_ok[i] = e < E;
-        wrow[i] = wg + (size_t)(e_ok[i] ? e : 0) * H;
+        wrow[i] = wg + (size_t)(e < E ? e : 0) * H;
     }
 
     // One chunk = 32 columns.  The raw loads of chunk c+1 are issued before chunk c is
@@ -114,15 +120,14 @@ __global__ __launch_bounds__(256) void router_partial_kernel(const XT *__restric
     auto fetch = [&](Chunk &ck, int c) {
         const int h = k0 + min(c, Hs - 32) + kg * 8;    // past the end: reload the last chunk
         ck.x = Row8<XT>::raw(xrow + h);
-        if (normed) ck.n = Row8<XT>::raw(norm_w + h);
+        if (NORMED) ck.n = Row8<XT>::raw(norm_w + h);
 #pragma unroll
         for (int i = 0; i < NE; ++i) ck.w[i] = Row8<XT>::raw(wrow[i] + h);
     };
-    auto consume = [&](const Chunk &ck, int c) {
-        const int h = k0 + c + kg * 8;
+    auto consume = [&](auto copy_c, const Chunk &ck, int c) {
         float xa[8];
         Row8<XT>::cvt(ck.x, xa);
-        if (normed) {
+        if (NORMED) {
             float nw[8];
             Row8<XT>::cvt(ck.n, nw);
 #pragma unroll
@@ -131,39 +136,41 @@ __global__ __launch_bounds__(256) void router_partial_kernel(const XT *__restric
                 xa[j] = ActIO<XT>::round(__fmul_rn(xn, nw[j]));
             }
         }
-        if (!t_ok) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) xa[j] = 0.0f;
-        }
-        if (x16 != nullptr && eg == 0 && t_ok) {
+        if (decltype(copy_c)::value) {
             half8_t o;
 #pragma unroll
             for (int j = 0; j < 8; ++j) o[j] = f32_to_f16_sat(xa[j]);
-            *(half8_t *)(x16 + (size_t)t * H + h) = o;
+            if (t_ok) *(half8_t *)(x16 + (size_t)t * H + k0 + c + kg * 8) = o;
         }
-        double xd[8];
+        // two accumulators in turn, so that the later rows' loads have until then to land
+        constexpr int IB = NE > 1 ? 2 : 1;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xd[j] = (double)xa[j];
+        for (int i0 = 0; i0 < NE; i0 += IB) {
+            float wa[IB][8];
 #pragma unroll
-        for (int i = 0; i < NE; ++i) {
-            float wa[8];
-            Row8<XT>::cvt(ck.w[i], wa);
+            for (int i = 0; i < IB; ++i) Row8<XT>::cvt(ck.w[i0 + i], wa[i]);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const double wd = e_ok[i] ? (double)wa[j] : 0.0;
-                acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(xd[j], wd, acc[i], 0, 0, 0);
-            }
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int i = 0; i < IB; ++i)
+                    acc[i0 + i] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xa[j], (double)wa[i][j], acc[i0 + i], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    Chunk ca, cb;
-    fetch(ca, 0);
-    for (int c = 0; c < Hs; c += 64) {
-        fetch(cb, c + 32);
-        consume(ca, c);
-        if (c + 32 >= Hs) break;
-        fetch(ca, c + 64);
-        consume(cb, c + 32);
-    }
+    auto reduce = [&](auto copy_c) {
+        Chunk ca, cb;
+        fetch(ca, 0);
+        int c = 0;
+        for (; c + 32 < Hs; c += 64) {
+            fetch(cb, c + 32);
+            consume(copy_c, ca, c);
+            fetch(ca, c + 64);
+            consume(copy_c, cb, c + 32);
+        }
+        if (c < Hs) consume(copy_c, ca, c);
+    };
+    if (x16 != nullptr && eg == 0) reduce(std::true_type{});
+    else reduce(std::false_type{});
 
     // When the K slices come in fours, the 4 wavefronts of this workgroup hold 4 consecutive
     // slices of the same tile: add them through LDS in slice order and write one partial.
@@ -372,7 +379,8 @@ static RouterPlan router_plan(const odsd_moe_shape *s, bool normed) {
     // Expert tiles per wavefront: more of them re-use a token chunk more often, fewer give more and
     // shorter wavefront units.  With few 16 x 16 output tiles the kernel is a latency chain and short
     // units win (E = 128: 4.6 against 6.9 us at T = 128, 6.5 against 7.1 at 256, 8.4 against 10.6 at
-    // 320); from ~512 tiles on the re-use wins (T = 4096, H = 4096: 94 against 117 us).  With the
+    // 320, with the kernel that the comment there calls "before"); from ~512 tiles on the re-use wins (T = 4096,
+    // H = 4096: 94 against 117 us).  With the
     // RMSNorm folded in, every expert group also repeats the normalisation of its token chunk (two
     // fp64 conversions per element): two tiles per wavefront are then the least (T = 256 in the
     // 48-layer stack: 8.2 us against 9.3 with one, 8.3 with four).
@@ -413,14 +421,16 @@ static void launch_partial(const RouterPlan &p, const odsd_moe_shape *s, const v
                            double *partial, void *x16, hipStream_t st, const double *norm_ss,
                            const void *norm_w, float eps) {
     const int n_units = p.TT * p.EG * p.S;
-    if (p.S % 4 == 0)
-        ODSD_LAUNCH(ODSD_KERNEL_ROUTER_LOGITS, (router_partial_kernel<XT, NE, true>), n_units / 4, 256, st,
-                    (const XT *)x, (const XT *)gw, partial, (half_t *)x16, s->T, s->H, s->E, p.S, p.EG,
-                    n_units, norm_ss, (const XT *)norm_w, (double)eps);
-    else
-        ODSD_LAUNCH(ODSD_KERNEL_ROUTER_LOGITS, (router_partial_kernel<XT, NE, false>), (n_units + 3) / 4, 256,
-                    st, (const XT *)x, (const XT *)gw, partial, (half_t *)x16, s->T, s->H, s->E, p.S, p.EG,
-                    n_units, norm_ss, (const XT *)norm_w, (double)eps);
+#define PARTIAL_GO(R4, NORMED)                                                                                       \
+    ODSD_LAUNCH(ODSD_KERNEL_ROUTER_LOGITS, (router_partial_kernel<XT, NE, R4, NORMED>), (n_units + 3) / 4, 256, st, \
+                (const XT *)x, (const XT *)gw, partial, (half_t *)x16, s->T, s->H, s->E, p.S, p.EG, n_units,         \
+                norm_ss, (const XT *)norm_w, (double)eps)
+    if (p.S % 4 == 0) {
+        if (norm_ss) PARTIAL_GO(true, true); else PARTIAL_GO(true, false);
+    } else {
+        if (norm_ss) PARTIAL_GO(false, true); else PARTIAL_GO(false, false);
+    }
+#undef PARTIAL_GO
 }
 
 int odsd_launch_router(const odsd_moe_shape *s, const void *x, const void *gate_w, int32_t *idx, float *w,
