@@ -22,7 +22,7 @@ struct AttnParams {
     // (contiguous, no block table); both null in paged mode
     const int32_t *cu_q, *cu_k;
     int n_wg;                  // streaming kernels: workgroups that share the work
-    int whole;                 // no unit is split
+    int whole;                 // no unit is split: row groups per (sequence, KV head); otherwise 0
     int v_once;                // V is read nontemporally
     float *part;               // its partial results, two slots per workgroup: [rows][HD + 4]
 };

@@ -41,13 +41,18 @@
 // Granularities of the list in keys: it is cut at multiples of FINE when that gives every workgroup at least
 // COARSE keys, otherwise at multiples of COARSE; with no sequence longer than WHOLE nothing is split and
 // there is nothing to merge.  (A merge costs 4 to 6 us, what a workgroup needs for WHOLE keys: 16 sequences
-// of 300 keys, decode, 7.7 us whole against 10.2 split.)
+// of 300 keys, decode, 7.7 us whole against 10.2 split.)  With more units nothing is split up to more
+// keys, and with MANY never: they fill the chip and level mixed lengths out by themselves.  (attn_keep_whole;
+// 32 / 4 heads of 128, split / whole, us.  Stream form: 40 sequences of up to 700 keys 15.2 / 12.6, 64 of 1000
+// 21.1 / 18.8, 384 of 700 67.9 / 58.2, but 128 of 2000 59.7 / 62.2.  Tile form, 8 queries each: 48 of 700 22.6 /
+// 24.7, 64 of 700 28.3 / 25.4, 64 of 1000 32.2 / 39.7, 128 of 700 46.4 / 34.0, 256 of 1500 151 / 129.)
 #define ATTN_STREAM_FINE 128
 #define ATTN_STREAM_COARSE 128
 #define ATTN_STREAM_WHOLE 512
 #define ATTN_TILE_FINE 32
 #define ATTN_TILE_COARSE 256
 #define ATTN_TILE_WHOLE 256
+#define ATTN_MANY (4 * ATTN_WG)
 
 // ---- how the work is dealt out -----------------------------------------------------------------------
 // A sequence is KVH * rg units, each of `steps` list steps of g keys (a sequence without keys still owns
@@ -108,7 +113,27 @@ __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int row
                                               const int coarse, const int who) {
     const int lane = lane_id();
     ListPlan pl;
-    pl.g = p.whole ? 1 << 30 : fine;          // (longer than any sequence: one step per unit, whatever its length)
+    if (p.whole) {
+        // A workgroup per (sequence, KV head, row group that a sequence can have), found without the list: with
+        // 512 sequences its scan cost every workgroup two rounds of 8 dependent loads (MANY, below).
+        pl.g = 1 << 30;                       // (longer than any sequence: one step per unit, whatever its length)
+        pl.total = 0x7fffffff;
+        pl.share = 1;
+        const int per_seq = p.KVH * p.whole, s = who / per_seq, l = who - s * per_seq;
+        const SeqCost c = seq_cost(p, s, rows_per_unit, pl.g);
+        pl.found = l < __builtin_amdgcn_readfirstlane(c.cost);
+        int tok = s;
+        if (p.cu_k) tok = p.cu_q[s] - p.cu_q[0];
+        else if (p.q_lens) {
+            tok = 0;
+            for (int i = lane; i < s; i += 64) tok += max(p.q_lens[i], 0);
+            tok = lane_value(wave_scan(tok), 63);
+        }
+        pl.at = SeqAt{s, __builtin_amdgcn_readfirstlane(c.L), __builtin_amdgcn_readfirstlane(c.ql),
+                      __builtin_amdgcn_readfirstlane(c.rg), 1, who - l, __builtin_amdgcn_readfirstlane(tok)};
+        return pl;
+    }
+    pl.g = fine;
     SeqCost c0 = seq_cost(p, lane, rows_per_unit, pl.g);
     int s0, total;
     for (;;) {
@@ -116,7 +141,7 @@ __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int row
         total = lane_value(s0, 63);
         for (int b = 64; b < p.n_seqs; b += 64)
             total += lane_value(wave_scan(seq_cost(p, b + lane, rows_per_unit, pl.g).cost), 63);
-        if (p.whole || pl.g == coarse || total >= (coarse / fine) * p.n_wg) break;
+        if (pl.g == coarse || total >= (coarse / fine) * p.n_wg) break;
         pl.g = coarse;
         seq_steps(p, c0, coarse);
     }
@@ -766,6 +791,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
 struct AttnForm {
     int rows;            // per unit
     int fine, whole;
+    bool tile;
 };
 static int64_t attn_kv_bytes(int64_t n_seqs, int64_t max_keys, int kvh, int head_dim) {
     return n_seqs * max_keys * kvh * head_dim * 4;
@@ -774,8 +800,15 @@ static AttnForm attn_form(int64_t rows, int64_t kv_bytes) {
     // 17 to 32 rows: two row blocks per wavefront pay with a lot of keys (64 sequences of up to 2000, 338 MB,
     // 5 queries of 4 heads: 62.6 against 68.3 us), the shared tiles with fewer (16 of up to 1000: 17.3 against 19.9)
     const bool wide = rows > 16 && rows <= 32 && kv_bytes > (256LL << 20);
-    if (rows <= 16 || wide) return AttnForm{wide ? 32 : 16, ATTN_STREAM_FINE, ATTN_STREAM_WHOLE};
-    return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_WHOLE};
+    if (rows <= 16 || wide) return AttnForm{wide ? 32 : 16, ATTN_STREAM_FINE, ATTN_STREAM_WHOLE, false};
+    return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_WHOLE, true};
+}
+
+// (row groups are not counted here: max_q_len may be far above what the sequences have)
+static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t max_keys) {
+    const int64_t units = n_seqs * kvh;
+    if (max_keys <= f.whole || units >= ATTN_MANY) return true;
+    return f.tile ? max_keys <= min(3 * units, (int64_t)2048) : units >= 128 && max_keys <= 1024;
 }
 
 extern "C" size_t odsd_paged_attention_workspace_bytes(int32_t n_seqs, int32_t max_q_len, int32_t num_heads,
@@ -788,7 +821,7 @@ extern "C" size_t odsd_paged_attention_workspace_bytes(int32_t n_seqs, int32_t m
     if ((rows + 63) / 64 > 65535) return 0;
     const int64_t max_keys = (int64_t)max_blocks * block_size;
     const AttnForm f = attn_form(rows, attn_kv_bytes(n_seqs, max_keys, num_kv_heads, head_dim));
-    if (max_keys <= f.whole) return 256;                              // every unit stays whole: nothing to merge
+    if (attn_keep_whole(f, n_seqs, num_kv_heads, max_keys)) return 256;   // nothing to merge
     return odsd_round_up((size_t)2 * ATTN_WG * f.rows * (head_dim + 4) * sizeof(float), 256);
 }
 
@@ -801,8 +834,12 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
     const int64_t rg = (rows + f.rows - 1) / f.rows;
     if (rg > 65535) return ODSD_ERR_UNSUPPORTED;                      // grid.y of the merge
     const int64_t steps = (max_keys + f.fine - 1) / f.fine;
-    const bool merge = max_keys > f.whole;
     const int64_t units = (int64_t)p.n_seqs * p.KVH * rg;
+    // a unit per workgroup slot, or at most 480 keys: splitting levels the lengths out, but these calls can do
+    // without it, and do when they bring no workspace for it
+    const bool can_do_without = units >= ATTN_WG || max_keys <= 480;
+    const bool no_workspace = !workspace || !odsd_aligned16(workspace) || workspace_bytes < need;
+    const bool merge = !attn_keep_whole(f, p.n_seqs, p.KVH, max_keys) && !(can_do_without && no_workspace);
     if (merge) {
         if (!workspace) return ODSD_ERR_NULL;
         if (!odsd_aligned16(workspace)) return ODSD_ERR_ALIGN;
@@ -811,8 +848,9 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         p.n_wg = ATTN_WG;
         p.whole = 0;
     } else {
-        p.n_wg = (int)min(units, (int64_t)0x7fffffff);                // each a workgroup of its own, finished in place
-        p.whole = 1;
+        if (units > 0x7fffffff) return ODSD_ERR_UNSUPPORTED;
+        p.n_wg = (int)units;                                          // each a workgroup of its own, finished in place
+        p.whole = (int)rg;
     }
     const unsigned grid = (unsigned)min((int64_t)p.n_wg, units * steps);
     // (keys that fit the 256 MB memory-side cache may still be there from the call before)

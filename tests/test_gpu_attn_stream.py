@@ -57,6 +57,11 @@ CASES = {
     # many sequences: the list is scanned 64 at a time; shares that span several of them
     "seqs150": (torch.bfloat16, 4, 2, 64, 32, [(1 + (i * 37) % 900, 1) for i in range(150)], 0),
     "seqs70_tile": (torch.float16, 16, 1, 64, 32, [(8 + (i * 53) % 700, 1 + i % 5) for i in range(70)], 0),
+    # 128 units and more with few keys, 2048 and more: nothing is split
+    "some": (torch.bfloat16, 4, 4, 64, 32, [(1 + (i * 37) % 1000, 1) for i in range(33)], 0),
+    "some_tile": (torch.bfloat16, 36, 4, 64, 32, [(9 + (i * 53) % 370, 2 + i % 5) for i in range(32)], 0),
+    "many": (torch.bfloat16, 8, 8, 64, 32, [(1 + (i * 37) % 700, 1) for i in range(256)], 0),
+    "many_tile": (torch.float16, 40, 8, 64, 32, [(7 + (i * 53) % 400, 1 + i % 7) for i in range(257)], 0),
     # no keys, no queries, fewer keys than queries
     "holes": (torch.bfloat16, 8, 2, 128, 32, [(0, 2), (700, 1), (3, 4), (40, 0), (1200, 2), (0, 1)], 0),
     "holes_tile": (torch.bfloat16, 24, 1, 128, 32, [(0, 2), (700, 3), (40, 0), (2, 3), (1200, 2), (0, 1)], 0),
@@ -89,3 +94,21 @@ def test_context_longer_than_its_table(dev):
     ctx["context_lens"] = torch.tensor([100, 1500], dtype=torch.int32, device=dev)
     out = odsd.paged_attention(q, kc, vc, ctx, 2, 32, max_q_len=mq)
     assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("name,seqs", [("units512", [(1040 - (i * 37) % 1000, 1) for i in range(256)]),
+                                       ("keys480", [(480, 9), (300, 9)])])
+def test_calls_that_can_do_without_a_workspace(dev, name, seqs):
+    """512 units, or at most 480 keys per sequence: a call without a workspace is carried out unsplit."""
+    from on_device_sd_amd import _lib
+    H, KVH, HD, bs = 8, 2, 64, 32
+    q, kc, vc, ctx, mq, ref = _case(dev, torch.bfloat16, H, KVH, HD, bs, seqs)
+    lib, bt, out = _lib.load(), ctx["block_tables"], torch.empty_like(q)
+    assert lib.odsd_paged_attention_workspace_bytes(len(seqs), mq, H, KVH, HD, bs, bt.shape[1]) > 256
+    print("attention without workspace", name, flush=True)
+    rc = lib.odsd_paged_attention(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), bt.data_ptr(), ctx["context_lens"].data_ptr(),
+                                  ctx["verify_query_lens"].data_ptr(), len(seqs), mq, H, KVH, HD, bs, bt.shape[1],
+                                  kc.shape[0], HD ** -0.5, _lib.DT_BF16, out.data_ptr(), None, 0, None)
+    torch.cuda.synchronize()
+    assert rc == 0
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
