@@ -386,7 +386,7 @@ def bench_attention(dev, steps, warmup, with_cpu):
         "sequences": n_seqs, "query_tokens_per_sequence": ql, "context_len": L, "heads": H, "kv_heads": KVH,
         "head_dim": HD, "block_size": bs, "tokens_per_s": round(n_tok / (graph_ms * 1e-3), 1),
         "ms_per_step": round(graph_ms, 5), "ms_per_step_eager_python": round(eager_ms, 5),
-        "roofline": {"bound": "hbm", "kernel": "paged_attn_kernel + paged_attn_merge_kernel", "achieved": round(ach, 1),
+        "roofline": {"bound": "hbm", "kernel": "attn_tile_kernel + attn_merge_kernel", "achieved": round(ach, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "algorithmic_bytes": kv_bytes, "kernel_ms": round(attn_ms, 5)},
     }
