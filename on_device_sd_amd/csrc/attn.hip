@@ -797,9 +797,11 @@ static int64_t attn_kv_bytes(int64_t n_seqs, int64_t max_keys, int kvh, int head
     return n_seqs * max_keys * kvh * head_dim * 4;
 }
 static AttnForm attn_form(int64_t rows, int64_t kv_bytes) {
-    // 17 to 32 rows: two row blocks per wavefront pay with a lot of keys (64 sequences of up to 2000, 338 MB,
-    // 5 queries of 4 heads: 62.6 against 68.3 us), the shared tiles with fewer (16 of up to 1000: 17.3 against 19.9)
-    const bool wide = rows > 16 && rows <= 32 && kv_bytes > (256LL << 20);
+    // 17 to 32 rows: two row blocks per wavefront pay with many keys, the shared tiles with fewer (us, shared / own:
+    // 32 / 8 heads, 64 sequences of up to 400 keys, 105 MB, 22.5 / 18.5, 700 31.5 / 25.9, 1000 41.4 / 34.0, 40 of
+    // 1500 40.9 / 42.5; 16 / 8 heads of 64, 64 of 1000 33.3 / 21.4; 32 / 4 heads, 64 of 2000 68.3 / 62.6, but 16 of
+    // 1000, 33 MB, 17.3 / 19.9)
+    const bool wide = rows > 16 && rows <= 32 && kv_bytes > (96LL << 20);
     if (rows <= 16 || wide) return AttnForm{wide ? 32 : 16, ATTN_STREAM_FINE, ATTN_STREAM_WHOLE, false};
     return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_WHOLE, true};
 }

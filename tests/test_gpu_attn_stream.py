@@ -65,7 +65,7 @@ CASES = {
     # no keys, no queries, fewer keys than queries
     "holes": (torch.bfloat16, 8, 2, 128, 32, [(0, 2), (700, 1), (3, 4), (40, 0), (1200, 2), (0, 1)], 0),
     "holes_tile": (torch.bfloat16, 24, 1, 128, 32, [(0, 2), (700, 3), (40, 0), (2, 3), (1200, 2), (0, 1)], 0),
-    # a table wide enough for 256 MB of keys: 17 to 32 rows in two row blocks
+    # a table wide enough for 96 MB of keys: 17 to 32 rows in two row blocks
     "wide": (torch.bfloat16, 32, 8, 128, 64, _edges([1500, 300, 129, 77], 5), 256),
     "wide_block48": (torch.float16, 24, 8, 64, 48, _edges([1500, 300, 129, 77], 8), 800),
 }
