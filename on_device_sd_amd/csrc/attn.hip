@@ -813,39 +813,65 @@ static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t 
     return f.tile ? max_keys <= min(3 * units, (int64_t)2048) : units >= 128 && max_keys <= 1024;
 }
 
+// What a call does, from its shape alone.  The size functions and the launch both ask here, with the same
+// number of keys: the form, whether units are split and the workspace belong together.
+struct AttnPlan {
+    AttnForm f;
+    int64_t rg, units, steps;     // row groups per (sequence, KV head), units, list steps of the longest unit
+    int64_t kv_bytes;
+    bool split;                   // units may be split: partial results and a merge
+    size_t bytes;                 // workspace that splitting takes
+};
+// rows: query rows per KV head of a sequence, max_keys: keys of a sequence, both at most
+static AttnPlan attn_plan(int64_t n_seqs, int64_t rows, int64_t max_keys, int kvh, int head_dim) {
+    AttnPlan pl;
+    pl.kv_bytes = attn_kv_bytes(n_seqs, max_keys, kvh, head_dim);
+    pl.f = attn_form(rows, pl.kv_bytes);
+    pl.rg = (rows + pl.f.rows - 1) / pl.f.rows;
+    pl.steps = (max_keys + pl.f.fine - 1) / pl.f.fine;
+    pl.units = n_seqs * kvh * pl.rg;
+    pl.split = !attn_keep_whole(pl.f, n_seqs, kvh, max_keys);
+    pl.bytes = pl.split ? odsd_round_up((size_t)2 * ATTN_WG * pl.f.rows * (head_dim + 4) * sizeof(float), 256) : 0;
+    return pl;
+}
+static bool attn_plan_shape_ok(int32_t n_seqs, int32_t max_q_len, int64_t max_keys, int32_t num_heads,
+                               int32_t num_kv_heads, int32_t head_dim) {
+    if (n_seqs <= 0 || max_q_len <= 0 || max_keys <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
+        num_heads % num_kv_heads || (head_dim != 64 && head_dim != 128))
+        return false;
+    return ((int64_t)max_q_len * (num_heads / num_kv_heads) + 63) / 64 <= 65535;
+}
+static size_t attn_workspace_bytes(int32_t n_seqs, int32_t max_q_len, int64_t max_keys, int32_t num_heads,
+                                   int32_t num_kv_heads, int32_t head_dim) {
+    if (!attn_plan_shape_ok(n_seqs, max_q_len, max_keys, num_heads, num_kv_heads, head_dim)) return 0;
+    const AttnPlan pl = attn_plan(n_seqs, (int64_t)max_q_len * (num_heads / num_kv_heads), max_keys, num_kv_heads, head_dim);
+    return pl.split ? pl.bytes : 256;
+}
+
 extern "C" size_t odsd_paged_attention_workspace_bytes(int32_t n_seqs, int32_t max_q_len, int32_t num_heads,
                                                        int32_t num_kv_heads, int32_t head_dim,
                                                        int32_t block_size, int32_t max_blocks) {
-    if (n_seqs <= 0 || max_q_len <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads ||
-        block_size <= 0 || max_blocks <= 0 || (head_dim != 64 && head_dim != 128))
-        return 0;
-    const int64_t rows = (int64_t)max_q_len * (num_heads / num_kv_heads);
-    if ((rows + 63) / 64 > 65535) return 0;
-    const int64_t max_keys = (int64_t)max_blocks * block_size;
-    const AttnForm f = attn_form(rows, attn_kv_bytes(n_seqs, max_keys, num_kv_heads, head_dim));
-    if (attn_keep_whole(f, n_seqs, num_kv_heads, max_keys)) return 256;   // nothing to merge
-    return odsd_round_up((size_t)2 * ATTN_WG * f.rows * (head_dim + 4) * sizeof(float), 256);
+    if (block_size <= 0 || max_blocks <= 0) return 0;
+    return attn_workspace_bytes(n_seqs, max_q_len, (int64_t)max_blocks * block_size, num_heads, num_kv_heads, head_dim);
 }
 
 // p: everything but Gq, n_wg, part; max_keys: no sequence has more
 static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_t rows, int64_t max_keys, bool aligned,
-                              void *workspace, size_t workspace_bytes, size_t need, hipStream_t st) {
-    const int64_t kv_bytes = attn_kv_bytes(p.n_seqs, max_keys, p.KVH, head_dim);
-    const AttnForm f = attn_form(rows, kv_bytes);
+                              void *workspace, size_t workspace_bytes, hipStream_t st) {
+    const AttnPlan pl = attn_plan(p.n_seqs, rows, max_keys, p.KVH, head_dim);
+    const AttnForm &f = pl.f;
+    const int64_t rg = pl.rg, units = pl.units, kv_bytes = pl.kv_bytes;
     p.Gq = p.H / p.KVH;
-    const int64_t rg = (rows + f.rows - 1) / f.rows;
     if (rg > 65535) return ODSD_ERR_UNSUPPORTED;                      // grid.y of the merge
-    const int64_t steps = (max_keys + f.fine - 1) / f.fine;
-    const int64_t units = (int64_t)p.n_seqs * p.KVH * rg;
     // a unit per workgroup slot, or at most 480 keys: splitting levels the lengths out, but these calls can do
     // without it, and do when they bring no workspace for it
     const bool can_do_without = units >= ATTN_WG || max_keys <= 480;
-    const bool no_workspace = !workspace || !odsd_aligned16(workspace) || workspace_bytes < need;
-    const bool merge = !attn_keep_whole(f, p.n_seqs, p.KVH, max_keys) && !(can_do_without && no_workspace);
+    const bool no_workspace = !workspace || !odsd_aligned16(workspace) || workspace_bytes < pl.bytes;
+    const bool merge = pl.split && !(can_do_without && no_workspace);
     if (merge) {
         if (!workspace) return ODSD_ERR_NULL;
         if (!odsd_aligned16(workspace)) return ODSD_ERR_ALIGN;
-        if (workspace_bytes < need) return ODSD_ERR_WORKSPACE;
+        if (workspace_bytes < pl.bytes) return ODSD_ERR_WORKSPACE;
         p.part = (float *)workspace;
         p.n_wg = ATTN_WG;
         p.whole = 0;
@@ -854,7 +880,7 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         p.n_wg = (int)units;                                          // each a workgroup of its own, finished in place
         p.whole = (int)rg;
     }
-    const unsigned grid = (unsigned)min((int64_t)p.n_wg, units * steps);
+    const unsigned grid = (unsigned)min((int64_t)p.n_wg, units * pl.steps);
     // (keys that fit the 256 MB memory-side cache may still be there from the call before)
     p.v_once = kv_bytes > (100 << 20);
     const dim3 mgrid((unsigned)(p.n_seqs * p.KVH), (unsigned)rg, (unsigned)((f.rows * head_dim + 1023) / 1024));
@@ -908,19 +934,15 @@ extern "C" int odsd_paged_attention(const void *q, const void *k_cache, const vo
     p.n_seqs = n_seqs; p.H = num_heads; p.KVH = num_kv_heads; p.max_blocks = max_blocks;
     p.block_size = block_size; p.num_slots = num_slots;
     p.scale_log2e = softmax_scale * 1.4426950408889634f;
-    const size_t need = odsd_paged_attention_workspace_bytes(n_seqs, max_q_len, num_heads, num_kv_heads, head_dim,
-                                                             block_size, max_blocks);
     return attn_stream_launch(p, dtype, head_dim, (int64_t)max_q_len * (num_heads / num_kv_heads),
-                              (int64_t)max_blocks * block_size, block_size % 32 == 0, workspace, workspace_bytes, need,
+                              (int64_t)max_blocks * block_size, block_size % 32 == 0, workspace, workspace_bytes,
                               (hipStream_t)stream);
 }
 
 // ---- variable-length (prefill) form ----------------------------------------------------------------
 extern "C" size_t odsd_varlen_attention_workspace_bytes(int32_t n_seqs, int32_t max_seqlen_q, int32_t max_seqlen_k,
                                                         int32_t num_heads, int32_t num_kv_heads, int32_t head_dim) {
-    if (max_seqlen_k <= 0) return 0;
-    return odsd_paged_attention_workspace_bytes(n_seqs, max_seqlen_q, num_heads, num_kv_heads, head_dim, 32,
-                                                (max_seqlen_k + 31) / 32);
+    return attn_workspace_bytes(n_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim);
 }
 
 extern "C" int odsd_varlen_attention(const void *q, const void *k, const void *v, const int32_t *cu_seqlens_q,
@@ -950,8 +972,5 @@ extern "C" int odsd_varlen_attention(const void *q, const void *k, const void *v
         ODSD_CHECK_LAUNCH();
         return ODSD_OK;
     }
-    const size_t need = odsd_varlen_attention_workspace_bytes(n_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads,
-                                                              head_dim);
-    return attn_stream_launch(p, dtype, head_dim, rows, max_seqlen_k, true, workspace, workspace_bytes, need,
-                              (hipStream_t)stream);
+    return attn_stream_launch(p, dtype, head_dim, rows, max_seqlen_k, true, workspace, workspace_bytes, (hipStream_t)stream);
 }
