@@ -300,7 +300,8 @@ size_t odsd_paged_attention_workspace_bytes(int32_t n_seqs, int32_t max_q_len, i
 /* Causal attention of a prefill step: variable-length sequences packed one after the other, keys
  * and values taken from the step's own k / v (no cache read).
  *   q [total_q, num_heads, head_dim], k / v [total_k, num_kv_heads, head_dim], contiguous
- *   cu_seqlens_q / cu_seqlens_k  int32 [n_seqs + 1]: row ranges of the sequences
+ *   cu_seqlens_q / cu_seqlens_k  int32 [n_seqs + 1]: row ranges of the sequences (they need not begin at 0:
+ *                part of a batch's offsets attends that part; other rows of out are not written)
  *   query i of a sequence attends keys 0 .. i + (k_len - q_len) of it (the mask is aligned to
  *   the bottom right corner when the lengths differ, as in flash-attn >= 2.1)
  * max_seqlen_q / max_seqlen_k: upper bounds of the lengths; softmax_scale > 0; head_dim 64 or 128;

@@ -98,7 +98,7 @@ __device__ __forceinline__ int lane_value(int v, int lane) { return __builtin_am
 struct SeqAt {
     int seq, L, ql, rg, steps;
     int first;       // list position of its first step
-    int q0;          // its first query token
+    int q0;          // its first query token (packed form: cu_q[seq], wherever the offsets begin)
 };
 struct ListPlan {
     int g;                   // keys per list step
@@ -123,7 +123,7 @@ __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int row
         const SeqCost c = seq_cost(p, s, rows_per_unit, pl.g);
         pl.found = l < __builtin_amdgcn_readfirstlane(c.cost);
         int tok = s;
-        if (p.cu_k) tok = p.cu_q[s] - p.cu_q[0];
+        if (p.cu_k) tok = p.cu_q[s];
         else if (p.q_lens) {
             tok = 0;
             for (int i = lane; i < s; i += 64) tok += max(p.q_lens[i], 0);
@@ -164,7 +164,7 @@ __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int row
             const int l = BY_SEQ ? who - b : __builtin_ctzll(__ballot(before + sc > target));
             pl.at = SeqAt{b + l, lane_value(c.L, l), lane_value(c.ql, l), lane_value(c.rg, l), lane_value(c.steps, l),
                           before + lane_value(sc, l) - lane_value(c.cost, l),
-                          tok + lane_value(tc, l) - lane_value(c.ql, l)};
+                          p.cu_k ? __builtin_amdgcn_readfirstlane(p.cu_q[b + l]) : tok + lane_value(tc, l) - lane_value(c.ql, l)};
             pl.found = true;
             return pl;
         }
@@ -182,8 +182,8 @@ __device__ __forceinline__ void next_unit(const AttnParams &p, SeqAt &sq, int &u
     unit = 0;
     sq.first += p.KVH * sq.rg * sq.steps;
     do {                                                   // (a sequence without queries has no units)
-        sq.q0 += sq.ql;
         ++sq.seq;
+        sq.q0 = p.cu_k ? __builtin_amdgcn_readfirstlane(p.cu_q[sq.seq]) : sq.q0 + sq.ql;
         const SeqCost nx = seq_cost(p, sq.seq, rows_per_unit, g);
         sq.L = __builtin_amdgcn_readfirstlane(nx.L);
         sq.ql = __builtin_amdgcn_readfirstlane(nx.ql);

@@ -112,3 +112,49 @@ def test_calls_that_can_do_without_a_workspace(dev, name, seqs):
     torch.cuda.synchronize()
     assert rc == 0
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+# (q_len, k_len) per sequence; 8 heads per KV head
+PACKED = {
+    "stream_whole": (2, [(1, 300), (2, 64), (1, 512)]),
+    "stream_split": (1, [(1, 1500), (2, 700), (0, 90), (1, 40), (2, 1100)]),
+    "tile_whole": (2, [(7, 200), (8, 33), (5, 256)]),
+    "tile_split": (1, [(7, 1500), (8, 700), (0, 90), (3, 40), (8, 1100)]),
+    "prefill": (4, [(300, 300), (65, 129), (200, 200)]),
+}
+
+
+@pytest.mark.parametrize("name", list(PACKED))
+def test_packed_offsets_that_do_not_begin_at_zero(dev, name):
+    """Part of a batch's offsets: rows are the absolute ranges of cu_seqlens, in every kernel, and rows
+    outside them are left alone."""
+    import on_device_sd_amd as odsd
+    from on_device_sd_amd import _lib
+    KVH, seqs = PACKED[name]
+    H, HD, q_first, k_first = 8 * KVH, 128, 13, 45
+    g = torch.Generator().manual_seed(len(name))
+    cu_q = np.concatenate([[0], np.cumsum([a for a, _ in seqs])]).astype(np.int32)
+    cu_k = np.concatenate([[0], np.cumsum([b for _, b in seqs])]).astype(np.int32)
+    nq, nk = int(cu_q[-1]), int(cu_k[-1])
+    q = torch.randn(nq + 2 * q_first, H, HD, generator=g).to(torch.bfloat16)
+    k = torch.randn(nk + 2 * k_first, KVH, HD, generator=g).to(torch.bfloat16)
+    v = torch.randn(nk + 2 * k_first, KVH, HD, generator=g).to(torch.bfloat16)
+    mq, mk = max(a for a, _ in seqs), max(b for _, b in seqs)
+    lib = _lib.load()
+    nbytes = lib.odsd_varlen_attention_workspace_bytes(len(seqs), mq, mk, H, KVH, HD)
+    assert (nbytes > 256) == (name.endswith("split") or name == "prefill")
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    cq, ck = torch.from_numpy(cu_q + q_first).to(dev), torch.from_numpy(cu_k + k_first).to(dev)
+    out = torch.full_like(qd, 77.0)
+    print("packed attention, offsets from", q_first, k_first, name, flush=True)
+    _lib.check(lib.odsd_varlen_attention(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), cq.data_ptr(), ck.data_ptr(), len(seqs), mq,
+                                         mk, H, KVH, HD, HD ** -0.5, _lib.DT_BF16, out.data_ptr(), ws.data_ptr(), nbytes, None),
+               "odsd_varlen_attention")
+    torch.cuda.synchronize()
+    ref = orc.varlen_attention(q[q_first:q_first + nq], k[k_first:k_first + nk], v[k_first:k_first + nk], cu_q, cu_k, HD ** -0.5)
+    out = out.float().cpu()
+    assert (out[q_first:q_first + nq] - ref).abs().max().item() <= 2e-2
+    assert (out[:q_first] == 77.0).all() and (out[q_first + nq:] == 77.0).all()
+    part = odsd.varlen_attention(qd, kd, vd, cq, ck, mq, mk).float().cpu()
+    assert torch.equal(part[q_first:q_first + nq], out[q_first:q_first + nq])
