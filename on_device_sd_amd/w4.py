@@ -117,7 +117,8 @@ class W4ExpertBank:
                     keep_canonical: bool = False):
         """Quantise one expert's [I,H], [I,H], [H,I] weights on the device and pack them: in one launch, or
         through the canonical arrays when the caller wants those as well."""
-        ws = [w if w.is_cuda else w.to(self.device) for w in (gate_w, up_w, down_w)]
+        here = self.gu_q.device                     # (with its index: another GPU's tensor has to move as well)
+        ws = [w if w.device == here else w.to(here) for w in (gate_w, up_w, down_w)]
         if keep_canonical:
             canon = tuple(ops.w4_quantize(w) for w in ws)
             self.load_canonical(e, *canon)

@@ -184,3 +184,29 @@ def test_bench_refuses_more_than_one_gpu():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0 and "one GPU" in r.stderr and r.stdout.strip() == ""
+
+
+def test_load_expert_brings_weights_to_the_bank(monkeypatch):
+    """Weights that live anywhere else, on another GPU as well as in host memory, are moved to the bank's device
+    before the kernels get their addresses; those that are there already are not copied."""
+    from on_device_sd_amd import ops
+
+    class Weight:
+        def __init__(self, device, shape, moved=False):
+            self.device, self.shape, self.moved = torch.device(device), torch.Size(shape), moved
+            self.is_cuda = self.device.type == "cuda"
+
+        def to(self, device):
+            return Weight(device, self.shape, moved=True)
+
+    bank = odsd.W4ExpertBank(2, 256, 128, "cpu")
+    bank.gu_q = Weight("cuda:0", bank.gu_q.shape)       # as if the bank lived on the first GPU
+    seen = []
+    monkeypatch.setattr(ops, "w4_load_expert", lambda *a: seen.append(a[:3]))
+    monkeypatch.setattr(ops, "w4_quantize", lambda w: w)
+    monkeypatch.setattr(bank, "load_canonical", lambda e, *ws: seen.append(ws))
+    for device in ("cuda:1", "cpu", "cuda:0"):
+        for keep in (False, True):
+            bank.load_expert(1, Weight(device, (128, 256)), Weight(device, (128, 256)), Weight(device, (256, 128)), keep_canonical=keep)
+            assert [w.device for w in seen[-1]] == [torch.device("cuda:0")] * 3
+            assert [w.moved for w in seen[-1]] == [device != "cuda:0"] * 3
