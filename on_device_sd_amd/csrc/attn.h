@@ -21,7 +21,8 @@ struct AttnParams {
     // variable-length mode (prefill): q / k / v rows of sequence s are q[cu_q[s] ..], k[cu_k[s] ..]
     // (contiguous, no block table); both null in paged mode
     const int32_t *cu_q, *cu_k;
-    int n_wg;                  // streaming kernels: workgroups that share the work
+    int max_keys, max_rg;      // streaming kernels: the keys and row groups of a sequence that the launch is sized for
+    int n_wg;                  // workgroups that share the work
     int whole;                 // no unit is split: row groups per (sequence, KV head); otherwise 0
     int v_once;                // V is read nontemporally
     float *part;               // its partial results, two slots per workgroup: [rows][HD + 4]

@@ -56,12 +56,14 @@
 
 // ---- how the work is dealt out -----------------------------------------------------------------------
 // A sequence is KVH * rg units, each of `steps` list steps of g keys (a sequence without keys still owns
-// output rows, which are written as zeros: one step).
+// output rows, which are written as zeros: one step).  A sequence takes no more of the list than the host sized
+// the launch for: a context longer than its table is walked by the last step of its units, and row groups
+// past the bound on the query lengths are left out, so that the others' shares stay where they are.
 struct SeqCost {
     int L, ql, rg, steps, cost;
 };
 __device__ __forceinline__ void seq_steps(const AttnParams &p, SeqCost &c, const int g) {
-    c.steps = max(1, (c.L + g - 1) / g);
+    c.steps = max(1, (min(c.L, p.max_keys) + g - 1) / g);
     c.cost = c.rg * p.KVH * c.steps;
 }
 __device__ __forceinline__ SeqCost seq_cost(const AttnParams &p, const int s, const int rows_per_unit, const int g) {
@@ -75,7 +77,7 @@ __device__ __forceinline__ SeqCost seq_cost(const AttnParams &p, const int s, co
             c.ql = p.q_lens ? p.q_lens[s] : 1;
         }
         c.ql = max(c.ql, 0);
-        c.rg = (c.ql * p.Gq + rows_per_unit - 1) / rows_per_unit;
+        c.rg = min((c.ql * p.Gq + rows_per_unit - 1) / rows_per_unit, p.max_rg);
         seq_steps(p, c, g);
     }
     return c;
@@ -319,7 +321,7 @@ __global__ __launch_bounds__(256, RB == 1 ? 3 : 2) void attn_stream_kernel(const
         // this wavefront's tiles: 32 keys from 32 * wave on, every STEP; 64 of them at a time (their
         // table entries sit one per lane)
         const char *kh = kc + kvh * (HD * 2), *vh = vc + kvh * (HD * 2);
-        const int key_end = min(L, pl.g * (step + n));
+        const int key_end = step + n == sq.steps ? L : pl.g * (step + n);
         for (int key0 = pl.g * step + 32 * wave; key0 < key_end; key0 += 64 * STEP) {
             const int nt = min(64, (key_end - key0 + STEP - 1) / STEP);
             // ALIGNED: the slot of each tile's first key and the last row of the tile that may be read, one
@@ -545,7 +547,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
     auto set_piece = [&](Cursor &q) {
         q.n = min(end - q.pos, q.sq.steps - q.step);
         q.key = pl.g * q.step;
-        q.key_end = min(q.sq.L, pl.g * (q.step + q.n));
+        q.key_end = q.step + q.n == q.sq.steps ? q.sq.L : pl.g * (q.step + q.n);
     };
     auto next_piece = [&](Cursor &q) {
         q.pos += q.n;
@@ -862,6 +864,8 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
     const AttnForm &f = pl.f;
     const int64_t rg = pl.rg, units = pl.units, kv_bytes = pl.kv_bytes;
     p.Gq = p.H / p.KVH;
+    p.max_keys = (int)min(max_keys, (int64_t)1 << 30);               // (rounding up to a step stays within 32 bits)
+    p.max_rg = (int)rg;
     if (rg > 65535) return ODSD_ERR_UNSUPPORTED;                      // grid.y of the merge
     // a unit per workgroup slot, or at most 480 keys: splitting levels the lengths out, but these calls can do
     // without it, and do when they bring no workspace for it

@@ -86,14 +86,46 @@ def test_paged_attention_shares(dev, name):
     assert torch.equal(out, odsd.paged_attention(q, kc, vc, ctx, KVH, bs, max_q_len=mq))
 
 
-def test_context_longer_than_its_table(dev):
-    """A context_len beyond the table's width (the positions past it read slot 0, as documented for entries
-    beyond the cache) stays inside the buffers: the bound that keeps units whole comes from the table."""
+@pytest.mark.parametrize("q_len,lens", [(1, [100, 64]), (1, [640, 640, 300]), (7, [640, 640, 300]), (8, [256, 90])])
+def test_context_longer_than_its_table(dev, q_len, lens):
+    """A context_len beyond the table's width: the positions past it read slot 0, as documented for entries
+    beyond the cache, and the other sequences are what they are without it.  Tables below and above the lengths
+    that keep units whole, both forms of the kernel; the list of shares is sized from the tables."""
     import on_device_sd_amd as odsd
-    q, kc, vc, ctx, mq, _ = _case(dev, torch.bfloat16, 8, 2, 128, 32, [(100, 1), (64, 1)])
-    ctx["context_lens"] = torch.tensor([100, 1500], dtype=torch.int32, device=dev)
-    out = odsd.paged_attention(q, kc, vc, ctx, 2, 32, max_q_len=mq)
-    assert torch.isfinite(out.float()).all()
+    KVH, bs, HD, long = 2, 32, 128, 1500
+    q, kc, vc, ctx, mq, _ = _case(dev, torch.bfloat16, 8 * KVH, KVH, HD, bs, _edges(lens, q_len))
+    over = [long] + lens[1:]
+    ctx["context_lens"] = torch.tensor(over, dtype=torch.int32, device=dev)
+    print("context longer than its table", q_len, lens, flush=True)
+    out = odsd.paged_attention(q, kc, vc, ctx, KVH, bs, max_q_len=mq).float().cpu()
+    bt = ctx["block_tables"].cpu()
+    slots = []
+    for s, L in enumerate(over):
+        pos = torch.arange(L)
+        here = pos // bs < bt.shape[1]
+        slots.append(torch.where(here, bt[s][(pos // bs).clamp(max=bt.shape[1] - 1)].long() * bs + pos % bs, 0))
+    rows = torch.cat(slots)
+    k, v = kc.cpu()[rows].view(-1, KVH, HD), vc.cpu()[rows].view(-1, KVH, HD)
+    cu_q = np.arange(len(over) + 1, dtype=np.int32) * q_len
+    cu_k = np.concatenate([[0], np.cumsum(over)]).astype(np.int32)
+    ref = orc.varlen_attention(q.cpu(), k, v, cu_q, cu_k, HD ** -0.5)
+    assert (out - ref).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("keys", [200, 1500])
+def test_query_longer_than_its_bound(dev, keys):
+    """A query length above max_q_len: its rows past the launch's row groups are not computed (documented), every
+    other row is, of all KV heads and of the sequences after it."""
+    import on_device_sd_amd as odsd
+    KVH, bs = 3, 32
+    for rows, mq in ((16, 2), (64, 8)):               # query rows per unit and max_q_len, 8 heads per KV head
+        seqs = [(keys, mq), (keys, mq + 7), (keys - 30, mq), (keys, 1)]
+        q, kc, vc, ctx, _, ref = _case(dev, torch.bfloat16, 8 * KVH, KVH, 64, bs, seqs)
+        print("query longer than its bound", keys, rows, flush=True)
+        out = odsd.paged_attention(q, kc, vc, ctx, KVH, bs, max_q_len=mq).float().cpu()
+        sure = torch.ones(q.shape[0], dtype=torch.bool)
+        sure[mq + rows // 8:2 * mq + 7] = False       # the long query's tokens past the first row group
+        assert (out - ref)[sure].abs().max().item() <= 2e-2
 
 
 @pytest.mark.parametrize("name,seqs", [("units512", [(1040 - (i * 37) % 1000, 1) for i in range(256)]),
