@@ -808,10 +808,11 @@ static AttnForm attn_form(int64_t rows, int64_t kv_bytes) {
     return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_WHOLE, true};
 }
 
-// (row groups are not counted here: max_q_len may be far above what the sequences have)
-static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t max_keys) {
-    const int64_t units = n_seqs * kvh;
-    if (max_keys <= f.whole || units >= ATTN_MANY) return true;
+// (row groups are not counted here: max_q_len may be far above what the sequences have.  But list positions are 32
+// bits wide: a list that could grow past 2^30 steps stays whole as well, with 2^18 units and more even on 131072 keys)
+static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t rg, int64_t max_keys) {
+    const int64_t units = n_seqs * kvh, steps = (max_keys + f.fine - 1) / f.fine;
+    if (max_keys <= f.whole || units >= ATTN_MANY || units * rg * steps > (1LL << 30)) return true;
     return f.tile ? max_keys <= min(3 * units, (int64_t)2048) : units >= 128 && max_keys <= 1024;
 }
 
@@ -832,7 +833,7 @@ static AttnPlan attn_plan(int64_t n_seqs, int64_t rows, int64_t max_keys, int kv
     pl.rg = (rows + pl.f.rows - 1) / pl.f.rows;
     pl.steps = (max_keys + pl.f.fine - 1) / pl.f.fine;
     pl.units = n_seqs * kvh * pl.rg;
-    pl.split = !attn_keep_whole(pl.f, n_seqs, kvh, max_keys);
+    pl.split = !attn_keep_whole(pl.f, n_seqs, kvh, pl.rg, max_keys);
     pl.bytes = pl.split ? odsd_round_up((size_t)2 * ATTN_WG * pl.f.rows * (head_dim + 4) * sizeof(float), 256) : 0;
     return pl;
 }

@@ -60,3 +60,12 @@ def test_a_launch_takes_what_the_size_function_says_and_no_less():
                 assert call(shape, at, need - 1) == ERR_WORKSPACE, shape
                 split += 1
     assert split > 100 and whole > 100
+
+
+def test_a_list_of_shares_fits_32_bits():
+    """A launch that would have to lay out more than 2^30 steps of 32 keys keeps its units whole."""
+    size = _lib.load().odsd_paged_attention_workspace_bytes
+    for n, q, blocks, split in ((256, 4096, 256, True), (256, 4096, 257, False), (256, 4096, 512, False), (1, 65535, 8193, False)):
+        steps = n * 4 * ((q * 8 + 63) // 64) * (blocks * 256 // 32)
+        assert (steps <= 1 << 30) == split
+        assert (size(n, q, 32, 4, 128, 256, blocks) > NOTHING) == split, (n, q, blocks)
