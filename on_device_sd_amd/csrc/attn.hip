@@ -110,12 +110,13 @@ struct ListPlan {
 };
 // fine, coarse: the two granularities.  The list is cut at multiples of `fine` keys when every workgroup gets at
 // least `coarse` keys that way; otherwise at multiples of `coarse`, so that short units stay whole.
-template <bool BY_SEQ>
+// SPLIT, UNSPLIT: the launches that the caller is compiled for.
+template <bool BY_SEQ, bool SPLIT, bool UNSPLIT>
 __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int rows_per_unit, const int fine,
                                               const int coarse, const int who) {
     const int lane = lane_id();
     ListPlan pl;
-    if (p.whole) {
+    if (UNSPLIT && (!SPLIT || p.whole)) {
         // A workgroup per (sequence, KV head, row group that a sequence can have), found without the list: with
         // 512 sequences its scan cost every workgroup two rounds of 8 dependent loads (MANY, below).
         pl.g = 1 << 30;                       // (longer than any sequence: one step per unit, whatever its length)
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(256, RB == 1 ? 3 : 2) void attn_stream_kernel(const
     float *xch = (float *)lds;
     auto vswz = [](int key) { return HD == 128 ? (key & 7) : ((key >> 1) & 3); };
 
-    const ListPlan pl = list_plan<false>(p, ROWS, ATTN_STREAM_FINE, ATTN_STREAM_COARSE, blockIdx.x);
+    const ListPlan pl = list_plan<false, true, true>(p, ROWS, ATTN_STREAM_FINE, ATTN_STREAM_COARSE, blockIdx.x);
     if (!pl.found) return;
     int pos = blockIdx.x * pl.share;                       // list position of the next step
     const int end = min(pl.total, pos + pl.share);
@@ -491,12 +492,15 @@ __global__ __launch_bounds__(256, RB == 1 ? 3 : 2) void attn_stream_kernel(const
     }
 }
 
-// The form for more than 32 rows per sequence (a verify step of a model with many query heads per KV head): a
-// wavefront cannot hold 64 rows next to its keys, so here the four wavefronts own 16 rows each and share
-// the keys through LDS, 32 at a time.  K and V rows are copied there asynchronously, three tiles ahead (a
-// ring of four, one barrier per tile, waits that leave the younger copies in flight) and on across the end
-// of a piece; the rows of the keys are looked up for many tiles at a time and kept in LDS.
-template <typename T, int HD>
+// The form for more rows per sequence than the stream form takes (a verify step of a model with many query heads per
+// KV head, a prompt chunk over the cache): a wavefront cannot hold 64 rows next to its keys, so here the four
+// wavefronts own 16 rows each and share the keys through LDS, 32 at a time.  K and V rows are copied there
+// asynchronously (a ring of tiles, one barrier per tile, waits that leave the younger copies in flight) and on across
+// the end of a piece; the rows of the keys are looked up for many tiles at a time and kept in LDS.
+// SPLIT: two workgroups per CU share all keys, with a ring of four.  Unsplit launches have workgroups to
+// spare: a ring of two, 36 KB, lets a CU hold four of them, whose copies overlap (ring of four / three / two, us, 32
+// / 4 heads: 256 sequences of 1500 keys x 8 144 / 138 / 121, 64 of 700 x 12, 32 / 8 heads, 33.4 / 32.6 / 27.0).
+template <typename T, int HD, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
     typedef typename AttnT<T>::V8 V8;
     constexpr int NJ = HD / 32, NDB = HD / 16;
@@ -505,8 +509,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
     constexpr int COPIES = 32 / RPC / 4; // copies per wavefront, tile and matrix
     constexpr int ROWS = 64, XROW = HD + 4;
     constexpr int TILEB = 32 * HD * 2;
-    constexpr int NBUF = 4;
-    constexpr int MOST = 64;             // tiles whose rows are looked up at a time
+    constexpr int NBUF = SPLIT ? 4 : 2;
+    constexpr int MOST = SPLIT ? 64 : 32;   // tiles whose rows are looked up at a time
     __shared__ __attribute__((aligned(16))) char lds[NBUF * 2 * TILEB];
     __shared__ uint32_t slots[MOST * 32];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -514,7 +518,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
     const int c = lane & 15, kq = lane >> 4;
     auto vswz = [](int key) { return HD == 128 ? (key & 7) : ((key >> 1) & 3); };
 
-    const ListPlan pl = list_plan<false>(p, ROWS, ATTN_TILE_FINE, ATTN_TILE_COARSE, blockIdx.x);
+    const ListPlan pl = list_plan<false, SPLIT, !SPLIT>(p, ROWS, ATTN_TILE_FINE, ATTN_TILE_COARSE, blockIdx.x);
     if (!pl.found) return;
     const int first_pos = blockIdx.x * pl.share, end = min(pl.total, first_pos + pl.share);
     const float sc = p.scale_log2e;
@@ -657,7 +661,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(qf[j]));
         auto copy_tile = [&](const int i) {
-            char *dst = lds + (i & (NBUF - 1)) * (2 * TILEB);
+            char *dst = lds + i % NBUF * (2 * TILEB);
             uint32_t sl[COPIES];
 #pragma unroll
             for (int u = 0; u < COPIES; ++u) sl[u] = slots[32 * i + RPC * (wave + 4 * u) + crow];
@@ -681,13 +685,13 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
             }
             if (fresh) begin_piece();
             // tile i has landed once only the copies of the younger tiles are outstanding
-            if (i + 2 < nt) ODSD_WAIT_VMCNT_LGKM0(2 * 2 * COPIES);
-            else if (i + 1 < nt) ODSD_WAIT_VMCNT_LGKM0(2 * COPIES);
+            if (NBUF > 3 && i + 2 < nt) ODSD_WAIT_VMCNT_LGKM0(2 * 2 * COPIES);
+            else if (NBUF > 2 && i + 1 < nt) ODSD_WAIT_VMCNT_LGKM0(2 * COPIES);
             else ODSD_WAIT_VMCNT_LGKM0(0);
             __builtin_amdgcn_s_barrier();                  // ... for every wavefront, and all are done with tile i - 1
             if (i + NBUF - 1 < nt) copy_tile(i + NBUF - 1);
             if (active) {
-                const char *kt = lds + (i & (NBUF - 1)) * (2 * TILEB), *vt = kt + TILEB;
+                const char *kt = lds + i % NBUF * (2 * TILEB), *vt = kt + TILEB;
                 const int k0 = now.key;
                 float4_t st[2];
 #pragma unroll
@@ -731,7 +735,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     constexpr int TPR = HD / 4, RPW = 256 / TPR;
     const int seq = blockIdx.x / p.KVH, kvh = blockIdx.x - seq * p.KVH;
     const int rg = blockIdx.y;
-    const ListPlan pl = list_plan<true>(p, ROWS, FINE, COARSE, seq);
+    const ListPlan pl = list_plan<true, true, false>(p, ROWS, FINE, COARSE, seq);
     const SeqAt &sq = pl.at;
     if (rg >= sq.rg) return;
     const int a = sq.first + (kvh * sq.rg + rg) * sq.steps;        // list positions of the unit's steps
@@ -900,7 +904,8 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         if (f.rows == 16) ATTN_GO(T, HDV, 1);                                                    \
         else if (f.rows == 32) ATTN_GO(T, HDV, 2);                                               \
         else {                                                                                   \
-            attn_tile_kernel<T, HDV><<<grid, 256, 0, st>>>(p);                                   \
+            if (merge) attn_tile_kernel<T, HDV, true><<<grid, 256, 0, st>>>(p);                  \
+            else attn_tile_kernel<T, HDV, false><<<grid, 256, 0, st>>>(p);                       \
             if (merge) attn_merge_kernel<T, HDV, 64, ATTN_TILE_FINE, ATTN_TILE_COARSE><<<mgrid, 256, 0, st>>>(p);              \
         }                                                                                        \
     } while (0)

@@ -62,6 +62,8 @@ CASES = {
     "some_tile": (torch.bfloat16, 36, 4, 64, 32, [(9 + (i * 53) % 370, 2 + i % 5) for i in range(32)], 0),
     "many": (torch.bfloat16, 8, 8, 64, 32, [(1 + (i * 37) % 700, 1) for i in range(256)], 0),
     "many_tile": (torch.float16, 40, 8, 64, 32, [(7 + (i * 53) % 400, 1 + i % 7) for i in range(257)], 0),
+    # unsplit with more keys than are looked up at a time (1024)
+    "long_unsplit": (torch.bfloat16, 36, 4, 64, 32, [(1300 - i if i % 40 == 0 else 9 + (i * 53) % 200, 4 + i % 4) for i in range(128)], 0),
     # no keys, no queries, fewer keys than queries
     "holes": (torch.bfloat16, 8, 2, 128, 32, [(0, 2), (700, 1), (3, 4), (40, 0), (1200, 2), (0, 1)], 0),
     "holes_tile": (torch.bfloat16, 24, 1, 128, 32, [(0, 2), (700, 3), (40, 0), (2, 3), (1200, 2), (0, 1)], 0),
