@@ -23,7 +23,8 @@ struct AttnParams {
     const int32_t *cu_q, *cu_k;
     int max_keys, max_rg;      // streaming kernels: the keys and row groups of a sequence that the launch is sized for
     int n_wg;                  // workgroups that share the work
-    int whole;                 // no unit is split: row groups per (sequence, KV head); otherwise 0
+    int whole;                 // no unit is split and a workgroup's number says which is its own: row groups per
+                               // (sequence, KV head); 0: the units are found in the list
     int v_once;                // V is read nontemporally
     float *part;               // its partial results, two slots per workgroup: [rows][HD + 4]
 };

@@ -110,33 +110,32 @@ struct ListPlan {
 };
 // fine, coarse: the two granularities.  The list is cut at multiples of `fine` keys when every workgroup gets at
 // least `coarse` keys that way; otherwise at multiples of `coarse`, so that short units stay whole.
-// SPLIT, UNSPLIT: the launches that the caller is compiled for.
+// SPLIT, UNSPLIT: the launches that the caller is compiled for (p.whole: its direct way to the unit).
 template <bool BY_SEQ, bool SPLIT, bool UNSPLIT>
 __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int rows_per_unit, const int fine,
                                               const int coarse, const int who) {
     const int lane = lane_id();
     ListPlan pl;
-    if (UNSPLIT && (!SPLIT || p.whole)) {
+    if (UNSPLIT && p.whole) {
         // A workgroup per (sequence, KV head, row group that a sequence can have), found without the list: with
         // 512 sequences its scan cost every workgroup two rounds of 8 dependent loads (MANY, below).
         pl.g = 1 << 30;                       // (longer than any sequence: one step per unit, whatever its length)
         pl.total = 0x7fffffff;
         pl.share = 1;
         const int per_seq = p.KVH * p.whole, s = who / per_seq, l = who - s * per_seq;
+        // (the query lengths before s in front of everything that waits for the sequence's own)
+        int tok = 0;
+        if (!p.cu_k && p.q_lens)
+            for (int i = lane; i < s; i += 64) tok += max(p.q_lens[i], 0);
         const SeqCost c = seq_cost(p, s, rows_per_unit, pl.g);
         pl.found = l < __builtin_amdgcn_readfirstlane(c.cost);
-        int tok = s;
         if (p.cu_k) tok = p.cu_q[s];
-        else if (p.q_lens) {
-            tok = 0;
-            for (int i = lane; i < s; i += 64) tok += max(p.q_lens[i], 0);
-            tok = lane_value(wave_scan(tok), 63);
-        }
+        else tok = p.q_lens ? lane_value(wave_scan(tok), 63) : s;
         pl.at = SeqAt{s, __builtin_amdgcn_readfirstlane(c.L), __builtin_amdgcn_readfirstlane(c.ql),
                       __builtin_amdgcn_readfirstlane(c.rg), 1, who - l, __builtin_amdgcn_readfirstlane(tok)};
         return pl;
     }
-    pl.g = fine;
+    pl.g = SPLIT ? fine : 1 << 30;                        // (unsplit: each unit is one step)
     SeqCost c0 = seq_cost(p, lane, rows_per_unit, pl.g);
     int s0, total;
     for (;;) {
@@ -144,7 +143,7 @@ __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int row
         total = lane_value(s0, 63);
         for (int b = 64; b < p.n_seqs; b += 64)
             total += lane_value(wave_scan(seq_cost(p, b + lane, rows_per_unit, pl.g).cost), 63);
-        if (pl.g == coarse || total >= (coarse / fine) * p.n_wg) break;
+        if (!SPLIT || pl.g == coarse || total >= (coarse / fine) * p.n_wg) break;
         pl.g = coarse;
         seq_steps(p, c0, coarse);
     }
@@ -552,6 +551,11 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
         q.n = min(end - q.pos, q.sq.steps - q.step);
         q.key = pl.g * q.step;
         q.key_end = q.step + q.n == q.sq.steps ? q.sq.L : pl.g * (q.step + q.n);
+        // (no further than the unit's last row sees: the row groups of a long query stop one after the other)
+        if (q.sq.rg > 1) {
+            const int r = q.sq.rg - 1 - q.unit % q.sq.rg, last = min(q.sq.ql, (ROWS * (r + 1) - 1) / p.Gq + 1);
+            q.key_end = min(q.key_end, q.sq.L - q.sq.ql + last);
+        }
     };
     auto next_piece = [&](Cursor &q) {
         q.pos += q.n;
@@ -577,7 +581,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
     float4_t o[NDB];
     auto begin_piece = [&]() {
         kvh = now.unit / now.sq.rg;
-        const int rg = now.unit - kvh * now.sq.rg;
+        const int rg = now.sq.rg - 1 - (now.unit - kvh * now.sq.rg);     // those with the most keys first
         const int rows_total = now.sq.ql * p.Gq, row0 = rg * ROWS + 16 * wave;
         const int row = row0 + c;
         active = row0 < rows_total;
@@ -738,7 +742,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     const ListPlan pl = list_plan<true, true, false>(p, ROWS, FINE, COARSE, seq);
     const SeqAt &sq = pl.at;
     if (rg >= sq.rg) return;
-    const int a = sq.first + (kvh * sq.rg + rg) * sq.steps;        // list positions of the unit's steps
+    const int a = sq.first + (kvh * sq.rg + sq.rg - 1 - rg) * sq.steps;        // list positions of the unit's steps
     const int wa = a / pl.share, wb = (a + sq.steps - 1) / pl.share;
     if (wa == wb) return;
     const int row = (int)blockIdx.z * RPW + (int)threadIdx.x / TPR, d = 4 * ((int)threadIdx.x % TPR);
@@ -812,11 +816,23 @@ static AttnForm attn_form(int64_t rows, int64_t kv_bytes) {
     return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_WHOLE, true};
 }
 
-// (row groups are not counted here: max_q_len may be far above what the sequences have.  But list positions are 32
-// bits wide: a list that could grow past 2^30 steps stays whole as well, with 2^18 units and more even on 131072 keys)
-static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t rg, int64_t max_keys) {
+// Long queries (row groups at sight of more and more keys): nothing is split once the units fill the chip, from
+// (keys - 320) / 4 units on, 300 at most (unsplit / split, us; 32 / 4 heads: 400 keys 50 units 13.2 / 13.9, 800 keys 68
+// 21.0 / 18.2, 128 21.3 / 23.1, 1600 keys 200 36.9 / 33.7, 400 43.9 / 53.2, 3200 keys 200 70 / 52, 400 81 / 92, 3200
+// 220 / 648).  But max_q_len may be far above what the sequences have, all tokens of the call by default; so only
+// where the query can be more than 1 / LONG of the keys (16 sequences of 4000 keys, 8 queries, bounded by 128: 34
+// split, 110 as one workgroup per unit before; the other way round 16 of 2000 keys with 100 queries of 4 heads take
+// 105 split and would take 87 unsplit).  With LONG_RG row groups and more the units are found in the list, at
+// most LISTED shares of them: workgroups without one end after its scan.
+// In the other rules row groups are not counted.  List positions are 32 bits wide: a list that could grow past 2^30
+// steps stays whole, with 2^18 units and more even on 131072 keys.
+#define ATTN_LONG 16
+#define ATTN_LONG_RG 4
+#define ATTN_LISTED 16384
+static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t rg, int64_t max_q, int64_t max_keys) {
     const int64_t units = n_seqs * kvh, steps = (max_keys + f.fine - 1) / f.fine;
     if (max_keys <= f.whole || units >= ATTN_MANY || units * rg * steps > (1LL << 30)) return true;
+    if (f.tile && ATTN_LONG * max_q > max_keys && 4 * units * rg >= min(max_keys - 320, (int64_t)1200)) return true;
     return f.tile ? max_keys <= min(3 * units, (int64_t)2048) : units >= 128 && max_keys <= 1024;
 }
 
@@ -829,15 +845,16 @@ struct AttnPlan {
     bool split;                   // units may be split: partial results and a merge
     size_t bytes;                 // workspace that splitting takes
 };
-// rows: query rows per KV head of a sequence, max_keys: keys of a sequence, both at most
-static AttnPlan attn_plan(int64_t n_seqs, int64_t rows, int64_t max_keys, int kvh, int head_dim) {
+// max_q, max_keys: query tokens and keys of a sequence at most; Gq: query heads per KV head
+static AttnPlan attn_plan(int64_t n_seqs, int64_t max_q, int Gq, int64_t max_keys, int kvh, int head_dim) {
     AttnPlan pl;
+    const int64_t rows = max_q * Gq;
     pl.kv_bytes = attn_kv_bytes(n_seqs, max_keys, kvh, head_dim);
     pl.f = attn_form(rows, pl.kv_bytes);
     pl.rg = (rows + pl.f.rows - 1) / pl.f.rows;
     pl.steps = (max_keys + pl.f.fine - 1) / pl.f.fine;
     pl.units = n_seqs * kvh * pl.rg;
-    pl.split = !attn_keep_whole(pl.f, n_seqs, kvh, pl.rg, max_keys);
+    pl.split = !attn_keep_whole(pl.f, n_seqs, kvh, pl.rg, max_q, max_keys);
     pl.bytes = pl.split ? odsd_round_up((size_t)2 * ATTN_WG * pl.f.rows * (head_dim + 4) * sizeof(float), 256) : 0;
     return pl;
 }
@@ -851,7 +868,7 @@ static bool attn_plan_shape_ok(int32_t n_seqs, int32_t max_q_len, int64_t max_ke
 static size_t attn_workspace_bytes(int32_t n_seqs, int32_t max_q_len, int64_t max_keys, int32_t num_heads,
                                    int32_t num_kv_heads, int32_t head_dim) {
     if (!attn_plan_shape_ok(n_seqs, max_q_len, max_keys, num_heads, num_kv_heads, head_dim)) return 0;
-    const AttnPlan pl = attn_plan(n_seqs, (int64_t)max_q_len * (num_heads / num_kv_heads), max_keys, num_kv_heads, head_dim);
+    const AttnPlan pl = attn_plan(n_seqs, max_q_len, num_heads / num_kv_heads, max_keys, num_kv_heads, head_dim);
     return pl.split ? pl.bytes : 256;
 }
 
@@ -863,9 +880,9 @@ extern "C" size_t odsd_paged_attention_workspace_bytes(int32_t n_seqs, int32_t m
 }
 
 // p: everything but Gq, n_wg, part; max_keys: no sequence has more
-static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_t rows, int64_t max_keys, bool aligned,
+static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_t max_q, int64_t max_keys, bool aligned,
                               void *workspace, size_t workspace_bytes, hipStream_t st) {
-    const AttnPlan pl = attn_plan(p.n_seqs, rows, max_keys, p.KVH, head_dim);
+    const AttnPlan pl = attn_plan(p.n_seqs, max_q, p.H / p.KVH, max_keys, p.KVH, head_dim);
     const AttnForm &f = pl.f;
     const int64_t rg = pl.rg, units = pl.units, kv_bytes = pl.kv_bytes;
     p.Gq = p.H / p.KVH;
@@ -886,8 +903,11 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         p.whole = 0;
     } else {
         if (units > 0x7fffffff) return ODSD_ERR_UNSUPPORTED;
-        p.n_wg = (int)units;                                          // each a workgroup of its own, finished in place
-        p.whole = (int)rg;
+        // each a workgroup of its own, finished in place; the bound on the row groups may be far above what there
+        // is, so with many of them the units are found in the list
+        const bool list = rg >= ATTN_LONG_RG;
+        p.n_wg = (int)(list ? min(units, (int64_t)ATTN_LISTED) : units);
+        p.whole = list ? 0 : (int)rg;
     }
     const unsigned grid = (unsigned)min((int64_t)p.n_wg, units * pl.steps);
     // (keys that fit the 256 MB memory-side cache may still be there from the call before)
@@ -906,7 +926,7 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         else {                                                                                   \
             if (merge) attn_tile_kernel<T, HDV, true><<<grid, 256, 0, st>>>(p);                  \
             else attn_tile_kernel<T, HDV, false><<<grid, 256, 0, st>>>(p);                       \
-            if (merge) attn_merge_kernel<T, HDV, 64, ATTN_TILE_FINE, ATTN_TILE_COARSE><<<mgrid, 256, 0, st>>>(p);              \
+            if (merge) attn_merge_kernel<T, HDV, 64, ATTN_TILE_FINE, ATTN_TILE_COARSE><<<mgrid, 256, 0, st>>>(p); \
         }                                                                                        \
     } while (0)
     if (dtype == ODSD_DT_F16) {
@@ -944,9 +964,8 @@ extern "C" int odsd_paged_attention(const void *q, const void *k_cache, const vo
     p.n_seqs = n_seqs; p.H = num_heads; p.KVH = num_kv_heads; p.max_blocks = max_blocks;
     p.block_size = block_size; p.num_slots = num_slots;
     p.scale_log2e = softmax_scale * 1.4426950408889634f;
-    return attn_stream_launch(p, dtype, head_dim, (int64_t)max_q_len * (num_heads / num_kv_heads),
-                              (int64_t)max_blocks * block_size, block_size % 32 == 0, workspace, workspace_bytes,
-                              (hipStream_t)stream);
+    return attn_stream_launch(p, dtype, head_dim, max_q_len, (int64_t)max_blocks * block_size, block_size % 32 == 0,
+                              workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 // ---- variable-length (prefill) form ----------------------------------------------------------------
@@ -982,5 +1001,5 @@ extern "C" int odsd_varlen_attention(const void *q, const void *k, const void *v
         ODSD_CHECK_LAUNCH();
         return ODSD_OK;
     }
-    return attn_stream_launch(p, dtype, head_dim, rows, max_seqlen_k, true, workspace, workspace_bytes, (hipStream_t)stream);
+    return attn_stream_launch(p, dtype, head_dim, max_seqlen_q, max_seqlen_k, true, workspace, workspace_bytes, (hipStream_t)stream);
 }

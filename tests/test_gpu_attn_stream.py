@@ -148,6 +148,69 @@ def test_calls_that_can_do_without_a_workspace(dev, name, seqs):
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
 
 
+# long queries: (heads, KV heads, head size, (context_len, q_len) per sequence); row groups of 64 rows see more keys one after
+# the other, and their steps in the list follow
+LONG = {
+    "whole_sequences": (8, 1, 64, [(900, 900), (333, 333), (64, 64)]),
+    "75_row_groups": (16, 2, 64, [(1500, 600), (700, 300), (1200, 1)]),
+    "3_heads": (6, 2, 128, [(1100, 400), (600, 23)]),
+    "more_queries_than_keys": (8, 1, 64, [(150, 400), (0, 70), (700, 500), (5, 130)]),
+    "coarse": (16, 2, 128, [(2000, 12), (1000, 40)]),
+    "unsplit": (16, 2, 64, [(250, 250), (100, 17), (256, 90)]),
+}
+
+
+@pytest.mark.parametrize("name", list(LONG))
+def test_paged_attention_long_queries(dev, name):
+    import on_device_sd_amd as odsd
+    H, KVH, HD, seqs = LONG[name]
+    print("attention, long queries", name, flush=True)
+    q, kc, vc, ctx, mq, ref = _case(dev, torch.bfloat16, H, KVH, HD, 32, seqs, seed=len(name))
+    out = odsd.paged_attention(q, kc, vc, ctx, KVH, 32, max_q_len=mq)
+    # probabilities and output are rounded to bf16: 2^-9 of values up to ~4
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+    again = odsd.paged_attention(q, kc, vc, ctx, KVH, 32)        # the default bound on the query lengths: all tokens
+    assert (again.float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+def test_more_units_than_workgroups(dev):
+    """16896 units in one unsplit call: a workgroup takes two of them in turn."""
+    import on_device_sd_amd as odsd
+    n, H, KVH, HD, bs, q_len = 64, 64, 8, 64, 32, 264
+    lens = [q_len + (i * 5) % 40 for i in range(n)]
+    nbs = [-(-L // bs) for L in lens]
+    first = np.concatenate([[0], np.cumsum(nbs)])
+    bt = torch.full((n, max(nbs)), -1, dtype=torch.int32)
+    for i in range(n):
+        bt[i, :nbs[i]] = torch.arange(first[i], first[i + 1]).flip(0)
+    g = torch.Generator(device=dev).manual_seed(7)
+    mk = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    q, kc, vc = mk(n * q_len, H, HD), mk(int(first[-1]) * bs, KVH * HD), mk(int(first[-1]) * bs, KVH * HD)
+    ctx = {"block_tables": bt.to(dev), "context_lens": torch.tensor(lens, dtype=torch.int32, device=dev),
+           "verify_query_lens": torch.full((n,), q_len, dtype=torch.int32, device=dev)}
+    print("more units than workgroups", flush=True)
+    out = odsd.paged_attention(q, kc, vc, ctx, KVH, bs, max_q_len=q_len)
+    kc, vc = kc.cpu(), vc.cpu()
+    for s in (0, 31, 63):
+        rows = slice(s * q_len, (s + 1) * q_len)
+        ref = orc.paged_attention(q[rows].cpu(), kc, vc, [bt[s].tolist()], [lens[s]], [q_len], KVH, bs, HD ** -0.5)
+        assert (out[rows].float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("keys", [250, 700])
+def test_rows_do_not_touch_keys_past_their_group(dev, keys):
+    """A row group stops at the 32-key tile of its last visible key: an infinity in a later V row does not reach it
+    as 0 x inf (unsplit, and in shares)."""
+    import on_device_sd_amd as odsd
+    q, kc, vc, ctx, mq, _ = _case(dev, torch.bfloat16, 8, 1, 64, 32, [(keys, keys)])
+    bt = ctx["block_tables"].cpu()[0]
+    last = keys // 32 * 32 + 1                        # a key of the last tile
+    vc[int(bt[last // 32]) * 32 + last % 32] = float("inf")
+    out = odsd.paged_attention(q, kc, vc, ctx, 1, 32, max_q_len=mq)
+    print("infinity in V at key", last, flush=True)
+    assert torch.isfinite(out[:keys // 32 * 32 - 8].float()).all()
+
+
 # (q_len, k_len) per sequence; 8 heads per KV head
 PACKED = {
     "stream_whole": (2, [(1, 300), (2, 64), (1, 512)]),
@@ -176,7 +239,7 @@ def test_packed_offsets_that_do_not_begin_at_zero(dev, name):
     mq, mk = max(a for a, _ in seqs), max(b for _, b in seqs)
     lib = _lib.load()
     nbytes = lib.odsd_varlen_attention_workspace_bytes(len(seqs), mq, mk, H, KVH, HD)
-    assert (nbytes > 256) == (name.endswith("split") or name == "prefill")
+    assert name == "prefill" or (nbytes > 256) == name.endswith("split")
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
     cq, ck = torch.from_numpy(cu_q + q_first).to(dev), torch.from_numpy(cu_k + k_first).to(dev)
