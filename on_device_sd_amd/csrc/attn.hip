@@ -733,18 +733,31 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
 // Merge of the pieces of a unit: out[row] = sum_s exp2(m_s - m) O_s / sum_s exp2(m_s - m) l_s, pieces in
 // order.  One workgroup per (sequence, KV head, unit, 1024 / HD rows): a thread owns 4 neighbouring output
 // elements of a row and walks the pieces, 4 at a time.  Units that were finished in place are left alone.
-template <typename T, int HD, int ROWS, int FINE, int COARSE>
+// BY_SHARE: one workgroup per bound between two shares instead, and 1024 / HD rows; the first bound inside a unit
+// does the work.  (For launches that allow for many row groups, which need not be there: 64 sequences of 8
+// queries with the query lengths bounded by the 512 tokens of the call only, 900 keys: 131072 workgroups
+// otherwise, 96 us the call.)
+template <typename T, int HD, int ROWS, int FINE, int COARSE, bool BY_SHARE = false>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     constexpr int XROW = HD + 4;
     constexpr int TPR = HD / 4, RPW = 256 / TPR;
-    const int seq = blockIdx.x / p.KVH, kvh = blockIdx.x - seq * p.KVH;
-    const int rg = blockIdx.y;
-    const ListPlan pl = list_plan<true, true, false>(p, ROWS, FINE, COARSE, seq);
+    int kvh, rg, a;                                                // a: list position of the unit's first step
+    const ListPlan pl = list_plan<!BY_SHARE, true, false>(p, ROWS, FINE, COARSE, BY_SHARE ? blockIdx.x + 1 : blockIdx.x / p.KVH);
     const SeqAt &sq = pl.at;
-    if (rg >= sq.rg) return;
-    const int a = sq.first + (kvh * sq.rg + sq.rg - 1 - rg) * sq.steps;        // list positions of the unit's steps
+    if (BY_SHARE) {
+        if (!pl.found) return;
+        const int at = ((int)blockIdx.x + 1) * pl.share - sq.first, unit = at / sq.steps;
+        kvh = unit / sq.rg;
+        rg = sq.rg - 1 - (unit - kvh * sq.rg);
+        a = sq.first + unit * sq.steps;
+    } else {
+        kvh = blockIdx.x % p.KVH;
+        rg = blockIdx.y;
+        if (rg >= sq.rg) return;
+        a = sq.first + (kvh * sq.rg + sq.rg - 1 - rg) * sq.steps;
+    }
     const int wa = a / pl.share, wb = (a + sq.steps - 1) / pl.share;
-    if (wa == wb) return;
+    if (wa == wb || (BY_SHARE && wa != (int)blockIdx.x)) return;
     const int row = (int)blockIdx.z * RPW + (int)threadIdx.x / TPR, d = 4 * ((int)threadIdx.x % TPR);
     const int r = rg * ROWS + row;
     if (row >= ROWS || r >= sq.ql * p.Gq) return;
@@ -926,7 +939,9 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         else {                                                                                   \
             if (merge) attn_tile_kernel<T, HDV, true><<<grid, 256, 0, st>>>(p);                  \
             else attn_tile_kernel<T, HDV, false><<<grid, 256, 0, st>>>(p);                       \
-            if (merge) attn_merge_kernel<T, HDV, 64, ATTN_TILE_FINE, ATTN_TILE_COARSE><<<mgrid, 256, 0, st>>>(p); \
+            if (merge && units > 2 * ATTN_WG)                                                    \
+                attn_merge_kernel<T, HDV, 64, ATTN_TILE_FINE, ATTN_TILE_COARSE, true><<<dim3(ATTN_WG - 1, 1, mgrid.z), 256, 0, st>>>(p); \
+            else if (merge) attn_merge_kernel<T, HDV, 64, ATTN_TILE_FINE, ATTN_TILE_COARSE><<<mgrid, 256, 0, st>>>(p); \
         }                                                                                        \
     } while (0)
     if (dtype == ODSD_DT_F16) {

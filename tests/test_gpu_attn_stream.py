@@ -173,6 +173,17 @@ def test_paged_attention_long_queries(dev, name):
     assert (again.float().cpu() - ref).abs().max().item() <= 2e-2
 
 
+def test_merge_with_a_loose_bound_on_the_queries(dev):
+    """Split units under a bound that allows for 38 row groups each: the merge walks the bounds of the shares."""
+    import on_device_sd_amd as odsd
+    seqs = [(40 + (i * 397) % 1500, 1 + (i * 7) % 20) for i in range(16)] + [(0, 3), (1500, 0), (7, 9)]
+    q, kc, vc, ctx, _, ref = _case(dev, torch.bfloat16, 16, 2, 64, 32, seqs, pad_blocks=160)
+    print("merge, loose bound on the queries", flush=True)
+    out = odsd.paged_attention(q, kc, vc, ctx, 2, 32, max_q_len=300)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+    assert torch.equal(out, odsd.paged_attention(q, kc, vc, ctx, 2, 32, max_q_len=300))
+
+
 def test_more_units_than_workgroups(dev):
     """16896 units in one unsplit call: a workgroup takes two of them in turn."""
     import on_device_sd_amd as odsd
