@@ -66,7 +66,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     [n_seqs, max_blocks], ``context_lens`` int32 [n_seqs] and, for a verify step,
     ``verify_query_lens`` int32 [n_seqs] (absent: one query token per sequence).  Returns
     [n_tokens, num_heads, head_dim] in the dtype of q.  ``max_q_len`` bounds the query lengths
-    (default: n_tokens, which is always safe)."""
+    (default: the context's ``max_query_len``, else n_tokens, which is always safe; a decode step needs none)."""
     if not (q.is_cuda and k_cache.is_cuda and v_cache.is_cuda):
         raise RuntimeError("paged attention runs on the GPU only (there is no CPU fallback)")
     n_tokens, num_heads, head_dim = q.shape
@@ -85,11 +85,12 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         return out
     scale = head_dim ** -0.5 if softmax_scale is None else softmax_scale
     lib = _lib.load()
-    # max_q_len sizes the launch: rows of a sequence beyond it would not be computed.  Without the
-    # caller's bound n_tokens is used (no sequence can hold more); a bound that came with the context
-    # (the builders below know the lengths on the host) is taken; lengths that are readable without a
-    # device synchronisation are checked against an explicit bound.
-    mq = max_q_len or context.get("max_query_len") or n_tokens
+    # max_q_len sizes the launch and chooses the kernel: rows of a sequence beyond it would not be
+    # computed.  Without query lengths there is one token per sequence; without the caller's bound
+    # n_tokens is used (no sequence can hold more); a bound that came with the context (the builders
+    # below know the lengths on the host) is taken; lengths that are readable without a device
+    # synchronisation are checked against an explicit bound.
+    mq = 1 if q_lens is None else max_q_len or context.get("max_query_len") or n_tokens
     if max_q_len and q_lens is not None and not q_lens.is_cuda and q_lens.numel() and int(q_lens.max()) > max_q_len:
         raise ValueError(f"max_q_len={max_q_len} is below the longest query ({int(q_lens.max())} tokens)")
     nbytes = lib.odsd_paged_attention_workspace_bytes(n_seqs, mq, num_heads, num_kv_heads, head_dim, block_size,

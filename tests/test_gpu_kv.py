@@ -122,6 +122,37 @@ def test_paged_attention_vs_oracle(dev, dtype, H, KVH, HD, bs, seqs):
     assert torch.equal(out, out2)
 
 
+@pytest.mark.parametrize("max_q_len", [None, 5])
+def test_decode_step_without_a_bound_is_one_token_per_sequence(dev, monkeypatch, max_q_len):
+    """A decode context that carries no max_query_len: the kernel is chosen for one query token per sequence,
+    not for all tokens of the call, whatever bound comes along."""
+    import on_device_sd_amd as odsd
+    from on_device_sd_amd import _lib
+    H, KVH, HD, bs, n = 16, 2, 128, 32, 24
+    g = torch.Generator().manual_seed(5)
+    lens = [1 + (i * 97) % 700 for i in range(n)]
+    bt = torch.arange(n * 22, dtype=torch.int32).view(n, 22)
+    kc, vc = (torch.randn(n * 22 * bs, KVH * HD, generator=g).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(n, H, HD, generator=g).to(torch.bfloat16)
+    lib, seen = _lib.load(), []
+
+    class Recorder:
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+        def odsd_paged_attention(self, *a):
+            seen.append(a[7])
+            return lib.odsd_paged_attention(*a)
+
+    monkeypatch.setattr(_lib, "load", lambda: Recorder())
+    ctx = {"block_tables": bt.to(dev), "context_lens": torch.tensor(lens, dtype=torch.int32, device=dev)}
+    print("decode without a bound", max_q_len, flush=True)
+    out = odsd.paged_attention(q.to(dev), kc.to(dev), vc.to(dev), ctx, KVH, bs, max_q_len=max_q_len)
+    ref = orc.paged_attention(q, kc, vc, bt.numpy(), lens, None, KVH, bs, HD ** -0.5)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+    assert seen == [1]
+
+
 VARLEN_CASES = [
     # dtype, H, KVH, HD, (q_len, k_len) per sequence
     (torch.bfloat16, 32, 4, 128, [(300, 300), (1, 1), (77, 77)]),            # Qwen3-30B-A3B heads, ragged prefill batch

@@ -161,8 +161,10 @@ def test_verify_step_equals_successive_decode_steps(dev):
         ctx_d = {"block_tables": bt, "context_lens": torch.tensor([c + j + 1 for c in cached], dtype=torch.int32, device=dev)}
         qj = q.view(len(cached), d, NHq, D)[:, j].contiguous()
         out_d = odsd.paged_attention(qj, kc, vc, ctx_d, KV, bs)
-        diff = (out_d.float() - out_v[:, j].float()).abs().max().item()
-        assert diff <= 4e-3, (j, diff)      # different key slicing and rounding points, same sums
+        diff = (out_d.float() - out_v[:, j].float()).abs()
+        # different kernels (8 query rows per KV head, 48 in the verify step), key slicing and rounding points, same sums: 4e-3 for those,
+        # and two sums that close may still round to neighbouring bf16 values, at most 2^-7 of the value apart
+        assert (diff <= 4e-3 + 2.0 ** -7 * out_v[:, j].float().abs()).all(), (j, diff.max().item())
 
 
 def test_verify_step_under_inference_mode(dev):
