@@ -813,7 +813,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
 // Form of the kernel by the query rows of a sequence and the bytes that the keys can have
 struct AttnForm {
     int rows;            // per unit
-    int fine, whole;
+    int fine, coarse, whole;
     bool tile;
 };
 static int64_t attn_kv_bytes(int64_t n_seqs, int64_t max_keys, int kvh, int head_dim) {
@@ -825,8 +825,8 @@ static AttnForm attn_form(int64_t rows, int64_t kv_bytes) {
     // 1500 40.9 / 42.5; 16 / 8 heads of 64, 64 of 1000 33.3 / 21.4; 32 / 4 heads, 64 of 2000 68.3 / 62.6, but 16 of
     // 1000, 33 MB, 17.3 / 19.9)
     const bool wide = rows > 16 && rows <= 32 && kv_bytes > (96LL << 20);
-    if (rows <= 16 || wide) return AttnForm{wide ? 32 : 16, ATTN_STREAM_FINE, ATTN_STREAM_WHOLE, false};
-    return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_WHOLE, true};
+    if (rows <= 16 || wide) return AttnForm{wide ? 32 : 16, ATTN_STREAM_FINE, ATTN_STREAM_COARSE, ATTN_STREAM_WHOLE, false};
+    return AttnForm{64, ATTN_TILE_FINE, ATTN_TILE_COARSE, ATTN_TILE_WHOLE, true};
 }
 
 // Long queries (row groups at sight of more and more keys): nothing is split once the units fill the chip, from
@@ -853,7 +853,8 @@ static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t 
 // number of keys: the form, whether units are split and the workspace belong together.
 struct AttnPlan {
     AttnForm f;
-    int64_t rg, units, steps;     // row groups per (sequence, KV head), units, list steps of the longest unit
+    int64_t rg, units;            // row groups per (sequence, KV head), units
+    int shares;                   // workgroups that can get a share of the list
     int64_t kv_bytes;
     bool split;                   // units may be split: partial results and a merge
     size_t bytes;                 // workspace that splitting takes
@@ -865,10 +866,13 @@ static AttnPlan attn_plan(int64_t n_seqs, int64_t max_q, int Gq, int64_t max_key
     pl.kv_bytes = attn_kv_bytes(n_seqs, max_keys, kvh, head_dim);
     pl.f = attn_form(rows, pl.kv_bytes);
     pl.rg = (rows + pl.f.rows - 1) / pl.f.rows;
-    pl.steps = (max_keys + pl.f.fine - 1) / pl.f.fine;
     pl.units = n_seqs * kvh * pl.rg;
     pl.split = !attn_keep_whole(pl.f, n_seqs, kvh, pl.rg, max_q, max_keys);
-    pl.bytes = pl.split ? odsd_round_up((size_t)2 * ATTN_WG * pl.f.rows * (head_dim + 4) * sizeof(float), 256) : 0;
+    // a list too short for the fine granularity is cut at the coarse one, and no workgroup has less than one step
+    int64_t total = pl.units * ((max_keys + pl.f.fine - 1) / pl.f.fine);
+    if (total < (int64_t)(pl.f.coarse / pl.f.fine) * ATTN_WG) total = pl.units * ((max_keys + pl.f.coarse - 1) / pl.f.coarse);
+    pl.shares = (int)min(total, (int64_t)ATTN_WG);
+    pl.bytes = pl.split ? odsd_round_up((size_t)2 * pl.shares * pl.f.rows * (head_dim + 4) * sizeof(float), 256) : 0;
     return pl;
 }
 static bool attn_plan_shape_ok(int32_t n_seqs, int32_t max_q_len, int64_t max_keys, int32_t num_heads,
@@ -922,7 +926,7 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         p.n_wg = (int)(list ? min(units, (int64_t)ATTN_LISTED) : units);
         p.whole = list ? 0 : (int)rg;
     }
-    const unsigned grid = (unsigned)min((int64_t)p.n_wg, units * pl.steps);
+    const unsigned grid = (unsigned)(merge ? pl.shares : p.n_wg);
     // (keys that fit the 256 MB memory-side cache may still be there from the call before)
     p.v_once = kv_bytes > (100 << 20);
     const dim3 mgrid((unsigned)(p.n_seqs * p.KVH), (unsigned)rg, (unsigned)((f.rows * head_dim + 1023) / 1024));

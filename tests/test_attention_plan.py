@@ -1,5 +1,7 @@
 """The workspace that an attention call asks for is the one that its launch uses (host side only, no GPU):
 sizes around the bounds where the kernel form and the splitting of units change."""
+import random
+
 import pytest
 import torch
 
@@ -69,3 +71,31 @@ def test_a_list_of_shares_fits_32_bits():
         steps = n * 4 * ((q * 8 + 63) // 64) * (blocks * 256 // 32)
         assert (steps <= 1 << 30) == split
         assert (size(n, q, 32, 4, 128, 256, blocks) > NOTHING) == split, (n, q, blocks)
+
+
+def test_the_workspace_holds_every_share_and_little_more():
+    """Two slots of partial results for each workgroup that gets a share: the list restated for random lengths
+    within the bounds (steps of 128 keys up to 32 query rows; above, of 32 keys when every workgroup gets 256
+    that way, else of 256; 512 workgroups)."""
+    size = _lib.load().odsd_paged_attention_workspace_bytes
+    rng = random.Random(1)
+    for n, q, heads, kvh, hd, keys in ((1, 8, 32, 4, 128, 4096), (1, 1, 32, 4, 128, 4000), (3, 5, 16, 2, 128, 1500),
+                                       (32, 8, 32, 4, 128, 2048), (2, 30, 8, 1, 64, 3000), (7, 1, 8, 8, 64, 700)):
+        group = heads // kvh
+        rows = 16 if q * group <= 16 else 64
+        slot = rows * (hd + 4) * 4
+        slots = size(n, q, heads, kvh, hd, 1, keys) / slot
+        fine, coarse = (128, 128) if rows == 16 else (32, 256)
+
+        def shares(lens, qs):
+            units = [kvh * -(-t * group // rows) for t in qs]
+            steps = lambda g: sum(u * max(1, -(-L // g)) for u, L in zip(units, lens))
+            total = steps(fine) if steps(fine) >= coarse // fine * 512 else steps(coarse)
+            share = max(1, -(-total // 512))
+            return -(-total // share)
+
+        assert 2 * shares([keys] * n, [q] * n) <= slots <= 1025
+        for _ in range(300):
+            assert 2 * shares([rng.randint(0, keys) for _ in range(n)], [rng.randint(0, q) for _ in range(n)]) <= slots
+    assert size(1, 8, 32, 4, 128, 256, 16) == 2 * 64 * 64 * 132 * 4          # one sequence of 4096 keys: 64 shares, 4.3 MB
+    assert size(32, 8, 32, 4, 128, 256, 8) == 2 * 512 * 64 * 132 * 4
