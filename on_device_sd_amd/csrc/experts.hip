@@ -736,6 +736,15 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
         int KS = 1;
         while (tiles_dn * p.PS_dn * KS < slots && KS * 2 <= G_dn / 4 && KS < 16) KS *= 2;
         p.KS = KS;
+        // Popular experts have several passes where the mean has one, and a workgroup that takes them in turn ends
+        // long after the others: four workgroups share them, whatever the mean (those without a pass come last
+        // and only look at the row count).  Layer, us, the streaming kernel's 128-row passes before / one / two / four /
+        // eight: E = 128, H = 2048, I = 768, Zipf, T = 1000 254 / 273 / 215 / 186 / 186, T = 2000 454 / 501 / 358 / 318 / 291,
+        // T = 4000 852 / 766 / 670 / 572 / 520; H = 4096, I = 1536, Zipf, T = 2000 1116 / 1145 / 988 / 925 / 885; on uniform
+        // routing four cost nothing (T = 1000 146 / 145), eight up to 1 % (H = 4096, T = 848 411 / 416).
+        const int share = 4;
+        p.PS_gu = p.PS_gu < share ? share : p.PS_gu;
+        p.PS_dn = p.PS_dn < share ? share : p.PS_dn;
     } else {
         const long wg_gu = active * ((2 * s->I / 16 + 15) / 16);
         if (wg_gu < 4 * slots) p.NB = 2;

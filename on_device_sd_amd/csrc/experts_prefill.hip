@@ -41,15 +41,17 @@ __global__ __launch_bounds__(256, 2) void w4_gemm_prefill_kernel(const GemmParam
     constexpr int XS_BUF = MAXNM * 32 * 256;   // one group of the token rows
     __shared__ __attribute__((aligned(16))) char xs[2 * XS_BUF];
 
-    // consecutive logical ids stay on one XCD: the row tiles of one expert share its token rows
+    // consecutive logical ids stay on one XCD: the row tiles of one expert share its token rows.  Everyone's
+    // first passes come before anyone's second: a workgroup without a pass then costs the end of the launch
+    // a look at the row count, and not the others a place.
     const int b = blockIdx.x;
-    const int L = (b & 7) * p.wg_per_xcd + (b >> 3);
+    const int ps = (b >> 3) / p.wg_per_xcd;
+    const int L = (b & 7) * p.wg_per_xcd + (b >> 3) - ps * p.wg_per_xcd;
     if (L >= p.n_wg) return;
     // row chunks innermost: neighbours share the token rows of one (expert, pass, K slice)
     const int chunk = L % p.nchunks;
     const int ks = (L / p.nchunks) % p.KS;
-    const int ps = (L / (p.nchunks * p.KS)) % p.PS;
-    const int e = L / (p.nchunks * p.KS * p.PS);
+    const int e = L / (p.nchunks * p.KS);
 
     // requested together: one round trip to memory instead of three dependent ones
     const uint64_t *trow = p.table + (size_t)e * ODSD_TABLE_COLS;
@@ -263,9 +265,9 @@ template <int MODE>
 void odsd_launch_gemm_prefill(GemmParams &gp, hipStream_t st) {
     gp.nchunks = (gp.NBLK + 15) / 16;
     if (gp.PS < 1) gp.PS = 1;
-    gp.n_wg = gp.E * gp.nchunks * gp.KS * gp.PS;
+    gp.n_wg = gp.E * gp.nchunks * gp.KS;
     gp.wg_per_xcd = (gp.n_wg + 7) / 8;
-    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_gemm_prefill_kernel<MODE>), gp.wg_per_xcd * 8, 256, st, gp);
+    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_gemm_prefill_kernel<MODE>), gp.wg_per_xcd * 8 * gp.PS, 256, st, gp);
 }
 
 template void odsd_launch_gemm_prefill<0>(GemmParams &, hipStream_t);

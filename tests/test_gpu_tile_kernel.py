@@ -13,6 +13,7 @@ COUNTS = {
     "blocks": [1, 31, 32, 33, 64, 65, 96, 97, 128, 0, 129, 160, 257, 385],
     "passes": [129, 255, 256, 300],
     "lone": [77],
+    "hot": [700, 3, 1090, 0, 60, 1],       # up to nine passes of one expert, shared by four workgroups
 }
 
 
