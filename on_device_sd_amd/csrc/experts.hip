@@ -69,10 +69,11 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
     __shared__ int32_t wsum[2][DISP ? WAVES : 1];        // DISP: per-wavefront totals (pairs of e, pairs below e)
 
     // workgroup -> (expert, row chunk, k split).  Hardware deals workgroups round-robin over
-    // the 8 XCDs: the chunks of one expert are spread over all of them.  (Keeping an expert's rows
+    // the 8 XCDs: the chunks of one expert are spread over all of them.  Keeping an expert's rows
     // in one L2 is worth nothing with few rows, and would leave an XCD idle for every expert
-    // without tokens.)
-    const int L = blockIdx.x;
+    // without tokens; with 128-row passes it is worth having.
+    const int b = blockIdx.x;
+    const int L = MB == 8 ? (b & 7) * p.wg_per_xcd + (b >> 3) : b;
     if (L >= p.n_wg) return;
     const int ks = L % p.KS;
     const int chunk = (L / p.KS) % p.nchunks;
@@ -688,13 +689,19 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     // streaming kernel's 64-row passes and the tile kernel, whole layer on uniform routing, us,
     // streaming / tile: Mixtral 25 rows per expert 180 / 202, 40 rows 200 / 215; Qwen3-30B 32 rows
     // 113 / 129, 62 rows 164 (128-row passes) / 157.
+    // A small gate_up (at most 512 pieces of 256 weight rows x 128 columns) leaves most CUs without a tile and its
+    // reduction ends before the tile kernel's pipeline is worth its start: there the streaming kernel takes up to 104
+    // rows in passes of 128 (128-row passes / tile: E = 8, H = 512, I = 1024 56 rows 28.2 / 30.0, 100 32.8 / 36.3, 134
+    // 39.9 / 36.6; H = I = 1024 64 rows 34.2 / 35.5; E = 32, H = I = 512 64 rows 31.1 / 32.5; twice the pieces: E = 8,
+    // H = 1024, I = 2048 64 rows 41.4 / 39.2, E = 64, H = I = 512 100 rows 53.0 / 48.4).
+    const long pieces_gu = (s->E < P ? s->E : P) * ((2 * s->I / 16 + 15) / 16) * (s->H / ODSD_GROUP);
     p.tile = 0;
     if (s->T <= 16) p.MB = 1;
     else if (s->T <= 32) p.MB = 2;
     else if (s->T <= 64) p.MB = 4;      // no expert can have more rows than a 64-row pass holds
     else if (mean_rows <= 16) p.MB = 2;
     else if (mean_rows <= 52) p.MB = 4;
-    else { p.MB = 8; p.tile = 1; }
+    else { p.MB = 8; p.tile = mean_rows > 104 || pieces_gu > 512; }
     const long active = s->E < P ? s->E : P;       // upper bound of experts with rows
     const long slots = 512;                        // 256 CUs x 2 workgroups
     const int G_gu = s->H / ODSD_GROUP, G_dn = s->I / ODSD_GROUP;
@@ -747,10 +754,11 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
         p.PS_dn = p.PS_dn < share ? share : p.PS_dn;
     } else {
         const long wg_gu = active * ((2 * s->I / 16 + 15) / 16);
-        if (wg_gu < 4 * slots) p.NB = 2;
+        if (wg_gu < 4 * slots || p.MB == 8) p.NB = 2;
         const int nchunks_dn = (s->H / 16 + 4 * p.NB - 1) / (4 * p.NB);
         int KS = 1;
-        while (KS * 2 <= G_dn / 2 && active * nchunks_dn * KS < 2 * slots && KS < 16) KS *= 2;   // up to 4 workgroups per CU
+        const long want = p.MB == 8 ? slots : 2 * slots;       // 2 workgroups per CU with eight token blocks, up to 4 with fewer
+        while (KS * 2 <= G_dn / 2 && active * nchunks_dn * KS < want && KS < 16) KS *= 2;
         p.KS = KS;
     }
     // every split must own at least one group
@@ -851,6 +859,8 @@ static void launch_gemm_plan(const ExpertsPlan &pl, GemmParams &gp, hipStream_t 
     } else if (pl.MB == 4) {
         if (pl.NB == 2) launch_gemm<2, 4, MODE, 2, 2, 1, false, 4>(gp, st);
         else launch_gemm<4, 4, MODE, 2, 2, 1, false, 2>(gp, st);
+    } else if (!pl.tile) {
+        launch_gemm<2, 8, MODE, 2, 2, 1, false, 2>(gp, st);
     } else {
         odsd_launch_gemm_prefill<MODE>(gp, st);
     }
@@ -870,7 +880,7 @@ static int experts_args_ok(const odsd_moe_shape *s) {
 static bool stream_dispatch_supported(const ExpertsPlan &pl, const odsd_moe_shape *s) {
     const int nb = pl.MB == 1 ? 2 : pl.NB;
     const int chunks = (2 * s->I / 16 + 4 * nb - 1) / (4 * nb);     // gate_up workgroups per expert
-    return !pl.tile && (pl.MB > 1 || pl.WK_gu == 0) && chunks <= STREAM_DISPATCH_CHUNKS && s->T * s->K <= 4 * 256;
+    return pl.MB <= 4 && (pl.MB > 1 || pl.WK_gu == 0) && chunks <= STREAM_DISPATCH_CHUNKS && s->T * s->K <= 4 * 256;
 }
 
 // idx + dispatch_out: the dispatch arrays have not been filled; the kernel dispatches for itself

@@ -1,5 +1,6 @@
-"""The tile kernel through the stage calls, with row counts that the caller sets: the edges of its 32-row blocks
-and 128-row passes, odd and single groups in the reduction, a weight matrix that ends inside a tile, a down
+"""The tile kernel, and the streaming kernel's 128-row passes that stand in for it where a call has few pieces of
+weights, through the stage calls with row counts that the caller sets: the edges of 16- and 32-row blocks and
+128-row passes, odd and single groups in the reduction, a weight matrix that ends inside a tile, a down
 reduction split over workgroups and passes shared by workgroups."""
 import numpy as np
 import pytest
@@ -10,7 +11,9 @@ from tests.helpers import canon_to_oracle
 pytestmark = pytest.mark.gpu
 
 COUNTS = {
+    # up to 104 rows per expert on average: 128-row passes of the streaming kernel (all sizes below)
     "blocks": [1, 31, 32, 33, 64, 65, 96, 97, 128, 0, 129, 160, 257, 385],
+    "tile_blocks": [1, 31, 32, 33, 64, 65, 96, 97, 128, 0, 129, 160, 257, 385, 500],
     "passes": [129, 255, 256, 300],
     "lone": [77],
     "hot": [700, 3, 1090, 0, 60, 1],       # up to nine passes of one expert, shared by four workgroups
