@@ -25,7 +25,7 @@ struct AttnParams {
     int n_wg;                  // workgroups that share the work
     int whole;                 // no unit is split and a workgroup's number says which is its own: row groups per
                                // (sequence, KV head); 0: the units are found in the list
-    int v_once;                // V is read nontemporally
+    int v_once;                // tile kernel: V is read nontemporally (the stream form always does)
     float *part;               // its partial results, two slots per workgroup: [rows][HD + 4]
 };
 
@@ -38,7 +38,6 @@ template <> struct AttnT<half_t> {
     __device__ static __forceinline__ float16_t mfma32(V8 a, V8 b, float16_t c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
-    __device__ static __forceinline__ uint16_t from_f32(float v) { return __builtin_bit_cast(uint16_t, (half_t)v); }
     // two values, round to nearest even, as one 32-bit word (a in the low half)
     __device__ static __forceinline__ uint32_t pack2(float a, float b) {
         typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -54,7 +53,6 @@ template <> struct AttnT<__bf16> {
     __device__ static __forceinline__ float16_t mfma32(V8 a, V8 b, float16_t c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
-    __device__ static __forceinline__ uint16_t from_f32(float v) { return f32_to_bf16(v); }
     __device__ static __forceinline__ uint32_t pack2(float a, float b) {   // v_cvt_pk_bf16_f32
         typedef __bf16 b2 __attribute__((ext_vector_type(2)));
         typedef float f2 __attribute__((ext_vector_type(2)));

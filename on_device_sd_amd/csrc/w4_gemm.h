@@ -126,8 +126,6 @@ __device__ __forceinline__ float silu_f32(float g) { return g / (1.0f + __expf(-
 // s_waitcnt vmcnt(N) only (gfx9 encoding: vmcnt = bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
 #define ODSD_WAIT_VMCNT_LGKM0(N) \
     __builtin_amdgcn_s_waitcnt(((N) & 0xF) | (((N) >> 4) << 14) | (7 << 4) | (0x0 << 8))
-#define ODSD_WAIT_LGKM0() \
-    __builtin_amdgcn_s_waitcnt(0xF | (3 << 14) | (7 << 4) | (0x0 << 8))
 #define ODSD_WAIT_VMCNT(N) \
     __builtin_amdgcn_s_waitcnt(((N) & 0xF) | (((N) >> 4) << 14) | (7 << 4) | (0xF << 8))
 

@@ -11,9 +11,9 @@ from tests.helpers import canon_to_oracle
 pytestmark = pytest.mark.gpu
 
 COUNTS = {
-    # up to 104 rows per expert on average: 128-row passes of the streaming kernel (all sizes below)
     "blocks": [1, 31, 32, 33, 64, 65, 96, 97, 128, 0, 129, 160, 257, 385],
-    "tile_blocks": [1, 31, 32, 33, 64, 65, 96, 97, 128, 0, 129, 160, 257, 385, 500],
+    # up to 104 rows per expert on average (and "lone"): the streaming kernel's passes
+    "stream_blocks": [1, 15, 16, 17, 31, 33, 64, 65, 96, 112, 113, 127, 128, 0, 129, 160, 257],
     "passes": [129, 255, 256, 300],
     "lone": [77],
     "hot": [700, 3, 1090, 0, 60, 1],       # up to nine passes of one expert, shared by four workgroups
