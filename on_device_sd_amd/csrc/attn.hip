@@ -4,8 +4,8 @@
 // A query row is one (token, query head) pair of a KV head's group; up to 16, 32 or 64 rows of one
 // (sequence, KV head) -- a unit -- are worked on together, so one pass over the keys serves a whole group
 // of query heads and all draft tokens.  What the kernels have to do is stream K and V from HBM.  The keys
-// of all units are laid end to end and dealt out in equal contiguous shares to as many workgroups as the
-// chip holds at once.  A share may begin and end in the middle of a unit: such pieces leave partial results
+// of all units are laid end to end and dealt out in equal contiguous shares to 512 workgroups, two per
+// CU.  A share may begin and end in the middle of a unit: such pieces leave partial results
 // that a second kernel merges, whole units are finished in place.  Sequences of mixed lengths then cost
 // what their bytes cost; with a fixed number of slices per sequence, as before, the longest sequence set
 // the time.  Two forms:
@@ -14,7 +14,8 @@
 //     memory straight into the registers that S^T = K Q^T wants as its A operand (v_mfma_f32_16x16x32); V
 //     goes through a piece of LDS that belongs to the wavefront, because O^T = V^T P^T needs its transpose
 //     (ds_read_b64_tr_b16).  A tile's registers are refilled as soon as it has been multiplied (K) or put
-//     into LDS (V); three wavefronts per SIMD hide what is left of the latency;
+//     into LDS (V); what is left of the latency is hidden by two wavefronts per SIMD, three (what registers and
+//     LDS allow) where nothing is split;
 //   * more rows, attn_tile_kernel: a wavefront cannot hold the rows next to its keys, so the workgroup
 //     shares the keys through LDS.
 // In both the scores of one query row stay in the 4 lanes that share lane % 16, in the order in which P^T
@@ -23,7 +24,9 @@
 // Measured (32 query / 4 KV heads of 128, bf16, kernel + merge, before -> now): 64 sequences of 750 to 3000
 // keys, one query each, 263 MB: 64.1 -> 47.5 us (the kernel alone 6.1 TB/s: bound by HBM); 64 of 2048
 // keys 53.3 -> 45.9; one of 4000 13.9 -> 13.0; 16 of 300 13.3 -> 7.7 (no merge).  32 sequences of 512 to 2048
-// keys x 8 queries, 85 MB: 31.8 -> 30.8: start-up, pieces and merge are as long as the stream there.
+// keys x 8 queries, 85 MB: 31.8 -> 30.8: start-up, pieces and merge are as long as the stream there.  Block sizes that
+// are no multiple of 32 (ALIGNED false) spill 28 bytes per lane at head size 128 and still gain: block size 16, 64
+// sequences of 750 to 3000 keys 68.5 -> 61.6, of 125 to 500 18.1 -> 13.6, with 32 / 8 heads 115 -> 106.5.
 //
 // Paged form: the cache is addressed through the sequence's block table exactly as the reference
 // gathers it: position p lives in slot block_table[p / block_size] * block_size + p % block_size.
@@ -44,8 +47,9 @@
 // of 300 keys, decode, 7.7 us whole against 10.2 split.)  With more units nothing is split up to more
 // keys, and with MANY never: they fill the chip and level mixed lengths out by themselves.  (attn_keep_whole;
 // 32 / 4 heads of 128, split / whole, us.  Stream form: 40 sequences of up to 700 keys 15.2 / 12.6, 64 of 1000
-// 21.1 / 18.8, 384 of 700 67.9 / 58.2, but 128 of 2000 59.7 / 62.2.  Tile form, 8 queries each: 48 of 700 22.6 /
-// 24.7, 64 of 700 28.3 / 25.4, 64 of 1000 32.2 / 39.7, 128 of 700 46.4 / 34.0, 256 of 1500 151 / 129.)
+// 21.1 / 18.8, 384 of 700 67.9 / 58.2, but 128 of 2000 59.7 / 62.2.  Tile form, 8 queries each: 16 of 300 15.0 /
+// 11.3, of 700 17.5 / 19.3; 32 of 700 20.4 / 19.5, of 1000 21.4 / 25.6; 48 of 1000 29.4 / 25.8, of 1500 34.1 / 40.3; 64 of
+// 1500 42.4 / 42.3; 96 of 2000 80 / 72; 128 of 700 48.3 / 28.9, of 2000 101 / 83; 256 of 1500 158 / 121.)
 #define ATTN_STREAM_FINE 128
 #define ATTN_STREAM_COARSE 128
 #define ATTN_STREAM_WHOLE 512
@@ -846,7 +850,7 @@ static bool attn_keep_whole(const AttnForm &f, int64_t n_seqs, int kvh, int64_t 
     const int64_t units = n_seqs * kvh, steps = (max_keys + f.fine - 1) / f.fine;
     if (max_keys <= f.whole || units >= ATTN_MANY || units * rg * steps > (1LL << 30)) return true;
     if (f.tile && ATTN_LONG * max_q > max_keys && 4 * units * rg >= min(max_keys - 320, (int64_t)1200)) return true;
-    return f.tile ? max_keys <= min(3 * units, (int64_t)2048) : units >= 128 && max_keys <= 1024;
+    return f.tile ? max_keys <= min(192 + 5 * units, (int64_t)2048) : units >= 128 && max_keys <= 1024;
 }
 
 // What a call does, from its shape alone.  The size functions and the launch both ask here, with the same
@@ -927,7 +931,9 @@ static int attn_stream_launch(AttnParams &p, int32_t dtype, int head_dim, int64_
         p.whole = list ? 0 : (int)rg;
     }
     const unsigned grid = (unsigned)(merge ? pl.shares : p.n_wg);
-    // (keys that fit the 256 MB memory-side cache may still be there from the call before)
+    // Up to 100 MB of keys may still be in the 256 MB memory-side cache from the call before; more are read past it:
+    // 32 sequences of 2048 keys, 134 MB, 37.3 us where other keys came before (41.6 without the hint), 36.8 where the
+    // same call did (34.2).  A model has other layers' keys in between.
     p.v_once = kv_bytes > (100 << 20);
     const dim3 mgrid((unsigned)(p.n_seqs * p.KVH), (unsigned)rg, (unsigned)((f.rows * head_dim + 1023) / 1024));
 #define ATTN_GO(T, HDV, RBV)                                                                     \
