@@ -80,6 +80,7 @@ class W4ExpertBank:
                        self.dn_q[e].data_ptr(), self.dn_sz[e].data_ptr())
                       for e in range(self.num_experts)]
         self._params: Dict[int, W4ExpertParams] = {}
+        self._device_index = self.gu_q.get_device()
 
     def clone(self) -> "W4ExpertBank":
         """A second copy of the packed weights in HBM (same contents, its own storage)."""
@@ -117,8 +118,8 @@ class W4ExpertBank:
                     keep_canonical: bool = False):
         """Quantise one expert's [I,H], [I,H], [H,I] weights on the device and pack them: in one launch, or
         through the canonical arrays when the caller wants those as well."""
-        here = self.gu_q.device                     # (with its index: another GPU's tensor has to move as well)
-        ws = [w if w.device == here else w.to(here) for w in (gate_w, up_w, down_w)]
+        # (by index, -1 for the host: another GPU's tensor has to move as well)
+        ws = [w if w.get_device() == self._device_index else w.to(self.gu_q.device) for w in (gate_w, up_w, down_w)]
         if keep_canonical:
             canon = tuple(ops.w4_quantize(w) for w in ws)
             self.load_canonical(e, *canon)

@@ -196,11 +196,14 @@ def test_load_expert_brings_weights_to_the_bank(monkeypatch):
             self.device, self.shape, self.moved = torch.device(device), torch.Size(shape), moved
             self.is_cuda = self.device.type == "cuda"
 
+        def get_device(self):
+            return self.device.index if self.is_cuda else -1
+
         def to(self, device):
             return Weight(device, self.shape, moved=True)
 
     bank = odsd.W4ExpertBank(2, 256, 128, "cpu")
-    bank.gu_q = Weight("cuda:0", bank.gu_q.shape)       # as if the bank lived on the first GPU
+    bank.gu_q, bank._device_index = Weight("cuda:0", bank.gu_q.shape), 0       # as if the bank lived on the first GPU
     seen = []
     monkeypatch.setattr(ops, "w4_load_expert", lambda *a: seen.append(a[:3]))
     monkeypatch.setattr(ops, "w4_quantize", lambda w: w)
