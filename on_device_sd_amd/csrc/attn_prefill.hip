@@ -14,9 +14,9 @@
 //   * V^T as the A operand through ds_read_b64_tr_b16 (no transposed copy).
 // Against the decode / verify kernel, which ran these calls before: twice the rows per wavefront, so a
 // fragment read from LDS feeds an MFMA of twice the flops, and a barrier covers four times the work.
-// Bound by the two wavefronts a SIMD has room for: matrix unit busy 55 % and vector issue 50 % of the
-// time, at a clock that the load takes down to 1.7 GHz; two thirds of the vector instructions are the
-// exponentials and their scaling.  (32-key tiles with three wavefronts per SIMD: + 3 % at 4096 tokens,
+// Bound by the two wavefronts a SIMD has room for: matrix unit busy 53 % and vector issue 41 % of the
+// cycles with workgroups (46 % and 36 % of all), no bank conflict; two thirds of the vector instructions
+// are the exponentials and their scaling.  (32-key tiles with three wavefronts per SIMD: + 3 % at 4096 tokens,
 // - 10 % below 2000; raised wavefront priority round the MFMAs: - 1 to - 5 %.)
 // Measured, causal flops, 32 query / 4 KV heads of 128, bf16, before -> now: 8192 tokens 812 -> 486 us
 // (1130 TFLOP/s), 4096 tokens 236 -> 137, three sequences of 1200 to 3000 206 -> 120, 300 tokens

@@ -19,10 +19,10 @@
 //
 // What bounds it: before, weights went expanded through LDS (192 KB read + 64 KB written per 64-column
 // stage of 2048 matrix cycles, the 128 bytes per cycle that LDS has).  Now LDS reads are half of that,
-// and the matrix unit is busy 58 % of the time at the 1.6 GHz that the load takes the clock down to
+// and the matrix unit is busy 71 % of the cycles (down: 63 %) at the 1.4 GHz that the load takes the clock down to
 // (Qwen3-235B experts, T = 4096: gate_up 987 -> 830 us, 990 TFLOP/s, down 578 -> 425 us, 970 TFLOP/s;
 // the library's fp16 product of 8192^3 reaches 1160 on the same card).  At 62 rows per expert vector
-// and matrix instructions share the time (57 % and 49 % of the cycles with workgroups).
+// and matrix instructions share the time (53 % each of the cycles with workgroups).
 // Variants: one wavefront per SIMD with 256 token rows per pass, i.e. half the expansion: 1.50 against
 // 1.45 ms for that layer (nothing runs under its barriers, prologue and epilogue).
 //

@@ -110,9 +110,9 @@ __global__ __launch_bounds__(256) void w4_pack_kernel(const uint8_t *__restrict_
 // kq = l/16) reads columns 32j + 8kq .. + 7 of row r (j = 0..3), which are exactly the codes of its
 // four packed words, so the group's minimum and maximum need two exchanges between lanes and the tile
 // leaves as one contiguous 1 KiB store.  Consecutive wavefronts take consecutive groups of a row
-// block.  16 experts of [768, 2048] in bf16: 115 us, bound by the host's 7 us per call (kernel 6.0 us,
-// 12 MB: launch, one round trip and the divisions; 7.4 us with the compiler's division).  As three
-// quantise and three pack launches with a canonical copy in between, 96 calls in all, 766 us.
+// block.  16 experts of [768, 2048] in bf16: 92.5 us, 16 kernels of 6.0 us minus what overlaps (12 MB each:
+// launch, one round trip and the divisions; 7.4 us with the compiler's division).  As three
+// quantise and three pack launches with a canonical copy in between, 96 calls in all, 715 us.
 // -----------------------------------------------------------------------------------------
 struct LoadMatrix {
     const void *w;
