@@ -670,6 +670,7 @@ struct ExpertsPlan {
     int tile;        // the tile kernel (experts_prefill.hip) instead of the streaming kernel
     int y_f16;       // down-projection outputs kept as fp16 (unsplit reduction) instead of fp32 partials
     int fused;       // whole-block calls run gate_up and down as one launch (experts_fused.hip)
+    int share;       // equal-share streaming kernel (experts_share.hip) for gate_up and down
     int S;           // fused: workgroups per expert = fp16 partial-sum slices of the down projection
     size_t h_bytes, y_bytes;
 };
@@ -678,6 +679,10 @@ struct ExpertsPlan {
 void odsd_launch_experts_fused(FusedParams &fp, int E, hipStream_t st);
 int odsd_fused_supported(int H, int I, int S, int E);
 int odsd_fused_dispatch_supported(int P);
+// equal-share streaming kernel (experts_share.hip)
+int odsd_share_supported(int H, int I, int E, int P);
+int odsd_share_down_splits(int I);
+void odsd_launch_share(int mode, GemmParams &gp, hipStream_t st);
 
 // Choices are functions of the shape only (the per-expert counts live on the device).
 static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
@@ -760,6 +765,18 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
         const long want = p.MB == 8 ? slots : 2 * slots;       // 2 workgroups per CU with eight token blocks, up to 4 with fewer
         while (KS * 2 <= G_dn / 2 && active * nchunks_dn * KS < want && KS < 16) KS *= 2;
         p.KS = KS;
+    }
+    // Equal shares (experts_share.hip) where its splits of the reductions exist and a pass of 16 rows holds most experts:
+    // up to 12 rows per expert on average.  Whole layer, us, the plan above / equal shares: H = 2048, I = 768, E = 128,
+    // K = 8: T = 1 30.7 / 24.5, T = 8 47.3 / 42.5, T = 24 69.5 / 59.6, T = 64 77.8 / 72.5, T = 112 77.2 / 74.2, Zipf
+    // T = 100 90.2 / 78.8; H = 4096, I = 1536: T = 4 77.4 / 66.6, T = 32 216 / 187, T = 160 256 / 235, T = 192 (12 rows)
+    // 259 / 248, T = 256 269 / 323; H = 4096, I = 14336, E = 8, K = 2: T = 1 58.8 / 50.1, T = 5 115.7 / 99.0, T = 40
+    // 152 / 135, T = 48 (12 rows) 153 / 146, T = 56 153 / 169.  From 14 rows on too many experts take a second pass
+    // over their weights, which the plan above saves with wider ones.
+    p.share = 0;
+    if (mean_rows <= 12 && odsd_share_supported(s->H, s->I, s->E, (int)P)) {
+        p.share = 1;
+        p.KS = odsd_share_down_splits(s->I);
     }
     // every split must own at least one group
     while (p.KS > 1 && ((G_dn + p.KS - 1) / p.KS) * (p.KS - 1) >= G_dn) p.KS--;
@@ -844,6 +861,7 @@ template <int MODE>
 static void launch_gemm_plan(const ExpertsPlan &pl, GemmParams &gp, hipStream_t st) {
     const int wk = MODE == 0 ? pl.WK_gu : pl.WK_dn;
     gp.y_f16 = pl.y_f16;
+    if (pl.share) { odsd_launch_share(MODE, gp, st); return; }
     if (pl.MB == 1 && wk == 0) {
         if (MODE == 0 || pl.NB_dn == 2) launch_gemm<2, 1, MODE, 3, 2, 1, false, 4>(gp, st);
         else if constexpr (MODE == 1) launch_gemm<1, 1, MODE, 3, 1, 1, false, 4>(gp, st);
@@ -878,6 +896,7 @@ static int experts_args_ok(const odsd_moe_shape *s) {
 // expert it costs gate_up more than the launch it saves: +7 us at the Mixtral T = 160 shape, +6 us
 // at T = 5, so those plans keep the dispatch kernel)
 static bool stream_dispatch_supported(const ExpertsPlan &pl, const odsd_moe_shape *s) {
+    if (pl.share) return true;
     const int nb = pl.MB == 1 ? 2 : pl.NB;
     const int chunks = (2 * s->I / 16 + 4 * nb - 1) / (4 * nb);     // gate_up workgroups per expert
     return pl.MB <= 4 && (pl.MB > 1 || pl.WK_gu == 0) && chunks <= STREAM_DISPATCH_CHUNKS && s->T * s->K <= 4 * 256;
