@@ -104,13 +104,18 @@ static int moe_forward_impl(const odsd_moe_shape *s, const void *x, const void *
     // expert ids themselves and leave counts / offsets / perm (inv and slot_token are not produced:
     // nothing after the experts reads them); otherwise the router launch dispatches as well (with few
     // tokens inside its top-k kernel, else by the dispatch kernel)
-    const OdsdDispatchOut inside{counts, offsets, perm, nullptr, nullptr};
+    OdsdDispatchOut inside{counts, offsets, perm, nullptr, nullptr};
     const OdsdDispatchOut outside{counts, offsets, perm, inv, slot_token};
     const bool dispatch_inside = odsd_experts_dispatch_inside(s) && odsd_aligned16(idx);
+    // (with few tokens the expert kernel does the top-k as well)
+    const bool route_inside = dispatch_inside && odsd_experts_route_inside(s);
+    int route_S = 0;
     int rc = odsd_launch_router(s, xin, gate_w, idx, w, nullptr, prepared ? nullptr : x16, ws + l.router,
                                 l.xn - l.router, st, fold ? row_sumsq_in : nullptr, norm_weight, eps,
-                                nullptr, dispatch_inside ? nullptr : &outside);
+                                nullptr, dispatch_inside ? nullptr : &outside, route_inside ? &route_S : nullptr);
     if (rc != ODSD_OK) return rc;
+    inside.partial = (const double *)(ws + l.router);
+    inside.route_S = route_S;
     // (the combine runs after this block's last reader of xn and x16, so it may overwrite them in place)
     const OdsdNextNorm nn{next_norm_w, eps, ws + l.xn, x16};
     return odsd_launch_experts(s, x16, table, idx, w, counts, offsets, perm, slot_token,

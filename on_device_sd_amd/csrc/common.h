@@ -127,6 +127,10 @@ struct OdsdDispatchOut {
     // (mirror_tag << 32) | counts[e], so a reader that knows the tag can tell when entry e has arrived
     int64_t *counts_mirror;
     uint32_t mirror_tag;
+    // dispatch inside the expert kernel: it routes as well (odsd_experts_route_inside), from the partial logits
+    // [route_S][T][E] that odsd_launch_router has left in the router's workspace, and fills idx and w
+    const double *partial;
+    int route_S;
 };
 // What the combine of a block leaves for the block after it when it is told that block's RMSNorm
 // (calls that run a stack of blocks): the normalised rows in the activation dtype and their fp16 copy.
@@ -135,11 +139,12 @@ struct OdsdNextNorm {
     float eps;
     void *xn, *x16;
 };
-// router (+ dispatch when `disp` is given)
+// router (+ dispatch when `disp` is given); logits_only: nothing but the partial logits, *logits_only of them per
+// logit, at the beginning of ws
 int odsd_launch_router(const odsd_moe_shape *s, const void *x, const void *gate_w, int32_t *idx,
                        float *w, int64_t *idx64, void *x16, void *ws, size_t ws_bytes,
                        hipStream_t st, const double *norm_ss, const void *norm_w, float eps,
-                       double *logits = nullptr, const OdsdDispatchOut *disp = nullptr);
+                       double *logits = nullptr, const OdsdDispatchOut *disp = nullptr, int *logits_only = nullptr);
 int odsd_launch_dispatch(const odsd_moe_shape *s, const int32_t *idx, int32_t *counts,
                          int32_t *offsets, int32_t *perm, int32_t *inv, int32_t *slot_token,
                          hipStream_t st, int64_t *counts_mirror = nullptr, uint32_t mirror_tag = 0u);
@@ -153,3 +158,4 @@ int odsd_launch_experts(const odsd_moe_shape *s, const void *x16, const uint64_t
                         const OdsdDispatchOut *dispatch_out = nullptr, const OdsdNextNorm *next_norm = nullptr);
 int odsd_combine_norm_supported(const odsd_moe_shape *s);
 int odsd_experts_dispatch_inside(const odsd_moe_shape *s);
+int odsd_experts_route_inside(const odsd_moe_shape *s);

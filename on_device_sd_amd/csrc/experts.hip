@@ -683,6 +683,7 @@ int odsd_fused_dispatch_supported(int P);
 int odsd_share_supported(int H, int I, int E, int P);
 int odsd_share_down_splits(int I);
 void odsd_launch_share(int mode, GemmParams &gp, hipStream_t st);
+int odsd_share_route_supported(int T, int E);
 
 // Choices are functions of the shape only (the per-expert counts live on the device).
 static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
@@ -904,9 +905,10 @@ static bool stream_dispatch_supported(const ExpertsPlan &pl, const odsd_moe_shap
 
 // idx + dispatch_out: the dispatch arrays have not been filled; the kernel dispatches for itself
 // and leaves counts / offsets / perm in dispatch_out
+// (route_S in dispatch_out: idx and w have not been filled either; the kernel leaves them there)
 static int launch_gate_up(const odsd_moe_shape *s, const void *x_f16, const uint64_t *table,
                           const int32_t *counts, const int32_t *offsets, const int32_t *slot_token,
-                          void *h_f16, hipStream_t st, const int32_t *idx, const OdsdDispatchOut *dispatch_out) {
+                          void *h_f16, hipStream_t st, const int32_t *idx, const float *w, const OdsdDispatchOut *dispatch_out) {
     const int rc = experts_args_ok(s);
     if (rc != ODSD_OK) return rc;
     if (s->T == 0) return ODSD_OK;
@@ -926,6 +928,12 @@ static int launch_gate_up(const odsd_moe_shape *s, const void *x_f16, const uint
         if (!odsd_aligned16(idx)) return ODSD_ERR_ALIGN;
         gu.idx = idx;
         gu.out_counts = dispatch_out->counts; gu.out_offsets = dispatch_out->offsets; gu.out_perm = dispatch_out->perm;
+        if (dispatch_out->route_S > 0) {
+            if (!pl.share || !odsd_share_route_supported(s->T, s->E)) return ODSD_ERR_UNSUPPORTED;
+            if (!w || !dispatch_out->partial) return ODSD_ERR_NULL;
+            gu.partial = dispatch_out->partial; gu.route_S = dispatch_out->route_S; gu.renorm = s->renorm; gu.T = s->T;
+            gu.route_idx = const_cast<int32_t *>(idx); gu.route_w = const_cast<float *>(w);
+        }
     }
     launch_gemm_plan<0>(pl, gu, st);
     ODSD_CHECK_LAUNCH();
@@ -935,7 +943,7 @@ static int launch_gate_up(const odsd_moe_shape *s, const void *x_f16, const uint
 extern "C" int odsd_w4_gate_up_silu(const odsd_moe_shape *s, const void *x_f16, const uint64_t *table,
                                     const int32_t *counts, const int32_t *offsets,
                                     const int32_t *slot_token, void *h_f16, void *stream) {
-    return launch_gate_up(s, x_f16, table, counts, offsets, slot_token, h_f16, (hipStream_t)stream, nullptr, nullptr);
+    return launch_gate_up(s, x_f16, table, counts, offsets, slot_token, h_f16, (hipStream_t)stream, nullptr, nullptr, nullptr);
 }
 
 extern "C" int32_t odsd_w4_down_splits(const odsd_moe_shape *s) {
@@ -1081,7 +1089,7 @@ int odsd_launch_experts(const odsd_moe_shape *s, const void *x16, const uint64_t
         ODSD_CHECK_LAUNCH();
         return launch_combine(s, y, idx, w, perm, table, residual, out_f32, out_act, row_ss, st, pl.S, nn);
     }
-    rc = launch_gate_up(s, x16, table, counts, offsets, slot_token, h16, st, idx, dispatch_out);
+    rc = launch_gate_up(s, x16, table, counts, offsets, slot_token, h16, st, idx, w, dispatch_out);
     if (rc != ODSD_OK) return rc;
     rc = odsd_w4_down(s, h16, table, counts, offsets, y, st);
     if (rc != ODSD_OK) return rc;
@@ -1094,6 +1102,13 @@ int odsd_experts_dispatch_inside(const odsd_moe_shape *s) {
     if (experts_check(s) != ODSD_OK) return 0;
     const ExpertsPlan pl = experts_plan(s);
     return pl.fused ? odsd_fused_dispatch_supported(s->T * s->K) : stream_dispatch_supported(pl, s);
+}
+
+// 1: it also does the top-k, from the router's partial logits
+int odsd_experts_route_inside(const odsd_moe_shape *s) {
+    if (experts_check(s) != ODSD_OK) return 0;
+    const ExpertsPlan pl = experts_plan(s);
+    return pl.share && !pl.fused && odsd_share_route_supported(s->T, s->E);
 }
 
 extern "C" int odsd_experts_w4(const odsd_moe_shape *s, const void *x_f16, const uint64_t *table,

@@ -26,6 +26,7 @@
 //   MODE 1  down: unit = RSUB * NB blocks of output rows, KS splits of the reduction across workgroups
 #include "w4_gemm.h"
 #include "w4_raw.h"
+#include "router_topk.h"
 
 #include <type_traits>
 
@@ -46,7 +47,8 @@ __device__ __forceinline__ int wave_prefix(int x) {
     return x;
 }
 
-template <int MODE, int GW, int WK, int NB, int DEPTH, bool DISP>
+// DISP  0: dispatch arrays are given; 1: from the id list; 2, 3: the top-k as well, E <= 64 / 128
+template <int MODE, int GW, int WK, int NB, int DEPTH, int DISP>
 __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const GemmParams p) {
     constexpr int WAVES = SHARE_WAVES, RSUB = WAVES / WK, UBLK = RSUB * NB;   // 16-row blocks of a unit
     constexpr int ROWS = 16, MAX_E = 64 * WAVES;     // one thread per expert in the prologue
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
     constexpr int MAXNI = DISP ? SHARE_MAX_P / (64 * WAVES) : 1;
     const int NI = DISP ? (p.P + 64 * WAVES - 1) / (64 * WAVES) : 0;
     int id[MAXNI], rank[MAXNI];
-    if (DISP) {
+    if (DISP == 1) {
 #pragma unroll
         for (int n = 0; n < MAXNI; ++n) {
             const int i = (wave * NI + n) * 64 + lane;
@@ -96,6 +98,21 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
     }
     if (MODE == 0 && !DISP)
         for (int i = tid; i < p.P; i += 64 * WAVES) list_lds[i] = (uint16_t)p.rowmap[i];
+    if (DISP >= 2) {
+        // every workgroup selects for every token; workgroup t leaves token t's experts and weights behind
+        for (int t = wave; t < p.T; t += WAVES) {
+            const bool mine = t == (int)blockIdx.x;
+            const int e = topk_token<(DISP >= 2 ? DISP - 1 : 1)>(p.partial, t, p.T, p.E, p.K, p.route_S, p.renorm, mine ? p.route_idx : nullptr,
+                                                                 mine ? p.route_w : nullptr, nullptr, nullptr);
+            if (lane < p.K) list_lds[t * p.K + lane] = (uint16_t)e;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < MAXNI; ++n) {
+            const int i = (wave * NI + n) * 64 + lane;
+            id[n] = n < NI && i < p.P ? (int)list_lds[i] : -1;
+        }
+    }
     if (DISP) {
         *(uint4_t *)&cntw_lds[wave][8 * lane] = uint4_t{0, 0, 0, 0};
 #pragma unroll
@@ -437,6 +454,10 @@ int odsd_share_supported(int H, int I, int E, int P) {
     return share_split(0, H / ODSD_GROUP, &u) && share_split(1, I / ODSD_GROUP, &d) && E <= 64 * SHARE_WAVES &&
            P <= SHARE_MAX_P && E + P / 16 <= SHARE_MAX_ITEMS;
 }
+// The top-k in gate_up's prologue, a token per wavefront: every workgroup repeats it, which costs less than the launch
+// it saves up to 8 tokens (layer, us, separate / inside: E = 128, H = 2048: T = 1 24.5 / 22.8, T = 8 42.5 / 41.7, T = 9
+// 44.1 / 44.7, T = 16 51.9 / 53.6; E = 8, H = 4096: T = 1 49.9 / 48.4, T = 5 99.4 / 97.2, T = 8 116.3 / 114.8).
+int odsd_share_route_supported(int T, int E) { return T <= SHARE_WAVES && E <= 128; }
 int odsd_share_down_splits(int I) {
     ShareSplit s;
     return share_split(1, I / ODSD_GROUP, &s) ? s.KS : 0;
@@ -450,11 +471,15 @@ static void share_go(GemmParams &gp, int KS, hipStream_t st) {
     gp.n_wg = SHARE_CUS / KS * KS;
     if constexpr (MODE == 0) {
         if (gp.idx) {
-            ODSD_LAUNCH(ODSD_KERNEL_GATE_UP, (w4_share_kernel<MODE, GW, WK, NB, DEPTH, true>), gp.n_wg, 64 * SHARE_WAVES, st, gp);
+#define SHARE_DISP_GO(DISP) ODSD_LAUNCH(ODSD_KERNEL_GATE_UP, (w4_share_kernel<MODE, GW, WK, NB, DEPTH, DISP>), gp.n_wg, 64 * SHARE_WAVES, st, gp)
+            if (gp.route_S == 0) SHARE_DISP_GO(1);
+            else if (gp.E <= 64) SHARE_DISP_GO(2);
+            else SHARE_DISP_GO(3);
+#undef SHARE_DISP_GO
             return;
         }
     }
-    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_share_kernel<MODE, GW, WK, NB, DEPTH, false>), gp.n_wg,
+    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_share_kernel<MODE, GW, WK, NB, DEPTH, 0>), gp.n_wg,
                 64 * SHARE_WAVES, st, gp);
 }
 

@@ -1,5 +1,5 @@
-// Pieces of the top-k selection shared by the router kernels: the order-preserving integer key of a
-// logit and the wavefront arg-max on (key, id).
+// The top-k selection shared by the router kernels and the expert kernels that route for themselves: the
+// order-preserving integer key of a logit, the wavefront arg-max on (key, id), the selection of a token.
 #pragma once
 #include "common.h"
 
@@ -62,4 +62,96 @@ __device__ __forceinline__ int wave_best(const uint64_t key, const int id) {
     const uint64_t who = __ballot(hi == top);
     if ((who & (who - 1)) == 0) return __builtin_amdgcn_readlane(id, __builtin_ctzll(who));
     return wave_argmax(key, id);
+}
+
+// V = logits per lane (experts lane, lane + 64, ...): 1, 2, 4 or 8 for E <= 64, 128, 256, 512
+// the selection for token t by one wavefront; lane k < K returns the k-th winner's expert id
+// (idx null: nothing but that)
+template <int V>
+__device__ __forceinline__ int topk_token(const double *__restrict__ partial, const int t, int T, int E,
+                                          int K, int S, int renorm, int32_t *__restrict__ idx,
+                                          float *__restrict__ w, int64_t *__restrict__ idx64,
+                                          double *__restrict__ logits) {
+    const int lane = lane_id();
+
+    double lg[V];
+    uint64_t key[V];
+    uint32_t taken = 0;   // bit v set: expert lane + 64 v already selected
+    // partial sums in slice order; the loads of one slice batch are independent of each other
+#pragma unroll
+    for (int v = 0; v < V; ++v) lg[v] = 0.0;
+    constexpr int SB = V <= 2 ? 8 : 4;   // slices loaded together
+    for (int s0 = 0; s0 < S; s0 += SB) {
+        double part[SB][V];
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const int e = lane + 64 * v;
+                part[u][v] = (e < E && s0 + u < S) ? partial[((size_t)(s0 + u) * T + t) * E + e] : 0.0;
+            }
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+#pragma unroll
+            for (int v = 0; v < V; ++v) lg[v] += part[u][v];
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        key[v] = order_key(lg[v]);
+        if (lane + 64 * v >= E) taken |= 1u << v;
+        else if (logits) logits[(size_t)t * E + lane + 64 * v] = lg[v];
+    }
+
+    int my_e = 0;          // lane k keeps the k-th winner
+    double my_l = 0.0;
+    double l_max = 0.0;
+    for (int k = 0; k < K; ++k) {
+        // best remaining candidate of this lane: largest key, then lowest expert.  A lane with
+        // nothing left offers key 0 (no finite logit maps to it) and the largest expert id.
+        uint64_t bk = 0;
+        int be = 0x7fffffff;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            if (!((taken >> v) & 1u)) {
+                if (be == 0x7fffffff || key[v] > bk) {
+                    bk = key[v];
+                    be = lane + 64 * v;
+                }
+            }
+        }
+        const int we = wave_best(bk, be);   // the same in every lane
+        // the winner's logit sits in lane (we & 63), slot (we >> 6)
+        double cand = lg[0];
+#pragma unroll
+        for (int v = 1; v < V; ++v) cand = (we >> 6) == v ? lg[v] : cand;
+        const uint64_t cb = (uint64_t)__double_as_longlong(cand);
+        const uint32_t wlo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cb, we & 63);
+        const uint32_t whi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cb >> 32), we & 63);
+        const double wl = __longlong_as_double((long long)(((uint64_t)whi << 32) | wlo));
+        if ((we & 63) == lane) taken |= 1u << (we >> 6);
+        if (lane == k) { my_e = we; my_l = wl; }
+        if (k == 0) l_max = wl;
+    }
+
+    if (!idx) return my_e;
+    // weights in fp32; differences are taken in fp64 before the cast
+    float num = 0.0f;
+    if (lane < K) num = expf((float)(my_l - l_max));
+    float den;
+    if (renorm) {
+        den = wave_sum(num);
+    } else {
+        float part = 0.0f;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (lane + 64 * v < E) part += expf((float)(lg[v] - l_max));
+        den = wave_sum(part);
+    }
+    if (lane < K) {
+        const size_t o = (size_t)t * K + lane;
+        idx[o] = my_e;
+        w[o] = num / den;
+        if (idx64) idx64[o] = (int64_t)my_e;
+    }
+    return my_e;
 }

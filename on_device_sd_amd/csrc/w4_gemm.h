@@ -35,6 +35,12 @@ struct GemmParams {
     const int32_t *idx;      // [P] expert id per (token, k) pair, or null
     int32_t *out_counts, *out_offsets, *out_perm;
     int K;
+    // ... and the routing too (route_S > 0): the fp64 partial logits [route_S][T][E]; the token's experts and
+    // weights are left in route_idx / route_w for the combine
+    const double *partial;
+    int route_S, renorm, T;
+    int32_t *route_idx;
+    float *route_w;
 };
 
 // Launch parameters of the one-launch expert kernel (experts_fused.hip)

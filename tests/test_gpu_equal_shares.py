@@ -1,7 +1,7 @@
 """Calls of few rows per expert at the edges of the equal-share kernel: fewer units than workgroups, shares that end
 inside an expert, experts with 16, 17 and more rows (further passes), experts without rows and without weights, every
 split of the two reductions that it has, the most experts and pairs it takes, the last average row count of its rule;
-with the dispatch inside (whole block) and with caller-made dispatch arrays (stage calls)."""
+with the routing (up to 8 tokens) and the dispatch inside (whole block) and with caller-made dispatch arrays (stage calls)."""
 import numpy as np
 import pytest
 import torch
@@ -34,6 +34,9 @@ def _bank(dev, H, E, I, g, distinct=6):
     (33, 2048, 16, 2, 768, 17),      # ... and with 17: a second pass of one row
     (96, 2048, 16, 2, 1536, 96),     # six passes over one expert; 12 rows on average, the last of the rule; 4 x 3 groups
     (7, 4096, 12, 3, 2048, 0),       # 32 groups in gate_up; 16 in down
+    (8, 2048, 128, 8, 768, 5),       # the most tokens that it routes for itself, and the most experts
+    (9, 2048, 65, 8, 768, 0),        # one token more
+    (8, 2048, 65, 64, 768, 0),       # the most choices per token
     (20, 4096, 8, 2, 4096, 18),      # two splits of the down reduction
     (40, 4096, 8, 2, 14336, 0),      # seven splits: 252 workgroups
     (64, 2048, 512, 8, 768, 3),      # the most experts
@@ -62,6 +65,7 @@ def test_equal_shares(dev, T, H, E, K, I, crowd):
     assert np.array_equal(out.counts.cpu().numpy(), counts)
     assert np.array_equal(out.offsets.cpu().numpy(), offsets)
     assert np.array_equal(out.perm.cpu().numpy(), perm)
+    assert np.allclose(out.w.cpu().numpy(), w, rtol=2e-6, atol=0)    # fp32 softmax of fp64 logits: a few units in the last place
     # h is rounded to fp16 once (2^-11): well inside the helper's 1e-2 of the largest and 2e-3 of the mean output
     check_output_relative(out.out_f32, ref)
     again = ops.moe_forward(xd, wgd, table, K, I, renorm=True)
