@@ -449,103 +449,84 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
 // out_act = cast(residual + cast(moe)): the reference rounds the MoE output to the
 // activation dtype before the residual add (qwen3_runner.py:295, :226).
 // ---------------------------------------------------------------------------------------------
-// KB > 0 (K a multiple of KB, KS == 1): the rows of KB pairs are fetched together -- slot, expert
-// and weight first, then KB independent row loads -- and added in k order; with the generic loop
-// every row load waits for the one before it (its address hangs on a branch), which is what the
-// kernel's time consists of at K = 8.
-// YH: 0 = y holds fp32 partial sums of KS slices; 1 = complete sums as fp16; 2 = KS fp16 slices (the
-// batched form, KB > 0, takes exactly two)
+// The rows of KB pairs (K is a multiple of KB) are fetched together -- slot, expert and weight first, then the
+// independent row loads of several slices -- and added in k order.  A row load that waits for the one before it
+// (with its address behind a branch, say) is what the kernel's time consists of: pair by pair, slice by slice / now,
+// us: K = 8, T = 256 7.6 / 6.3; K = 2: seven slices, T = 5 6.6 / 5.0; four, T = 160 6.9 / 5.3; two, T = 32, H = 512
+// 5.5 / 3.3.
+// YH: 0 = y holds fp32 partial sums of KS slices; 1 = complete sums as fp16; 2 = KS fp16 slices
 // Gather-sum of one token's columns c .. c+3: sum over k of w[t,k] * (sum over slices of y[slice][slot(t,k)]).
 template <int YH, int KB>
 __device__ __forceinline__ float4_t combine_gather(const float *__restrict__ y, const int32_t *__restrict__ idx,
                                                    const float *__restrict__ w, const int32_t *__restrict__ perm,
                                                    const uint64_t *__restrict__ table, const int t, const int c,
                                                    const int H, const int K, const int E, const int KS, const int P) {
-        float4_t acc = {0.f, 0.f, 0.f, 0.f};
-        if (KB > 0) {
-            for (int k0 = 0; k0 < K; k0 += KB) {
-                int slot[KB > 0 ? KB : 1];
-                float wk[KB > 0 ? KB : 1];
-                bool ok[KB > 0 ? KB : 1];
-                uint64_t tq[KB > 0 ? KB : 1];      // first table entry of the pair's expert: 0 = no weights
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < K; k0 += KB) {
+        int slot[KB];
+        float wk[KB];
+        bool ok[KB];
+        uint64_t tq[KB];      // first table entry of the pair's expert: 0 = no weights
 #pragma unroll
-                for (int u = 0; u < KB; ++u) {
-                    const int pr = t * K + k0 + u;
-                    const int sl = perm[pr];
-                    const int e = idx[pr];
-                    wk[u] = w[pr];
-                    // (the row's address must not wait for the table entry: that would be a third
-                    // dependent round trip to memory -- slot, then table, then row -- in a kernel that
-                    // consists of little else; a pair in range always has a row that exists)
-                    const bool in_range = sl >= 0 && e >= 0 && e < E;
-                    tq[u] = table[(size_t)(in_range ? e : 0) * ODSD_TABLE_COLS];
-                    ok[u] = in_range;
-                    slot[u] = in_range ? sl : 0;   // a row that exists; its values are discarded below
-                }
-                float4_t v[KB > 0 ? KB : 1];
-                if (YH == 2) {
-                    // two fp16 slices: all 2 KB row loads are issued before the first is used
-                    half4_t h0[KB > 0 ? KB : 1], h1[KB > 0 ? KB : 1];
+        for (int u = 0; u < KB; ++u) {
+            const int pr = t * K + k0 + u;
+            const int sl = perm[pr];
+            const int e = idx[pr];
+            wk[u] = w[pr];
+            // (the row's address must not wait for the table entry: that would be a third
+            // dependent round trip to memory -- slot, then table, then row -- in a kernel that
+            // consists of little else; a pair in range always has a row that exists)
+            const bool in_range = sl >= 0 && e >= 0 && e < E;
+            tq[u] = table[(size_t)(in_range ? e : 0) * ODSD_TABLE_COLS];
+            ok[u] = in_range;
+            slot[u] = in_range ? sl : 0;   // a row that exists; its values are discarded below
+        }
+        float4_t v[KB];
+        if (YH == 1 || (YH == 0 && KS == 1)) {
 #pragma unroll
-                    for (int u = 0; u < KB; ++u) {
-                        h0[u] = *(const half4_t *)((const half_t *)y + (size_t)slot[u] * H + c);
-                        h1[u] = *(const half4_t *)((const half_t *)y + ((size_t)P + slot[u]) * H + c);
-                    }
-#pragma unroll
-                    for (int u = 0; u < KB; ++u) {
-                        v[u] = float4_t{(float)h0[u].x, (float)h0[u].y, (float)h0[u].z, (float)h0[u].w};
-                        v[u] += float4_t{(float)h1[u].x, (float)h1[u].y, (float)h1[u].z, (float)h1[u].w};
-                    }
+            for (int u = 0; u < KB; ++u) {
+                if (YH) {
+                    const half4_t hv = *(const half4_t *)((const half_t *)y + (size_t)slot[u] * H + c);
+                    v[u] = float4_t{(float)hv.x, (float)hv.y, (float)hv.z, (float)hv.w};
                 } else {
-#pragma unroll
-                for (int u = 0; u < KB; ++u) {
-                    if (YH) {
-                        const half4_t hv = *(const half4_t *)((const half_t *)y + (size_t)slot[u] * H + c);
-                        v[u] = float4_t{(float)hv.x, (float)hv.y, (float)hv.z, (float)hv.w};
-                    } else {
-                        v[u] = *(const float4_t *)(y + (size_t)slot[u] * H + c);
-                    }
-                }
-                }
-#pragma unroll
-                for (int u = 0; u < KB; ++u) {
-                    if (ok[u] && tq[u] != 0) {
-                        acc.x = fmaf(wk[u], v[u].x, acc.x);
-                        acc.y = fmaf(wk[u], v[u].y, acc.y);
-                        acc.z = fmaf(wk[u], v[u].z, acc.z);
-                        acc.w = fmaf(wk[u], v[u].w, acc.w);
-                    }
+                    v[u] = *(const float4_t *)(y + (size_t)slot[u] * H + c);
                 }
             }
         } else {
-        for (int k = 0; k < K; ++k) {
-            const int pr = t * K + k;
-            const int slot = perm[pr];
-            const int e = idx[pr];
-            if (slot < 0 || e < 0 || e >= E || table[(size_t)e * ODSD_TABLE_COLS] == 0) continue;
-            float4_t v;
-            if (YH) {
-                // fp16 values: complete sums (YH == 1) or the partial sums of KS slices (YH == 2)
-                const half4_t hv = *(const half4_t *)((const half_t *)y + (size_t)slot * H + c);
-                v = float4_t{(float)hv.x, (float)hv.y, (float)hv.z, (float)hv.w};
-                if (YH == 2) {
-                    for (int sl = 1; sl < KS; ++sl) {      // further slices, in slice order
-                        const half4_t hs = *(const half4_t *)((const half_t *)y + ((size_t)sl * P + slot) * H + c);
-                        v += float4_t{(float)hs.x, (float)hs.y, (float)hs.z, (float)hs.w};
+            // slices in order, SB of them and all KB rows requested before the first is used (slices past the
+            // last repeat it and are not added)
+            typedef typename std::conditional<YH == 0, float4_t, half4_t>::type Part;
+            typedef typename std::conditional<YH == 0, float, half_t>::type Elt;
+            constexpr int SB = KB == 4 ? 2 : 4;
+            const Elt *yp = (const Elt *)y;
+            for (int s0 = 0; s0 < KS; s0 += SB) {
+                Part part[SB][KB];
+#pragma unroll
+                for (int i = 0; i < SB; ++i)
+#pragma unroll
+                    for (int u = 0; u < KB; ++u)
+                        part[i][u] = *(const Part *)(yp + ((size_t)min(s0 + i, KS - 1) * P + slot[u]) * H + c);
+#pragma unroll
+                for (int i = 0; i < SB; ++i)
+#pragma unroll
+                    for (int u = 0; u < KB; ++u) {
+                        const float4_t t = {(float)part[i][u].x, (float)part[i][u].y, (float)part[i][u].z, (float)part[i][u].w};
+                        if (i == 0 && s0 == 0) v[u] = t;
+                        else if (s0 + i < KS) v[u] += t;
                     }
-                }
-            } else {
-                v = *(const float4_t *)(y + (size_t)slot * H + c);
-                for (int s = 1; s < KS; ++s) v += *(const float4_t *)(y + ((size_t)s * P + slot) * H + c);
             }
-            const float wk = w[pr];
-            acc.x = fmaf(wk, v.x, acc.x);
-            acc.y = fmaf(wk, v.y, acc.y);
-            acc.z = fmaf(wk, v.z, acc.z);
-            acc.w = fmaf(wk, v.w, acc.w);
         }
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            if (ok[u] && tq[u] != 0) {
+                acc.x = fmaf(wk[u], v[u].x, acc.x);
+                acc.y = fmaf(wk[u], v[u].y, acc.y);
+                acc.z = fmaf(wk[u], v[u].z, acc.z);
+                acc.w = fmaf(wk[u], v[u].w, acc.w);
+            }
         }
-        return acc;
+    }
+    return acc;
 }
 
 // What a token's 4 columns become once the sum is there: residual add and the roundings of the
@@ -1000,39 +981,37 @@ static int launch_combine(const odsd_moe_shape *s, const void *y_, const int32_t
     const int nchunk = (s->H / 4 + 255) / 256;
     if ((int64_t)nchunk * s->T > 0x7fffffffLL) return ODSD_ERR_UNSUPPORTED;
     const dim3 grid((unsigned)(nchunk * s->T));
-    // rows of 4 pairs fetched together (8: no faster): complete sums, or two fp16 slices
-    const bool batched = (pl.KS == 1 || (pl.y_f16 && pl.KS == 2)) && s->K % 4 == 0;
+    const int kb = s->K % 4 == 0 ? 4 : (s->K % 2 == 0 ? 2 : 1);     // rows of 4 pairs fetched together (8: no faster)
     if (nn) {
         // the whole-row form: the next block's normalised input instead of the row statistic
         if (!odsd_combine_norm_supported(s)) return ODSD_ERR_UNSUPPORTED;
         if (!out_act || out_f32 || row_ss || !nn->norm_w || !nn->xn || !nn->x16) return ODSD_ERR_NULL;
         if (!odsd_aligned16(nn->x16) || !odsd_aligned16(nn->xn)) return ODSD_ERR_ALIGN;
     }
-#define COMBINE_GO(XT, YH, ST)                                                                          \
-    do {                                                                                                \
-        if (batched)                                                                                    \
-            ODSD_LAUNCH(ODSD_KERNEL_COMBINE, (combine_kernel<XT, YH, ST, 4>), grid, 256, st, y, idx, w, perm, \
-                        table, (const XT *)residual, out_f32, (XT *)out_act, row_ss, s->T, s->H, s->K,  \
-                        s->E, pl.KS, P, nchunk);                                                        \
-        else                                                                                            \
-            ODSD_LAUNCH(ODSD_KERNEL_COMBINE, (combine_kernel<XT, YH, ST, 0>), grid, 256, st, y, idx, w, perm, \
-                        table, (const XT *)residual, out_f32, (XT *)out_act, row_ss, s->T, s->H, s->K,  \
-                        s->E, pl.KS, P, nchunk);                                                        \
-    } while (0)
-#define COMBINE_NORM_N(XT, YH, KB)                                                                      \
+#define COMBINE_KB(XT, YH, ST, KB)                                                                      \
+    ODSD_LAUNCH(ODSD_KERNEL_COMBINE, (combine_kernel<XT, YH, ST, KB>), grid, 256, st, y, idx, w, perm, table, \
+                (const XT *)residual, out_f32, (XT *)out_act, row_ss, s->T, s->H, s->K, s->E, pl.KS, P, nchunk)
+#define COMBINE_NORM_KB(XT, YH, KB)                                                                     \
     ODSD_LAUNCH(ODSD_KERNEL_COMBINE, (combine_norm_kernel<XT, YH, KB>), dim3((unsigned)s->T), 256 * nchunk, st, y, idx, w, \
                 perm, table, (const XT *)residual, (XT *)out_act, s->T, s->H, s->K, s->E, pl.KS, P,     \
                 (const XT *)nn->norm_w, (double)nn->eps, (XT *)nn->xn, (half_t *)nn->x16)
-#define COMBINE_Y(XT, ST)                                    \
-    do {                                                     \
-        if (nn) {                                            \
-            if (pl.y_f16 && pl.KS >= 2) { if (batched) COMBINE_NORM_N(XT, 2, 4); else COMBINE_NORM_N(XT, 2, 0); } \
-            else if (pl.y_f16) { if (batched) COMBINE_NORM_N(XT, 1, 4); else COMBINE_NORM_N(XT, 1, 0); }          \
-            else { if (batched) COMBINE_NORM_N(XT, 0, 4); else COMBINE_NORM_N(XT, 0, 0); }                        \
-        }                                                    \
-        else if (pl.y_f16 && pl.KS >= 2) COMBINE_GO(XT, 2, ST);   \
-        else if (pl.y_f16) COMBINE_GO(XT, 1, ST);            \
-        else COMBINE_GO(XT, 0, ST);                          \
+#define COMBINE_GO(XT, YH, ST)                                                       \
+    do {                                                                             \
+        if (nn) {                                                                    \
+            if (kb == 4) COMBINE_NORM_KB(XT, YH, 4);                                 \
+            else if (kb == 2) COMBINE_NORM_KB(XT, YH, 2);                            \
+            else COMBINE_NORM_KB(XT, YH, 1);                                         \
+        } else {                                                                     \
+            if (kb == 4) COMBINE_KB(XT, YH, ST, 4);                                  \
+            else if (kb == 2) COMBINE_KB(XT, YH, ST, 2);                             \
+            else COMBINE_KB(XT, YH, ST, 1);                                          \
+        }                                                                            \
+    } while (0)
+#define COMBINE_Y(XT, ST)                                       \
+    do {                                                        \
+        if (pl.y_f16 && pl.KS >= 2) COMBINE_GO(XT, 2, ST);      \
+        else if (pl.y_f16) COMBINE_GO(XT, 1, ST);               \
+        else COMBINE_GO(XT, 0, ST);                             \
     } while (0)
     if (s->act_dtype == ODSD_DT_BF16) {
         if (row_ss) COMBINE_Y(uint16_t, true);
@@ -1042,8 +1021,9 @@ static int launch_combine(const odsd_moe_shape *s, const void *y_, const int32_t
         else COMBINE_Y(float, false);
     }
 #undef COMBINE_Y
-#undef COMBINE_NORM_N
 #undef COMBINE_GO
+#undef COMBINE_NORM_KB
+#undef COMBINE_KB
     ODSD_CHECK_LAUNCH();
     return ODSD_OK;
 }
