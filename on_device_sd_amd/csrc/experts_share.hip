@@ -47,12 +47,15 @@ __device__ __forceinline__ int wave_prefix(int x) {
     return x;
 }
 
-// DISP  0: dispatch arrays are given; 1: from the id list; 2, 3: the top-k as well, E <= 64 / 128
-template <int MODE, int GW, int WK, int NB, int DEPTH, int DISP>
+// NI    0: dispatch arrays are given; otherwise the kernel dispatches for itself, up to 512 NI pairs
+// ROUTE 1, 2: it does the top-k as well, E <= 64 / 128
+template <int MODE, int GW, int WK, int NB, int DEPTH, int NI, int ROUTE>
 __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const GemmParams p) {
     constexpr int WAVES = SHARE_WAVES, RSUB = WAVES / WK, UBLK = RSUB * NB;   // 16-row blocks of a unit
+    constexpr bool DISP = NI > 0;
     constexpr int ROWS = 16, MAX_E = 64 * WAVES;     // one thread per expert in the prologue
     constexpr int SPU = GW * NB / 2;                      // steps (one group of two blocks) per unit
+    static_assert(SPU % DEPTH == 0, "every unit begins on ring slot 0");
     static_assert(MODE == 1 || UBLK == 2, "gate_up: a gate block and its up block");
     static_assert(!DISP || MODE == 0, "gate_up dispatches");
     __shared__ __attribute__((aligned(16))) float red[2][WK][UBLK][256];
@@ -74,14 +77,12 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
     // w * 64 NI .., 64 at a time; a pair's rank among the earlier pairs of its expert is what lies before it in the
     // wavefront's batch (a match by ballots over the bits of the id), plus the wavefront's earlier batches, plus the
     // wavefronts before it.
-    constexpr int MAXNI = DISP ? SHARE_MAX_P / (64 * WAVES) : 1;
-    const int NI = DISP ? (p.P + 64 * WAVES - 1) / (64 * WAVES) : 0;
-    int id[MAXNI], rank[MAXNI];
-    if (DISP == 1) {
+    int id[DISP ? NI : 1], rank[DISP ? NI : 1];
+    if (DISP && ROUTE == 0) {
 #pragma unroll
-        for (int n = 0; n < MAXNI; ++n) {
+        for (int n = 0; n < NI; ++n) {
             const int i = (wave * NI + n) * 64 + lane;
-            id[n] = n < NI && i < p.P ? p.idx[i] : -1;
+            id[n] = i < p.P ? p.idx[i] : -1;
         }
     }
     uint64_t q = 0, sz = 0;
@@ -98,26 +99,26 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
     }
     if (MODE == 0 && !DISP)
         for (int i = tid; i < p.P; i += 64 * WAVES) list_lds[i] = (uint16_t)p.rowmap[i];
-    if (DISP >= 2) {
+    if (ROUTE > 0) {
         // every workgroup selects for every token; workgroup t leaves token t's experts and weights behind
         for (int t = wave; t < p.T; t += WAVES) {
             const bool mine = t == (int)blockIdx.x;
-            const int e = topk_token<(DISP >= 2 ? DISP - 1 : 1)>(p.partial, t, p.T, p.E, p.K, p.route_S, p.renorm, mine ? p.route_idx : nullptr,
+            const int e = topk_token<(ROUTE > 0 ? ROUTE : 1)>(p.partial, t, p.T, p.E, p.K, p.route_S, p.renorm, mine ? p.route_idx : nullptr,
                                                                  mine ? p.route_w : nullptr, nullptr, nullptr);
             if (lane < p.K) list_lds[t * p.K + lane] = (uint16_t)e;
         }
         __syncthreads();
 #pragma unroll
-        for (int n = 0; n < MAXNI; ++n) {
+        for (int n = 0; n < NI; ++n) {
             const int i = (wave * NI + n) * 64 + lane;
-            id[n] = n < NI && i < p.P ? (int)list_lds[i] : -1;
+            id[n] = i < p.P ? (int)list_lds[i] : -1;
         }
     }
     if (DISP) {
         *(uint4_t *)&cntw_lds[wave][8 * lane] = uint4_t{0, 0, 0, 0};
 #pragma unroll
-        for (int n = 0; n < MAXNI; ++n) {
-            if (n < NI) {
+        for (int n = 0; n < NI; ++n) {
+            {
                 const int x = (uint32_t)id[n] < (uint32_t)p.E ? id[n] : -1;   // others belong to nobody
                 id[n] = x;
                 uint64_t same = __ballot(x >= 0);
@@ -166,8 +167,8 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
     __syncthreads();
     if (DISP) {
 #pragma unroll
-        for (int n = 0; n < MAXNI; ++n) {
-            if (n < NI && id[n] >= 0) {
+        for (int n = 0; n < NI; ++n) {
+            if (id[n] >= 0) {
                 const int i = (wave * NI + n) * 64 + lane;
                 const int slot = off_lds[id[n]] + cntw_lds[wave][id[n]] + rank[n];
                 list_lds[slot] = (uint16_t)((uint32_t)i / (uint32_t)p.K);
@@ -345,7 +346,8 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
     const int rd_comp = lane & 3, rd_kq = (lane >> 2) & 3, rd_r = lane >> 4;
     constexpr int QUADS = (MODE == 0 ? 1 : UBLK) * 4;   // 4 rows x 16 outputs each
     int turn = 0;                                         // which wavefronts sum up: moves on with the unit
-    auto finish = [&](const int buf) {
+    auto finish = [&]() {
+        const int buf = turn & 1;
 #pragma unroll
         for (int i = 0; i < NB; ++i) *(float4_t *)&red[buf][kpart][rsub * NB + i][red_w] = acc[i];
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -374,62 +376,39 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
     };
 
     // ---- the stream ------------------------------------------------------------------------------------------
-    // units per trip so that ring slots and reduction buffers are compile-time
-    constexpr int UB = DEPTH % SPU == 0 ? DEPTH / SPU * (DEPTH / SPU % 2 ? 2 : 1) : DEPTH * (DEPTH % 2 ? 2 : 1);
-    static_assert(UB * SPU % DEPTH == 0 && UB % 2 == 0 && UB <= 4, "whole trips round ring and buffers");
+    // One loop with one exit and one copy of a unit (unrolled trips and what is left behind them cost a first pass 7 us in
+    // instruction fetches, and a break between two units would count as a way back to the loop's top: the wait counts
+    // there would allow for the ring as that way leaves it).
     int base_n = 0, mcnt_n = 0;
-    auto unit = [&](auto k_c) {
-        constexpr int k = decltype(k_c)::value;
-        if constexpr (k < UB) {
-            if (in == U) {
-                in = 0;
-                ++item;
-                if constexpr (AHEAD) {
-                    base = base_n;
-                    mcnt = mcnt_n;
+    for (int left = u1 - u0; left > 0; --left) {
+        if (in == U) {
+            in = 0;
+            ++item;
+            if constexpr (AHEAD) {
+                base = base_n;
+                mcnt = mcnt_n;
 #pragma unroll
-                    for (int g = 0; g < GW; ++g)
+                for (int g = 0; g < GW; ++g)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) bx[g][j] = bn[g][j];
-                    group_sums();
-                } else {
-                    rows_now(item);
-                    group_sums();
-                    // nothing of the rows is outstanding from here on, whichever way was taken (or the wait counts
-                    // of the stream would have to allow for it, at the cost of half the ring)
-                    ODSD_WAIT_VMCNT(0);
-                }
+                    for (int j = 0; j < 4; ++j) bx[g][j] = bn[g][j];
+                group_sums();
+            } else {
+                rows_now(item);
+                group_sums();
+                // nothing of the rows is outstanding from here on, whichever way was taken (or the wait counts
+                // of the stream would have to allow for it, at the cost of half the ring)
+                ODSD_WAIT_VMCNT(0);
             }
-            if constexpr (AHEAD)
-                if (in == U - 1 && item < last_item) {
-                    item_rows(item + 1, base_n, mcnt_n);
-                    fetch_rows(base_n, mcnt_n, bn);
-                }
+        }
+        if constexpr (AHEAD)
+            if (in == U - 1 && item < last_item) {
+                item_rows(item + 1, base_n, mcnt_n);
+                fetch_rows(base_n, mcnt_n, bn);
+            }
 #pragma unroll
-            for (int s = 0; s < SPU; ++s) step((k * SPU + s) % DEPTH, s);
-            finish(k & 1);
-            ++in;
-        }
-    };
-    // whole trips in a loop with one exit (a break between two units would count as a way back to its top, and
-    // the wait counts there would allow for the ring as that way leaves it), the remaining units behind it
-    typedef std::integral_constant<int, 0> K0;
-    typedef std::integral_constant<int, 1> K1;
-    typedef std::integral_constant<int, 2> K2;
-    typedef std::integral_constant<int, 3> K3;
-    int left = u1 - u0;
-    for (; left >= UB; left -= UB) {
-        unit(K0{});
-        unit(K1{});
-        unit(K2{});
-        unit(K3{});
-    }
-    if (left > 0) {
-        unit(K0{});
-        if (UB > 2 && left > 1) {
-            unit(K1{});
-            if (left > 2) unit(K2{});
-        }
+        for (int s = 0; s < SPU; ++s) step(s % DEPTH, s);
+        finish();
+        ++in;
     }
 }
 
@@ -469,29 +448,32 @@ static void share_go(GemmParams &gp, int KS, hipStream_t st) {
     constexpr int NB = 2;
     gp.nchunks = gp.NBLK / (SHARE_WAVES / WK * NB);        // units per item
     gp.n_wg = SHARE_CUS / KS * KS;
+#define SHARE_GO(NI, ROUTE)                                                                                        \
+    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_share_kernel<MODE, GW, WK, NB, DEPTH, NI, ROUTE>), \
+                gp.n_wg, 64 * SHARE_WAVES, st, gp)
     if constexpr (MODE == 0) {
         if (gp.idx) {
-#define SHARE_DISP_GO(DISP) ODSD_LAUNCH(ODSD_KERNEL_GATE_UP, (w4_share_kernel<MODE, GW, WK, NB, DEPTH, DISP>), gp.n_wg, 64 * SHARE_WAVES, st, gp)
-            if (gp.route_S == 0) SHARE_DISP_GO(1);
-            else if (gp.E <= 64) SHARE_DISP_GO(2);
-            else SHARE_DISP_GO(3);
-#undef SHARE_DISP_GO
+            if (gp.route_S > 0 && gp.E <= 64) SHARE_GO(1, 1);          // (at most 8 tokens of 64 choices)
+            else if (gp.route_S > 0) SHARE_GO(1, 2);
+            else if (gp.P <= 512) SHARE_GO(1, 0);
+            else if (gp.P <= 1024) SHARE_GO(2, 0);
+            else SHARE_GO(SHARE_MAX_P / 512, 0);
             return;
         }
     }
-    ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN, (w4_share_kernel<MODE, GW, WK, NB, DEPTH, 0>), gp.n_wg,
-                64 * SHARE_WAVES, st, gp);
+    SHARE_GO(0, 0);
+#undef SHARE_GO
 }
 
-// Steps in flight per wavefront (2 KiB each): 4; 3 where a unit has 3 steps (H = 2048, I = 768: T = 24 17.7 us against
-// 17.9 with 4 and 18.8 with 6, T = 128 24.0 / 25.2 / 24.7).
+// Steps in flight per wavefront (2 KiB each): 2 to 4, no more than a unit has; more do not stream faster (H = 2048,
+// I = 768, T = 24: gate_up 2 / 3 / 4 / 6 steps 27.5 / 27.8 / 27.8 / 28.7 us; down 3 / 4 / 6 17.7 / 17.9 / 18.8).
 void odsd_launch_share(int mode, GemmParams &gp, hipStream_t st) {
     ShareSplit s;
     if (!share_split(mode, gp.G, &s)) return;
     if (mode == 0) {
-        if (s.GW == 2) share_go<0, 2, 8, 4>(gp, s.KS, st);
+        if (s.GW == 2) share_go<0, 2, 8, 2>(gp, s.KS, st);
         else share_go<0, 4, 8, 4>(gp, s.KS, st);
     } else if (s.WK == 2) share_go<1, 3, 2, 3>(gp, s.KS, st);
     else if (s.WK == 4) share_go<1, 3, 4, 3>(gp, s.KS, st);
-    else share_go<1, 2, 8, 4>(gp, s.KS, st);
+    else share_go<1, 2, 8, 2>(gp, s.KS, st);
 }
