@@ -639,6 +639,7 @@ __global__ __launch_bounds__(1024) void combine_norm_kernel(const float *__restr
 }
 
 #define STREAM_DISPATCH_CHUNKS 32   // most gate_up workgroups per expert that each scan the ids (stream_dispatch_supported)
+#define STREAM_DISPATCH_PAIRS 1024  // most ids: 4 per thread
 
 // ---- host side ---------------------------------------------------------------------------------
 struct ExpertsPlan {
@@ -652,6 +653,7 @@ struct ExpertsPlan {
     int y_f16;       // down-projection outputs kept as fp16 (unsplit reduction) instead of fp32 partials
     int fused;       // whole-block calls run gate_up and down as one launch (experts_fused.hip)
     int share;       // equal-share streaming kernel (experts_share.hip) for gate_up and down
+    int mid;         // 48-row streaming kernel (experts_mid.hip) for gate_up and down
     int S;           // fused: workgroups per expert = fp16 partial-sum slices of the down projection
     size_t h_bytes, y_bytes;
 };
@@ -665,6 +667,8 @@ int odsd_share_supported(int H, int I, int E, int P);
 int odsd_share_down_splits(int I);
 void odsd_launch_share(int mode, GemmParams &gp, hipStream_t st);
 int odsd_share_route_supported(int T, int E);
+// 48-row streaming kernel (experts_mid.hip)
+void odsd_launch_mid(int mode, GemmParams &gp, hipStream_t st);
 
 // Choices are functions of the shape only (the per-expert counts live on the device).
 static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
@@ -682,7 +686,7 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     // 39.9 / 36.6; H = I = 1024 64 rows 34.2 / 35.5; E = 32, H = I = 512 64 rows 31.1 / 32.5; twice the pieces: E = 8,
     // H = 1024, I = 2048 64 rows 41.4 / 39.2, E = 64, H = I = 512 100 rows 53.0 / 48.4).
     const long pieces_gu = (s->E < P ? s->E : P) * ((2 * s->I / 16 + 15) / 16) * (s->H / ODSD_GROUP);
-    p.tile = 0;
+    p.tile = p.mid = 0;
     if (s->T <= 16) p.MB = 1;
     else if (s->T <= 32) p.MB = 2;
     else if (s->T <= 64) p.MB = 4;      // no expert can have more rows than a 64-row pass holds
@@ -742,9 +746,18 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     } else {
         const long wg_gu = active * ((2 * s->I / 16 + 15) / 16);
         if (wg_gu < 4 * slots || p.MB == 8) p.NB = 2;
+        // 13 to 34 rows per expert of models whose token rows are 32 groups or longer: the 48-row kernel.  Whole layer,
+        // us, 32- or 64-row passes of the other one / this one: H = 4096, I = 14336, E = 8, K = 2: T = 56 157 / 142,
+        // T = 72 167 / 155, T = 100 173 / 164, T = 128 189 / 182, T = 140 (35 rows) 195 / 189, T = 160 (40) 201 / 208;
+        // H = 4096, I = 1536, E = 128, K = 8: T = 224 273 / 254, T = 320 297 / 279, T = 450 323 / 309, T = 550 (35)
+        // 349 / 346, T = 800 (50) 413 / 507, Zipf T = 256 380 / 302, T = 400 396 / 357.  With 16 groups (H = 2048, I = 768) it is no faster (T = 400 103 / 103),
+        // from 35 rows on too many experts take a second pass.  Not where the other kernel dispatches for itself.
+        p.mid = p.MB >= 2 && p.MB <= 4 && mean_rows >= 13 && mean_rows <= 34 && G_gu >= 32 &&
+                (P > STREAM_DISPATCH_PAIRS || (2 * s->I / 16 + 4 * p.NB - 1) / (4 * p.NB) > STREAM_DISPATCH_CHUNKS);
+        if (p.mid) p.NB = 4;
         const int nchunks_dn = (s->H / 16 + 4 * p.NB - 1) / (4 * p.NB);
         int KS = 1;
-        const long want = p.MB == 8 ? slots : 2 * slots;       // 2 workgroups per CU with eight token blocks, up to 4 with fewer
+        const long want = p.MB == 8 || p.mid ? slots : 2 * slots;       // 2 workgroups per CU with eight token blocks or four weight blocks, up to 4 with fewer
         while (KS * 2 <= G_dn / 2 && active * nchunks_dn * KS < want && KS < 16) KS *= 2;
         p.KS = KS;
     }
@@ -844,6 +857,7 @@ static void launch_gemm_plan(const ExpertsPlan &pl, GemmParams &gp, hipStream_t 
     const int wk = MODE == 0 ? pl.WK_gu : pl.WK_dn;
     gp.y_f16 = pl.y_f16;
     if (pl.share) { odsd_launch_share(MODE, gp, st); return; }
+    if (pl.mid) { odsd_launch_mid(MODE, gp, st); return; }
     if (pl.MB == 1 && wk == 0) {
         if (MODE == 0 || pl.NB_dn == 2) launch_gemm<2, 1, MODE, 3, 2, 1, false, 4>(gp, st);
         else if constexpr (MODE == 1) launch_gemm<1, 1, MODE, 3, 1, 1, false, 4>(gp, st);
@@ -881,7 +895,7 @@ static bool stream_dispatch_supported(const ExpertsPlan &pl, const odsd_moe_shap
     if (pl.share) return true;
     const int nb = pl.MB == 1 ? 2 : pl.NB;
     const int chunks = (2 * s->I / 16 + 4 * nb - 1) / (4 * nb);     // gate_up workgroups per expert
-    return pl.MB <= 4 && (pl.MB > 1 || pl.WK_gu == 0) && chunks <= STREAM_DISPATCH_CHUNKS && s->T * s->K <= 4 * 256;
+    return pl.MB <= 4 && (pl.MB > 1 || pl.WK_gu == 0) && chunks <= STREAM_DISPATCH_CHUNKS && s->T * s->K <= STREAM_DISPATCH_PAIRS && !pl.mid;
 }
 
 // idx + dispatch_out: the dispatch arrays have not been filled; the kernel dispatches for itself
