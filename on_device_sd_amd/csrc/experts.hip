@@ -73,7 +73,10 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
     // in one L2 is worth nothing with few rows, and would leave an XCD idle for every expert
     // without tokens; with 128-row passes it is worth having.
     const int b = blockIdx.x;
-    const int L = MB == 8 ? (b & 7) * p.wg_per_xcd + (b >> 3) : b;
+    // SHARED: several workgroups share the passes over a tile, everyone's first passes come before anyone's second
+    constexpr bool SHARED = !DISP && (MB == 2 || MB == 4);
+    const int ps = SHARED ? b / p.n_wg : 0, PS = SHARED ? p.PS : 1;
+    const int L = MB == 8 ? (b & 7) * p.wg_per_xcd + (b >> 3) : b - ps * p.n_wg;
     if (L >= p.n_wg) return;
     const int ks = L % p.KS;
     const int chunk = (L / p.KS) % p.nchunks;
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
         M_e = p.counts[e];
         base = p.offsets[e];
     }
-    if (M_e == 0 || t_present == 0) return;
+    if (M_e <= ps * 16 * MB || t_present == 0) return;
     // addresses from the table are global memory: say so, or the loads become flat loads
     // whose LDS-side counter forces every wait to drain
     const global_char *qp_c = (const global_char *)t_q;
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
 #pragma unroll
     for (int j = 0; j < 4; ++j) lds_frag[j] = (uint32_t)((r * 16 + ((4 * j + kq) ^ r)) * 16);
 
-    for (int m0 = 0; m0 < M_e; m0 += 16 * MB) {
+    for (int m0 = ps * 16 * MB; m0 < M_e; m0 += PS * 16 * MB) {
         const int mcnt = min(M_e - m0, 16 * MB);
         const int nmb = (mcnt + 15) >> 4;
         const int mcnt_s = MB == 1 ? mcnt : scalar_int(mcnt);
@@ -648,7 +651,7 @@ struct ExpertsPlan {
     int NB_dn;       // MB == 1, LDS path: the same of the down projection
     int WK_gu, WK_dn;  // MB == 1: wavefronts of a workgroup that split K on the direct path, 0: the LDS path
     int KS;          // split of the down projection's reduction dimension across workgroups
-    int PS_gu, PS_dn;  // prefill tile kernel: workgroups sharing the row passes of one tile
+    int PS_gu, PS_dn;  // workgroups sharing the row passes of one tile
     int tile;        // the tile kernel (experts_prefill.hip) instead of the streaming kernel
     int y_f16;       // down-projection outputs kept as fp16 (unsplit reduction) instead of fp32 partials
     int fused;       // whole-block calls run gate_up and down as one launch (experts_fused.hip)
@@ -668,6 +671,7 @@ int odsd_share_down_splits(int I);
 void odsd_launch_share(int mode, GemmParams &gp, hipStream_t st);
 int odsd_share_route_supported(int T, int E);
 // 48-row streaming kernel (experts_mid.hip)
+#define ODSD_MID_ROWS 48
 void odsd_launch_mid(int mode, GemmParams &gp, hipStream_t st);
 
 // Choices are functions of the shape only (the per-expert counts live on the device).
@@ -760,6 +764,14 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
         const long want = p.MB == 8 || p.mid ? slots : 2 * slots;       // 2 workgroups per CU with eight token blocks or four weight blocks, up to 4 with fewer
         while (KS * 2 <= G_dn / 2 && active * nchunks_dn * KS < want && KS < 16) KS *= 2;
         p.KS = KS;
+        // A popular expert's passes side by side instead of in turn: four workgroups share them, no more than there can
+        // be passes.  Layer, us, one / two / four: E = 128, H = 2048, I = 768, Zipf, T = 400 154 / 135 / 122, T = 600
+        // 195 / 165 / 146, T = 800 248 / 203 / 177; H = 4096, I = 1536, Zipf, T = 800 631 / 564 / 534; E = 8, I = 14336,
+        // Zipf, T = 160 248 / 233 / 233; uniform T = 400 105 / 105 / 105, T = 800 143 / 138 / 138.
+        if (p.MB <= 4) {
+            const int rows = p.mid ? ODSD_MID_ROWS : 16 * p.MB, most = (s->T + rows - 1) / rows;
+            p.PS_gu = p.PS_dn = most < 4 ? most : 4;
+        }
     }
     // Equal shares (experts_share.hip) where its splits of the reductions exist and a pass of 16 rows holds most experts:
     // up to 12 rows per expert on average.  Whole layer, us, the plan above / equal shares: H = 2048, I = 768, E = 128,
@@ -845,8 +857,10 @@ static void launch_gemm(GemmParams &gp, hipStream_t st) {
             return;
         }
     }
+    if (MB != 2 && MB != 4) gp.PS = 1;
     ODSD_LAUNCH(MODE == 0 ? ODSD_KERNEL_GATE_UP : ODSD_KERNEL_DOWN,
-                (w4_gemm_kernel<NB, MB, MODE, DEPTH, NA, WK, DIRECT, OCC, WAVES, false>), gp.wg_per_xcd * 8, 64 * WAVES, st, gp);
+                (w4_gemm_kernel<NB, MB, MODE, DEPTH, NA, WK, DIRECT, OCC, WAVES, false>),
+                MB == 8 ? gp.wg_per_xcd * 8 : gp.n_wg * gp.PS, 64 * WAVES, st, gp);
 }
 
 // prefill-shaped tile kernel (experts_prefill.hip)

@@ -13,7 +13,7 @@
 //     layer, us: H = 4096, I = 14336, E = 8, T = 56 165 / 142, T = 100 177 / 164; I = 1536, E = 128, T = 256 296 / 257.
 //     Neighbours on one XCD (every eighth workgroup) are 5 groups apart, XCDs one.  Apart by one in launch order,
 //     i.e. an XCD's all at the same L2 channels: 266 for the last.
-//   * Four workgroups share the passes over a tile: a popular expert's passes run side by side instead of in turn, the
+//   * Up to four workgroups share the passes over a tile: a popular expert's passes run side by side instead of in turn, the
 //     workgroups without one come last and only look at the row count.  Zipf-distributed routing, E = 128, one / four,
 //     layer, us: T = 256 352 / 302, T = 400 464 / 357; uniform routing does not notice (256 / 256, 291 / 293).
 //
@@ -31,7 +31,6 @@
 #define MID_WAVES 4
 #define MID_MB 3               // token blocks of a pass: 48 rows
 #define MID_XB 3               // token-row buffers
-#define MID_PS 4               // workgroups that share the passes over one tile
 
 template <int MODE, int NB>
 __global__ __launch_bounds__(64 * MID_WAVES, 2) void w4_mid_kernel(const GemmParams p) {
@@ -234,7 +233,7 @@ __global__ __launch_bounds__(64 * MID_WAVES, 2) void w4_mid_kernel(const GemmPar
             }
         }
     };
-    for (int m0 = ps * 16 * MID_MB; m0 < M_e; m0 += MID_PS * 16 * MID_MB) {
+    for (int m0 = ps * 16 * MID_MB; m0 < M_e; m0 += p.PS * 16 * MID_MB) {
         const int mcnt = min(M_e - m0, 16 * MID_MB);
         if (mcnt <= 16) pass(std::integral_constant<int, 1>{}, m0, mcnt);
         else if (mcnt <= 32) pass(std::integral_constant<int, 2>{}, m0, mcnt);
@@ -246,6 +245,6 @@ void odsd_launch_mid(int mode, GemmParams &gp, hipStream_t st) {
     constexpr int NB = 4;
     gp.nchunks = (gp.NBLK + MID_WAVES * NB - 1) / (MID_WAVES * NB);
     gp.n_wg = gp.E * gp.nchunks * gp.KS;
-    if (mode == 0) ODSD_LAUNCH(ODSD_KERNEL_GATE_UP, (w4_mid_kernel<0, NB>), gp.n_wg * MID_PS, 64 * MID_WAVES, st, gp);
-    else ODSD_LAUNCH(ODSD_KERNEL_DOWN, (w4_mid_kernel<1, NB>), gp.n_wg * MID_PS, 64 * MID_WAVES, st, gp);
+    if (mode == 0) ODSD_LAUNCH(ODSD_KERNEL_GATE_UP, (w4_mid_kernel<0, NB>), gp.n_wg * gp.PS, 64 * MID_WAVES, st, gp);
+    else ODSD_LAUNCH(ODSD_KERNEL_DOWN, (w4_mid_kernel<1, NB>), gp.n_wg * gp.PS, 64 * MID_WAVES, st, gp);
 }

@@ -23,7 +23,7 @@ struct GemmParams {
     int nchunks;             // workgroup tiles along the rows
     int KS;                  // splits of the reduction dimension
     int gper;                // groups per split
-    int PS;                  // tile kernel: workgroups sharing the row passes of one tile
+    int PS;                  // workgroups sharing the row passes of one tile
     int ldo;                 // I (MODE 0) or H (MODE 1)
     int P;
     int E;

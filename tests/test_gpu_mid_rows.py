@@ -1,6 +1,7 @@
 """The 48-row streaming kernel at its edges: experts with 1, 16, 17, 32, 33, 48, 49 and more rows (every number of token
 blocks, a second and a third pass), without rows and without weights, the ends of its rule, weight rows that end inside a
-workgroup's 16 blocks, unsplit and split down reductions, splits of unequal length."""
+workgroup's 16 blocks, unsplit and split down reductions, splits of unequal length; and the 32- and 64-row kernel where
+several workgroups share an expert's passes, at the edges of those."""
 import numpy as np
 import pytest
 import torch
@@ -18,6 +19,9 @@ pytestmark = pytest.mark.gpu
     (129, 4096, 64, 9, 128, (100,)),                 # 1161 pairs: more than the other kernel scans; one group in down
     (600, 4224, 40, 2, 256, (47, 16)),               # 33 groups; 264 blocks of output rows: the last workgroup has 8
     (100, 8192, 4, 1, 4608, (31, 2)),                # 64 groups
+    (600, 512, 32, 2, 384, (600, 257, 256, 65)),     # 64-row passes: ten, five, four and two of them for four workgroups
+    (600, 512, 96, 2, 384, (129, 128, 33, 32)),      # 32-row passes
+    (65, 512, 8, 4, 384, (65, 64)),                  # two workgroups in down, the dispatch inside gate_up
 ])
 def test_mid_rows(dev, T, H, E, K, I, crowd):
     from on_device_sd_amd import ops
@@ -33,8 +37,8 @@ def test_mid_rows(dev, T, H, E, K, I, crowd):
         wg[c] = 0.0
         wg[c, c] = 1.0
         x[:, c] = -40.0
-        x[at:at + rows, c] = 40.0
-        at = at + rows if K == 1 else 0
+        x[(at + torch.arange(rows)) % T, c] = 40.0      # one after the other, round and round: at most K of them per token
+        at += rows
     bank, experts = _bank(dev, H, E, I, g, distinct=3)
     xd, wgd, table = x.to(dev), wg.to(dev), bank.table()
     out = ops.moe_forward(xd, wgd, table, K, I, renorm=True)
