@@ -29,7 +29,7 @@ struct MoeLayout {
     size_t router, xn, x16, idx, w, counts, offsets, perm, inv, slot_token, experts, total;
 };
 
-static MoeLayout moe_layout(const odsd_moe_shape *s) {
+static MoeLayout moe_layout(const odsd_moe_shape *s, const size_t experts_bytes) {
     MoeLayout l;
     const size_t T = s->T > 0 ? s->T : 1, P = T * s->K;
     const size_t act = s->act_dtype == ODSD_DT_F32 ? 4 : 2;
@@ -45,10 +45,13 @@ static MoeLayout moe_layout(const odsd_moe_shape *s) {
     l.perm = take(P * 4);
     l.inv = take(P * 4);
     l.slot_token = take(P * 4);
-    l.experts = take(odsd_experts_workspace_bytes(s));
+    l.experts = take(experts_bytes);
     l.total = o;
     return l;
 }
+static MoeLayout moe_layout(const odsd_moe_shape *s) { return moe_layout(s, odsd_experts_workspace_bytes(s)); }
+// the block's workspace without that of the expert kernels (for a plan that depends on what is left)
+size_t odsd_moe_bytes_around_experts(const odsd_moe_shape *s) { return moe_layout(s, 0).total; }
 
 extern "C" size_t odsd_moe_workspace_bytes(const odsd_moe_shape *s) {
     if (!s) return 0;

@@ -157,5 +157,6 @@ int odsd_launch_experts(const odsd_moe_shape *s, const void *x16, const uint64_t
                         size_t ws_bytes, hipStream_t st, double *row_ss,
                         const OdsdDispatchOut *dispatch_out = nullptr, const OdsdNextNorm *next_norm = nullptr);
 int odsd_combine_norm_supported(const odsd_moe_shape *s);
+size_t odsd_moe_bytes_around_experts(const odsd_moe_shape *s);
 int odsd_experts_dispatch_inside(const odsd_moe_shape *s);
 int odsd_experts_route_inside(const odsd_moe_shape *s);

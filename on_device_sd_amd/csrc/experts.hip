@@ -773,6 +773,12 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
             p.PS_gu = p.PS_dn = most < 4 ? most : 4;
         }
     }
+    // every split must own at least one group
+    while (p.KS > 1 && ((G_dn + p.KS - 1) / p.KS) * (p.KS - 1) >= G_dn) p.KS--;
+    p.h_bytes = odsd_round_up((size_t)(P > 0 ? P : 1) * s->I * sizeof(half_t), 256);
+    auto y_need = [&](const int KS) {
+        return odsd_round_up((size_t)KS * (size_t)(P > 0 ? P : 1) * s->H * (KS == 1 || p.MB >= 2 ? sizeof(half_t) : sizeof(float)), 256);
+    };
     // Equal shares (experts_share.hip) where its splits of the reductions exist and a pass of 16 rows holds most experts:
     // up to 12 rows per expert on average.  Whole layer, us, the plan above / equal shares: H = 2048, I = 768, E = 128,
     // K = 8: T = 1 30.7 / 24.5, T = 8 47.3 / 42.5, T = 24 69.5 / 59.6, T = 64 77.8 / 72.5, T = 112 77.2 / 74.2, Zipf
@@ -780,13 +786,18 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     // 259 / 248, T = 256 269 / 323; H = 4096, I = 14336, E = 8, K = 2: T = 1 58.8 / 50.1, T = 5 115.7 / 99.0, T = 40
     // 152 / 135, T = 48 (12 rows) 153 / 146, T = 56 153 / 169.  From 14 rows on too many experts take a second pass
     // over their weights, which the plan above saves with wider ones.
+    // Its splits of the down projection follow from the reduction alone, so with many rows of a long one it can need more
+    // partial sums than the plan above: not where that takes a block out of the library's static array.
     p.share = 0;
     if (mean_rows <= 12 && odsd_share_supported(s->H, s->I, s->E, (int)P)) {
-        p.share = 1;
-        p.KS = odsd_share_down_splits(s->I);
+        const int KS = odsd_share_down_splits(s->I);
+        const size_t y_this = y_need(KS), y_other = y_need(p.KS);
+        const size_t others = y_this > y_other ? odsd_moe_bytes_around_experts(s) + p.h_bytes : 0, most = ODSD_STATIC_SCRATCH_BYTES;
+        if (y_this <= y_other || others + y_this <= most || others + y_other > most) {
+            p.share = 1;
+            p.KS = KS;
+        }
     }
-    // every split must own at least one group
-    while (p.KS > 1 && ((G_dn + p.KS - 1) / p.KS) * (p.KS - 1) >= G_dn) p.KS--;
     // The down projection's outputs are stored as fp16 (3 more bits than the bf16 the reference keeps
     // its expert outputs in): half the bytes to write and to read back in the combine (at prefill
     // shapes fp32 would be 0.5 GB per layer each way) -- complete sums without a split of the
@@ -794,8 +805,7 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     // Mixtral T = 160 shape the fp32 form wrote and re-read 21 MB per layer).  Calls with at most 16
     // tokens keep fp32 partial sums: they split deepest (up to 16 slices) and move next to nothing.
     p.y_f16 = p.KS == 1 || p.MB >= 2;
-    p.h_bytes = odsd_round_up((size_t)(P > 0 ? P : 1) * s->I * sizeof(half_t), 256);
-    p.y_bytes = odsd_round_up((size_t)p.KS * (size_t)(P > 0 ? P : 1) * s->H * (p.y_f16 ? sizeof(half_t) : sizeof(float)), 256);
+    p.y_bytes = y_need(p.KS);
     // The one-launch expert kernel serves calls where nearly every expert has rows and a pass holds
     // them all (8 to 20 rows per expert on average, at most 32 per pass; measured against the
     // two-launch plan on uniform routing it wins up to 20 and loses from 24 on, where many experts
