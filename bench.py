@@ -140,7 +140,7 @@ def _roofline(wl, kernel_ms, algorithmic_bytes, kernel=None):
                 "traffic": traffic, "algorithmic_flops": gu_flops}
     else:
         ach = algorithmic_bytes / (kernel_ms * 1e-3) / 1e9
-        roof = {"bound": "hbm", "kernel": kernel or "w4_gemm_kernel<gate_up>", "achieved": round(ach, 1),
+        roof = {"bound": "hbm", "kernel": kernel or "gate_up (streaming kernel of the plan)", "achieved": round(ach, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                 "traffic": traffic, "algorithmic_bytes": int(algorithmic_bytes)}
     if commit:
@@ -237,7 +237,7 @@ def bench_layer(wl, dev, steps, warmup, with_cpu):
                                     "frac": round(ach / MFMA_F16_PEAK_TFLOPS, 4), "kernel_ms": round(k["down"], 5)}
         else:
             ach = down_bytes / (k["down"] * 1e-3) / 1e9
-            res["down_roofline"] = {"bound": "hbm", "kernel": "w4_gemm_kernel<down>", "achieved": round(ach, 1),
+            res["down_roofline"] = {"bound": "hbm", "kernel": "down (streaming kernel of the plan)", "achieved": round(ach, 1),
                                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                                     "algorithmic_bytes": int(down_bytes), "kernel_ms": round(k["down"], 5)}
     del runner, placements, plan, banks, tables
