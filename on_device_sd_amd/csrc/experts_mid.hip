@@ -18,8 +18,9 @@
 //     layer, us: T = 256 352 / 302, T = 400 464 / 357; uniform routing does not notice (256 / 256, 291 / 293).
 //
 // Bound by issue at 33 to 48 rows (matrix cores busy 38 %, vector instructions 31 % of the cycles, 1.75 rounds of
-// workgroups at E = 8), by HBM at up to 16 (5.8 TB/s).  Measured and not kept: no interleaving of vector and matrix
-// instructions (T = 160: 208 / 204), 64-row passes (254 registers without the interleaving, spills with it).
+// workgroups at E = 8), by HBM at up to 16 (about 6 TB/s).  Measured and not kept: no interleaving of vector and matrix
+// instructions (before the workgroups started on different groups, E = 128, T = 400: 318 / 309 with it; E = 8, T = 160
+// 208 / 211).  Passes of 64 rows take 254 registers without the interleaving and leave none for it.
 //
 //   MODE 0  gate_up: h = SiLU(gate) * up -> fp16
 //   MODE 1  down: KS splits of the reduction across workgroups, fp16 sums
