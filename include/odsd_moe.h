@@ -202,7 +202,8 @@ int odsd_experts_w4(const odsd_moe_shape *s, const void *x_f16, const uint64_t *
  *   h_f16 fp16 [P, I] in slot order; y: a buffer of odsd_w4_down_splits(s)*P*H*4 bytes that
  *   odsd_w4_down fills and odsd_combine reads -- [splits][P][H] partial sums over slices of I,
  *   which odsd_combine adds in slice order: fp16 values (a value beyond +-65504 saturates), except
- *   for calls with T <= 16, which keep float partial sums when the reduction is split.
+ *   for calls with T <= 16, which keep float sums wherever I is large enough for a split reduction
+ *   to be of use (from I = 2048 on, when the experts alone do not fill the chip).
  * They stand in for the three F.linear calls of mlp.py:227-230 (gate/up fused with
  * SiLU*mul, then down) and the indexed "+=" of qwen3_runner.py:363. */
 int     odsd_w4_gate_up_silu(const odsd_moe_shape *s, const void *x_f16, const uint64_t *table,

@@ -776,9 +776,17 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     // every split must own at least one group
     while (p.KS > 1 && ((G_dn + p.KS - 1) / p.KS) * (p.KS - 1) >= G_dn) p.KS--;
     p.h_bytes = odsd_round_up((size_t)(P > 0 ? P : 1) * s->I * sizeof(half_t), 256);
-    auto y_need = [&](const int KS) {
-        return odsd_round_up((size_t)KS * (size_t)(P > 0 ? P : 1) * s->H * (KS == 1 || p.MB >= 2 ? sizeof(half_t) : sizeof(float)), 256);
+    // The down projection's outputs are stored as fp16 (3 more bits than the bf16 the reference keeps
+    // its expert outputs in): half the bytes to write and to read back in the combine (at prefill
+    // shapes fp32 would be 0.5 GB per layer each way) -- complete sums without a split of the
+    // reduction, one fp16 partial sum per slice with one (added in slice order by the combine; at the
+    // Mixtral T = 160 shape the fp32 form wrote and re-read 21 MB per layer).  Calls with at most 16
+    // tokens whose reduction is split keep fp32 sums: they split deepest (up to 16 slices) and move next to nothing.
+    p.y_f16 = p.KS == 1 || p.MB >= 2;
+    auto y_need = [&](const int KS, const int f16) {
+        return odsd_round_up((size_t)KS * (size_t)(P > 0 ? P : 1) * s->H * (f16 ? sizeof(half_t) : sizeof(float)), 256);
     };
+    p.y_bytes = y_need(p.KS, p.y_f16);
     // Equal shares (experts_share.hip) where its splits of the reductions exist and a pass of 16 rows holds most experts:
     // up to 12 rows per expert on average.  Whole layer, us, the plan above / equal shares: H = 2048, I = 768, E = 128,
     // K = 8: T = 1 30.7 / 24.5, T = 8 47.3 / 42.5, T = 24 69.5 / 59.6, T = 64 77.8 / 72.5, T = 112 77.2 / 74.2, Zipf
@@ -791,21 +799,17 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     p.share = 0;
     if (mean_rows <= 12 && odsd_share_supported(s->H, s->I, s->E, (int)P)) {
         const int KS = odsd_share_down_splits(s->I);
-        const size_t y_this = y_need(KS), y_other = y_need(p.KS);
-        const size_t others = y_this > y_other ? odsd_moe_bytes_around_experts(s) + p.h_bytes : 0, most = ODSD_STATIC_SCRATCH_BYTES;
-        if (y_this <= y_other || others + y_this <= most || others + y_other > most) {
+        // sums that the plan above keeps as fp32 stay fp32, also where this one leaves a single slice of them
+        const int y_f16 = p.y_f16 && (KS == 1 || p.MB >= 2);
+        const size_t y_this = y_need(KS, y_f16);
+        const size_t others = y_this > p.y_bytes ? odsd_moe_bytes_around_experts(s) + p.h_bytes : 0, most = ODSD_STATIC_SCRATCH_BYTES;
+        if (y_this <= p.y_bytes || others + y_this <= most || others + p.y_bytes > most) {
             p.share = 1;
             p.KS = KS;
+            p.y_f16 = y_f16;
+            p.y_bytes = y_this;
         }
     }
-    // The down projection's outputs are stored as fp16 (3 more bits than the bf16 the reference keeps
-    // its expert outputs in): half the bytes to write and to read back in the combine (at prefill
-    // shapes fp32 would be 0.5 GB per layer each way) -- complete sums without a split of the
-    // reduction, one fp16 partial sum per slice with one (added in slice order by the combine; at the
-    // Mixtral T = 160 shape the fp32 form wrote and re-read 21 MB per layer).  Calls with at most 16
-    // tokens keep fp32 partial sums: they split deepest (up to 16 slices) and move next to nothing.
-    p.y_f16 = p.KS == 1 || p.MB >= 2;
-    p.y_bytes = y_need(p.KS);
     // The one-launch expert kernel serves calls where nearly every expert has rows and a pass holds
     // them all (8 to 20 rows per expert on average, at most 32 per pass; measured against the
     // two-launch plan on uniform routing it wins up to 20 and loses from 24 on, where many experts

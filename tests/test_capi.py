@@ -4,6 +4,8 @@ import ctypes as C
 import os
 import re
 
+import pytest
+
 from on_device_sd_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -48,6 +50,17 @@ def test_one_launch_plan_follows_shape_and_max_rows():
     # the workspace answer does not depend on the statement (one buffer serves either plan)
     ws = lambda mr: lib.odsd_experts_workspace_bytes(C.byref(_lib.MoeShape(256, 2048, 128, 8, 768, 1, _lib.DT_BF16, mr)))
     assert ws(0) == ws(40) > 0
+
+
+@pytest.mark.parametrize("T,H,E,K,I", [(1, 2048, 4, 1, 2048), (8, 2048, 8, 2, 2048), (16, 4096, 16, 2, 2048), (5, 4096, 8, 2, 14336)])
+def test_sums_of_split_reductions_stay_fp32_up_to_16_tokens(T, H, E, K, I):
+    """Calls of at most 16 tokens whose experts leave CUs idle split the reduction of the down projection and keep its
+    sums in fp32; a plan that needs fewer slices of them keeps them in fp32 all the same."""
+    lib = _lib.load()
+    s = _lib.MoeShape(T, H, E, K, I, 1, _lib.DT_BF16, 0)
+    up = lambda n: -(-n // 256) * 256  # noqa: E731
+    P = T * K
+    assert lib.odsd_experts_workspace_bytes(C.byref(s)) == up(P * I * 2) + up(lib.odsd_w4_down_splits(C.byref(s)) * P * H * 4)
 
 
 def test_argument_checks_need_no_gpu():

@@ -12,12 +12,12 @@ from tests.helpers import canon_to_oracle, check_output_relative
 pytestmark = pytest.mark.gpu
 
 
-def _bank(dev, H, E, I, g, distinct=6):
+def _bank(dev, H, E, I, g, distinct=6, w_down=0.05):
     """Bank of E experts; the weights repeat after `distinct` of them (the oracle then quantises few)."""
     import on_device_sd_amd as odsd
     bank = odsd.W4ExpertBank(E, H, I, dev)
-    mk = lambda r, c: torch.randn(r, c, generator=g) * 0.05  # noqa: E731
-    ws = [(mk(I, H), mk(I, H), mk(H, I)) for _ in range(min(E, distinct))]
+    mk = lambda r, c, scale=0.05: torch.randn(r, c, generator=g) * scale  # noqa: E731
+    ws = [(mk(I, H), mk(I, H), mk(H, I, w_down)) for _ in range(min(E, distinct))]
     experts = {}
     for e in range(E):
         if e < distinct:
@@ -79,3 +79,23 @@ def test_equal_shares(dev, T, H, E, K, I, crowd):
     got, _ = ops.experts_w4(x16, hole, i32, wd, disp, I, torch.bfloat16, want_f32=True, want_act=False)
     ref_hole = orc.moe_forward(x, idx, np.where(idx == gone, 0.0, w).astype(np.float32), experts)
     check_output_relative(got, ref_hole)
+
+
+@pytest.mark.parametrize("T,H,E,K,I", [
+    (8, 2048, 8, 2, 2048),       # one slice of sums where the reduction was to be split
+    (16, 4096, 16, 2, 2048),
+    (5, 4096, 8, 2, 14336),      # seven slices
+])
+def test_few_tokens_keep_fp32_sums(dev, T, H, E, K, I):
+    """Expert outputs far beyond fp16's largest value: fp32 sums carry them, fp16 ones would be clamped to 65504."""
+    from on_device_sd_amd import ops
+    print("equal shares, large outputs", T, H, E, K, I, flush=True)
+    g = torch.Generator().manual_seed(T + H + I)
+    wg = (torch.randn(E, H, generator=g) * 0.02).to(torch.bfloat16)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    bank, experts = _bank(dev, H, E, I, g, distinct=3, w_down=8000.0)
+    out = ops.moe_forward(x.to(dev), wg.to(dev), bank.table(), K, I, renorm=True)
+    ref, idx, _ = orc.moe_block(x, wg, experts, K, True)
+    assert np.array_equal(out.idx.cpu().numpy(), idx)
+    assert (ref.abs() > 65504).float().mean() > 0.5       # (weights of at most 1: the sums themselves are larger still)
+    check_output_relative(out.out_f32, ref)
