@@ -414,18 +414,28 @@ __global__ __launch_bounds__(64 * SHARE_WAVES, 2) void w4_share_kernel(const Gem
 
 // ---- host side -----------------------------------------------------------------------------------
 // How the wavefronts of a workgroup split a reduction of G groups: WK parts of GW groups, KS splits across workgroups.
-// The token rows of a part live in registers, 16 GW of them.
+// The token rows of a part live in registers, 16 GW of them (207 in all at GW = 3, where the next item's rows are fetched
+// ahead, 194 at GW = 4): 2 to 4 groups.  One group per part would make a unit of gate_up a single step, with a barrier
+// every 2 KiB of a wavefront's stream.  gate_up (8 parts, both blocks of a unit): 16, 24 or 32 groups.  down: the most
+// parts that divide the reduction, two groups before three, and what is left over across workgroups.
+// Layer, us, the plan without equal shares / this: H = 3072, E = 128, I = 768, K = 8: T = 1 34.1 / 25.3, T = 64 102.5 / 93.4,
+// T = 176 114.6 / 111.4; H = 2048, I = 512, E = 512, K = 10, T = 64 166 / 119; I = 1024, E = 64, K = 8: T = 8 53.3 / 42.6,
+// T = 88 63.1 / 58.6; I = 2560 (5 splits), E = 16, K = 2: T = 8 37.8 / 30.1, T = 88 47.9 / 43.4; H = 4096, I = 3072, E = 32,
+// K = 2: T = 24 116 / 93; I = 5632 (11 splits), E = 16: T = 24 125 / 104, T = 88 130 / 126.
 struct ShareSplit { int WK, GW, KS; };
 static bool share_split(int mode, int G, ShareSplit *s) {
     if (mode == 0) {
-        if (G != 16 && G != 32) return false;
+        if (G % 8 || G < 16 || G > 32) return false;
         *s = {8, G / 8, 1};
-    } else {
-        if (G == 6 || G == 12) *s = {G / 3, 3, 1};
-        else if (G % 16 == 0 && G / 16 <= 16) *s = {8, 2, G / 16};
-        else return false;
+        return true;
     }
-    return true;
+    static const int parts[][2] = {{8, 2}, {8, 3}, {4, 3}, {4, 2}, {2, 3}, {2, 2}};
+    for (const auto &w : parts)
+        if (G % (w[0] * w[1]) == 0 && G / (w[0] * w[1]) <= 16) {
+            *s = {w[0], w[1], G / (w[0] * w[1])};
+            return true;
+        }
+    return false;
 }
 
 int odsd_share_supported(int H, int I, int E, int P) {
@@ -472,8 +482,15 @@ void odsd_launch_share(int mode, GemmParams &gp, hipStream_t st) {
     if (!share_split(mode, gp.G, &s)) return;
     if (mode == 0) {
         if (s.GW == 2) share_go<0, 2, 8, 2>(gp, s.KS, st);
+        else if (s.GW == 3) share_go<0, 3, 8, 3>(gp, s.KS, st);
         else share_go<0, 4, 8, 4>(gp, s.KS, st);
-    } else if (s.WK == 2) share_go<1, 3, 2, 3>(gp, s.KS, st);
-    else if (s.WK == 4) share_go<1, 3, 4, 3>(gp, s.KS, st);
-    else share_go<1, 2, 8, 2>(gp, s.KS, st);
+    } else if (s.GW == 2) {
+        if (s.WK == 2) share_go<1, 2, 2, 2>(gp, s.KS, st);
+        else if (s.WK == 4) share_go<1, 2, 4, 2>(gp, s.KS, st);
+        else share_go<1, 2, 8, 2>(gp, s.KS, st);
+    } else {
+        if (s.WK == 2) share_go<1, 3, 2, 3>(gp, s.KS, st);
+        else if (s.WK == 4) share_go<1, 3, 4, 3>(gp, s.KS, st);
+        else share_go<1, 3, 8, 3>(gp, s.KS, st);
+    }
 }

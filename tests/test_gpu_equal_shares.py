@@ -41,6 +41,15 @@ def _bank(dev, H, E, I, g, distinct=6, w_down=0.05):
     (40, 4096, 8, 2, 14336, 0),      # seven splits: 252 workgroups
     (64, 2048, 512, 8, 768, 3),      # the most experts
     (511, 2048, 384, 8, 768, 40),    # nearly the most pairs
+    (8, 3072, 8, 2, 512, 0),         # 24 groups in gate_up, the top-k inside; 2 x 2 in down
+    (6, 3072, 96, 8, 1024, 4),       # more than 64 experts to choose from; 4 x 2
+    (70, 3072, 64, 8, 512, 17),      # 560 pairs
+    (200, 3072, 256, 8, 512, 33),    # 1600 pairs
+    (40, 2048, 16, 2, 3072, 21),     # 8 x 3 groups
+    (9, 3072, 16, 2, 2304, 0),       # 2 x 3 groups and three splits: 255 workgroups
+    (20, 4096, 8, 2, 2560, 17),      # 2 x 2 groups and five splits
+    (33, 2048, 16, 2, 4608, 16),     # 4 x 3 groups and three splits
+    (12, 2048, 8, 2, 1280, 0),       # ten groups: no split of theirs; the other plan
 ])
 def test_equal_shares(dev, T, H, E, K, I, crowd):
     from on_device_sd_amd import ops

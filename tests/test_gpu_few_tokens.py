@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
     (16, 128, 3, 3, 512),       # a single group in the gate_up reduction, 16 rows on every expert; 4 groups
     (7, 640, 40, 7, 640),       # 49 pairs, 5 groups either way
     (16, 384, 24, 8, 896),      # 3 and 7 groups
-    (16, 2048, 64, 8, 1024),    # two weight blocks per wavefront in the down projection
+    (16, 2048, 64, 8, 1024),    # equal shares: 4 parts of 2 groups in the down projection
+    (16, 2176, 64, 8, 1024),    # two weight blocks per wavefront in the down projection
     (5, 1024, 8, 2, 4608),      # too many workgroups per expert to dispatch inside; split down reduction
     (1, 512, 64, 48, 512),      # one token with 48 pairs
 ])
