@@ -127,7 +127,8 @@ def _small_stack(dev, T, Hs, Es, Ks, Is, L, dtype, renorm=False, seed=1):
 @pytest.mark.parametrize("T,Hs,Es,Ks,Is,dtype", [
     (40, 512, 8, 2, 256, torch.bfloat16), (24, 4096, 8, 2, 256, torch.bfloat16), (33, 384, 8, 2, 128, torch.float32),
     (16, 1280, 16, 4, 256, torch.bfloat16), (20, 3072, 8, 2, 128, torch.float32), (9, 128, 4, 1, 128, torch.bfloat16),
-    (8, 5120, 8, 2, 128, torch.bfloat16)])
+    (8, 5120, 8, 2, 128, torch.bfloat16),
+    (6, 2048, 8, 2, 512, torch.float32), (18, 3072, 8, 2, 512, torch.float32)])      # equal shares
 def test_stack_call_equals_layer_calls_on_other_shapes(dev, T, Hs, Es, Ks, Is, dtype):
     print("stack call, shape", T, Hs, Es, Ks, Is, dtype, flush=True)
     st, x0 = _small_stack(dev, T, Hs, Es, Ks, Is, 3, dtype, renorm=Ks > 1, seed=T)
@@ -142,6 +143,42 @@ def test_stack_call_equals_layer_calls_on_other_shapes(dev, T, Hs, Es, Ks, Is, d
                     out_act=h[(l + 1) & 1])
     torch.cuda.synchronize()
     assert torch.equal(a, h[st.L & 1])
+
+
+# few rows per expert: the equal-share kernel, which up to 8 tokens takes the router's partial logits and does the top-k
+# (with rows that the previous block's combine prepared, and with a folded RMSNorm), and from 9 on dispatches
+@pytest.mark.parametrize("T", [1, 5, 8, 9, 24, 100])
+def test_stack_call_of_few_tokens(dev, layer, T):
+    print("stack call, few tokens", T, flush=True)
+    import on_device_sd_amd as odsd
+    bank, experts = layer
+    L = 3
+    cfg = odsd.MoEConfig(hidden_size=H, num_hidden_layers=L, num_experts=E, num_experts_per_token=K,
+                         moe_intermediate_size=I, norm_topk_prob=True)
+    gates = _gates(L, 300 + T, False)
+    g = torch.Generator().manual_seed(T)
+    norms = [(1 + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16) for _ in range(L)]
+    x0 = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    st = odsd.MoEOnlyStack(cfg, gates, norms, [bank] * L, T)
+    a = st.forward(x0.to(dev)).clone()
+    assert torch.equal(a, st.forward_layers(x0.to(dev)))
+    # every layer with the stand-alone RMSNorm kernel in front, held to the oracle as well
+    h = [x0.to(dev), torch.empty_like(a)]
+    for l in range(L):
+        before = h[l & 1].cpu()
+        st.plan.run(h[l & 1], st.gate[l], st.tables[l], st.norm[l], st.config.rms_norm_eps, add_residual=True,
+                    out_act=h[(l + 1) & 1])
+        normed = orc.rmsnorm(before, norms[l], EPS)
+        idx, w = orc.route(orc.router_logits(normed, gates[l]), K, True)
+        ref = (before.float() + orc.moe_forward(normed, idx, w, experts).to(torch.bfloat16).float()).to(torch.bfloat16)
+        check_output(h[(l + 1) & 1].float().cpu() - before.float(), ref.float() - before.float())
+    assert torch.equal(a, h[L & 1])
+    st.capture()
+    for _ in range(3):
+        r = st.forward(x0.to(dev))
+        torch.cuda.synchronize()
+        assert torch.equal(r, a)
+        st.forward_layers(x0.to(dev))
 
 
 def test_stack_call_small_shape_and_arguments(dev):

@@ -241,6 +241,10 @@ EXPERT_CASES = [
     (100, 256, 2, 2, 128, torch.bfloat16),    # 100 rows per expert: one partial 128-row streaming pass
     (600, 256, 2, 2, 1024, torch.bfloat16),   # few tiles: passes shared by workgroups, down reduction split in 2
     (260, 256, 1, 1, 1280, torch.bfloat16),   # one expert, 10 groups in down: two slices of 5 (odd start, odd length)
+    # fp32 activations: equal shares with the top-k inside and with the dispatch inside, 48-row kernel
+    (5, 2048, 8, 2, 512, torch.float32),
+    (24, 2048, 8, 2, 768, torch.float32),
+    (600, 4096, 40, 2, 256, torch.float32),
 ]
 
 
@@ -275,6 +279,9 @@ OFFSET_CASES = [
     (40, 512, 4, 2, 384, -0.5, 0.01),
     (6, 1024, 4, 2, 256, 0.3, 0.02),        # direct path
     (600, 256, 2, 2, 384, 0.15, 0.01),      # tile kernel (fp16 y: keep the outputs inside fp16 range)
+    (24, 2048, 8, 2, 768, 0.1, 0.02),       # equal shares
+    (6, 4096, 8, 2, 2048, -0.1, 0.01),      # equal shares, the top-k inside, fp32 sums
+    (600, 4096, 40, 2, 256, 0.1, 0.02),     # 48-row kernel
 ]
 
 
@@ -446,15 +453,17 @@ def test_bank_unpacks_to_the_canonical_arrays(dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H", [128, 1280, 2048])
-def test_rmsnorm_folded_into_router_matches_standalone(dev, H):
+@pytest.mark.parametrize("T,H,I", [(37, 128, 256), (37, 1280, 256), (37, 2048, 256),
+                                   (5, 2048, 768), (8, 4096, 512),       # the top-k inside the equal-share kernel
+                                   (20, 2048, 768)])                     # the dispatch inside it
+def test_rmsnorm_folded_into_router_matches_standalone(dev, T, H, I):
     """Two chained blocks: the first block's combine leaves per-row sums of squares, the second
     block folds its RMSNorm into the router kernel with them.  The result must equal, bit for
     bit, the run in which the second block runs the stand-alone RMSNorm kernel, and the
     statistic must be the sum of squares of the rows that were stored."""
     import on_device_sd_amd as odsd
     from on_device_sd_amd import ops
-    T, E, K, I = 37, 8, 2, 256
+    E, K = 8, 2
     g = torch.Generator().manual_seed(11)
     x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
     gate = (0.02 * torch.randn(E, H, generator=g)).to(torch.bfloat16).to(dev)

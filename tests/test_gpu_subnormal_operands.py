@@ -14,7 +14,7 @@ SHAPES = [
     (24, 2048, 16, 2, 768),        # equal shares; down in two parts of three groups
     (5, 4096, 8, 2, 2048),         # equal shares with the top-k inside; down in eight parts of two groups
     (160, 2048, 128, 8, 768),      # the one-launch kernel
-    (104, 4096, 8, 1, 1024),       # the 48-row kernel
+    (600, 4096, 40, 2, 256),       # the 48-row kernel (1200 pairs: more than the streaming kernel dispatches for itself)
 ]
 
 
