@@ -121,6 +121,14 @@ def _traffic(wl_name, kernel=None):
         return None, None
 
 
+def _recorded_kernel(wl_name, key, mode):
+    """The streaming kernel that the workload ran when its traffic was recorded (the plan chooses among several)."""
+    try:
+        return json.load(open(TRAFFIC_FILE))[wl_name][key]
+    except (OSError, KeyError, ValueError):
+        return f"{mode} (streaming kernel of the plan)"
+
+
 def _dominant(wl, k, active_experts, launches=1):
     """The dominant kernel of a workload, its time per launch and the algorithmic bytes of one launch:
     the one-launch expert kernel (gate_up + down weights of the active experts) where the library
@@ -140,7 +148,7 @@ def _roofline(wl, kernel_ms, algorithmic_bytes, kernel=None):
                 "traffic": traffic, "algorithmic_flops": gu_flops}
     else:
         ach = algorithmic_bytes / (kernel_ms * 1e-3) / 1e9
-        roof = {"bound": "hbm", "kernel": kernel or "gate_up (streaming kernel of the plan)", "achieved": round(ach, 1),
+        roof = {"bound": "hbm", "kernel": kernel or _recorded_kernel(wl.name, "kernel", "gate_up"), "achieved": round(ach, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                 "traffic": traffic, "algorithmic_bytes": int(algorithmic_bytes)}
     if commit:
@@ -237,7 +245,7 @@ def bench_layer(wl, dev, steps, warmup, with_cpu):
                                     "frac": round(ach / MFMA_F16_PEAK_TFLOPS, 4), "kernel_ms": round(k["down"], 5)}
         else:
             ach = down_bytes / (k["down"] * 1e-3) / 1e9
-            res["down_roofline"] = {"bound": "hbm", "kernel": "down (streaming kernel of the plan)", "achieved": round(ach, 1),
+            res["down_roofline"] = {"bound": "hbm", "kernel": _recorded_kernel(wl.name, "down_kernel", "down"), "achieved": round(ach, 1),
                                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                                     "algorithmic_bytes": int(down_bytes), "kernel_ms": round(k["down"], 5)}
     del runner, placements, plan, banks, tables

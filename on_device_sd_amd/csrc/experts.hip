@@ -10,7 +10,7 @@
 //
 //   MODE 0  gate_up: rows of the fused [2I, H] matrix alternate 16 gate rows / 16 up rows,
 //           so one lane holds gate and up of the same feature; epilogue h = silu(g)*u -> fp16
-//   MODE 1  down:    y[ks][slot][H] fp32 partials over KS slices of the reduction dimension
+//   MODE 1  down:    y[ks][slot][H] partial sums (fp32 or fp16) over KS slices of the reduction dimension
 //                    (summed in a fixed order by the combine, so split-K stays deterministic)
 //
 // Token rows of one expert are shared by the 4 wavefronts of a workgroup through LDS
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void w4_gemm_kernel(const GemmPara
 // (with its address behind a branch, say) is what the kernel's time consists of: pair by pair, slice by slice / now,
 // us: K = 8, T = 256 7.6 / 6.3; K = 2: seven slices, T = 5 6.6 / 5.0; four, T = 160 6.9 / 5.3; two, T = 32, H = 512
 // 5.5 / 3.3.
-// YH: 0 = y holds fp32 partial sums of KS slices; 1 = complete sums as fp16; 2 = KS fp16 slices
+// YH: 0 = y holds fp32 sums of KS slices (one or more); 1 = complete sums as fp16; 2 = KS fp16 slices
 // Gather-sum of one token's columns c .. c+3: sum over k of w[t,k] * (sum over slices of y[slice][slot(t,k)]).
 template <int YH, int KB>
 __device__ __forceinline__ float4_t combine_gather(const float *__restrict__ y, const int32_t *__restrict__ idx,
@@ -653,7 +653,7 @@ struct ExpertsPlan {
     int KS;          // split of the down projection's reduction dimension across workgroups
     int PS_gu, PS_dn;  // workgroups sharing the row passes of one tile
     int tile;        // the tile kernel (experts_prefill.hip) instead of the streaming kernel
-    int y_f16;       // down-projection outputs kept as fp16 (unsplit reduction) instead of fp32 partials
+    int y_f16;       // down-projection outputs kept as fp16 instead of fp32
     int fused;       // whole-block calls run gate_up and down as one launch (experts_fused.hip)
     int share;       // equal-share streaming kernel (experts_share.hip) for gate_up and down
     int mid;         // 48-row streaming kernel (experts_mid.hip) for gate_up and down
@@ -767,7 +767,9 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
         // A popular expert's passes side by side instead of in turn: four workgroups share them, no more than there can
         // be passes.  Layer, us, one / two / four: E = 128, H = 2048, I = 768, Zipf, T = 400 154 / 135 / 122, T = 600
         // 195 / 165 / 146, T = 800 248 / 203 / 177; H = 4096, I = 1536, Zipf, T = 800 631 / 564 / 534; E = 8, I = 14336,
-        // Zipf, T = 160 248 / 233 / 233; uniform T = 400 105 / 105 / 105, T = 800 143 / 138 / 138.
+        // Zipf, T = 160 248 / 233 / 233; uniform T = 400 105 / 105 / 105, T = 800 143 / 138 / 138.  The workgroups without a
+        // pass show where there are thousands and the rest is short: H = I = 512, E = 512, K = 8, T = 256, one / four, uniform
+        // 81.8 / 83.8, Zipf 120 / 66.6; E = 256, T = 200 46.6 / 47.7, Zipf 82.4 / 46.3.
         if (p.MB <= 4) {
             const int rows = p.mid ? ODSD_MID_ROWS : 16 * p.MB, most = (s->T + rows - 1) / rows;
             p.PS_gu = p.PS_dn = most < 4 ? most : 4;
@@ -795,7 +797,10 @@ static ExpertsPlan experts_plan(const odsd_moe_shape *s) {
     // 152 / 135, T = 48 (12 rows) 153 / 146, T = 56 153 / 169.  From 14 rows on too many experts take a second pass
     // over their weights, which the plan above saves with wider ones.
     // Its splits of the down projection follow from the reduction alone, so with many rows of a long one it can need more
-    // partial sums than the plan above: not where that takes a block out of the library's static array.
+    // partial sums than the plan above: not where that takes a block out of the library's static array.  A block that is
+    // past the array either way takes them: at most 16 slices of at most 12 rows per expert are under 3 % of the weights
+    // (H = 4096, I = 14336, E = 128, K = 2, T = 768, seven slices 2237 / 2149; I = 5632, E = 512, K = 8, T = 512, eleven
+    // 3470 / 3097).
     p.share = 0;
     if (mean_rows <= 12 && odsd_share_supported(s->H, s->I, s->E, (int)P)) {
         const int KS = odsd_share_down_splits(s->I);

@@ -17,10 +17,10 @@
 //     workgroups without one come last and only look at the row count.  Zipf-distributed routing, E = 128, one / four,
 //     layer, us: T = 256 352 / 302, T = 400 464 / 357; uniform routing does not notice (256 / 256, 291 / 293).
 //
-// Bound by issue at 33 to 48 rows (matrix cores busy 38 %, vector instructions 31 % of the cycles, 1.75 rounds of
-// workgroups at E = 8), by HBM at up to 16 (about 6 TB/s).  Measured and not kept: no interleaving of vector and matrix
-// instructions (before the workgroups started on different groups, E = 128, T = 400: 318 / 309 with it; E = 8, T = 160
-// 208 / 211).  Passes of 64 rows take 254 registers without the interleaving and leave none for it.
+// Bound by issue from some 25 rows on: H = 4096, I = 14336, E = 8, T = 136 (34 rows) matrix cores busy 37 % of the cycles, other
+// vector instructions issuing 35 %, 1.75 rounds of workgroups; T = 100 32 % and 34 %.  At up to 16 rows by HBM.  Measured and
+// not kept: no interleaving of vector and matrix instructions (before the workgroups started on different groups, E = 128,
+// T = 400: 318 / 309 with it; E = 8, T = 160 208 / 211).  Passes of 64 rows take 254 registers without the interleaving and leave none for it.
 //
 //   MODE 0  gate_up: h = SiLU(gate) * up -> fp16
 //   MODE 1  down: KS splits of the reduction across workgroups, fp16 sums
@@ -35,7 +35,7 @@
 
 template <int MODE, int NB>
 __global__ __launch_bounds__(64 * MID_WAVES, 2) void w4_mid_kernel(const GemmParams p) {
-    constexpr int XS = 16 * MID_MB * 256;                // bytes of a token-row buffer: 64 rows of one group
+    constexpr int XS = 16 * MID_MB * 256;                // bytes of a token-row buffer: 48 rows of one group
     __shared__ __attribute__((aligned(16))) char xs_raw[MID_XB * XS];
     // everyone's first passes come before anyone's second
     const int b = (int)blockIdx.x % p.n_wg, ps = (int)blockIdx.x / p.n_wg;

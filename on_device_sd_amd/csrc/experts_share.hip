@@ -1,8 +1,11 @@
 // Streaming W4 GEMM in equal shares: experts with few rows on average.
 //
-// The weights of the experts with rows are one long list of units -- (expert, pass of 16 rows, blocks of 16 weight rows) -- and every workgroup takes the same number of consecutive units, whichever experts they belong to:
-// one workgroup per CU, no second round of workgroups, no CU left over because its expert has no rows, and an
-// expert with more rows than a pass holds is just more units of the list.
+// The weights of the experts with rows are one long list of units -- (expert, pass of 16 rows, blocks of 16 weight rows) --
+// and every workgroup takes the same number of consecutive units, one more or less, whichever experts they belong to: one
+// workgroup per CU, no second round of workgroups, no CU left over because its expert has no rows, and an expert with more
+// rows than a pass holds is just more units of the list.  Where a unit is large and a share short that one unit shows: down
+// at I = 768 has units of 51 KB, 6.3 to 7.1 per CU at T = 24 to 64, so the slowest, with 7 or 8, takes 11 to 13 % longer
+// than the mean.
 //
 // The wavefronts of a workgroup split the reduction: a wavefront owns GW groups of 128 columns of every unit, so
 // the token rows it needs -- its columns of the expert's rows -- stay in registers as MFMA B operands for as long
@@ -13,17 +16,16 @@
 // Codes go to the matrix cores as they are, scale and zero point are applied to each group's sum (as in
 // w4_expert_fused_kernel: 5 vector instructions per 8 weights instead of 13).
 //
-// Bound by HBM once it streams: at H = 2048, I = 768, E = 128, T = 24 a unit of gate_up (34 KB with its scales) takes
-// a workgroup 1.14 us, 7.6 TB/s over the chip, against 4.4 TB/s for the kernel whose workgroups own (expert, 128
-// rows).  The rest is start-up: 2.8 us until the list is there, 1 to 2 until the first rows and weights are.  Kernel
-// times there, before / now: gate_up 39.3 / 29.6 us (169 MB), down 20.1 / 17.7 (84 MB); H = 4096, I = 14336, T = 5:
-// 59.4 / 48.6 and 30.7 / 27.7.  Measured and not kept: reading a unit's sums behind the next unit's steps (no change),
-// one wavefront per whole reduction without a barrier (its rows are then read eight times, 20.2), 6 wavefronts with
-// one group each (21.9: two SIMDs have twice the work of the others), 16 wavefronts per CU with 3 steps in flight
-// each (23.5), two token blocks per pass (T = 256: 47 + 34).
+// Bound by HBM once it streams: 3.5 GB of gate_up (H = 4096, I = 14336, 56 experts) take 496 us, 7.0 TB/s.  Short streams are
+// mostly start-up: 2.8 us until the list is there, 1 to 2 until the first rows and weights are.  H = 2048, I = 768, E = 128,
+// T = 24, the kernel whose workgroups own (expert, 128 rows) / this: gate_up 39.3 / 29.8 us (169 MB, 5.7 TB/s), down
+// 20.1 / 18.2 (84 MB, 4.6 TB/s); H = 4096, I = 14336, T = 5: 59.4 / 48.6 and 30.7 / 27.7.  Measured and not kept: reading a
+// unit's sums behind the next unit's steps (no change), one wavefront per whole reduction without a barrier (down there 20.2:
+// its rows are then read eight times), 6 wavefronts with one group each (21.9: two SIMDs have twice the work of the others),
+// 16 wavefronts per CU with 3 steps in flight each (23.5), two token blocks per pass (T = 256: 47 + 34).
 //
 //   MODE 0  gate_up: unit = a gate block and its up block, h = SiLU(gate) * up -> fp16
-//   MODE 1  down: unit = RSUB * NB blocks of output rows, KS splits of the reduction across workgroups
+//   MODE 1  down: unit = RSUB * NB blocks of output rows, KS splits of the reduction across workgroups, fp32 or fp16 sums
 #include "w4_gemm.h"
 #include "w4_raw.h"
 #include "router_topk.h"
@@ -475,8 +477,9 @@ static void share_go(GemmParams &gp, int KS, hipStream_t st) {
 #undef SHARE_GO
 }
 
-// Steps in flight per wavefront (2 KiB each): 2 to 4, no more than a unit has; more do not stream faster (H = 2048,
-// I = 768, T = 24: gate_up 2 / 3 / 4 / 6 steps 27.5 / 27.8 / 27.8 / 28.7 us; down 3 / 4 / 6 17.7 / 17.9 / 18.8).
+// Steps in flight per wavefront (2 KiB each): 2 to 4, as many as a unit has, so that every unit begins on ring slot 0.  More
+// did not stream faster in an earlier form whose ring ran on over several units (H = 2048, I = 768, T = 24: gate_up
+// 2 / 3 / 4 / 6 steps 27.5 / 27.8 / 27.8 / 28.7 us; down 3 / 4 / 6 17.7 / 17.9 / 18.8).
 void odsd_launch_share(int mode, GemmParams &gp, hipStream_t st) {
     ShareSplit s;
     if (!share_split(mode, gp.G, &s)) return;

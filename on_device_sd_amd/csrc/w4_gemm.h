@@ -27,7 +27,8 @@ struct GemmParams {
     int ldo;                 // I (MODE 0) or H (MODE 1)
     int P;
     int E;
-    int n_wg;                // E * nchunks * KS (* PS)
+    int n_wg;                // E * nchunks * KS: the grid is PS times that where workgroups share a tile's passes
+                             // (equal shares: all workgroups)
     int wg_per_xcd;          // ceil(n_wg / 8)
     // gate_up with the dispatch inside (idx given; counts / offsets / rowmap are then NOT inputs):
     // every workgroup finds its expert's pairs in the id list itself, and the first workgroup of
