@@ -15,12 +15,14 @@ from . import _lib
 from ._lib import MoeShape
 
 
+_DTYPE_CODES = {torch.float32: _lib.DT_F32, torch.bfloat16: _lib.DT_BF16}
+
+
 def _dtype_code(dt: torch.dtype) -> int:
-    if dt == torch.float32:
-        return _lib.DT_F32
-    if dt == torch.bfloat16:
-        return _lib.DT_BF16
-    raise TypeError(f"activation dtype {dt} is not supported (float32 or bfloat16)")
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        raise TypeError(f"activation dtype {dt} is not supported (float32 or bfloat16)")
+    return code
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -30,12 +32,14 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 # The raw handle of torch's current stream.  torch.cuda.current_stream() builds a Stream object through
 # several Python layers (8 us per call, three calls per layer on the engine path); the C entry point
 # torch's own compiled-graph runtime uses for the same question takes a fraction of a microsecond.
+# (The same for the device: its C entry point, which needs the runtime to be up, as it is once a tensor is there.)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _stream() -> int:
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_raw_device())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -111,17 +115,25 @@ def w4_load_expert(gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor,
                    dst: Tuple[int, int, int, int]) -> None:
     """gate [I,H], up [I,H], down [H,I] (float32 / bfloat16) -> the streaming layout at the four device
     addresses ``dst`` (gate_up codes, gate_up (scale, zero), down codes, down (scale, zero)), in one launch."""
-    _require_cuda(gate, up, down)
-    I, H = gate.shape
-    if up.shape != gate.shape or down.shape != (H, I):
+    # (a model load calls this thousands of times for kernels of 5 us: a launch takes the host 3.3, and what is written
+    # out here in place of helper calls took 1.5)
+    if not (gate.is_cuda and up.is_cuda and down.is_cuda):
+        _require_cuda(gate, up, down)
+    shape = gate.shape
+    I, H = shape
+    if up.shape != shape or down.shape != (H, I):
         raise ValueError(f"expert weights do not belong together: {tuple(gate.shape)}, {tuple(up.shape)}, {tuple(down.shape)}")
     gate, up, down = gate.contiguous(), up.contiguous(), down.contiguous()
     a, b, c = gate.data_ptr(), up.data_ptr(), down.data_ptr()
-    if (a | b | c) % 16:                                          # the kernel reads 16 bytes at a time
+    if (a | b | c) & 15:                                          # the kernel reads 16 bytes at a time
         gate, up, down = gate.clone(), up.clone(), down.clone()
         a, b, c = gate.data_ptr(), up.data_ptr(), down.data_ptr()
-    _lib.check(_lib.load().odsd_w4_load_expert(a, _dtype_code(gate.dtype), b, _dtype_code(up.dtype), c,
-                                               _dtype_code(down.dtype), H, I, *dst, _stream()), "odsd_w4_load_expert")
+    t, u, v = gate.dtype, up.dtype, down.dtype
+    ct = _dtype_code(t)
+    cu, cv = (ct if u is t else _dtype_code(u)), (ct if v is t else _dtype_code(v))
+    rc = _lib.load().odsd_w4_load_expert(a, ct, b, cu, c, cv, H, I, *dst, _stream())
+    if rc:
+        _lib.check(rc, "odsd_w4_load_expert")
 
 
 # ------------------------------------------------------------------------------------------

@@ -119,14 +119,16 @@ class W4ExpertBank:
         """Quantise one expert's [I,H], [I,H], [H,I] weights on the device and pack them: in one launch, or
         through the canonical arrays when the caller wants those as well."""
         # (by index, -1 for the host: another GPU's tensor has to move as well)
-        ws = [w if w.get_device() == self._device_index else w.to(self.gu_q.device) for w in (gate_w, up_w, down_w)]
+        at = self._device_index
+        if gate_w.get_device() != at or up_w.get_device() != at or down_w.get_device() != at:
+            gate_w, up_w, down_w = (w if w.get_device() == at else w.to(self.gu_q.device) for w in (gate_w, up_w, down_w))
         if keep_canonical:
-            canon = tuple(ops.w4_quantize(w) for w in ws)
+            canon = tuple(ops.w4_quantize(w) for w in (gate_w, up_w, down_w))
             self.load_canonical(e, *canon)
             return canon
-        if ws[0].shape != (self.inter, self.hidden):
-            raise ValueError(f"expert weights of shape {tuple(ws[0].shape)}: this bank holds [{self.inter}, {self.hidden}]")
-        ops.w4_load_expert(*ws, self._ptrs[e])
+        if gate_w.shape != (self.inter, self.hidden):
+            raise ValueError(f"expert weights of shape {tuple(gate_w.shape)}: this bank holds [{self.inter}, {self.hidden}]")
+        ops.w4_load_expert(gate_w, up_w, down_w, self._ptrs[e])
         self.mark_loaded(e)
         return None
 
