@@ -16,6 +16,7 @@
 // (:210-216) and GPUOperators.router (demo/src/operators/gpu_operators.py:48-69).
 #include "common.h"
 #include "router_topk.h"
+#include "w4_gemm.h"
 
 #include <type_traits>
 
@@ -226,6 +227,406 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const double *__restri
     topk_token<V>(partial, t, T, E, K, S, renorm, idx, w, idx64, logits);
 }
 
+// -----------------------------------------------------------------------------------------
+// Many tokens, bf16: the logits on the bf16 matrix cores, and in fp64 only where the choice hangs on more.
+//
+// v_mfma_f32_16x16x32_bf16 multiplies exactly and runs 30 times as fast as the fp64 product.  Two products of 32
+// columns, each from zero, are added in fp32, and everything above them in fp64, so a logit is off by at most
+//     SCREEN_ERR * |x| * |w|,  SCREEN_ERR = 35 * 2^-23
+// (32 additions of a product and the one of two products, each off by no more than a unit in the last place of the
+// sum of the magnitudes so far -- whatever order the matrix core adds in, and whether it rounds or truncates -- then
+// Cauchy-Schwarz; the norms' own rounding and flushed subnormals are in the remaining 6 %).  The top-k kernel takes
+// neighbours in the order that are further apart than twice this bound as they are, and computes the others anew in
+// fp64: the indices are those of the exact logits.  On N(0, 1) tokens that is one token in thirty, two or three dot products
+// each.  The weights come from these logits through fp64 exponentials and are rounded to fp32 once: 4e-8 off
+// (2-norm; 5.3e-8 with fp64 logits and fp32 exponentials).
+//
+// A workgroup of 8 wavefronts owns 32 tokens x 128 experts over one K slice, 128 columns a step; a wavefront 64 of the
+// experts and a quarter of the columns; the quarters meet in LDS.  Rows arrive by asynchronous copies two steps ahead,
+// 256 bytes of a row together: fragments loaded straight into registers, 64 bytes of each of 16 rows 8 KB apart, took
+// 32 us at T = 4096, H = 4096 where this takes 22.  The sums of two steps go to the fp64 accumulators together
+// (conversion and addition are the larger part of the vector work).
+// -----------------------------------------------------------------------------------------
+#define SCREEN_NT 2
+#define SCREEN_NE 4
+#define SCREEN_EXPERTS (2 * 16 * SCREEN_NE)   // of a workgroup
+#define SCREEN_ERR (35.0 / 8388608.0)
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+// sum of squares of 8 bf16, and whether any of them is not zero
+__device__ __forceinline__ float sumsq8(const uint4_t &u, float acc, uint32_t &bits) {
+    float v[8];
+    Row8<uint16_t>::cvt(u, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc = __builtin_fmaf(v[j], v[j], acc);
+    bits |= (u.x | u.y | u.z | u.w) & 0x7fff7fffu;
+    return acc;
+}
+// what stands for a norm: 0 only for a row of zeros (squares may vanish where the row has not)
+__device__ __forceinline__ float nonzero_sq(const float ss, const bool any) { return any ? fmaxf(ss, 1.17549435e-38f) : 0.0f; }
+
+template <bool NORMED>
+__global__ __launch_bounds__(512, 2) void router_screen_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg,
+                                                            double *__restrict__ partial, float *__restrict__ xsq,
+                                                            float *__restrict__ wsq, half_t *__restrict__ x16, int T,
+                                                            int H, int E, int S, int EG,
+                                                            const double *__restrict__ norm_ss,
+                                                            const uint16_t *__restrict__ norm_w, double eps) {
+    constexpr int XB = 16 * SCREEN_NT * 256, BUF = XB + SCREEN_EXPERTS * 256, N_DMA = BUF / 8192;
+    constexpr int NTILE = SCREEN_NT * SCREEN_NE;
+    __shared__ __attribute__((aligned(16))) char rows[3 * BUF];   // token rows, then expert rows, of 128 columns
+    __shared__ float red_ss[4][16 * SCREEN_NT], red_w[8];
+    static_assert(8 * N_DMA * 1024 == BUF && 4 * 2 * (NTILE - NTILE / 4) * 2048 <= 3 * BUF, "whole copies; partial sums take the rows' place");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+    const int unit = blockIdx.x;
+    const int s = unit % S, eg = (unit / S) % EG, tt = unit / (S * EG);
+    const int Hs = H / S, k0 = s * Hs, ng = Hs / ODSD_GROUP;
+    const int r = lane & 15, kg = lane >> 4;
+    const int eh = wave & 1, q = wave >> 1;              // the wavefront's 64 experts and its 32 of the 128 columns
+    // copies: 4 rows x 256 B each, 16-byte segments XORed with the row as in the expert kernels
+    uint32_t off[N_DMA];
+#pragma unroll
+    for (int i = 0; i < N_DMA; ++i) {
+        const int row = (wave * N_DMA + i) * 4 + kg;     // token rows first
+        const int t = tt * 16 * SCREEN_NT + row, e = eg * SCREEN_EXPERTS + row - 16 * SCREEN_NT;
+        const int src = row < 16 * SCREEN_NT ? (t < T ? t : 0) : (e < E ? e : 0);
+        off[i] = ((uint32_t)src * (uint32_t)H + (uint32_t)(k0 + ((r ^ (row & 15)) * 8))) * 2u;
+    }
+    auto dma = [&](const int buf, const int g) {
+        const global_char *xb = (const global_char *)x + (size_t)g * (2 * ODSD_GROUP), *wb = (const global_char *)wg + (size_t)g * (2 * ODSD_GROUP);
+#pragma unroll
+        for (int i = 0; i < N_DMA; ++i) {
+            const int piece = wave * N_DMA + i;
+            dma16_to_lds(piece < 4 * SCREEN_NT ? xb : wb, off[i], (lds_void *)(rows + buf * BUF + piece * 1024));
+        }
+    };
+    int t_of[SCREEN_NT];
+    double rstd[SCREEN_NT];
+#pragma unroll
+    for (int i = 0; i < SCREEN_NT; ++i) {
+        const int t = (tt * SCREEN_NT + i) * 16 + r;
+        t_of[i] = t < T ? t : -1;
+        rstd[i] = 1.0;
+        if (NORMED) {                                    // as in router_partial_kernel
+            const int nchunk = (H + 1023) / 1024;
+            double tot = 0.0;
+            for (int c = 0; c < nchunk; ++c) tot += norm_ss[(size_t)(t < T ? t : 0) * nchunk + c];
+            rstd[i] = 1.0 / sqrt(tot / (double)H + eps);
+        }
+    }
+    double4_t acc[NTILE];
+#pragma unroll
+    for (int m = 0; m < NTILE; ++m) acc[m] = double4_t{0.0, 0.0, 0.0, 0.0};
+    float ss[SCREEN_NT] = {};
+    uint32_t bits[SCREEN_NT] = {};
+    const uint32_t frag = (uint32_t)((r * 16 + ((4 * q + kg) ^ r)) * 16);
+
+    dma(0, 0);
+    if (ng > 1) dma(1, 1);
+    // the experts' norms, one expert a workgroup while the rows travel
+    for (int e = unit; e < E; e += gridDim.x) {
+        float sw = 0.f;
+        uint32_t bw = 0;
+        for (int h = (int)threadIdx.x * 8; h < H; h += 4096) sw = sumsq8(*(const uint4_t *)(wg + (size_t)e * H + h), sw, bw);
+        sw = nonzero_sq(wave_sum(sw), __any(bw != 0));
+        if (lane == 0) red_w[wave] = sw;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            float tot = 0.f;
+            for (int i = 0; i < 8; ++i) tot += red_w[i];
+            wsq[e] = tot;
+        }
+        __syncthreads();
+    }
+    int buf = 0;
+    float4_t pend[NTILE];
+    // one group; the sums of two groups go to the fp64 accumulators together
+    auto step = [&](const int g, const bool second) {
+        // (loads land in order, and no more than the next group's are left; the stores of the copy only make this stricter)
+        if (g + 1 < ng) ODSD_WAIT_VMCNT(N_DMA);
+        else ODSD_WAIT_VMCNT(0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (g + 2 < ng) dma(buf == 0 ? 2 : buf - 1, g + 2);      // what the step before this one read
+        const char *base = rows + buf * BUF + frag;
+        uint4_t xf[SCREEN_NT], wf[SCREEN_NE];
+#pragma unroll
+        for (int i = 0; i < SCREEN_NT; ++i) xf[i] = *(const uint4_t *)(base + i * 4096);
+#pragma unroll
+        for (int j = 0; j < SCREEN_NE; ++j) wf[j] = *(const uint4_t *)(base + XB + (eh * SCREEN_NE + j) * 4096);
+        if (NORMED) {
+            float nw[8];
+            Row8<uint16_t>::cvt(*(const uint4_t *)(norm_w + k0 + g * ODSD_GROUP + 32 * q + 8 * kg), nw);
+#pragma unroll
+            for (int i = 0; i < SCREEN_NT; ++i) {
+                float v[8];
+                Row8<uint16_t>::cvt(xf[i], v);
+                uint32_t o[4];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float xn = ActIO<uint16_t>::round((float)((double)v[k] * rstd[i]));
+                    const uint32_t b = f32_to_bf16(__fmul_rn(xn, nw[k]));
+                    o[k >> 1] = (k & 1) ? o[k >> 1] | (b << 16) : b;
+                }
+                xf[i] = uint4_t{o[0], o[1], o[2], o[3]};
+            }
+        }
+        const float4_t z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < SCREEN_NE; ++j)
+#pragma unroll
+            for (int i = 0; i < SCREEN_NT; ++i) {
+                const int m = i * SCREEN_NE + j;
+                const float4_t v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xf[i]),
+                                                                          __builtin_bit_cast(bf16x8_t, wf[j]), z, 0, 0, 0);
+                if (second) {
+                    acc[m].x += (double)(pend[m].x + v.x);
+                    acc[m].y += (double)(pend[m].y + v.y);
+                    acc[m].z += (double)(pend[m].z + v.z);
+                    acc[m].w += (double)(pend[m].w + v.w);
+                } else {
+                    pend[m] = v;
+                }
+            }
+        // expert group 0: norms and the fp16 copy of x, token block i by the wavefronts of expert half i
+        if (eg == 0) {
+#pragma unroll
+            for (int i = 0; i < SCREEN_NT; ++i) {
+                if (i != eh) continue;
+                ss[i] = sumsq8(xf[i], ss[i], bits[i]);
+                if (x16 != nullptr && t_of[i] >= 0) {
+                    float v[8];
+                    Row8<uint16_t>::cvt(xf[i], v);
+                    half8_t o;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) o[k] = f32_to_f16_sat(v[k]);
+                    *(half8_t *)(x16 + (size_t)t_of[i] * H + k0 + g * ODSD_GROUP + 32 * q + 8 * kg) = o;
+                }
+            }
+        }
+        buf = buf == 2 ? 0 : buf + 1;
+    };
+    for (int g = 0; g < ng; g += 2) {
+        step(g, false);
+        if (g + 1 < ng) {
+            step(g + 1, true);
+        } else {
+#pragma unroll
+            for (int m = 0; m < NTILE; ++m) {
+                acc[m].x += (double)pend[m].x;
+                acc[m].y += (double)pend[m].y;
+                acc[m].z += (double)pend[m].z;
+                acc[m].w += (double)pend[m].w;
+            }
+        }
+    }
+    // The four quarters of the columns meet in LDS, in the rows' place: each wavefront leaves the tiles that it does not
+    // finish, and finishes two.
+    __syncthreads();
+    double *red = (double *)rows;
+    constexpr int OWN = NTILE / 4;
+    auto slot = [&](const int from, const int m) {       // tile m of wavefront (from, eh): m without the tiles that `from` owns
+        const int k = m < from * OWN ? m : m - OWN;
+        return red + ((size_t)((from * 2 + eh) * (NTILE - OWN) + k) * 4) * 64 + lane;
+    };
+#pragma unroll
+    for (int m = 0; m < NTILE; ++m) {
+        if (m / OWN == q) continue;
+        double *o = slot(q, m);
+        o[0] = acc[m].x; o[64] = acc[m].y; o[128] = acc[m].z; o[192] = acc[m].w;
+    }
+    if (eg == 0) {
+#pragma unroll
+        for (int i = 0; i < SCREEN_NT; ++i) {
+            if (i != eh) continue;
+            ss[i] += __shfl_xor(ss[i], 16, 64);
+            ss[i] += __shfl_xor(ss[i], 32, 64);
+            bits[i] |= (uint32_t)__shfl_xor((int)bits[i], 16, 64);
+            bits[i] |= (uint32_t)__shfl_xor((int)bits[i], 32, 64);
+            if (kg == 0) red_ss[q][i * 16 + r] = nonzero_sq(ss[i], bits[i] != 0);
+        }
+    }
+    __syncthreads();
+    if (eg == 0 && wave == 0 && lane < 16 * SCREEN_NT) {
+        const int t = tt * 16 * SCREEN_NT + lane;
+        if (t < T) xsq[(size_t)s * T + t] = (red_ss[0][lane] + red_ss[1][lane]) + (red_ss[2][lane] + red_ss[3][lane]);
+    }
+#pragma unroll
+    for (int m = 0; m < NTILE; ++m) {
+        if (m / OWN != q) continue;
+        double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int from = 0; from < 4; ++from) {
+            const double *o = slot(from, m);
+            if (from == q) {
+                v[0] += acc[m].x; v[1] += acc[m].y; v[2] += acc[m].z; v[3] += acc[m].w;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] += o[64 * k];
+            }
+        }
+        // lane: tokens 4 kg .. of the block, expert r
+        const int e = eg * SCREEN_EXPERTS + (eh * SCREEN_NE + m % SCREEN_NE) * 16 + r;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int t = (tt * SCREEN_NT + m / SCREEN_NE) * 16 + kg * 4 + k;
+            if (t < T && e < E) partial[((size_t)s * T + t) * E + e] = v[k];
+        }
+    }
+}
+
+// One wavefront per token, as router_topk_kernel, on the logits of router_screen_kernel.  K < E and K < 64.
+// The logits to be computed anew go on a list of the workgroup, and its four wavefronts share them: a token that needs
+// any needs two or three, and with each of them on a wavefront of its own the kernel ends one dot product later, not three.
+#define SCREENED_WAVES 4
+template <int V, bool NORMED>
+__global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kernel(
+    const double *__restrict__ partial, const float *__restrict__ xsq, const float *__restrict__ wsq,
+    const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg, int T, int H, int E, int K, int S, int renorm,
+    int32_t *__restrict__ idx, float *__restrict__ w, int64_t *__restrict__ idx64, const double *__restrict__ norm_ss,
+    const uint16_t *__restrict__ norm_w, double eps) {
+    __shared__ double anew[SCREENED_WAVES * 64 * V];
+    __shared__ uint32_t list[SCREENED_WAVES * 64 * V];
+    __shared__ int n_list;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+    const int t = blockIdx.x * SCREENED_WAVES + wave;
+    const bool mine = t < T;
+    if (threadIdx.x == 0) n_list = 0;
+    double lg[V];
+    float nx = 0.f, nw = 0.f;
+    bool odd = false;
+    double near = 0.0;
+    if (mine) {
+        for (int s = 0; s < S; ++s) nx += xsq[(size_t)s * T + t];
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (lane + 64 * v < E) nw = fmaxf(nw, wsq[lane + 64 * v]);
+        sum_logits<V>(partial, t, T, E, S, lg);
+        nw = wave_max(nw);
+        // what two logits may be apart and still change places.  Everything is computed anew where the norms have left the
+        // range in which the argument for the bound holds (2^-80: below, flushed products could matter) and where a logit
+        // is not finite.
+        near = 2.0 * SCREEN_ERR * sqrt((double)nx) * sqrt((double)nw);
+        odd = !(near < (double)INFINITY) || (nx > 0.f && nx < 8.2718061e-25f) || (nw > 0.f && nw < 8.2718061e-25f);
+#pragma unroll
+        for (int v = 0; v < V; ++v) odd |= lane + 64 * v < E && !(__builtin_fabs(lg[v]) < (double)INFINITY);
+        odd = __any(odd);
+    }
+    __syncthreads();
+    int my_e = 0;
+    double my_l = 0.0, l_max = 0.0;
+    bool again = false;
+    for (int pass = 0; pass < 2; ++pass) {
+        uint32_t taken = 0;
+        // the winners and the best of the others, which lane K holds
+        if (pass == 0 ? mine : again) taken = select_top<V>(lg, K + 1, E, my_e, my_l, l_max);
+        if (pass == 1) break;
+        uint32_t flag = 0;                               // bit v: expert lane + 64 v is computed anew
+        if (odd) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) flag |= (lane + 64 * v < E ? 1u : 0u) << v;
+        } else if (mine && near > 0.0) {
+            const double below = __shfl_down(my_l, 1, 64);
+            if (__any(lane < K && my_l - below <= near)) {
+                for (int k = 0; k <= K; ++k) {
+                    const double wl = __shfl(my_l, k, 64);
+                    const int we = __builtin_amdgcn_readlane(my_e, k);
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        const int e = lane + 64 * v;
+                        // (against the runner-up only winners are compared, and it against them)
+                        const bool counts = e < E && e != we && (k < K || ((taken >> v) & 1u));
+                        if (counts && __builtin_fabs(lg[v] - wl) <= near) flag |= 1u << v;
+                    }
+                }
+            }
+        }
+        int at[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const uint64_t m = __ballot((flag >> v) & 1u);
+            at[v] = 0;
+            if (m) {
+                again = true;
+                int base = 0;
+                if (lane == 0) base = atomicAdd(&n_list, __popcll(m));
+                at[v] = __builtin_amdgcn_readfirstlane(base) + mask_rank(m);
+                if ((flag >> v) & 1u) list[at[v]] = (uint32_t)(wave << 16 | (lane + 64 * v));
+            }
+        }
+        __syncthreads();
+        const int n = n_list;
+        if (n == 0) break;
+        for (int i = wave; i < n; i += SCREENED_WAVES) {
+            const uint32_t job = __builtin_amdgcn_readfirstlane(list[i]);
+            const int tj = blockIdx.x * SCREENED_WAVES + (int)(job >> 16);
+            const uint16_t *xr = x + (size_t)tj * H, *wr = wg + (size_t)(job & 0xffffu) * H;
+            double rstd = 1.0;
+            if (NORMED) {
+                const int nchunk = (H + 1023) / 1024;
+                double tot = 0.0;
+                for (int c = 0; c < nchunk; ++c) tot += norm_ss[(size_t)tj * nchunk + c];
+                rstd = 1.0 / sqrt(tot / (double)H + eps);
+            }
+            double d = 0.0;
+            for (int h0 = 0; h0 < H; h0 += 2048) {       // four pieces of 512 columns on their way together
+                uint4_t xa[4], wa[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int h = h0 + 512 * u + lane * 8;
+                    xa[u] = wa[u] = uint4_t{0u, 0u, 0u, 0u};
+                    if (h < H) {
+                        xa[u] = *(const uint4_t *)(xr + h);
+                        wa[u] = *(const uint4_t *)(wr + h);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    float a[8], b[8];
+                    Row8<uint16_t>::cvt(xa[u], a);
+                    Row8<uint16_t>::cvt(wa[u], b);
+                    if (NORMED) {
+                        const int h = min(h0 + 512 * u + lane * 8, H - 8);
+                        float g[8];
+                        Row8<uint16_t>::cvt(*(const uint4_t *)(norm_w + h), g);
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const float xn = ActIO<uint16_t>::round((float)((double)a[j] * rstd));
+                            a[j] = ActIO<uint16_t>::round(__fmul_rn(xn, g[j]));
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) d = __builtin_fma((double)a[j], (double)b[j], d);
+                }
+            }
+            d = wave_sum(d);
+            if (__builtin_isnan(d)) d = __builtin_nan("");       // one key for every NaN
+            if (lane == 0) anew[i] = d;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if ((flag >> v) & 1u) lg[v] = anew[at[v]];
+    }
+    if (!mine) return;
+    double den = 0.0;
+    const double num = lane < K ? exp(my_l - l_max) : 0.0;
+    if (renorm) {
+        den = num;
+    } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (lane + 64 * v < E) den += exp(lg[v] - l_max);
+    }
+    den = wave_sum(den);
+    if (lane < K) {
+        const size_t o = (size_t)t * K + lane;
+        idx[o] = my_e;
+        w[o] = (float)(num / den);
+        if (idx64) idx64[o] = (int64_t)my_e;
+    }
+}
+
 // Few tokens (T <= 16, P = T * K <= ROUTER_SMALL_PAIRS): one workgroup, one wavefront per token, and
 // behind a barrier the same workgroup sorts the pairs by expert -- the dispatch of dispatch.hip on a
 // list that fits LDS, without its launch (decode and short verify steps: 4 us of a 107 us layer at
@@ -309,6 +710,26 @@ static RouterPlan router_plan(const odsd_moe_shape *s, bool normed) {
     return p;
 }
 
+// Slices of K for router_screen_kernel, or 0 where the fp64 kernel runs.  As many as give every CU a workgroup (two steps
+// of 128 columns and 8 MB of partial sums are the price at T = 1000).  The line lies where the two meet: the fp64 kernel
+// grows with the products, the screened pair has 13 us of top-k with a dot product behind it at any size.  Both kernels
+// together, K = 8, fp64 / screened, us: E = 128, H = 2048: T = 700 17.4 / 20.9, T = 1000 20.7 / 21.7, T = 2000 33.0 / 24.4,
+// T = 4096 50.4 / 28.0; H = 4096: T = 400 19.9 / 23.1, T = 1000 31.2 / 26.8, T = 4096 88.8 / 36.3; E = 512, H = 4096, T = 1000
+// 91.5 / 41.9.
+#define SCREEN_MIN_PRODUCTS 4.5e8
+#define SCREEN_WGS 256
+static int screen_slices(const odsd_moe_shape *s, const RouterPlan &p) {
+    if (s->act_dtype != ODSD_DT_BF16 || s->E <= 64 || s->K >= s->E || s->K >= 64) return 0;
+    if ((double)s->T * s->E * s->H < SCREEN_MIN_PRODUCTS) return 0;
+    if ((size_t)s->T * s->H * 2 > 0xffffffffull || (size_t)s->E * s->H * 2 > 0xffffffffull) return 0;
+    const long tiles = (long)((s->T + 16 * SCREEN_NT - 1) / (16 * SCREEN_NT)) * ((s->E + SCREEN_EXPERTS - 1) / SCREEN_EXPERTS);
+    int S = 1;
+    while (s->H % (S * 2 * ODSD_GROUP) == 0 && tiles * S * 2 <= SCREEN_WGS) S *= 2;
+    // its logits and norms take no more room than the fp64 kernel's
+    const size_t need = (size_t)S * s->T * ((size_t)s->E * sizeof(double) + sizeof(float)) + (size_t)s->E * sizeof(float);
+    return need <= p.partial_bytes ? S : 0;
+}
+
 static int router_check(const odsd_moe_shape *s) {
     if (!s) return ODSD_ERR_NULL;
     if (s->T < 0 || s->H <= 0 || s->E <= 0 || s->K <= 0) return ODSD_ERR_SHAPE;
@@ -360,6 +781,35 @@ int odsd_launch_router(const odsd_moe_shape *s, const void *x, const void *gate_
     const RouterPlan p = router_plan(s, norm_ss != nullptr);
     if (ws_bytes < p.partial_bytes) return ODSD_ERR_WORKSPACE;
     double *partial = (double *)ws;
+    const int screen_S = logits || logits_only ? 0 : screen_slices(s, p);
+    if (screen_S) {
+        const int S = screen_S, EG = (s->E + SCREEN_EXPERTS - 1) / SCREEN_EXPERTS, TT = (s->T + 16 * SCREEN_NT - 1) / (16 * SCREEN_NT);
+        float *xsq = (float *)(partial + (size_t)S * s->T * s->E), *wsq = xsq + (size_t)S * s->T;
+#define SCREEN_GO(NORMED)                                                                                                   \
+        ODSD_LAUNCH(ODSD_KERNEL_ROUTER_LOGITS, router_screen_kernel<NORMED>, TT * EG * S, 512, st,                          \
+                    (const uint16_t *)x, (const uint16_t *)gate_w, partial, xsq, wsq, (half_t *)x16, s->T, s->H, s->E, S,   \
+                    EG, norm_ss, (const uint16_t *)norm_w, (double)eps)
+#define SCREENED_GO(VV, NORMED)                                                                                             \
+        ODSD_LAUNCH(ODSD_KERNEL_ROUTER_TOPK, (router_topk_screened_kernel<VV, NORMED>),                               \
+                    (s->T + SCREENED_WAVES - 1) / SCREENED_WAVES, 64 * SCREENED_WAVES, st, (const double *)partial, (const float *)xsq, (const float *)wsq, (const uint16_t *)x,   \
+                    (const uint16_t *)gate_w, s->T, s->H, s->E, s->K, S, s->renorm, idx, w, idx64, norm_ss,             \
+                    (const uint16_t *)norm_w, (double)eps)
+#define SCREENED_BOTH(VV) do { if (norm_ss) SCREENED_GO(VV, true); else SCREENED_GO(VV, false); } while (0)
+        if (norm_ss) SCREEN_GO(true); else SCREEN_GO(false);
+        ODSD_CHECK_LAUNCH();
+        if (s->E <= 64) SCREENED_BOTH(1);
+        else if (s->E <= 128) SCREENED_BOTH(2);
+        else if (s->E <= 256) SCREENED_BOTH(4);
+        else SCREENED_BOTH(8);
+#undef SCREENED_BOTH
+#undef SCREENED_GO
+#undef SCREEN_GO
+        ODSD_CHECK_LAUNCH();
+        if (disp)
+            return odsd_launch_dispatch(s, idx, disp->counts, disp->offsets, disp->perm, disp->inv, disp->slot_token, st,
+                                        disp->counts_mirror, disp->mirror_tag);
+        return ODSD_OK;
+    }
     const bool bf = s->act_dtype == ODSD_DT_BF16;
 #define ROUTER_GO(NEV)                                                                   \
     do {                                                                                 \

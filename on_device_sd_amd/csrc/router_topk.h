@@ -65,19 +65,10 @@ __device__ __forceinline__ int wave_best(const uint64_t key, const int id) {
 }
 
 // V = logits per lane (experts lane, lane + 64, ...): 1, 2, 4 or 8 for E <= 64, 128, 256, 512
-// the selection for token t by one wavefront; lane k < K returns the k-th winner's expert id
-// (idx null: nothing but that)
+// Token t's logits into the lanes: partial sums in slice order; the loads of one slice batch are independent of each other.
 template <int V>
-__device__ __forceinline__ int topk_token(const double *__restrict__ partial, const int t, int T, int E,
-                                          int K, int S, int renorm, int32_t *__restrict__ idx,
-                                          float *__restrict__ w, int64_t *__restrict__ idx64,
-                                          double *__restrict__ logits) {
+__device__ __forceinline__ void sum_logits(const double *__restrict__ partial, const int t, int T, int E, int S, double (&lg)[V]) {
     const int lane = lane_id();
-
-    double lg[V];
-    uint64_t key[V];
-    uint32_t taken = 0;   // bit v set: expert lane + 64 v already selected
-    // partial sums in slice order; the loads of one slice batch are independent of each other
 #pragma unroll
     for (int v = 0; v < V; ++v) lg[v] = 0.0;
     constexpr int SB = V <= 2 ? 8 : 4;   // slices loaded together
@@ -95,17 +86,24 @@ __device__ __forceinline__ int topk_token(const double *__restrict__ partial, co
 #pragma unroll
             for (int v = 0; v < V; ++v) lg[v] += part[u][v];
     }
+}
+
+// The n largest logits in descending order, ties to the lower expert: lane k < n keeps the k-th winner and its logit.
+// Returns the bits of this lane's experts that were taken (those past E among them).
+template <int V>
+__device__ __forceinline__ uint32_t select_top(const double (&lg)[V], const int n, const int E, int &my_e, double &my_l, double &l_max) {
+    const int lane = lane_id();
+    uint64_t key[V];
+    uint32_t taken = 0;   // bit v set: expert lane + 64 v already selected
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         key[v] = order_key(lg[v]);
         if (lane + 64 * v >= E) taken |= 1u << v;
-        else if (logits) logits[(size_t)t * E + lane + 64 * v] = lg[v];
     }
-
-    int my_e = 0;          // lane k keeps the k-th winner
-    double my_l = 0.0;
-    double l_max = 0.0;
-    for (int k = 0; k < K; ++k) {
+    my_e = 0;
+    my_l = 0.0;
+    l_max = 0.0;
+    for (int k = 0; k < n; ++k) {
         // best remaining candidate of this lane: largest key, then lowest expert.  A lane with
         // nothing left offers key 0 (no finite logit maps to it) and the largest expert id.
         uint64_t bk = 0;
@@ -132,6 +130,28 @@ __device__ __forceinline__ int topk_token(const double *__restrict__ partial, co
         if (lane == k) { my_e = we; my_l = wl; }
         if (k == 0) l_max = wl;
     }
+    return taken;
+}
+
+// the selection for token t by one wavefront; lane k < K returns the k-th winner's expert id
+// (idx null: nothing but that)
+template <int V>
+__device__ __forceinline__ int topk_token(const double *__restrict__ partial, const int t, int T, int E,
+                                          int K, int S, int renorm, int32_t *__restrict__ idx,
+                                          float *__restrict__ w, int64_t *__restrict__ idx64,
+                                          double *__restrict__ logits) {
+    const int lane = lane_id();
+
+    double lg[V];
+    sum_logits<V>(partial, t, T, E, S, lg);
+    if (logits) {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (lane + 64 * v < E) logits[(size_t)t * E + lane + 64 * v] = lg[v];
+    }
+    int my_e;              // lane k keeps the k-th winner
+    double my_l, l_max;
+    select_top<V>(lg, K, E, my_e, my_l, l_max);
 
     if (!idx) return my_e;
     // weights in fp32; differences are taken in fp64 before the cast

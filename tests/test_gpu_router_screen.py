@@ -1,0 +1,98 @@
+"""The router's path for many bf16 tokens: logits on the bf16 matrix cores with an error bound, the choice that hangs on more
+anew in fp64.  Indices are those of the exact logits, whatever the tokens look like; the weights are no further from
+64 bits than with fp64 logits (rounding to fp32: 2^-25 on average, the blocks' sums some 2^-25 of a logit)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,H,E,K,renorm", [
+    (1000, 4096, 128, 8, True),
+    (2017, 2048, 128, 8, False),     # ragged token tile
+    (27500, 128, 128, 4, True),      # one step
+    (5300, 384, 224, 3, False),      # an odd number of steps, experts that do not fill a workgroup
+    (1300, 5248, 66, 63, True),      # most winners, one expert more than they
+    (1100, 1024, 512, 1, False),     # eight logits per lane
+])
+def test_indices_and_weights(dev, T, H, E, K, renorm):
+    from on_device_sd_amd import ops
+    print("router screen", T, H, E, K, renorm, flush=True)
+    g = torch.Generator().manual_seed(T + E)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    wg = (torch.randn(E, H, generator=g) * 0.02).to(torch.bfloat16)
+    # exact ties and ties up to the last bit of one weight, among the popular experts as well
+    wg[E // 2] = wg[1]
+    wg[E - 1] = wg[3]
+    wg[E - 1, 5] = wg[3, 5] * (1 + 2.0 ** -7)
+    wg[2] = wg[4]
+    wg[2, H - 1] = wg[4, H - 1] * (1 + 2.0 ** -7)
+    x[0] = 0.0                                            # every logit is zero
+    x[1] = x[1] * 1e-30                                   # squares vanish, the row has not
+    x[2] = x[2] * 2.0 ** 124                              # sums beyond fp32
+    x[3, 7] = 3000.0                                      # an outlier
+    x[4, 1:] = 0.0                                        # one product per logit
+    x[5] = x[6]
+    x[T - 1] = x[T - 1] * 1e-20
+    idx, w, idx64, x16 = ops.router_topk(x.to(dev), wg.to(dev), K, renorm, want_f16=True, want_int64=True)
+    lo = orc.router_logits(x, wg)
+    idx_o, w_o = orc.route(lo, K, renorm)
+    assert np.array_equal(idx.cpu().numpy(), idx_o)
+    assert np.array_equal(idx64.cpu().numpy(), idx_o.astype(np.int64))
+    # the oracle's weights are fp32 from fp64 logits: half a unit each, one for exp, and the logits' own error
+    rows = np.r_[0:2, 3:T]
+    np.testing.assert_allclose(w.cpu().numpy()[rows], w_o[rows], rtol=2e-6, atol=1e-7)
+    sel = lo.double().numpy()[np.arange(T)[:, None], idx_o]
+    p = np.exp(sel - sel[:, :1])
+    p /= p.sum(1, keepdims=True) if renorm else np.exp(lo.double().numpy() - sel[:, :1]).sum(1, keepdims=True)
+    err = np.linalg.norm(w.cpu().numpy()[rows] - p[rows]) / np.linalg.norm(p[rows])
+    print("weights against 64 bits %.2e" % err, flush=True)
+    assert err < 6e-8
+    assert torch.equal(x16.cpu(), torch.clamp(x.float(), -65504.0, 65504.0).to(torch.float16))
+    again = ops.router_topk(x.to(dev), wg.to(dev), K, renorm)
+    assert torch.equal(again[0], idx) and torch.equal(again[1].view(torch.int32), w.view(torch.int32))
+
+
+def test_tokens_that_are_not_finite_leave_the_others_alone(dev):
+    from on_device_sd_amd import ops
+    T, H, E, K = 1100, 4096, 128, 8
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    wg = (torch.randn(E, H, generator=g) * 0.02).to(torch.bfloat16)
+    x[7, 9] = float("nan")
+    x[8, 11] = float("inf")
+    idx, w, _, _ = ops.router_topk(x.to(dev), wg.to(dev), K, True)
+    good = np.r_[0:7, 9:T]
+    idx_o, w_o = orc.route(orc.router_logits(x[good], wg), K, True)
+    assert np.array_equal(idx.cpu().numpy()[good], idx_o)
+    np.testing.assert_allclose(w.cpu().numpy()[good], w_o, rtol=2e-6, atol=1e-7)
+    assert idx.min() >= 0 and idx.max() < E
+    assert idx[7].tolist() == list(range(K))              # every logit is a NaN: a tie
+    pos = (wg[:, 11].float() > 0).nonzero().flatten()[:K].tolist()
+    assert idx[8].tolist() == pos                         # and here every logit is one of the infinities
+
+
+def test_norm_folded_in_gives_the_same_bits(dev):
+    """The RMSNorm applied on the fly from row statistics against the stand-alone one in front of the router."""
+    import on_device_sd_amd as odsd
+    from on_device_sd_amd import ops
+    T, H, E, K, I = 1025, 4096, 128, 8, 128
+    g = torch.Generator().manual_seed(12)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+    gate = (0.02 * torch.randn(E, H, generator=g)).to(torch.bfloat16).to(dev)
+    gate[9] = gate[4]
+    norm = (1 + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16).to(dev)
+    bank = odsd.W4ExpertBank(E, H, I, dev)
+    for e in range(E):
+        bank.load_expert(e, *(0.02 * torch.randn(*s, generator=g) for s in ((I, H), (I, H), (H, I))))
+    plan = ops.MoeForwardPlan(T, H, E, K, I, True, torch.bfloat16, dev)
+    ss = ops.row_stats(T, H, dev)
+    h1, a, b = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x)
+    plan.run(x, gate, bank.table(), norm, 1e-6, add_residual=True, out_act=h1, row_sumsq_out=ss)
+    ra = plan.run(h1, gate, bank.table(), norm, 1e-6, add_residual=True, out_act=a)
+    idx_a, w_a = ra.idx.clone(), ra.w.clone()
+    rb = plan.run(h1, gate, bank.table(), norm, 1e-6, add_residual=True, out_act=b, row_sumsq_in=ss)
+    assert torch.equal(idx_a, rb.idx) and torch.equal(w_a.view(torch.int32), rb.w.view(torch.int32)) and torch.equal(a, b)
