@@ -711,23 +711,26 @@ static RouterPlan router_plan(const odsd_moe_shape *s, bool normed) {
 }
 
 // Slices of K for router_screen_kernel, or 0 where the fp64 kernel runs.  As many as give every CU a workgroup (two steps
-// of 128 columns and 8 MB of partial sums are the price at T = 1000).  The line lies where the two meet: the fp64 kernel
-// grows with the products, the screened pair has 13 us of top-k with a dot product behind it at any size.  Both kernels
-// together, K = 8, fp64 / screened, us: E = 128, H = 2048: T = 700 17.4 / 20.9, T = 1000 20.7 / 21.7, T = 2000 33.0 / 24.4,
-// T = 4096 50.4 / 28.0; H = 4096: T = 400 19.9 / 23.1, T = 1000 31.2 / 26.8, T = 4096 88.8 / 36.3; E = 512, H = 4096, T = 1000
-// 91.5 / 41.9.
-#define SCREEN_MIN_PRODUCTS 4.5e8
+// of 128 columns and 8 MB of partial sums are the price at T = 1000).  The line lies where the two meet inside a layer: the fp64
+// kernel grows with the products, the screened pair has a top-k of 13 us with a dot product behind it at any size.  Both
+// kernels together, back to back, K = 8, fp64 / screened, us: E = 128, H = 2048: T = 700 17.4 / 21.9, T = 1000 20.7 / 24.2,
+// T = 2000 33.0 / 24.4, T = 4096 50.4 / 28.0; H = 4096: T = 1000 31.2 / 26.8, T = 4096 88.8 / 36.3; E = 512, H = 4096,
+// T = 1000 91.5 / 41.9.  Layers: H = 2048, I = 768: T = 850 146.1 / 147.7, T = 1000 156.2 / 158.3, T = 1300 188.8 / 183.8,
+// T = 1600 207.2 / 197.3; H = 4096, I = 1536: T = 400 287 / 288, T = 600 351.8 / 350.0, T = 800 399.3 / 395.8.
+#define SCREEN_MIN_PRODUCTS 3e8
 #define SCREEN_WGS 256
-static int screen_slices(const odsd_moe_shape *s, const RouterPlan &p) {
+static int screen_slices(const odsd_moe_shape *s) {
     if (s->act_dtype != ODSD_DT_BF16 || s->E <= 64 || s->K >= s->E || s->K >= 64) return 0;
     if ((double)s->T * s->E * s->H < SCREEN_MIN_PRODUCTS) return 0;
     if ((size_t)s->T * s->H * 2 > 0xffffffffull || (size_t)s->E * s->H * 2 > 0xffffffffull) return 0;
     const long tiles = (long)((s->T + 16 * SCREEN_NT - 1) / (16 * SCREEN_NT)) * ((s->E + SCREEN_EXPERTS - 1) / SCREEN_EXPERTS);
     int S = 1;
     while (s->H % (S * 2 * ODSD_GROUP) == 0 && tiles * S * 2 <= SCREEN_WGS) S *= 2;
-    // its logits and norms take no more room than the fp64 kernel's
+    // its logits and norms take no more room than the fp64 kernel's, with the RMSNorm folded in and without: the choice depends on
+    // the shape alone
+    const size_t a = router_plan(s, false).partial_bytes, b = router_plan(s, true).partial_bytes;
     const size_t need = (size_t)S * s->T * ((size_t)s->E * sizeof(double) + sizeof(float)) + (size_t)s->E * sizeof(float);
-    return need <= p.partial_bytes ? S : 0;
+    return need <= (a < b ? a : b) ? S : 0;
 }
 
 static int router_check(const odsd_moe_shape *s) {
@@ -781,7 +784,7 @@ int odsd_launch_router(const odsd_moe_shape *s, const void *x, const void *gate_
     const RouterPlan p = router_plan(s, norm_ss != nullptr);
     if (ws_bytes < p.partial_bytes) return ODSD_ERR_WORKSPACE;
     double *partial = (double *)ws;
-    const int screen_S = logits || logits_only ? 0 : screen_slices(s, p);
+    const int screen_S = logits || logits_only ? 0 : screen_slices(s);
     if (screen_S) {
         const int S = screen_S, EG = (s->E + SCREEN_EXPERTS - 1) / SCREEN_EXPERTS, TT = (s->T + 16 * SCREEN_NT - 1) / (16 * SCREEN_NT);
         float *xsq = (float *)(partial + (size_t)S * s->T * s->E), *wsq = xsq + (size_t)S * s->T;
@@ -797,8 +800,7 @@ int odsd_launch_router(const odsd_moe_shape *s, const void *x, const void *gate_
 #define SCREENED_BOTH(VV) do { if (norm_ss) SCREENED_GO(VV, true); else SCREENED_GO(VV, false); } while (0)
         if (norm_ss) SCREEN_GO(true); else SCREEN_GO(false);
         ODSD_CHECK_LAUNCH();
-        if (s->E <= 64) SCREENED_BOTH(1);
-        else if (s->E <= 128) SCREENED_BOTH(2);
+        if (s->E <= 128) SCREENED_BOTH(2);      // E > 64 here
         else if (s->E <= 256) SCREENED_BOTH(4);
         else SCREENED_BOTH(8);
 #undef SCREENED_BOTH
