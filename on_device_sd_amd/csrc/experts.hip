@@ -641,6 +641,10 @@ __global__ __launch_bounds__(1024) void combine_norm_kernel(const float *__restr
     }
 }
 
+// combine for many tokens (combine.hip)
+void odsd_launch_combine_wide(const odsd_moe_shape *s, const half_t *y, const int32_t *idx, const float *w, const int32_t *perm,
+                              const uint64_t *table, const void *residual, float *out_f32, void *out_act, hipStream_t st);
+#define COMBINE_WIDE_MIN 8000000     // elements of y from which on the wide combine runs
 #define STREAM_DISPATCH_CHUNKS 32   // most gate_up workgroups per expert that each scan the ids (stream_dispatch_supported)
 #define STREAM_DISPATCH_PAIRS 1024  // most ids: 4 per thread
 
@@ -1034,6 +1038,15 @@ static int launch_combine(const odsd_moe_shape *s, const void *y_, const int32_t
         if (!odsd_combine_norm_supported(s)) return ODSD_ERR_UNSUPPORTED;
         if (!out_act || out_f32 || row_ss || !nn->norm_w || !nn->xn || !nn->x16) return ODSD_ERR_NULL;
         if (!odsd_aligned16(nn->x16) || !odsd_aligned16(nn->xn)) return ODSD_ERR_ALIGN;
+    }
+    // Layer, us, combine_kernel / combine_wide_kernel, E = 128, K = 8: H = 2048: T = 300 86.8 / 86.9, T = 500 111.9 / 112.1, T = 900
+    // 148.7 / 147.9, T = 2000 228.2 / 226.1; H = 4096: T = 100 218.3 / 218.9, T = 256 251.0 / 250.6, T = 400 284.9 / 282.7,
+    // T = 4096 1367 / 1357.  Below the line the kernel's own 2 us are launch and first loads either way.
+    if (!nn && !row_ss && pl.y_f16 && pl.KS == 1 && (int64_t)P * s->H >= COMBINE_WIDE_MIN && (!out_act || odsd_aligned16(out_act)) &&
+        (!residual || odsd_aligned16(residual))) {
+        odsd_launch_combine_wide(s, (const half_t *)y_, idx, w, perm, table, residual, out_f32, out_act, st);
+        ODSD_CHECK_LAUNCH();
+        return ODSD_OK;
     }
 #define COMBINE_KB(XT, YH, ST, KB)                                                                      \
     ODSD_LAUNCH(ODSD_KERNEL_COMBINE, (combine_kernel<XT, YH, ST, KB>), grid, 256, st, y, idx, w, perm, table, \
