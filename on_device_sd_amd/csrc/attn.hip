@@ -57,6 +57,7 @@
 #define ATTN_TILE_COARSE 256
 #define ATTN_TILE_WHOLE 256
 #define ATTN_MANY (4 * ATTN_WG)
+#define ATTN_XCD_GROUP 8     // row groups of a (sequence, KV head) that go to one XCD together, at most
 
 // ---- how the work is dealt out -----------------------------------------------------------------------
 // A sequence is KVH * rg units, each of `steps` list steps of g keys (a sequence without keys still owns
@@ -110,16 +111,37 @@ struct ListPlan {
     int g;                   // keys per list step
     int total, share;        // steps in all, steps per workgroup
     SeqAt at;
+    int me;                  // the share (unit) that is this workgroup's
     bool found;
 };
+// Workgroups go round the 8 XCDs, each with an L2 of its own, and the row groups of a (sequence, KV head) read the same
+// keys.  Unsplit units: `group` neighbours of the list go to workgroups that are 8 apart, in whole periods of 8 groups
+// (what is left at the end stays as it is), so that the groups still go round.  (32 / 4 heads of 128, 8 queries a row group, us,
+// workgroup = unit or share / so: unsplit, 64 sequences of 1024 keys x 16 queries 40.2 / 35.9, 100 of 900 x 12 55.7 / 45.0; split, 8
+// of 3000 x 16 29.3 / 27.9, x 40 43.9 / 40.8, 30 of 1777 x 9 39.2 / 38.4; one row group each: no difference.)
+__device__ __forceinline__ int unit_of_workgroup(const int wg, const int n, const int group) {
+    if (group <= 1) return wg;
+    const int period = 8 * group, o = wg % period;
+    return wg - o + period > n ? wg : wg - o + (o & 7) * group + (o >> 3);
+}
+// Shares, which cost the same: a contiguous eighth of the `used` ones to each XCD, so that the pieces of a unit and the units of
+// a sequence are neighbours there.  Not below `used`: a workgroup without a share.
+__device__ __forceinline__ int share_of_workgroup(const int wg, const int used) {
+    if (wg >= used) return wg;
+    const int q = used >> 3, r = used & 7, x = wg & 7;
+    return x * q + min(x, r) + (wg >> 3);
+}
 // fine, coarse: the two granularities.  The list is cut at multiples of `fine` keys when every workgroup gets at
 // least `coarse` keys that way; otherwise at multiples of `coarse`, so that short units stay whole.
-// SPLIT, UNSPLIT: the launches that the caller is compiled for (p.whole: its direct way to the unit).
-template <bool BY_SEQ, bool SPLIT, bool UNSPLIT>
+// SPLIT, UNSPLIT: the launches that the caller is compiled for (p.whole: its direct way to the unit).  BY_XCD: `who` is a
+// workgroup, and its share or unit is chosen by the two functions above.
+template <bool BY_SEQ, bool SPLIT, bool UNSPLIT, bool BY_XCD = false>
 __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int rows_per_unit, const int fine,
-                                              const int coarse, const int who) {
+                                              const int coarse, int who) {
     const int lane = lane_id();
     ListPlan pl;
+    if (BY_XCD && !SPLIT) who = unit_of_workgroup(who, p.n_wg, min(p.max_rg, ATTN_XCD_GROUP));
+    pl.me = who;
     if (UNSPLIT && p.whole) {
         // A workgroup per (sequence, KV head, row group that a sequence can have), found without the list: with
         // 512 sequences its scan cost every workgroup two rounds of 8 dependent loads (MANY, below).
@@ -154,6 +176,7 @@ __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int row
     pl.total = total;
     pl.share = max(1, (total + p.n_wg - 1) / p.n_wg);
     pl.found = false;
+    if (BY_XCD && SPLIT) pl.me = who = share_of_workgroup(who, (total + pl.share - 1) / pl.share);
     const int target = BY_SEQ ? 0 : who * pl.share;
     if (!BY_SEQ && target >= total) return pl;
     int before = 0, tok = 0;
@@ -521,9 +544,9 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
     const int c = lane & 15, kq = lane >> 4;
     auto vswz = [](int key) { return HD == 128 ? (key & 7) : ((key >> 1) & 3); };
 
-    const ListPlan pl = list_plan<false, SPLIT, !SPLIT>(p, ROWS, ATTN_TILE_FINE, ATTN_TILE_COARSE, blockIdx.x);
+    const ListPlan pl = list_plan<false, SPLIT, !SPLIT, true>(p, ROWS, ATTN_TILE_FINE, ATTN_TILE_COARSE, blockIdx.x);
     if (!pl.found) return;
-    const int first_pos = blockIdx.x * pl.share, end = min(pl.total, first_pos + pl.share);
+    const int first_pos = pl.me * pl.share, end = min(pl.total, first_pos + pl.share);
     const float sc = p.scale_log2e;
 
     // copies: row RPC * (wave + 4 i) + lane / NP of a tile, stored piece lane % NP (16-byte pieces of a K row and
@@ -622,7 +645,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnParams p) {
                                                      AttnT<T>::pack2(o[db].z * inv, o[db].w * inv)};
             } else {
                 // (a piece that begins where its workgroup's share begins goes to the workgroup's first slot)
-                float *part = p.part + (size_t)(2 * blockIdx.x + (now.pos > first_pos ? 1 : 0)) * (ROWS * XROW) + (16 * wave + c) * XROW;
+                float *part = p.part + (size_t)(2 * pl.me + (now.pos > first_pos ? 1 : 0)) * (ROWS * XROW) + (16 * wave + c) * XROW;
 #pragma unroll
                 for (int db = 0; db < NDB; ++db) *(float4_t *)(part + 16 * db + 4 * kq) = o[db];
                 if (kq == 0) {
