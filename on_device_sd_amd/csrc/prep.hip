@@ -106,16 +106,15 @@ __global__ __launch_bounds__(256) void w4_pack_kernel(const uint8_t *__restrict_
 
 // -----------------------------------------------------------------------------------------
 // Quantise-on-load of one expert: gate, up and down weights -> streaming layout in ONE launch, with no
-// canonical copy in between.  A workgroup takes four consecutive [16 rows x 128 columns] tiles of a row block
-// (or of two, where a block ends among them: every lane knows its own tile's); a wavefront reads four of the
-// 16 rows, 1 KiB of each per load.  16 lanes hold a row's group, 8 columns each, which are the 8 codes of one
-// packed word.  The words change lanes through LDS, and each wavefront stores one tile as 1 KiB.
-//   * Runs of 1 KiB, not a tile's 16 pieces of 64 bytes, per load: moving the bytes without any arithmetic
-//     takes 3.95 us against 5.00 per expert of [768, 2048] in bf16 (12 MB; an empty kernel 2.4).
-//   * Nontemporal stores: nothing is left in L2 to be written back when the launch ends (5.60 -> 5.19).
-//   * The lanes of a quad compute the parameters of one row each and hand them round: three divisions per
-//     lane, as if the lane had one row.
-//   * Half as many rows per wavefront and twice as many wavefronts: 5.19 as well (instruction issue).
+// canonical copy in between.  A wavefront takes one [16 rows x 128 columns] tile; its lane (r = l%16,
+// kq = l/16) reads columns 32j + 8kq .. + 7 of row r (j = 0..3), which are exactly the codes of its
+// four packed words, so the group's minimum and maximum need two exchanges between lanes and the tile
+// leaves as one contiguous 1 KiB store.  Consecutive wavefronts take consecutive groups of a row
+// block.  Bound by one launch with one round trip and the divisions behind it.  16 experts of [768, 2048] in bf16, 12 MB
+// each, weights that no cache holds, the launches queued up: 88.0 us (92.7 with ordinary stores, whose lines the end of a launch
+// writes back; nontemporal loads besides 90.7).  Rows read in runs of 1 KiB, the words turned through LDS: 96 (83 only where
+// the same 12 MB come again and again).  As three quantise and three pack launches with a canonical copy in
+// between, 96 calls in all, 715 us.
 // -----------------------------------------------------------------------------------------
 struct LoadMatrix {
     const void *w;
@@ -123,77 +122,58 @@ struct LoadMatrix {
     uint32_t *sz;
     int f32;                     // 1: fp32 weights, 0: bf16
     int G;                       // groups per row
-    int first;                   // first tile of this matrix in the launch (a multiple of LOAD_TILES)
+    int first;                   // first tile of this matrix in the launch
     int bstride, boffset;        // destination block = b * bstride + boffset
 };
 struct LoadParams {
     LoadMatrix m[3];
+    int n_tiles;
 };
-#define LOAD_TILES 4             // of a workgroup
-template <int CTRL> __device__ __forceinline__ float dpp_f32(const float v) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
-}
-#define DPP_QUAD_XOR1 0xB1
-#define DPP_QUAD_XOR2 0x4E
-#define DPP_QUAD_LANE(i) ((i) * 0x55)
-#define DPP_ROW_ROR(n) (0x120 + (n))
-__global__ __launch_bounds__(64 * LOAD_TILES) void w4_load_expert_kernel(const LoadParams p) {
-    __shared__ __attribute__((aligned(16))) uint32_t words[LOAD_TILES][256];
-    const int tile = blockIdx.x * LOAD_TILES;
+__global__ __launch_bounds__(256) void w4_load_expert_kernel(const LoadParams p) {
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tile >= p.n_tiles) return;
     const int which = __builtin_amdgcn_readfirstlane((tile >= p.m[1].first) + (tile >= p.m[2].first));
     const LoadMatrix m = p.m[which];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = lane_id(), c = lane & 15, ti = lane >> 4;
-    const int t0 = tile - m.first, t = t0 + ti;                 // this lane's tile: row block b, group g
+    const int t = tile - m.first;
     const int b = t / m.G, g = t - b * m.G;
-    const size_t at = ((size_t)(b * 16 + 4 * wave) * m.G + g) * ODSD_GROUP + c * 8, ld = (size_t)m.G * ODSD_GROUP;
-    float w[4][8];                                              // rows 4 wave + i, columns 8 c .. of the group
+    const int lane = lane_id(), r = lane & 15, kq = lane >> 4;
+    const size_t at = ((size_t)(b * 16 + r) * m.G + g) * ODSD_GROUP + kq * 8;
+    float w[4][8];
     if (m.f32) {
         const float *src = (const float *)m.w + at;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4_t lo = *(const float4_t *)(src + i * ld), hi = *(const float4_t *)(src + i * ld + 4);
-            w[i][0] = lo.x; w[i][1] = lo.y; w[i][2] = lo.z; w[i][3] = lo.w;
-            w[i][4] = hi.x; w[i][5] = hi.y; w[i][6] = hi.z; w[i][7] = hi.w;
+        for (int j = 0; j < 4; ++j) {
+            const float4_t lo = *(const float4_t *)(src + 32 * j), hi = *(const float4_t *)(src + 32 * j + 4);
+            w[j][0] = lo.x; w[j][1] = lo.y; w[j][2] = lo.z; w[j][3] = lo.w;
+            w[j][4] = hi.x; w[j][5] = hi.y; w[j][6] = hi.z; w[j][7] = hi.w;
         }
     } else {
         const uint16_t *src = (const uint16_t *)m.w + at;
-        uint4_t v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = *(const uint4_t *)(src + i * ld);
+        for (int j = 0; j < 4; ++j) {
+            const uint4_t v = *(const uint4_t *)(src + 32 * j);
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t u[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                w[i][2 * k] = __uint_as_float(u[k] << 16);
-                w[i][2 * k + 1] = __uint_as_float(u[k] & 0xffff0000u);
+            for (int i = 0; i < 4; ++i) {
+                w[j][2 * i] = __uint_as_float(u[i] << 16);
+                w[j][2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
             }
         }
     }
-    // minimum and maximum: over the lane's columns and its quad for all four rows, then every lane goes on with the
-    // row of its place in the quad (rotations by 4 and 8 keep that place)
-    float mn[4], mx[4];
+    float mn = w[0][0], mx = w[0][0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        mn[i] = mx[i] = w[i][0];
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int k = 1; k < 8; ++k) {
-            mn[i] = fminf(mn[i], w[i][k]);
-            mx[i] = fmaxf(mx[i], w[i][k]);
+        for (int i = 0; i < 8; ++i) {
+            mn = fminf(mn, w[j][i]);
+            mx = fmaxf(mx, w[j][i]);
         }
-        mn[i] = fminf(mn[i], dpp_f32<DPP_QUAD_XOR1>(mn[i]));
-        mx[i] = fmaxf(mx[i], dpp_f32<DPP_QUAD_XOR1>(mx[i]));
-        mn[i] = fminf(mn[i], dpp_f32<DPP_QUAD_XOR2>(mn[i]));
-        mx[i] = fmaxf(mx[i], dpp_f32<DPP_QUAD_XOR2>(mx[i]));
+#pragma unroll
+    for (int d = 16; d <= 32; d <<= 1) {
+        mn = fminf(mn, __shfl_xor(mn, d, ODSD_WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, d, ODSD_WAVE));
     }
-    float lo = (c & 2) ? ((c & 1) ? mn[3] : mn[2]) : ((c & 1) ? mn[1] : mn[0]);
-    float hi = (c & 2) ? ((c & 1) ? mx[3] : mx[2]) : ((c & 1) ? mx[1] : mx[0]);
-    lo = fminf(lo, dpp_f32<DPP_ROW_ROR(4)>(lo));
-    hi = fmaxf(hi, dpp_f32<DPP_ROW_ROR(4)>(hi));
-    lo = fminf(lo, dpp_f32<DPP_ROW_ROR(8)>(lo));
-    hi = fmaxf(hi, dpp_f32<DPP_ROW_ROR(8)>(hi));
-    const QuantParams qp = quant_params(lo, hi);
+    const QuantParams qp = quant_params(mn, mx);
     // w / scale, correctly rounded, in three instructions: q0 = w y with y = 1 / scale correctly rounded is
     // within 1.5 units of the quotient, its residual w - q0 scale is exact, and one correction leaves an
     // error below 2^-23 units before the last rounding.  scale has 11 significant bits (it is an fp16
@@ -201,53 +181,32 @@ __global__ __launch_bounds__(64 * LOAD_TILES) void w4_load_expert_kernel(const L
     // from that point, and no 24-bit w has a quotient exactly there: the last rounding is the right one.
     // (Quotients too small for that argument vanish when the zero point is added.)  Groups with
     // infinities take the division.
-    const bool finite = hi - lo < INFINITY;
+    const bool finite = mx - mn < INFINITY;
     const float y = __fdiv_rn(1.0f, qp.sf);
-    const float ys[4] = {dpp_f32<DPP_QUAD_LANE(0)>(y), dpp_f32<DPP_QUAD_LANE(1)>(y), dpp_f32<DPP_QUAD_LANE(2)>(y),
-                         dpp_f32<DPP_QUAD_LANE(3)>(y)};
-    const float ss[4] = {dpp_f32<DPP_QUAD_LANE(0)>(qp.sf), dpp_f32<DPP_QUAD_LANE(1)>(qp.sf), dpp_f32<DPP_QUAD_LANE(2)>(qp.sf),
-                         dpp_f32<DPP_QUAD_LANE(3)>(qp.sf)};
-    const float zs[4] = {dpp_f32<DPP_QUAD_LANE(0)>(qp.zf), dpp_f32<DPP_QUAD_LANE(1)>(qp.zf), dpp_f32<DPP_QUAD_LANE(2)>(qp.zf),
-                         dpp_f32<DPP_QUAD_LANE(3)>(qp.zf)};
-    constexpr int pos[8] = {0, 16, 4, 20, 8, 24, 12, 28};      // permute_nibbles: code i -> bit position
-    // 1.5 * 2^23 + code: the sum's last bits are the code, rounded to even as rintf does; what the upper bits of
-    // eight such words leave in a packed word is a constant
-    constexpr float MAGIC = 12582912.0f;
-    constexpr uint32_t MBITS = 0x4B400000u, MSUM = (MBITS << 0) + (MBITS << 16) + (MBITS << 4) + (MBITS << 20) + (MBITS << 8) +
-                                                   (MBITS << 24) + (MBITS << 12) + (MBITS << 28);
     uint32_t out[4];
+    constexpr int pos[8] = {0, 16, 4, 20, 8, 24, 12, 28};      // permute_nibbles: code i -> bit position
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] = 0;
     if (__all(finite)) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t o = 0u - MSUM;
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const float q0 = __fmul_rn(w[i][k], ys[i]);
-                const float q = fmaf(fmaf(-q0, ss[i], w[i][k]), ys[i], q0);
-                const float code = __builtin_amdgcn_fmed3f(__fadd_rn(q, zs[i]), 0.0f, 15.0f);
-                o += __float_as_uint(__fadd_rn(code, MAGIC)) << pos[k];
+            for (int i = 0; i < 8; ++i) {
+                const float q0 = __fmul_rn(w[j][i], y);
+                const float q = fmaf(fmaf(-q0, qp.sf, w[j][i]), y, q0);
+                const float t = rintf(__fadd_rn(q, qp.zf));
+                out[j] |= (uint32_t)__builtin_amdgcn_fmed3f(t, 0.0f, 15.0f) << pos[i];
             }
-            out[i] = o;
-        }
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const QuantParams row{qp.s16, qp.z16, ss[i], zs[i]};
-            out[i] = 0;
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) out[i] |= quant_code(w[i][k], row) << pos[k];
-        }
+            for (int i = 0; i < 8; ++i) out[j] |= quant_code(w[j][i], qp) << pos[i];
     }
-    if (c < 4)
-        m.sz[((size_t)(b * m.bstride + m.boffset) * m.G + g) * 16 + 4 * wave + c] =
-            (uint32_t)__builtin_bit_cast(uint16_t, qp.s16) | ((uint32_t)__builtin_bit_cast(uint16_t, qp.z16) << 16);
-    // columns 8 c ..: word c / 4 of lane (c % 4) * 16 + row of the tile
-#pragma unroll
-    for (int i = 0; i < 4; ++i) words[ti][((c & 3) * 16 + 4 * wave + i) * 4 + (c >> 2)] = out[i];
-    __syncthreads();
-    const int t2 = t0 + wave, b2 = t2 / m.G, g2 = t2 - b2 * m.G;
-    __builtin_nontemporal_store(*(const uint4_t *)&words[wave][lane * 4],
-                                &m.qp[((size_t)(b2 * m.bstride + m.boffset) * m.G + g2) * 64 + lane]);
+    const size_t dst = (size_t)(b * m.bstride + m.boffset) * m.G + g;
+    __builtin_nontemporal_store(uint4_t{out[0], out[1], out[2], out[3]}, &m.qp[dst * 64 + lane]);
+    if (kq == 0)
+        m.sz[dst * 16 + r] = (uint32_t)__builtin_bit_cast(uint16_t, qp.s16) | ((uint32_t)__builtin_bit_cast(uint16_t, qp.z16) << 16);
 }
 
 // -----------------------------------------------------------------------------------------
@@ -446,9 +405,9 @@ extern "C" int odsd_w4_load_expert(const void *gate, int32_t gate_dtype, const v
     const int Gu = (int)(H / ODSD_GROUP), Gd = (int)(I / ODSD_GROUP);
     const LoadParams p{{{gate, (uint4_t *)gu_q, (uint32_t *)gu_sz, gate_dtype == ODSD_DT_F32, Gu, 0, 2, 0},
                         {up, (uint4_t *)gu_q, (uint32_t *)gu_sz, up_dtype == ODSD_DT_F32, Gu, (int)tiles, 2, 1},
-                        {down, (uint4_t *)dn_q, (uint32_t *)dn_sz, down_dtype == ODSD_DT_F32, Gd, (int)(2 * tiles), 1, 0}}};
-    // H and I are multiples of 128, so a matrix has a multiple of 8 tiles and a workgroup's tiles are of one matrix
-    w4_load_expert_kernel<<<dim3((unsigned)((2 * tiles + tiles_dn) / LOAD_TILES)), 64 * LOAD_TILES, 0, (hipStream_t)stream>>>(p);
+                        {down, (uint4_t *)dn_q, (uint32_t *)dn_sz, down_dtype == ODSD_DT_F32, Gd, (int)(2 * tiles), 1, 0}},
+                       (int)(2 * tiles + tiles_dn)};
+    w4_load_expert_kernel<<<dim3((unsigned)((p.n_tiles + 3) / 4)), 256, 0, (hipStream_t)stream>>>(p);
     ODSD_CHECK_LAUNCH();
     return ODSD_OK;
 }
