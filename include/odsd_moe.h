@@ -136,7 +136,7 @@ int odsd_add_rmsnorm(const void *x, const void *residual, const void *weight, in
 
 /* ---- Router ------------------------------------------------------------------------- */
 size_t odsd_router_workspace_bytes(const odsd_moe_shape *s);
-/* x [T,H], gate_w [E,H] in act_dtype.  Logits are accumulated in fp64.
+/* x [T,H], gate_w [E,H] in act_dtype.  The choice is that of logits accumulated in fp64.
  * out_idx  int32 [T,K] experts in descending logit order, ties to the lower index
  * out_w    float [T,K]
  * out_idx64 (optional) the same indices as int64, the dtype torch.topk returns
@@ -326,7 +326,7 @@ size_t odsd_varlen_attention_workspace_bytes(int32_t n_seqs, int32_t max_seqlen_
  * the other slots are not touched.  Results are those of odsd_moe_forward. */
 enum {
     ODSD_KERNEL_NORM = 0,           /* stand-alone RMSNorm                          */
-    ODSD_KERNEL_ROUTER_LOGITS = 1,  /* fp64 logit partials (+ fp16 copy of x)       */
+    ODSD_KERNEL_ROUTER_LOGITS = 1,  /* logit partials (+ fp16 copy of x)            */
     ODSD_KERNEL_ROUTER_TOPK = 2,
     ODSD_KERNEL_DISPATCH = 3,
     ODSD_KERNEL_GATE_UP = 4,

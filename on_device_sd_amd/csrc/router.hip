@@ -1,6 +1,7 @@
 // Router: logits = x . Wg^T accumulated in fp64, then softmax / top-k per token.
 //
-// Two kernels.
+// Two kernels (for many bf16 tokens another pair with the same choices: router_screen_kernel and
+// router_topk_screened_kernel, below).
 //  1. router_partial_kernel: a split-K [T,H]x[H,E] product on the fp64 matrix cores
 //     (v_mfma_f64_16x16x4_f64).  One wavefront owns a tile of 16 tokens x (16*NE) experts
 //     over one K slice and writes fp64 partial logits.  fp64 accumulation makes the logits
