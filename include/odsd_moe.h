@@ -136,7 +136,7 @@ int odsd_add_rmsnorm(const void *x, const void *residual, const void *weight, in
 
 /* ---- Router ------------------------------------------------------------------------- */
 size_t odsd_router_workspace_bytes(const odsd_moe_shape *s);
-/* x [T,H], gate_w [E,H] in act_dtype.  The choice is that of logits accumulated in fp64.
+/* x [T,H], gate_w [E,H] in act_dtype.  Choice and weights are those of logits accumulated in fp64.
  * out_idx  int32 [T,K] experts in descending logit order, ties to the lower index
  * out_w    float [T,K]
  * out_idx64 (optional) the same indices as int64, the dtype torch.topk returns

@@ -1,6 +1,6 @@
 // Router: logits = x . Wg^T accumulated in fp64, then softmax / top-k per token.
 //
-// Two kernels (for many bf16 tokens another pair with the same choices: router_screen_kernel and
+// Two kernels (for many bf16 tokens another pair with the same choices and weights: router_screen_kernel and
 // router_topk_screened_kernel, below).
 //  1. router_partial_kernel: a split-K [T,H]x[H,E] product on the fp64 matrix cores
 //     (v_mfma_f64_16x16x4_f64).  One wavefront owns a tile of 16 tokens x (16*NE) experts
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const double *__restri
 }
 
 // -----------------------------------------------------------------------------------------
-// Many tokens, bf16: the logits on the bf16 matrix cores, and in fp64 only where the choice hangs on more.
+// Many tokens, bf16: the logits on the bf16 matrix cores, and in fp64 only the winners' and those that the choice hangs on.
 //
 // v_mfma_f32_16x16x32_bf16 multiplies exactly and runs 30 times as fast as the fp64 product.  Two products of 32
 // columns, each from zero, are added in fp32, and everything above them in fp64, so a logit is off by at most
@@ -239,8 +239,8 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const double *__restri
 // Cauchy-Schwarz; the norms' own rounding and flushed subnormals are in the remaining 6 %).  The top-k kernel takes
 // neighbours in the order that are further apart than twice this bound as they are, and computes the others anew in
 // fp64: the indices are those of the exact logits.  On N(0, 1) tokens that is one token in thirty, two or three dot products
-// each.  The weights come from these logits through fp64 exponentials and are rounded to fp32 once: 4e-8 off
-// (2-norm; 5.3e-8 with fp64 logits and fp32 exponentials).
+// each.  The winners' logits are computed anew in any case, for the weights; those of a softmax over all experts
+// (renorm = 0) hang on all logits, and such calls take the fp64 kernels.
 //
 // A workgroup of 8 wavefronts owns 32 tokens x 128 experts over one K slice, 128 columns a step; a wavefront 64 of the
 // experts and a quarter of the columns; the quarters meet in LDS.  Rows arrive by asynchronous copies two steps ahead,
@@ -477,27 +477,33 @@ __global__ __launch_bounds__(512, 2) void router_screen_kernel(const uint16_t *_
 }
 
 // One wavefront per token, as router_topk_kernel, on the logits of router_screen_kernel.  K < E and K < 64.
-// The logits to be computed anew go on a list of the workgroup, and its four wavefronts share them: a token that needs
-// any needs two or three, and with each of them on a wavefront of its own the kernel ends one dot product later, not three.
+// The weights come from the winners' logits, so these are computed anew in fp64 with those that the order hangs on: the weights are
+// those of the fp64 kernels, whatever the tokens look like.  (From the screened logits they would be off by what 64 columns'
+// fp32 sum is: with a column of 300 that all experts share 1.2e-5 in the 2-norm where this has 5.1e-8.)  What is to be computed
+// goes on a list of the token, and the wavefronts of the workgroup share all its tokens' lists, SCREENED_ROWS experts of one token
+// at a time.  That reads T K rows of gate_w from L2: T = 4096, H = 4096, E = 128, K = 8, both kernels 60 us, 43 of it
+// without the winners (2 experts at a time 63, 8 61, 4 with 1024 columns on their way 61, with 2048 68).
 #define SCREENED_WAVES 4
+#define SCREENED_ROWS 4
 template <int V, bool NORMED>
 __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kernel(
     const double *__restrict__ partial, const float *__restrict__ xsq, const float *__restrict__ wsq,
-    const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg, int T, int H, int E, int K, int S, int renorm,
+    const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg, int T, int H, int E, int K, int S,
     int32_t *__restrict__ idx, float *__restrict__ w, int64_t *__restrict__ idx64, const double *__restrict__ norm_ss,
     const uint16_t *__restrict__ norm_w, double eps) {
-    __shared__ double anew[SCREENED_WAVES * 64 * V];
-    __shared__ uint32_t list[SCREENED_WAVES * 64 * V];
-    __shared__ int n_list;
+    __shared__ double anew[SCREENED_WAVES][64 * V];
+    __shared__ uint16_t list[SCREENED_WAVES][64 * V];
+    __shared__ int n_list[SCREENED_WAVES];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
     const int t = blockIdx.x * SCREENED_WAVES + wave;
     const bool mine = t < T;
-    if (threadIdx.x == 0) n_list = 0;
     double lg[V];
-    float nx = 0.f, nw = 0.f;
-    bool odd = false;
-    double near = 0.0;
+    int my_e = 0, n_mine = 0, at[V];
+    double my_l = 0.0, l_max = 0.0;
+    uint32_t flag = 0;                                   // bit v: expert lane + 64 v is computed anew
+    bool again = false;                                  // the order may change by it
     if (mine) {
+        float nx = 0.f, nw = 0.f;
         for (int s = 0; s < S; ++s) nx += xsq[(size_t)s * T + t];
 #pragma unroll
         for (int v = 0; v < V; ++v)
@@ -507,28 +513,20 @@ __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kern
         // what two logits may be apart and still change places.  Everything is computed anew where the norms have left the
         // range in which the argument for the bound holds (2^-80: below, flushed products could matter) and where a logit
         // is not finite.
-        near = 2.0 * SCREEN_ERR * sqrt((double)nx) * sqrt((double)nw);
-        odd = !(near < (double)INFINITY) || (nx > 0.f && nx < 8.2718061e-25f) || (nw > 0.f && nw < 8.2718061e-25f);
+        const double near = 2.0 * SCREEN_ERR * sqrt((double)nx) * sqrt((double)nw);
+        bool odd = !(near < (double)INFINITY) || (nx > 0.f && nx < 8.2718061e-25f) || (nw > 0.f && nw < 8.2718061e-25f);
 #pragma unroll
         for (int v = 0; v < V; ++v) odd |= lane + 64 * v < E && !(__builtin_fabs(lg[v]) < (double)INFINITY);
-        odd = __any(odd);
-    }
-    __syncthreads();
-    int my_e = 0;
-    double my_l = 0.0, l_max = 0.0;
-    bool again = false;
-    for (int pass = 0; pass < 2; ++pass) {
-        uint32_t taken = 0;
         // the winners and the best of the others, which lane K holds
-        if (pass == 0 ? mine : again) taken = select_top<V>(lg, K + 1, E, my_e, my_l, l_max);
-        if (pass == 1) break;
-        uint32_t flag = 0;                               // bit v: expert lane + 64 v is computed anew
-        if (odd) {
+        const uint32_t taken = select_top<V>(lg, K + 1, E, my_e, my_l, l_max);
+        if (__any(odd)) {
+            again = true;
 #pragma unroll
             for (int v = 0; v < V; ++v) flag |= (lane + 64 * v < E ? 1u : 0u) << v;
-        } else if (mine && near > 0.0) {
+        } else if (near > 0.0) {                         // (otherwise every logit is zero)
             const double below = __shfl_down(my_l, 1, 64);
-            if (__any(lane < K && my_l - below <= near)) {
+            again = __any(lane < K && my_l - below <= near);
+            if (again) {
                 for (int k = 0; k <= K; ++k) {
                     const double wl = __shfl(my_l, k, 64);
                     const int we = __builtin_amdgcn_readlane(my_e, k);
@@ -541,91 +539,91 @@ __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kern
                     }
                 }
             }
+            // the weights come from the winners' logits
+            const int other = __builtin_amdgcn_readlane(my_e, K);
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                if (lane + 64 * v < E && lane + 64 * v != other) flag |= taken & (1u << v);
         }
-        int at[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             const uint64_t m = __ballot((flag >> v) & 1u);
-            at[v] = 0;
-            if (m) {
-                again = true;
-                int base = 0;
-                if (lane == 0) base = atomicAdd(&n_list, __popcll(m));
-                at[v] = __builtin_amdgcn_readfirstlane(base) + mask_rank(m);
-                if ((flag >> v) & 1u) list[at[v]] = (uint32_t)(wave << 16 | (lane + 64 * v));
-            }
+            at[v] = n_mine + mask_rank(m);
+            n_mine += __popcll(m);
+            if ((flag >> v) & 1u) list[wave][at[v]] = (uint16_t)(lane + 64 * v);
         }
-        __syncthreads();
-        const int n = n_list;
-        if (n == 0) break;
-        for (int i = wave; i < n; i += SCREENED_WAVES) {
-            const uint32_t job = __builtin_amdgcn_readfirstlane(list[i]);
-            const int tj = blockIdx.x * SCREENED_WAVES + (int)(job >> 16);
-            const uint16_t *xr = x + (size_t)tj * H, *wr = wg + (size_t)(job & 0xffffu) * H;
-            double rstd = 1.0;
+    }
+    if (lane == 0) n_list[wave] = n_mine;
+    __syncthreads();
+    int n_of[SCREENED_WAVES];
+#pragma unroll
+    for (int i = 0; i < SCREENED_WAVES; ++i) n_of[i] = __builtin_amdgcn_readfirstlane(n_list[i]);
+    for (int unit = wave;; unit += SCREENED_WAVES) {     // (at most as many as the lists have experts)
+        int who = 0, first = unit;
+        while (who < SCREENED_WAVES && first >= (n_of[who] + SCREENED_ROWS - 1) / SCREENED_ROWS)
+            first -= (n_of[who++] + SCREENED_ROWS - 1) / SCREENED_ROWS;
+        if (who == SCREENED_WAVES) break;
+        first *= SCREENED_ROWS;
+        const int tj = blockIdx.x * SCREENED_WAVES + who, n = min(SCREENED_ROWS, n_of[who] - first);
+        const uint16_t *xr = x + (size_t)tj * H, *wr[SCREENED_ROWS];
+#pragma unroll
+        for (int j = 0; j < SCREENED_ROWS; ++j)          // (past the end: the last one again)
+            wr[j] = wg + (size_t)__builtin_amdgcn_readfirstlane(list[who][first + min(j, n - 1)]) * H;
+        double rstd = 1.0;
+        if (NORMED) {
+            const int nchunk = (H + 1023) / 1024;
+            double tot = 0.0;
+            for (int c = 0; c < nchunk; ++c) tot += norm_ss[(size_t)tj * nchunk + c];
+            rstd = 1.0 / sqrt(tot / (double)H + eps);
+        }
+        double d[SCREENED_ROWS] = {};
+        for (int h = lane * 8; h < H; h += 512) {
+            uint4_t wa[SCREENED_ROWS];
+            const uint4_t xa = *(const uint4_t *)(xr + h);
+#pragma unroll
+            for (int j = 0; j < SCREENED_ROWS; ++j) wa[j] = *(const uint4_t *)(wr[j] + h);
+            float a[8];
+            Row8<uint16_t>::cvt(xa, a);
             if (NORMED) {
-                const int nchunk = (H + 1023) / 1024;
-                double tot = 0.0;
-                for (int c = 0; c < nchunk; ++c) tot += norm_ss[(size_t)tj * nchunk + c];
-                rstd = 1.0 / sqrt(tot / (double)H + eps);
-            }
-            double d = 0.0;
-            for (int h0 = 0; h0 < H; h0 += 2048) {       // four pieces of 512 columns on their way together
-                uint4_t xa[4], wa[4];
+                float g[8];
+                Row8<uint16_t>::cvt(*(const uint4_t *)(norm_w + h), g);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int h = h0 + 512 * u + lane * 8;
-                    xa[u] = wa[u] = uint4_t{0u, 0u, 0u, 0u};
-                    if (h < H) {
-                        xa[u] = *(const uint4_t *)(xr + h);
-                        wa[u] = *(const uint4_t *)(wr + h);
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    float a[8], b[8];
-                    Row8<uint16_t>::cvt(xa[u], a);
-                    Row8<uint16_t>::cvt(wa[u], b);
-                    if (NORMED) {
-                        const int h = min(h0 + 512 * u + lane * 8, H - 8);
-                        float g[8];
-                        Row8<uint16_t>::cvt(*(const uint4_t *)(norm_w + h), g);
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) {
-                            const float xn = ActIO<uint16_t>::round((float)((double)a[j] * rstd));
-                            a[j] = ActIO<uint16_t>::round(__fmul_rn(xn, g[j]));
-                        }
-                    }
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) d = __builtin_fma((double)a[j], (double)b[j], d);
+                for (int i = 0; i < 8; ++i) {
+                    const float xn = ActIO<uint16_t>::round((float)((double)a[i] * rstd));
+                    a[i] = ActIO<uint16_t>::round(__fmul_rn(xn, g[i]));
                 }
             }
-            d = wave_sum(d);
-            if (__builtin_isnan(d)) d = __builtin_nan("");       // one key for every NaN
-            if (lane == 0) anew[i] = d;
+#pragma unroll
+            for (int j = 0; j < SCREENED_ROWS; ++j) {
+                float b[8];
+                Row8<uint16_t>::cvt(wa[j], b);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[j] = __builtin_fma((double)a[i], (double)b[i], d[j]);
+            }
         }
-        __syncthreads();
 #pragma unroll
-        for (int v = 0; v < V; ++v)
-            if ((flag >> v) & 1u) lg[v] = anew[at[v]];
+        for (int j = 0; j < SCREENED_ROWS; ++j) {
+            double l = wave_sum(d[j]);
+            if (__builtin_isnan(l)) l = __builtin_nan("");       // one key for every NaN
+            if (lane == 0 && j < n) anew[who][first + j] = l;
+        }
     }
+    __syncthreads();
     if (!mine) return;
-    double den = 0.0;
-    const double num = lane < K ? exp(my_l - l_max) : 0.0;
-    if (renorm) {
-        den = num;
-    } else {
 #pragma unroll
-        for (int v = 0; v < V; ++v)
-            if (lane + 64 * v < E) den += exp(lg[v] - l_max);
+    for (int v = 0; v < V; ++v)
+        if ((flag >> v) & 1u) lg[v] = anew[wave][at[v]];
+    if (again) {
+        select_top<V>(lg, K, E, my_e, my_l, l_max);
+    } else {                                             // the same winners, with their logits as they are now
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const double l = __shfl(lg[v], my_e & 63, 64);
+            if (my_e >> 6 == v) my_l = l;
+        }
+        l_max = __shfl(my_l, 0, 64);
     }
-    den = wave_sum(den);
-    if (lane < K) {
-        const size_t o = (size_t)t * K + lane;
-        idx[o] = my_e;
-        w[o] = (float)(num / den);
-        if (idx64) idx64[o] = (int64_t)my_e;
-    }
+    topk_weights<V>(lg, my_e, my_l, l_max, t, E, K, 1, idx, w, idx64);
 }
 
 // Few tokens (T <= 16, P = T * K <= ROUTER_SMALL_PAIRS): one workgroup, one wavefront per token, and
@@ -721,7 +719,7 @@ static RouterPlan router_plan(const odsd_moe_shape *s, bool normed) {
 #define SCREEN_MIN_PRODUCTS 3e8
 #define SCREEN_WGS 256
 static int screen_slices(const odsd_moe_shape *s) {
-    if (s->act_dtype != ODSD_DT_BF16 || s->E <= 64 || s->K >= s->E || s->K >= 64) return 0;
+    if (s->act_dtype != ODSD_DT_BF16 || !s->renorm || s->E <= 64 || s->K >= s->E || s->K >= 64) return 0;
     if ((double)s->T * s->E * s->H < SCREEN_MIN_PRODUCTS) return 0;
     if ((size_t)s->T * s->H * 2 > 0xffffffffull || (size_t)s->E * s->H * 2 > 0xffffffffull) return 0;
     const long tiles = (long)((s->T + 16 * SCREEN_NT - 1) / (16 * SCREEN_NT)) * ((s->E + SCREEN_EXPERTS - 1) / SCREEN_EXPERTS);
@@ -796,7 +794,7 @@ int odsd_launch_router(const odsd_moe_shape *s, const void *x, const void *gate_
 #define SCREENED_GO(VV, NORMED)                                                                                             \
         ODSD_LAUNCH(ODSD_KERNEL_ROUTER_TOPK, (router_topk_screened_kernel<VV, NORMED>),                               \
                     (s->T + SCREENED_WAVES - 1) / SCREENED_WAVES, 64 * SCREENED_WAVES, st, (const double *)partial, (const float *)xsq, (const float *)wsq, (const uint16_t *)x,   \
-                    (const uint16_t *)gate_w, s->T, s->H, s->E, s->K, S, s->renorm, idx, w, idx64, norm_ss,             \
+                    (const uint16_t *)gate_w, s->T, s->H, s->E, s->K, S, idx, w, idx64, norm_ss,             \
                     (const uint16_t *)norm_w, (double)eps)
 #define SCREENED_BOTH(VV) do { if (norm_ss) SCREENED_GO(VV, true); else SCREENED_GO(VV, false); } while (0)
         if (norm_ss) SCREEN_GO(true); else SCREEN_GO(false);

@@ -133,6 +133,32 @@ __device__ __forceinline__ uint32_t select_top(const double (&lg)[V], const int 
     return taken;
 }
 
+// What lane k < K holds of the k-th winner, and its weight: in fp32, differences are taken in fp64 before the cast.
+template <int V>
+__device__ __forceinline__ void topk_weights(const double (&lg)[V], const int my_e, const double my_l, const double l_max,
+                                             const int t, int E, int K, int renorm, int32_t *__restrict__ idx,
+                                             float *__restrict__ w, int64_t *__restrict__ idx64) {
+    const int lane = lane_id();
+    float num = 0.0f;
+    if (lane < K) num = expf((float)(my_l - l_max));
+    float den;
+    if (renorm) {
+        den = wave_sum(num);
+    } else {
+        float part = 0.0f;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (lane + 64 * v < E) part += expf((float)(lg[v] - l_max));
+        den = wave_sum(part);
+    }
+    if (lane < K) {
+        const size_t o = (size_t)t * K + lane;
+        idx[o] = my_e;
+        w[o] = num / den;
+        if (idx64) idx64[o] = (int64_t)my_e;
+    }
+}
+
 // the selection for token t by one wavefront; lane k < K returns the k-th winner's expert id
 // (idx null: nothing but that)
 template <int V>
@@ -154,24 +180,6 @@ __device__ __forceinline__ int topk_token(const double *__restrict__ partial, co
     select_top<V>(lg, K, E, my_e, my_l, l_max);
 
     if (!idx) return my_e;
-    // weights in fp32; differences are taken in fp64 before the cast
-    float num = 0.0f;
-    if (lane < K) num = expf((float)(my_l - l_max));
-    float den;
-    if (renorm) {
-        den = wave_sum(num);
-    } else {
-        float part = 0.0f;
-#pragma unroll
-        for (int v = 0; v < V; ++v)
-            if (lane + 64 * v < E) part += expf((float)(lg[v] - l_max));
-        den = wave_sum(part);
-    }
-    if (lane < K) {
-        const size_t o = (size_t)t * K + lane;
-        idx[o] = my_e;
-        w[o] = num / den;
-        if (idx64) idx64[o] = (int64_t)my_e;
-    }
+    topk_weights<V>(lg, my_e, my_l, l_max, t, E, K, renorm, idx, w, idx64);
     return my_e;
 }

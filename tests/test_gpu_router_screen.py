@@ -1,6 +1,5 @@
-"""The router's path for many bf16 tokens: logits on the bf16 matrix cores with an error bound, the choice that hangs on more
-anew in fp64.  Indices are those of the exact logits, whatever the tokens look like; the weights are no further from
-64 bits than with fp64 logits (rounding to fp32: 2^-25 on average, the blocks' sums some 2^-25 of a logit)."""
+"""The router's path for many bf16 tokens: logits on the bf16 matrix cores with an error bound; the winners, and what the choice
+hangs on, anew in fp64.  Indices are those of the exact logits and weights those of fp64 logits, whatever the tokens look like."""
 import numpy as np
 import pytest
 import torch
@@ -54,6 +53,59 @@ def test_indices_and_weights(dev, T, H, E, K, renorm):
     assert torch.equal(x16.cpu(), torch.clamp(x.float(), -65504.0, 65504.0).to(torch.float16))
     again = ops.router_topk(x.to(dev), wg.to(dev), K, renorm)
     assert torch.equal(again[0], idx) and torch.equal(again[1].view(torch.int32), w.view(torch.int32))
+
+
+# What the tokens and the router have in common in a trained model, and what makes a sum of 32 columns in fp32 lose the rest.
+def _rows(kind, T, H, E):
+    g = torch.Generator().manual_seed(T + H + E + len(kind))
+    x, wg = torch.randn(T, H, generator=g), torch.randn(E, H, generator=g) * 0.02
+    if kind == "residual_stream":
+        x *= 8
+    elif kind == "large_columns":
+        x[:, [12, 99]] *= 1000.0
+    elif kind == "common_component":
+        x += 1.0
+        wg += 0.02 * torch.randn(H, generator=g).abs()
+    elif kind == "shared_column":                         # that all experts weight alike
+        x[:, 33] = 300.0 * (1 + 0.1 * torch.randn(T, generator=g))
+        wg[:, 33] = 0.5
+    elif kind == "cancelling":
+        # Two columns of every 32 cancel exactly and take the last bits of the others, which make the choice, with them; so
+        # large that half of the neighbours are closer than what the screen leaves open, 35 * 2^-22 |x||w|, and half a few times that apart.
+        for c in range(0, H, 32):
+            x[:, c + 3], x[:, c + 20] = 10300 / H ** 0.5, -10300 / H ** 0.5
+            wg[:, c + 3] = wg[:, c + 20] = 0.125
+    return x.to(torch.bfloat16), wg.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("kind", ["residual_stream", "large_columns", "common_component", "shared_column", "cancelling"])
+@pytest.mark.parametrize("T,H,E,K", [(1700, 4096, 128, 8), (5300, 384, 224, 3), (2100, 1024, 512, 8)])
+def test_weights_are_those_of_fp64_logits(dev, T, H, E, K, kind):
+    from on_device_sd_amd import ops
+    print("router screen, weights", T, H, E, K, kind, flush=True)
+    x, wg = _rows(kind, T, H, E)
+    x, wg = x.to(dev), wg.to(dev)
+    idx, w, _, _ = ops.router_topk(x, wg, K, True)
+    lo = x.double() @ wg.double().t()
+    val, pos = lo.topk(K, dim=1)
+    sel = lo.gather(1, idx.long())
+    # (two fp64 sums of H products may order neighbours differently only within their own rounding)
+    slack = H * 2.0 ** -53 * (x.double().abs() @ wg.double().abs().t()).amax(1, keepdim=True)
+    assert ((sel - val).abs() <= slack).all()
+    # Each weight against 64 bits.  num: the difference rounded to fp32 and exp's own unit; den: the same of its terms, weighted, and
+    # K - 1 additions; the division.  In units of 2^-24 of the weight.
+    d = sel - sel[:, :1]
+    p = d.exp()
+    p = p / p.sum(1, keepdim=True)
+    units = d.abs() + 2 + (p * (d.abs() + 2)).sum(1, keepdim=True) + (K - 1) + 1
+    err = (w.double() - p).abs()
+    print("worst weight %.2e of itself" % (err / p).max().item(), flush=True)
+    assert (err <= p * (units * 2.0 ** -24) + 2.0 ** -149).all()
+    # the call that returns the logits has them in fp64: a weight differs only where their last bits turn a rounding
+    lg = torch.empty(T, E, dtype=torch.float64, device=dev)
+    idx2, w2, _, _ = ops.router_topk(x, wg, K, True, logits_out=lg)
+    assert torch.equal(idx, idx2)
+    assert (w.view(torch.int32) != w2.view(torch.int32)).sum().item() <= 1e-4 * T * K
 
 
 def test_tokens_that_are_not_finite_leave_the_others_alone(dev):
