@@ -136,6 +136,10 @@ int odsd_add_rmsnorm(const void *x, const void *residual, const void *weight, in
 
 /* ---- Router ------------------------------------------------------------------------- */
 size_t odsd_router_workspace_bytes(const odsd_moe_shape *s);
+/* 1 where odsd_router_topk and the calls built on it take the logits of this shape from the bf16 matrix cores and compute in fp64
+ * what choice and weights hang on, 0 where they compute all in fp64.  The same results either way.  normed: with the RMSNorm folded
+ * into the router (row_sumsq_in of odsd_moe_forward). */
+int odsd_router_screened(const odsd_moe_shape *s, int32_t normed);
 /* x [T,H], gate_w [E,H] in act_dtype.  Choice and weights are those of logits accumulated in fp64.
  * out_idx  int32 [T,K] experts in descending logit order, ties to the lower index
  * out_w    float [T,K]

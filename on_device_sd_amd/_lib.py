@@ -42,6 +42,7 @@ SIGNATURES = {
     "odsd_rmsnorm": (C.c_int, [_P, _P, C.c_int32, C.c_int32, C.c_int32, C.c_float, _P, _P]),
     "odsd_add_rmsnorm": (C.c_int, [_P, _P, _P, C.c_int32, C.c_int32, C.c_int32, C.c_float, _P, _P, _P]),
     "odsd_router_workspace_bytes": (C.c_size_t, [_SP]),
+    "odsd_router_screened": (C.c_int, [_SP, C.c_int32]),
     "odsd_router_topk": (C.c_int, [_SP, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
     "odsd_router_topk_logits": (C.c_int, [_SP, _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
     "odsd_route_dispatch": (C.c_int, [_SP, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),

@@ -323,7 +323,7 @@ __global__ __launch_bounds__(512, 2) void router_screen_kernel(const uint16_t *_
     const uint32_t frag = (uint32_t)((r * 16 + ((4 * q + kg) ^ r)) * 16);
 
     dma(0, 0);
-    if (ng > 1) dma(1, 1);
+    dma(1, 1);                                           // (ng >= 2, screen_slices)
     // the experts' norms, one expert a workgroup while the rows travel
     for (int e = unit; e < E; e += gridDim.x) {
         float sw = 0.f;
@@ -480,17 +480,18 @@ __global__ __launch_bounds__(512, 2) void router_screen_kernel(const uint16_t *_
 // The weights come from the winners' logits, so these are computed anew in fp64 with those that the order hangs on: the weights are
 // those of the fp64 kernels, whatever the tokens look like.  (From the screened logits they would be off by what 64 columns'
 // fp32 sum is: with a column of 300 that all experts share 1.2e-5 in the 2-norm where this has 5.1e-8.)  What is to be computed
-// goes on a list of the token, and the wavefronts of the workgroup share all its tokens' lists, SCREENED_ROWS experts of one token
+// goes on a list of the token, and the wavefronts of the workgroup share all its tokens' lists, four or eight experts of one token
 // at a time.  That reads T K rows of gate_w from L2: T = 4096, H = 4096, E = 128, K = 8, both kernels 60 us, 43 of it
 // without the winners (2 experts at a time 63, 8 61, 4 with 1024 columns on their way 61, with 2048 68).
 #define SCREENED_WAVES 4
-#define SCREENED_ROWS 4
+#define SCREENED_MAX_K 16
 template <int V, bool NORMED>
 __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kernel(
     const double *__restrict__ partial, const float *__restrict__ xsq, const float *__restrict__ wsq,
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg, int T, int H, int E, int K, int S,
     int32_t *__restrict__ idx, float *__restrict__ w, int64_t *__restrict__ idx64, const double *__restrict__ norm_ss,
     const uint16_t *__restrict__ norm_w, double eps) {
+    constexpr int ROWS = NORMED ? 8 : 4;                 // (a group repeats the normalisation of its token)
     __shared__ double anew[SCREENED_WAVES][64 * V];
     __shared__ uint16_t list[SCREENED_WAVES][64 * V];
     __shared__ int n_list[SCREENED_WAVES];
@@ -560,14 +561,14 @@ __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kern
     for (int i = 0; i < SCREENED_WAVES; ++i) n_of[i] = __builtin_amdgcn_readfirstlane(n_list[i]);
     for (int unit = wave;; unit += SCREENED_WAVES) {     // (at most as many as the lists have experts)
         int who = 0, first = unit;
-        while (who < SCREENED_WAVES && first >= (n_of[who] + SCREENED_ROWS - 1) / SCREENED_ROWS)
-            first -= (n_of[who++] + SCREENED_ROWS - 1) / SCREENED_ROWS;
+        while (who < SCREENED_WAVES && first >= (n_of[who] + ROWS - 1) / ROWS)
+            first -= (n_of[who++] + ROWS - 1) / ROWS;
         if (who == SCREENED_WAVES) break;
-        first *= SCREENED_ROWS;
-        const int tj = blockIdx.x * SCREENED_WAVES + who, n = min(SCREENED_ROWS, n_of[who] - first);
-        const uint16_t *xr = x + (size_t)tj * H, *wr[SCREENED_ROWS];
+        first *= ROWS;
+        const int tj = blockIdx.x * SCREENED_WAVES + who, n = min(ROWS, n_of[who] - first);
+        const uint16_t *xr = x + (size_t)tj * H, *wr[ROWS];
 #pragma unroll
-        for (int j = 0; j < SCREENED_ROWS; ++j)          // (past the end: the last one again)
+        for (int j = 0; j < ROWS; ++j)          // (past the end: the last one again)
             wr[j] = wg + (size_t)__builtin_amdgcn_readfirstlane(list[who][first + min(j, n - 1)]) * H;
         double rstd = 1.0;
         if (NORMED) {
@@ -576,12 +577,12 @@ __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kern
             for (int c = 0; c < nchunk; ++c) tot += norm_ss[(size_t)tj * nchunk + c];
             rstd = 1.0 / sqrt(tot / (double)H + eps);
         }
-        double d[SCREENED_ROWS] = {};
+        double d[ROWS] = {};
         for (int h = lane * 8; h < H; h += 512) {
-            uint4_t wa[SCREENED_ROWS];
+            uint4_t wa[ROWS];
             const uint4_t xa = *(const uint4_t *)(xr + h);
 #pragma unroll
-            for (int j = 0; j < SCREENED_ROWS; ++j) wa[j] = *(const uint4_t *)(wr[j] + h);
+            for (int j = 0; j < ROWS; ++j) wa[j] = *(const uint4_t *)(wr[j] + h);
             float a[8];
             Row8<uint16_t>::cvt(xa, a);
             if (NORMED) {
@@ -594,7 +595,7 @@ __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kern
                 }
             }
 #pragma unroll
-            for (int j = 0; j < SCREENED_ROWS; ++j) {
+            for (int j = 0; j < ROWS; ++j) {
                 float b[8];
                 Row8<uint16_t>::cvt(wa[j], b);
 #pragma unroll
@@ -602,7 +603,7 @@ __global__ __launch_bounds__(64 * SCREENED_WAVES) void router_topk_screened_kern
             }
         }
 #pragma unroll
-        for (int j = 0; j < SCREENED_ROWS; ++j) {
+        for (int j = 0; j < ROWS; ++j) {
             double l = wave_sum(d[j]);
             if (__builtin_isnan(l)) l = __builtin_nan("");       // one key for every NaN
             if (lane == 0 && j < n) anew[who][first + j] = l;
@@ -709,24 +710,33 @@ static RouterPlan router_plan(const odsd_moe_shape *s, bool normed) {
     return p;
 }
 
-// Slices of K for router_screen_kernel, or 0 where the fp64 kernel runs.  As many as give every CU a workgroup (two steps
-// of 128 columns and 8 MB of partial sums are the price at T = 1000).  The line lies where the two meet inside a layer: the fp64
-// kernel grows with the products, the screened pair has a top-k of 13 us with a dot product behind it at any size.  Both
-// kernels together, back to back, K = 8, fp64 / screened, us: E = 128, H = 2048: T = 700 17.4 / 21.9, T = 1000 20.7 / 24.2,
-// T = 2000 33.0 / 24.4, T = 4096 50.4 / 28.0; H = 4096: T = 1000 31.2 / 26.8, T = 4096 88.8 / 36.3; E = 512, H = 4096,
-// T = 1000 91.5 / 41.9.  Layers: H = 2048, I = 768: T = 850 146.1 / 147.7, T = 1000 156.2 / 158.3, T = 1300 188.8 / 183.8,
-// T = 1600 207.2 / 197.3; H = 4096, I = 1536: T = 400 287 / 288, T = 600 351.8 / 350.0, T = 800 399.3 / 395.8.
-#define SCREEN_MIN_PRODUCTS 3e8
+// Slices of K for router_screen_kernel, or 0 where the fp64 kernels run.  Slices: as many as still give no CU a second workgroup (two
+// steps of 128 columns and 8 MB of partial sums are the price at T = 1000).  The choice: from an estimate of either pair, us, because both
+// go in steps, the fp64 kernel with the units of work per SIMD, the screen with the workgroups per CU and, where H / 128 is odd,
+// with the whole row in one slice.  fp64: 12 + 9.4 for 1000 columns x 16 experts of a SIMD.  Screened: 10, 1 for a step, the winners' rows
+// from L2 (10 for 1e8 columns, 32 for 1e5 columns one after the other, 4 experts at a time), the partial sums, the winners' selection.
+// 3 us between them are left to the fp64 kernels, 17 with the RMSNorm folded in, which the dot products repeat.  Measured, fp64 /
+// screened, K = 8: E = 128: H = 2048: T = 1600 32.5 / 29.4, T = 2000 33.1 / 30.7, T = 2600 41.4 / 34.7, T = 4096 49.8 / 38.8; H = 4096: T = 1000
+// 31.0 / 35.8, T = 1300 41.4 / 39.4, T = 2000 51.3 / 41.0, T = 4096 89.1 / 59.8; H = 3968: T = 600 34.5 / 55.4, T = 2000 50.8 / 55.2, T = 4096
+// 86.5 / 68.1; E = 66, H = 4096, T = 4096 88.7 / 58.6; E = 512, H = 4096, T = 1000 91.7 / 53.7.  K = 16: E = 128, H = 4096: T = 2000 52.9 / 57.9,
+// T = 4096 91.2 / 85.3; E = 512, H = 2048, T = 1000 58.6 / 56.3.  More winners: E = 128, H = 4096, K = 30, T = 4096 96 / 130; K = 24, T = 8991 245 / 227; E = 256,
+// K = 48, T = 7710 341 / 383.  Layers with the RMSNorm folded in, K = 8, I = 128: E = 128, H = 4096: T = 2000 214 / 217, T = 4096 412 / 374; E = 256, H = 4096: T = 600
+// 145 / 158, T = 2000 284 / 256.  Of 200 shapes drawn where this says screened, 4 were slower, all short of 512 tokens (up to 15 %: too few wavefronts
+// behind the winners' rows; hence the bound), the others took 71 % of the time on average.
 #define SCREEN_WGS 256
-static int screen_slices(const odsd_moe_shape *s) {
-    if (s->act_dtype != ODSD_DT_BF16 || !s->renorm || s->E <= 64 || s->K >= s->E || s->K >= 64) return 0;
-    if ((double)s->T * s->E * s->H < SCREEN_MIN_PRODUCTS) return 0;
+static int screen_slices(const odsd_moe_shape *s, bool normed) {
+    if (s->act_dtype != ODSD_DT_BF16 || !s->renorm || s->E <= 64 || s->K >= s->E || s->K > SCREENED_MAX_K || s->T < 512) return 0;
     if ((size_t)s->T * s->H * 2 > 0xffffffffull || (size_t)s->E * s->H * 2 > 0xffffffffull) return 0;
     const long tiles = (long)((s->T + 16 * SCREEN_NT - 1) / (16 * SCREEN_NT)) * ((s->E + SCREEN_EXPERTS - 1) / SCREEN_EXPERTS);
     int S = 1;
     while (s->H % (S * 2 * ODSD_GROUP) == 0 && tiles * S * 2 <= SCREEN_WGS) S *= 2;
-    // its logits and norms take no more room than the fp64 kernel's, with the RMSNorm folded in and without: the choice depends on
-    // the shape alone
+    if (s->H / S < 2 * ODSD_GROUP) return 0;             // the kernel has two groups on their way
+    const RouterPlan p = router_plan(s, false);
+    const double mega = 1e-6 * s->T, steps = (double)((tiles * S + SCREEN_WGS - 1) / SCREEN_WGS) * (s->H / S / ODSD_GROUP);
+    const double fp64 = 12 + 9.4e-3 * (((long)p.TT * p.EG * p.S + 1023) / 1024) * (s->H / p.S) * p.NE;
+    const double screened = 10 + steps + mega * s->K * s->H / 10 + 3.2e-4 * s->H * ((s->K + 3) / 4) + 6.5 * mega * s->E * S + 1.3 * s->K;
+    if (fp64 < screened + (normed ? 17 : 3)) return 0;
+    // its logits and norms take no more room than the fp64 kernel's, with the RMSNorm folded in and without
     const size_t a = router_plan(s, false).partial_bytes, b = router_plan(s, true).partial_bytes;
     const size_t need = (size_t)S * s->T * ((size_t)s->E * sizeof(double) + sizeof(float)) + (size_t)s->E * sizeof(float);
     return need <= (a < b ? a : b) ? S : 0;
@@ -747,6 +757,10 @@ extern "C" size_t odsd_router_workspace_bytes(const odsd_moe_shape *s) {
     // (the split of K, and with it the partial sums, depends on whether the RMSNorm is folded in)
     const size_t a = router_plan(s, false).partial_bytes, b = router_plan(s, true).partial_bytes;
     return a > b ? a : b;
+}
+
+extern "C" int odsd_router_screened(const odsd_moe_shape *s, int32_t normed) {
+    return router_check(s) == ODSD_OK && screen_slices(s, normed != 0) > 0;
 }
 
 template <typename XT, int NE>
@@ -783,7 +797,7 @@ int odsd_launch_router(const odsd_moe_shape *s, const void *x, const void *gate_
     const RouterPlan p = router_plan(s, norm_ss != nullptr);
     if (ws_bytes < p.partial_bytes) return ODSD_ERR_WORKSPACE;
     double *partial = (double *)ws;
-    const int screen_S = logits || logits_only ? 0 : screen_slices(s);
+    const int screen_S = logits || logits_only ? 0 : screen_slices(s, norm_ss != nullptr);
     if (screen_S) {
         const int S = screen_S, EG = (s->E + SCREEN_EXPERTS - 1) / SCREEN_EXPERTS, TT = (s->T + 16 * SCREEN_NT - 1) / (16 * SCREEN_NT);
         float *xsq = (float *)(partial + (size_t)S * s->T * s->E), *wsq = xsq + (size_t)S * s->T;

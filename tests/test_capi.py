@@ -35,6 +35,22 @@ def test_version_and_status_strings():
         assert len(lib.odsd_status_string(code)) > 3
 
 
+def test_router_screens_where_the_fp64_pair_takes_longer():
+    """bf16, renorm, more than 64 experts, from 512 tokens on; not where the screen has too few workgroups (a row of H / 128 odd is one
+    slice), where the winners are many, or where its results would not fit the workspace that the fp64 kernels ask for."""
+    lib = _lib.load()
+    q = lambda T, H, E=128, K=8, renorm=1, dt=_lib.DT_BF16, normed=0: lib.odsd_router_screened(
+        C.byref(_lib.MoeShape(T, H, E, K, 128, renorm, dt, 0)), normed)
+    assert q(4096, 4096) == q(2400, 2048) == q(4096, 2048) == q(2000, 4096) == q(16368, 4096) == q(4096, 4096, 66) == q(1000, 4096, 512) == 1
+    assert q(600, 3968) == q(2000, 3968) == 0 and q(4096, 3968) == 1
+    assert q(4096, 4096, K=17) == q(2000, 4096, K=16) == 0 and q(4096, 4096, K=16) == 1
+    assert q(4096, 4096, normed=1) == 1 and q(2000, 4096, normed=1) == 0
+    assert q(511, 4096, 512) == 0 and q(513, 4096, 512) == 1
+    assert q(1000, 4096) == q(1600, 2048) == q(16369, 4096) == 0
+    assert q(4096, 4096, 64) == q(4096, 4096, renorm=0) == q(4096, 4096, dt=_lib.DT_F32) == q(4096, 4096, 512, 64) == 0
+    assert q(0, 4096) == q(4096, 4000) == q(4096, 4096, 513) == 0
+
+
 def test_one_launch_plan_follows_shape_and_max_rows():
     """The whole-block experts calls take the one-launch kernel at the Qwen3-30B expert shape with
     8 to 20 rows per expert on average, unless the caller says that some expert has more rows than

@@ -9,17 +9,31 @@ from oracle import moe_oracle as orc
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("T,H,E,K,renorm", [
-    (1000, 4096, 128, 8, True),
-    (2017, 2048, 128, 8, False),     # ragged token tile
-    (27500, 128, 128, 4, True),      # one step
-    (5300, 384, 224, 3, False),      # an odd number of steps, experts that do not fill a workgroup
-    (1300, 5248, 66, 63, True),      # most winners, one expert more than they
-    (1100, 1024, 512, 1, False),     # eight logits per lane
+def _screened(T, H, E, K, renorm=True, normed=False):
+    import ctypes as C
+    from on_device_sd_amd import _lib, ops
+    return bool(_lib.load().odsd_router_screened(C.byref(ops.make_shape(T, H, E, K, 128, renorm, torch.bfloat16)), normed))
+
+
+@pytest.mark.parametrize("T,H,E,K,renorm,screened", [
+    (1700, 4096, 128, 8, True, True),
+    (2317, 2048, 128, 8, True, True),      # ragged token tile
+    (4100, 384, 224, 3, True, True),       # an odd number of steps, experts that do not fill a workgroup; four logits per lane
+    (700, 2048, 512, 4, True, True),       # two steps in the first slice and the last
+    (1500, 4096, 512, 16, True, True),     # most winners, eight logits per lane
+    (8200, 4096, 66, 1, True, True),       # one winner and its runner-up
+    # and their neighbours in fp64
+    (1000, 4096, 128, 8, True, False),
+    (2017, 2048, 128, 8, False, False),
+    (27500, 128, 128, 4, True, False),
+    (5300, 384, 224, 3, False, False),
+    (1300, 5248, 66, 63, True, False),
+    (1100, 1024, 512, 1, False, False),
 ])
-def test_indices_and_weights(dev, T, H, E, K, renorm):
+def test_indices_and_weights(dev, T, H, E, K, renorm, screened):
     from on_device_sd_amd import ops
     print("router screen", T, H, E, K, renorm, flush=True)
+    assert _screened(T, H, E, K, renorm) == screened
     g = torch.Generator().manual_seed(T + E)
     x = torch.randn(T, H, generator=g).to(torch.bfloat16)
     wg = (torch.randn(E, H, generator=g) * 0.02).to(torch.bfloat16)
@@ -79,10 +93,11 @@ def _rows(kind, T, H, E):
 
 
 @pytest.mark.parametrize("kind", ["residual_stream", "large_columns", "common_component", "shared_column", "cancelling"])
-@pytest.mark.parametrize("T,H,E,K", [(1700, 4096, 128, 8), (5300, 384, 224, 3), (2100, 1024, 512, 8)])
+@pytest.mark.parametrize("T,H,E,K", [(1700, 4096, 128, 8), (4100, 384, 224, 3), (2100, 1024, 512, 8)])
 def test_weights_are_those_of_fp64_logits(dev, T, H, E, K, kind):
     from on_device_sd_amd import ops
     print("router screen, weights", T, H, E, K, kind, flush=True)
+    assert _screened(T, H, E, K)
     x, wg = _rows(kind, T, H, E)
     x, wg = x.to(dev), wg.to(dev)
     idx, w, _, _ = ops.router_topk(x, wg, K, True)
@@ -110,7 +125,8 @@ def test_weights_are_those_of_fp64_logits(dev, T, H, E, K, kind):
 
 def test_tokens_that_are_not_finite_leave_the_others_alone(dev):
     from on_device_sd_amd import ops
-    T, H, E, K = 1100, 4096, 128, 8
+    T, H, E, K = 1600, 4096, 128, 8
+    assert _screened(T, H, E, K)
     g = torch.Generator().manual_seed(3)
     x = torch.randn(T, H, generator=g).to(torch.bfloat16)
     wg = (torch.randn(E, H, generator=g) * 0.02).to(torch.bfloat16)
@@ -127,11 +143,13 @@ def test_tokens_that_are_not_finite_leave_the_others_alone(dev):
     assert idx[8].tolist() == pos                         # and here every logit is one of the infinities
 
 
-def test_norm_folded_in_gives_the_same_bits(dev):
+# (an odd number of winners: the last group of a token's experts is not full)
+@pytest.mark.parametrize("T,H,E,K,I", [(3601, 4096, 128, 8, 128), (2501, 4096, 512, 11, 128)])
+def test_norm_folded_in_gives_the_same_bits(dev, T, H, E, K, I):
     """The RMSNorm applied on the fly from row statistics against the stand-alone one in front of the router."""
     import on_device_sd_amd as odsd
     from on_device_sd_amd import ops
-    T, H, E, K, I = 1025, 4096, 128, 8, 128
+    assert _screened(T, H, E, K) and _screened(T, H, E, K, normed=True)
     g = torch.Generator().manual_seed(12)
     x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
     gate = (0.02 * torch.randn(E, H, generator=g)).to(torch.bfloat16).to(dev)
