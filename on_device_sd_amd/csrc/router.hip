@@ -343,9 +343,11 @@ __global__ __launch_bounds__(512, 2) void router_screen_kernel(const uint16_t *_
     float4_t pend[NTILE];
     // one group; the sums of two groups go to the fp64 accumulators together
     auto step = [&](const int g, const bool second) {
-        // (loads land in order, and no more than the next group's are left; the stores of the copy only make this stricter)
-        if (g + 1 < ng) ODSD_WAIT_VMCNT(N_DMA);
-        else ODSD_WAIT_VMCNT(0);
+        // This group's rows have landed: loads land in order, and no more than the next group's are left (the stores of the copy only
+        // make this stricter).  And this wavefront has the last step's fragments in registers: behind the barrier their buffer is
+        // written again.
+        if (g + 1 < ng) ODSD_WAIT_VMCNT_LGKM0(N_DMA);
+        else ODSD_WAIT_VMCNT_LGKM0(0);
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (g + 2 < ng) dma(buf == 0 ? 2 : buf - 1, g + 2);      // what the step before this one read
