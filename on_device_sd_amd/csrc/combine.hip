@@ -2,26 +2,26 @@
 // "+=" of demo/src/model/qwen3_runner.py:363, with the residual add of :226).
 #include "common.h"
 
-// Many tokens, complete fp16 sums: 8 columns per thread, so that a row of a pair is a load of 16 bytes per lane, the rows of up to
-// 8 pairs on their way together, read past the caches that a layer's sums would only sweep.  Bound by HBM (T = 4096, H = 4096,
-// K = 8: 60 -> 50 us for 336 MB).  The sums are those of combine_kernel, bit for bit.  In a file of its own: the code of the
-// expert kernels behind it in experts.hip moved and ran up to 5 % slower (w4_gemm_kernel at T = 600, H = 2048: 56.1 -> 58.9 us).
-template <typename XT, int KB>
+// Many tokens, complete fp16 sums, bf16 output: 8 columns per thread, so that a row of a pair is a load of 16 bytes per lane, the
+// rows of up to 8 pairs on their way together, read past the caches that a layer's sums would only sweep.  Bound by HBM
+// (T = 4096, H = 4096, K = 8: 60 -> 50 us for 336 MB).  The sums are those of combine_kernel, bit for bit.  In a file of its own: the code of
+// the expert kernels behind it in experts.hip moved and ran up to 5 % slower (w4_gemm_kernel at T = 600, H = 2048: 56.1 -> 58.9 us).
+template <int KB>
 __global__ __launch_bounds__(256) void combine_wide_kernel(const half_t *__restrict__ y, const int32_t *__restrict__ idx,
                                                            const float *__restrict__ w, const int32_t *__restrict__ perm,
                                                            const uint64_t *__restrict__ table,
-                                                           const XT *__restrict__ residual, float *__restrict__ out_f32,
-                                                           XT *__restrict__ out_act, int H, int K, int E, int nchunk) {
+                                                           const uint16_t *__restrict__ residual,
+                                                           uint16_t *__restrict__ out_act, int H, int K, int E, int nchunk) {
     const int t = blockIdx.x / nchunk, chunk = blockIdx.x - t * nchunk;
     const int c = (chunk * (int)blockDim.x + (int)threadIdx.x) * 8;
     if (c >= H) return;
     const size_t o = (size_t)t * H + c;
     float acc[8] = {}, res[8] = {};
+    typedef uint16_t act8 __attribute__((ext_vector_type(8)));
     if (residual) {
-        typedef XT xt8 __attribute__((ext_vector_type(8)));
-        const xt8 rv = *(const xt8 *)(residual + o);
+        const act8 rv = *(const act8 *)(residual + o);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { const XT e = rv[i]; res[i] = ActIO<XT>::load(&e, 0); }
+        for (int i = 0; i < 8; ++i) { const uint16_t e = rv[i]; res[i] = ActIO<uint16_t>::load(&e, 0); }
     }
     for (int k0 = 0; k0 < K; k0 += KB) {
         int slot[KB];
@@ -46,39 +46,26 @@ __global__ __launch_bounds__(256) void combine_wide_kernel(const half_t *__restr
                 for (int i = 0; i < 8; ++i) acc[i] = fmaf(wk[u], (float)v[u][i], acc[i]);
             }
     }
-    if (out_f32) {
-        *(float4_t *)(out_f32 + o) = float4_t{acc[0] + res[0], acc[1] + res[1], acc[2] + res[2], acc[3] + res[3]};
-        *(float4_t *)(out_f32 + o + 4) = float4_t{acc[4] + res[4], acc[5] + res[5], acc[6] + res[6], acc[7] + res[7]};
-    }
-    if (out_act) {
-        typedef XT xt8 __attribute__((ext_vector_type(8)));
-        xt8 st;
+    act8 st;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float m = ActIO<XT>::round(acc[i]);
-            XT e;
-            ActIO<XT>::store(&e, 0, residual ? __fadd_rn(res[i], m) : m);
-            st[i] = e;
-        }
-        *(xt8 *)(out_act + o) = st;
+    for (int i = 0; i < 8; ++i) {
+        const float m = ActIO<uint16_t>::round(acc[i]);
+        uint16_t e;
+        ActIO<uint16_t>::store(&e, 0, residual ? __fadd_rn(res[i], m) : m);
+        st[i] = e;
     }
+    *(act8 *)(out_act + o) = st;
 }
 
 void odsd_launch_combine_wide(const odsd_moe_shape *s, const half_t *y, const int32_t *idx, const float *w, const int32_t *perm,
-                              const uint64_t *table, const void *residual, float *out_f32, void *out_act, hipStream_t st) {
+                              const uint64_t *table, const void *residual, void *out_act, hipStream_t st) {
     const int threads = s->H >= 2048 ? 256 : (s->H / 8 + 63) / 64 * 64, nchunk = (s->H / 8 + threads - 1) / threads;
-#define COMBINE_WIDE(XT, KB)                                                                                                   \
-    ODSD_LAUNCH(ODSD_KERNEL_COMBINE, (combine_wide_kernel<XT, KB>), dim3((unsigned)(nchunk * s->T)), threads, st, y, idx, w,    \
-                perm, table, (const XT *)residual, out_f32, (XT *)out_act, s->H, s->K, s->E, nchunk)
-#define COMBINE_WIDE_K(XT)                           \
-    do {                                             \
-        if (s->K % 8 == 0) COMBINE_WIDE(XT, 8);      \
-        else if (s->K % 4 == 0) COMBINE_WIDE(XT, 4); \
-        else if (s->K % 2 == 0) COMBINE_WIDE(XT, 2); \
-        else COMBINE_WIDE(XT, 1);                    \
-    } while (0)
-    if (s->act_dtype == ODSD_DT_BF16) COMBINE_WIDE_K(uint16_t);
-    else COMBINE_WIDE_K(float);
-#undef COMBINE_WIDE_K
+#define COMBINE_WIDE(KB)                                                                                                      \
+    ODSD_LAUNCH(ODSD_KERNEL_COMBINE, combine_wide_kernel<KB>, dim3((unsigned)(nchunk * s->T)), threads, st, y, idx, w, perm,   \
+                table, (const uint16_t *)residual, (uint16_t *)out_act, s->H, s->K, s->E, nchunk)
+    if (s->K % 8 == 0) COMBINE_WIDE(8);
+    else if (s->K % 4 == 0) COMBINE_WIDE(4);
+    else if (s->K % 2 == 0) COMBINE_WIDE(2);
+    else COMBINE_WIDE(1);
 #undef COMBINE_WIDE
 }

@@ -643,8 +643,10 @@ __global__ __launch_bounds__(1024) void combine_norm_kernel(const float *__restr
 
 // combine for many tokens (combine.hip)
 void odsd_launch_combine_wide(const odsd_moe_shape *s, const half_t *y, const int32_t *idx, const float *w, const int32_t *perm,
-                              const uint64_t *table, const void *residual, float *out_f32, void *out_act, hipStream_t st);
-#define COMBINE_WIDE_MIN 8000000     // elements of y from which on the wide combine runs
+                              const uint64_t *table, const void *residual, void *out_act, hipStream_t st);
+// elements of y and of the output from which on the wide combine runs
+#define COMBINE_WIDE_MIN_Y 8000000
+#define COMBINE_WIDE_MIN_OUT 2000000
 #define STREAM_DISPATCH_CHUNKS 32   // most gate_up workgroups per expert that each scan the ids (stream_dispatch_supported)
 #define STREAM_DISPATCH_PAIRS 1024  // most ids: 4 per thread
 
@@ -1041,10 +1043,14 @@ static int launch_combine(const odsd_moe_shape *s, const void *y_, const int32_t
     }
     // Layer, us, combine_kernel / combine_wide_kernel, E = 128, K = 8: H = 2048: T = 300 86.8 / 86.9, T = 500 111.9 / 112.1, T = 900
     // 148.7 / 147.9, T = 2000 228.2 / 226.1; H = 4096: T = 100 218.3 / 218.9, T = 256 251.0 / 250.6, T = 400 284.9 / 282.7,
-    // T = 4096 1367 / 1357.  Below the line the kernel's own 2 us are launch and first loads either way.
-    if (!nn && !row_ss && pl.y_f16 && pl.KS == 1 && (int64_t)P * s->H >= COMBINE_WIDE_MIN && (!out_act || odsd_aligned16(out_act)) &&
+    // T = 4096 1367 / 1357.  The kernels alone, y from memory, with a residual: T = 500, H = 2048, K = 8 5.9 / 6.4, T = 400, H = 4096 8.0 / 7.9,
+    // T = 1000, H = 2048 9.0 / 8.6, T = 600, H = 4096 11.0 / 9.7; K = 4: T = 500, H = 4096 6.6 / 6.2; K = 2: T = 1000, H = 4096 8.2 / 7.2; K = 1: T = 2000 12.1 /
+    // 10.3.  So from 1000 workgroups on.  fp32 stores, two of 16 bytes a thread with gaps between the lanes, take that back: fp32 output
+    // besides, K = 2, T = 2000, H = 4096 17.0 / 20.2, K = 8, T = 600 11.7 / 11.9; fp32 activations, K = 2 16.0 / 20.4.
+    if (!nn && !row_ss && !out_f32 && s->act_dtype == ODSD_DT_BF16 && pl.y_f16 && pl.KS == 1 &&
+        (int64_t)P * s->H >= COMBINE_WIDE_MIN_Y && (int64_t)s->T * s->H >= COMBINE_WIDE_MIN_OUT && odsd_aligned16(out_act) &&
         (!residual || odsd_aligned16(residual))) {
-        odsd_launch_combine_wide(s, (const half_t *)y_, idx, w, perm, table, residual, out_f32, out_act, st);
+        odsd_launch_combine_wide(s, (const half_t *)y_, idx, w, perm, table, residual, out_act, st);
         ODSD_CHECK_LAUNCH();
         return ODSD_OK;
     }
