@@ -125,7 +125,9 @@ __device__ __forceinline__ int unit_of_workgroup(const int wg, const int n, cons
     return wg - o + period > n ? wg : wg - o + (o & 7) * group + (o >> 3);
 }
 // Shares, which cost the same: a contiguous eighth of the `used` ones to each XCD, so that the pieces of a unit and the units of
-// a sequence are neighbours there.  Not below `used`: a workgroup without a share.
+// a sequence are neighbours there.  Not below `used`: a workgroup without a share.  Shares of one step stay as they are (9 sequences
+// of 1225 keys x 24 24.3 / 25.0; others no difference).  With more, as above; two of 15 such lose (2 of 1939 x 160, 16 / 2 heads, 26.2 / 27.0,
+// 7 of 1294 x 24, 64 / 4 heads of 64, 22.9 / 23.7).
 __device__ __forceinline__ int share_of_workgroup(const int wg, const int used) {
     if (wg >= used) return wg;
     const int q = used >> 3, r = used & 7, x = wg & 7;
@@ -176,7 +178,7 @@ __device__ __forceinline__ ListPlan list_plan(const AttnParams &p, const int row
     pl.total = total;
     pl.share = max(1, (total + p.n_wg - 1) / p.n_wg);
     pl.found = false;
-    if (BY_XCD && SPLIT) pl.me = who = share_of_workgroup(who, (total + pl.share - 1) / pl.share);
+    if (BY_XCD && SPLIT && pl.share > 1) pl.me = who = share_of_workgroup(who, (total + pl.share - 1) / pl.share);
     const int target = BY_SEQ ? 0 : who * pl.share;
     if (!BY_SEQ && target >= total) return pl;
     int before = 0, tok = 0;
