@@ -56,14 +56,14 @@ def test_indices_and_weights(dev, T, H, E, K, renorm, screened):
     assert np.array_equal(idx.cpu().numpy(), idx_o)
     assert np.array_equal(idx64.cpu().numpy(), idx_o.astype(np.int64))
     # the oracle's weights are fp32 from fp64 logits: half a unit each, one for exp, and the logits' own error
-    rows = np.r_[0:2, 3:T]
-    np.testing.assert_allclose(w.cpu().numpy()[rows], w_o[rows], rtol=2e-6, atol=1e-7)
+    np.testing.assert_allclose(w.cpu().numpy(), w_o, rtol=2e-6, atol=1e-7)
     sel = lo.double().numpy()[np.arange(T)[:, None], idx_o]
     p = np.exp(sel - sel[:, :1])
     p /= p.sum(1, keepdims=True) if renorm else np.exp(lo.double().numpy() - sel[:, :1]).sum(1, keepdims=True)
-    err = np.linalg.norm(w.cpu().numpy()[rows] - p[rows]) / np.linalg.norm(p[rows])
-    print("weights against 64 bits %.2e" % err, flush=True)
-    assert err < 6e-8
+    err = np.linalg.norm(w.cpu().numpy() - p, axis=1) / np.linalg.norm(p, axis=1)
+    print("weights against 64 bits, worst token %.2e" % err.max(), flush=True)
+    # K - 1 additions, exp's unit, the division, and a logit's distance from the largest in fp32 (under 17 where a weight counts)
+    assert np.all(err[np.arange(T) != 2] < (K + 2 + 2 * 17) * 2.0 ** -24) and err[2] < 1e-6
     assert torch.equal(x16.cpu(), torch.clamp(x.float(), -65504.0, 65504.0).to(torch.float16))
     again = ops.router_topk(x.to(dev), wg.to(dev), K, renorm)
     assert torch.equal(again[0], idx) and torch.equal(again[1].view(torch.int32), w.view(torch.int32))
