@@ -22,6 +22,7 @@ def _screened(T, H, E, K, renorm=True, normed=False):
     (700, 2048, 512, 4, True, True),       # two steps in the first slice and the last
     (1500, 4096, 512, 16, True, True),     # most winners, eight logits per lane
     (8200, 4096, 66, 1, True, True),       # one winner and its runner-up
+    (1500, 2048, 300, 6, True, True),      # eight logits per lane, some past the experts
     # and their neighbours in fp64
     (1000, 4096, 128, 8, True, False),
     (2017, 2048, 128, 8, False, False),
@@ -89,10 +90,15 @@ def _rows(kind, T, H, E):
         for c in range(0, H, 32):
             x[:, c + 3], x[:, c + 20] = 10300 / H ** 0.5, -10300 / H ** 0.5
             wg[:, c + 3] = wg[:, c + 20] = 0.125
+    elif kind == "swallowed":
+        # One product of 1 in every 32, the others below half a unit in its last place in fp32 and all that tells the experts apart:
+        # what a sum of 32 loses at most, which the bound has to leave open.
+        x, wg = 2.0 ** -13 * (1 + torch.rand(T, H, generator=g)), 2.0 ** -12 * torch.rand(E, H, generator=g)
+        x[:, ::32] = wg[:, ::32] = 1.0
     return x.to(torch.bfloat16), wg.to(torch.bfloat16)
 
 
-@pytest.mark.parametrize("kind", ["residual_stream", "large_columns", "common_component", "shared_column", "cancelling"])
+@pytest.mark.parametrize("kind", ["residual_stream", "large_columns", "common_component", "shared_column", "cancelling", "swallowed"])
 @pytest.mark.parametrize("T,H,E,K", [(1700, 4096, 128, 8), (4100, 384, 224, 3), (2100, 1024, 512, 8)])
 def test_weights_are_those_of_fp64_logits(dev, T, H, E, K, kind):
     from on_device_sd_amd import ops
